@@ -14,9 +14,9 @@
 #include "internal.h"
 #include "plan.h"
 
-int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s);
+int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s, const JobSet *jobs = nullptr);
 int nttm_run_fused(const PassArgs &a, const PassGeom &g, hipStream_t s);
-int nttm_run_fused2(const PassArgs &a, const PassArgs &bq, const PassGeom &g, hipStream_t s);
+int nttm_run_fused2(const PassArgs &a, const FusedB &fb, const PassGeom &g, hipStream_t s, const FusedSet &js);
 bool nttm_fwd_pass_streams(const PassArgs &a, const PassGeom &g);
 void nttm_set_pts(int pts);
 int nttm_get_pts(void);
@@ -37,6 +37,11 @@ int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which
                         const PrimeK *pk, const double2 *scale, hipStream_t s);
 int nttm_crt_launch_batch(const void *desc_dev, uint64_t nprod, uint64_t nblocks, int np, const CrtConst &cc,
                           uint32_t *scratch, hipStream_t s, double alg_bytes, int per = 8);
+/* the two halves of nttm_crt_launch_batch: the limbs of products whose blocks are [blk0, blk0 + nblk) of the launch's
+ * block numbering, for a carry in of 0; then every block's carry */
+int nttm_crt_launch_limbs(const void *desc_dev, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np, const CrtConst &cc,
+                          uint32_t *scratch, hipStream_t s, double alg_bytes, int per);
+int nttm_crt_launch_carry(const void *desc_dev, uint64_t nprod, uint64_t nblocks, uint32_t *scratch, hipStream_t s, int per);
 uint64_t nttm_crt_blocks(uint64_t nc, int per = 8);      /* per: CRT limbs per thread, 8 (2048-limb blocks) or 1 (256) */
 uint64_t nttm_crt_scratch_words(uint64_t nblocks);
 int nttm_run_norm(const void *desc_dev, uint64_t nprod, uint64_t *ncn_dev, hipStream_t s);
@@ -44,9 +49,7 @@ int nttm_run_fill_x(const void *desc_dev, uint64_t nprod, hipStream_t s);
 int nttm_run_dft16_mfma(const uint64_t *x, double *y, int logn, uint64_t batch, const void *etab, const double *tlo,
                         const double *thi, const double *consts, double p, hipStream_t s);
 int nttm_run_add_carry(uint64_t *c, uint64_t n, const uint64_t *carry, hipStream_t s);
-int nttm_run_r3(bool inv, double *x, uint64_t batch, int logk, const PrimeK &pk, const double2 *b3,
-                const uint64_t *limbs, uint64_t nlimbs, const LoadDesc *ldesc, int which, const double2 *scale,
-                hipStream_t s);
+int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s);
 
 /* ---- errors ----------------------------------------------------------------------------------------------------- */
 /* per host thread: the library's own helper threads (the e pipeline's download preparation) may fail too */
@@ -109,8 +112,6 @@ struct Ctx {
     void *dfree[8]; int ndfree;              /* buffers the planned tree outgrew, freed after its final synchronization */
     void *hfree[4]; int nhfree;
     hipEvent_t tev[8];                       /* the last copies on tcs, in turn */
-    hipStream_t ps[NTTM_MAX_PRIMES - 1];     /* primes 1.. of a small product, beside the caller's stream (prime 0) */
-    hipEvent_t pfev, pjev[NTTM_MAX_PRIMES - 1];   /* their fork from and join to the caller's stream */
     uint64_t *hpin; size_t hpin_bytes;       /* pinned host staging (descriptors, flags) */
     char *stage; size_t stage_bytes;         /* device copies of host-resident operands and results */
     size_t stage_chunk;                      /* staged bytes per sub-batch of a batch */
@@ -130,6 +131,19 @@ static int g_no_defer;                       /* NTTM_NO_DEFER=1: every pass appl
 static int g_tree_levelwise;                 /* NTTM_TREE_LEVELWISE=1: the tree level by level (for comparison) */
 static int g_fused_bits_env;                 /* NTTM_FUSED_BITS=10|11|12: that last-pass width for every product
                                               * transform above it (for comparison measurements) */
+
+/* Products of at most g_par_points points per prime run each pass as ONE launch for all primes and both operands, each
+ * prime with a B plane of its own (2 np planes); longer ones run prime after prime through np + 1 planes.  A launch
+ * costs about 6 us beside its work (the gap, the blocks' tables, the last tiles), and one prime's pass of 2^21 points has one
+ * tile per CU: nothing to fetch ahead.  Measured per call, prime after prime against one launch for all: 32 K-limb
+ * operands 163 -> 86 us, 2^20 276 -> 202, 2^22 840 -> 724, 2^23 (2^24 points) 1529 -> 1405; at 2^25 points the two are
+ * equal (2.77 and 2.75 ms) and the planes twice as large.  NTTM_PAR_POINTS overrides it, 0 turns it off. */
+static uint64_t g_par_points = (uint64_t)1 << 24;
+/* points of one prime per chunk of a batch group: a group's products run chunk after chunk through the same planes, so
+ * that the planes stay below 2 np 128 MiB.  Smaller chunks, whose planes would fit the last-level cache, are slower:
+ * the 4096 leaves' replay takes 5.83 ms at 2^24 points, 5.91 at 2^22, 6.71 at 2^21, 8.41 at 2^20 (four more launches
+ * per chunk).  NTTM_CHUNK_POINTS overrides it. */
+static uint64_t g_chunk_points = (uint64_t)1 << 24;
 
 /* the workspace of nttm_mul_noalloc: a file-scope device array, one copy per GPU, held until the process ends.  Host
  * code never uses its name as an address (on the host it is a stand-in, not the device address): nttm_init looks up
@@ -413,6 +427,11 @@ extern "C" int nttm_init(int device, const nttm_config *cfg)
         g_no_defer = e && e[0] == '1';
     }
     {
+        const char *e = getenv("NTTM_PAR_POINTS"), *c = getenv("NTTM_CHUNK_POINTS");
+        g_par_points = e ? strtoull(e, nullptr, 0) : (uint64_t)1 << 24;
+        g_chunk_points = c && strtoull(c, nullptr, 0) ? strtoull(c, nullptr, 0) : (uint64_t)1 << 24;
+    }
+    {
         const char *e = getenv("NTTM_TREE_LEVELWISE");
         g_tree_levelwise = e && e[0] == '1';
     }
@@ -450,11 +469,6 @@ extern "C" void nttm_shutdown(void)
     for (int k = 0; k < 2; k++) if (g.bev[k]) (void)hipEventDestroy(g.bev[k]);
     for (int k = 0; k < 8; k++) if (g.tev[k]) (void)hipEventDestroy(g.tev[k]);
     if (g.tcs) (void)hipStreamDestroy(g.tcs);
-    for (int k = 0; k < NTTM_MAX_PRIMES - 1; k++) {
-        if (g.ps[k]) (void)hipStreamDestroy(g.ps[k]);
-        if (g.pjev[k]) (void)hipEventDestroy(g.pjev[k]);
-    }
-    if (g.pfev) (void)hipEventDestroy(g.pfev);
     free_deferred();
     for (int i = 0; i < 4; i++) (void)hipEventDestroy(g.ev[i]);
     for (int i = 0; i < 2 * NTTM_MAX_PRIMES; i++) if (g.pev[i]) (void)hipEventDestroy(g.pev[i]);
@@ -558,8 +572,7 @@ static void product_plan(Plan *pl, int logn, uint64_t batch, int tile_log)
 
 /* the transforms of cnt products of one length: 2^logn points (r3 = 0), or 3 2^logn points (r3 = 1: a radix-3 layer,
  * reading the limbs, and the 2^logn engine on the 3 cnt thirds).  Plane i of A holds the cnt transforms of prime i back
- * to back.  After it, A holds the cyclic convolutions mod each prime, natural order.  B has one plane, reused by every
- * prime: B's transform of prime i is made just before A's (np + 1 planes in all instead of 2 np).
+ * to back.  After it, A holds the cyclic convolutions mod each prime, natural order.
  * Shared B operands (bmap non-null): B's plane holds the cnt_b distinct operands of ldesc_b; A's engine transform t
  * pairs with B's engine transform bmap[t] in the double-fused pass.
  * pev (or null): 2 np events recorded around B's transform of each prime. */
@@ -572,24 +585,27 @@ static bool defer_ok(const PassArgs &q, const Plan &pl, int last)
     PassArgs nx = q; nx.limbs = nullptr; nx.ldesc = nullptr; nx.do_in_scale = 0;
     return nttm_fwd_pass_streams(q, pl.p[0]) && nttm_fwd_pass_streams(nx, pl.p[1]) && pl.p[1].m >= 4;
 }
-/* the deferral's flags for pass j of the plan (q carries pass 0's in_scale until pass 0 has run) */
+/* the deferral's flags for pass j of the plan (a job's dfr_scale goes with the pass that has dfr_in) */
 static void defer_set(PassArgs &q, const Plan &pl, int j, bool on)
 {
     q.dfr_out = on && j == 0;
-    if (on && j == 1) {
-        q.dfr_in = 1; q.dfr_lom = pl.p[0].lo + pl.p[0].m; q.dfr_gm = pl.p[0].m;
-    } else q.dfr_in = 0;
-    if (on && j == 0) { q.dfr_do_scale = q.do_in_scale; q.dfr_scale = q.in_scale; }
-    if (j > 1) q.dfr_do_scale = 0;
+    q.dfr_in = on && j == 1;
+    if (q.dfr_in) { q.dfr_lom = pl.p[0].lo + pl.p[0].m; q.dfr_gm = pl.p[0].m; }
 }
-/* ps: prime i's work on stream ps[i] with its own B plane at Bp + i bstride (the caller forks and joins them); null:
- * every prime on s, one after another, through the one B plane at Bp */
-static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A, double *Bp, const uint64_t *a,
-                              uint64_t na, const uint64_t *b, uint64_t nb, const LoadDesc *ldesc, hipStream_t s0,
-                              hipEvent_t *pev, uint64_t cnt_b = 0, const LoadDesc *ldesc_b = nullptr,
-                              const uint32_t *bmap = nullptr, const hipStream_t *ps = nullptr, uint64_t bstride = 0)
+/* a job of prime i on plane x, in one direction */
+static PassJob prime_job(int i, double *x, uint64_t batch, bool inv)
 {
-    double *const Bp0 = Bp;
+    PassJob j; memset(&j, 0, sizeof j);
+    j.x = x; j.batch = batch; j.p = g.pk[i].p; j.pinv = g.pk[i].pinv; j.tw = inv ? g.twi[i] : g.twf[i];
+    return j;
+}
+/* bstride = 0: one prime after another, sharing the one B plane at Bp; bstride > 0: one launch per pass for every prime
+ * and both operands, prime i's B plane at Bp + i bstride */
+static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A, double *Bp, uint64_t bstride,
+                              const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb, const LoadDesc *ldesc,
+                              hipStream_t s, hipEvent_t *pev, uint64_t cnt_b = 0, const LoadDesc *ldesc_b = nullptr,
+                              const uint32_t *bmap = nullptr)
+{
     if (!bmap) { cnt_b = cnt; ldesc_b = ldesc; }
     const uint64_t tb = r3 ? 3 * cnt : cnt, tbb = r3 ? 3 * cnt_b : cnt_b;   /* engine transforms of 2^logn points */
     Plan pl; product_plan(&pl, logn, tb, product_tile_log(logn));
@@ -598,46 +614,77 @@ static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A,
     const int last = pl.npass - 1;
     if (bmap && (plb.npass != pl.npass || pl.p[last].m + pl.p[last].logh > logn || (last == 0 && !r3)))
         return nttm_fail(NTTM_EINVAL, "internal: shared B operands on this length");
-    for (int i = 0; i < np; i++) {
-        double *Ai = A + (size_t)i * plane;
-        const uint64_t p = NTTM_PRIMES[i];
-        const hipStream_t s = ps ? ps[i] : s0;
-        Bp = ps ? Bp0 + (size_t)i * bstride : Bp0;
-        /* B, prime i, all passes but the last */
-        if (pev) HIPCK(hipEventRecord(pev[2 * i], s));
-        const double2 ninv = h_shoup(h_inv(ntot % p, p), p);     /* the inverse's 1/length, folded into B */
-        PassArgs fb = base_args(i, Bp, logn, tbb, false);
-        if (r3) RCK(nttm_run_r3(false, Bp, cnt_b, logn, g.pk[i], g.twf[i].b3, ldesc_b ? nullptr : b, nb, ldesc_b, 1, &ninv, s));
-        else { fb.limbs = ldesc_b ? nullptr : b; fb.nlimbs = nb; fb.ldesc = ldesc_b; fb.which = 1; fb.in_scale = ninv; fb.do_in_scale = 1; }
-        const bool dfb = !r3 && defer_ok(fb, plb, last);
-        for (int j = 0; j < last; j++) {
-            defer_set(fb, plb, j, dfb);
-            RCK(nttm_run_pass(false, fb, plb.p[j], s));
-            fb.limbs = nullptr; fb.ldesc = nullptr; fb.do_in_scale = 0;
+    /* both operands' strided passes in one launch where their geometry is the same (it differs only in the blocks a
+     * tile spans, by the powers of two in the two batch counts) */
+    bool pair = bstride > 0;
+    for (int j = 0; j < last; j++) if (memcmp(&pl.p[j], &plb.p[j], sizeof(PassGeom))) pair = false;
+    const int step = bstride ? np : 1;
+    for (int i0 = 0; i0 < np; i0 += step) {
+        JobSet jb, ja, ji;                                         /* B, A, A's inverse */
+        FusedSet jf;                                               /* the double-fused pass */
+        memset(&jb, 0, sizeof jb); memset(&ja, 0, sizeof ja); memset(&jf, 0, sizeof jf); memset(&ji, 0, sizeof ji);
+        jb.n = ja.n = jf.n = ji.n = step;
+        for (int k = 0; k < step; k++) {
+            const int i = i0 + k;
+            const uint64_t p = NTTM_PRIMES[i];
+            double *Ai = A + (size_t)i * plane, *Bi = Bp + (size_t)i * bstride;
+            const double2 ninv = h_shoup(h_inv(ntot % p, p), p);     /* the inverse's 1/length, folded into B */
+            jb.j[k] = prime_job(i, Bi, tbb, false);
+            jb.j[k].limbs = ldesc_b ? nullptr : b; jb.j[k].nlimbs = nb; jb.j[k].ldesc = ldesc_b; jb.j[k].which = 1;
+            jb.j[k].in_scale = ninv; jb.j[k].do_in_scale = 1;
+            ja.j[k] = prime_job(i, Ai, tb, false);
+            ja.j[k].limbs = ldesc ? nullptr : a; ja.j[k].nlimbs = na; ja.j[k].ldesc = ldesc; ja.j[k].which = 0;
+            jf.j[k] = FusedJob{Ai, Bi, g.pk[i].p, g.pk[i].pinv, g.twf[i].stage, g.twi[i].stage, ninv};
+            ji.j[k] = prime_job(i, Ai, tb, true);
         }
-        if (pev) HIPCK(hipEventRecord(pev[2 * i + 1], s));
-        /* A, prime i */
-        PassArgs fa = base_args(i, Ai, logn, tb, false);
-        if (r3) RCK(nttm_run_r3(false, Ai, cnt, logn, g.pk[i], g.twf[i].b3, ldesc ? nullptr : a, na, ldesc, 0, nullptr, s));
-        else { fa.limbs = ldesc ? nullptr : a; fa.nlimbs = na; fa.ldesc = ldesc; fa.which = 0; }
-        const bool dfa = !r3 && defer_ok(fa, pl, last);
-        for (int j = 0; j < last; j++) {
-            defer_set(fa, pl, j, dfa);
-            RCK(nttm_run_pass(false, fa, pl.p[j], s));
-            fa.limbs = nullptr; fa.ldesc = nullptr;
+        /* the forward passes but the last, of the given jobs; the first reads the operand limbs (a radix-3 layer does
+         * where there is one).  j0: the jobs as the caller set them up */
+        auto forward = [&](JobSet js, const Plan &q) -> int {
+            auto limbs_done = [&]() { for (int k = 0; k < js.n; k++) { PassJob &j = js.j[k]; j.limbs = nullptr; j.ldesc = nullptr; j.do_in_scale = 0; } };
+            if (r3) {
+                JobSet r = js;
+                for (int k = 0; k < r.n; k++) r.j[k].batch /= 3;
+                RCK(nttm_run_r3(false, logn, r, s));
+                limbs_done();
+            }
+            PassArgs f = base_args(i0, js.j[0].x, logn, js.j[0].batch, false);
+            f.limbs = js.j[0].limbs; f.nlimbs = js.j[0].nlimbs; f.ldesc = js.j[0].ldesc;
+            const bool dfr = !r3 && defer_ok(f, q, last);
+            for (int j = 0; j < last; j++) {
+                defer_set(f, q, j, dfr);
+                if (dfr && j == 0) for (int k = 0; k < js.n; k++) js.j[k].dfr_do_scale = js.j[k].do_in_scale;
+                RCK(nttm_run_pass(false, f, q.p[j], s, &js));
+                f.limbs = nullptr; f.ldesc = nullptr;
+                limbs_done();
+            }
+            return 0;
+        };
+        if (pair && (last > 0 || r3)) {
+            JobSet all = jb;
+            for (int k = 0; k < step; k++) all.j[all.n++] = ja.j[k];
+            if (pev) HIPCK(hipEventRecord(pev[2 * i0], s));
+            RCK(forward(all, pl));
+            if (pev) HIPCK(hipEventRecord(pev[2 * i0 + 1], s));
+        } else {
+            if (pev) HIPCK(hipEventRecord(pev[2 * i0], s));
+            if (last > 0 || r3) RCK(forward(jb, plb));
+            if (pev) HIPCK(hipEventRecord(pev[2 * i0 + 1], s));
+            if (last > 0 || r3) RCK(forward(ja, pl));
         }
-        fa.dfr_in = 0;
         /* B's last forward pass, A's last forward pass, the pointwise product and A's first inverse pass */
-        PassArgs fbl = base_args(i, Bp, logn, tb, false);
-        fbl.bmap = bmap;
-        if (last == 0 && !r3) {                                  /* a single-pass transform reads B's limbs here */
-            fbl.limbs = ldesc ? nullptr : b; fbl.nlimbs = nb; fbl.ldesc = ldesc; fbl.which = 1;
-            fbl.in_scale = h_shoup(h_inv(n % p, p), p); fbl.do_in_scale = 1;
+        PassArgs fa = base_args(i0, jf.j[0].x, logn, tb, false);
+        FusedB fb{nullptr, 0, nullptr, bmap};
+        if (last == 0 && !r3) {                                  /* a single-pass transform reads both operands here */
+            fa.limbs = ldesc ? nullptr : a; fa.nlimbs = na; fa.ldesc = ldesc; fa.which = 0;
+            fb.limbs = ldesc ? nullptr : b; fb.nlimbs = nb; fb.ldesc = ldesc;
         }
-        RCK(nttm_run_fused2(fa, fbl, pl.p[last], s));
-        PassArgs ia = base_args(i, Ai, logn, tb, true);
-        for (int j = last - 1; j >= 0; j--) RCK(nttm_run_pass(true, ia, pl.p[j], s));
-        if (r3) RCK(nttm_run_r3(true, Ai, cnt, logn, g.pk[i], g.twi[i].b3, nullptr, 0, nullptr, 0, nullptr, s));
+        RCK(nttm_run_fused2(fa, fb, pl.p[last], s, jf));
+        PassArgs ia = base_args(i0, ji.j[0].x, logn, tb, true);
+        for (int j = last - 1; j >= 0; j--) RCK(nttm_run_pass(true, ia, pl.p[j], s, &ji));
+        if (r3) {
+            for (int k = 0; k < step; k++) ji.j[k].batch = cnt;
+            RCK(nttm_run_r3(true, logn, ji, s));
+        }
     }
     return 0;
 }
@@ -699,20 +746,7 @@ static bool fits_one(size_t na, size_t nb, size_t nc)
 
 /* the workspace of a one-transform product: the planes, its CRT descriptor and the CRT's scratch (bytes from ws) */
 struct CoreLayout { int np, logn, r3, par; uint64_t n, ncoef; size_t nc, nc_full, off_desc, off_crt, bytes; };
-/* transforms of at most this many points run their primes concurrently (a launch of one prime's pass has too few tiles
- * to fill the device); NTTM_PAR_POINTS overrides it, 0 turns it off */
-static uint64_t par_points(void)
-{
-    static uint64_t v = 0;
-    static bool set = false;
-    if (!set) {
-        const char *e = getenv("NTTM_PAR_POINTS");
-        v = e ? strtoull(e, nullptr, 0) : ((uint64_t)1 << 22);
-        set = true;
-    }
-    return v;
-}
-/* allow_par: the primes may run concurrently, each with its own B plane (the library's workspace, not captured) */
+/* allow_par: one launch per pass for all primes, each with its own B plane (in the library's workspace) */
 static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout *L, bool allow_par = false)
 {
     L->nc_full = na + nb + (has_x ? 1 : 0); L->nc = L->nc_full < wcut ? L->nc_full : wcut;
@@ -722,15 +756,15 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
     choose_len(ncoef_full, &L->logn, &L->r3);
     if (L->logn > NTTM_LOGN_MAX) return nttm_fail(NTTM_EBOUND, "transform length 2^%d above 2^%d", L->logn, NTTM_LOGN_MAX);
     L->n = (uint64_t)(L->r3 ? 3 : 1) << L->logn;                  /* points per plane */
-    /* np planes of A and one of B: B's transform of each prime is made just before A's of that prime; concurrent
-     * primes take a B plane each */
+    /* np planes of A and one of B: B's transform of each prime is made just before A's of that prime; primes in one
+     * launch take a B plane each */
     const size_t crt_words = nttm_crt_scratch_words(nttm_crt_blocks(L->nc));
-    for (int par = allow_par && L->np > 1 && L->n <= par_points(); par >= 0; par--) {
+    for (int par = allow_par && L->np > 1 && L->n <= g_par_points; par >= 0; par--) {
         const size_t planes_bytes = (size_t)(par ? 2 * L->np : L->np + 1) * L->n * 8;
         L->par = par;
         L->off_desc = align_up(planes_bytes, 256); L->off_crt = L->off_desc + 256;
         L->bytes = L->off_crt + crt_words * 4 + 256;
-        if (!g.cfg.workspace_bytes || L->bytes <= g.cfg.workspace_bytes) break;   /* concurrent only within the cap */
+        if (!g.cfg.workspace_bytes || L->bytes <= g.cfg.workspace_bytes) break;   /* together only within the cap */
     }
     return 0;
 }
@@ -756,9 +790,7 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
         return 0;
     }
     if (!nc) return 0;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (!ws && hipStreamIsCapturing(s, &cap) != hipSuccess) { (void)hipGetLastError(); cap = hipStreamCaptureStatusActive; }
-    CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws && cap == hipStreamCaptureStatusNone));
+    CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws));
     if (ws) {
         if (L.bytes > ws_cap) return nttm_fail(NTTM_EINVAL, "the product needs %zu bytes of workspace, above the %zu given", L.bytes, ws_cap);
     } else {
@@ -771,23 +803,7 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     char *hs = (char *)g.hpin + 128 * slot;                       /* pinned: the descriptor, then (at 96) the flags */
 
     if (sync) HIPCK(hipEventRecord(g.ev[0], s));
-    hipStream_t ps[NTTM_MAX_PRIMES];
-    if (L.par) {                                                 /* prime 0 on s, the others forked from it */
-        if (!g.pfev) {
-            HIPCK(hipEventCreateWithFlags(&g.pfev, hipEventDisableTiming));
-            for (int k = 0; k < NTTM_MAX_PRIMES - 1; k++) {
-                HIPCK(hipStreamCreateWithFlags(&g.ps[k], hipStreamNonBlocking));
-                HIPCK(hipEventCreateWithFlags(&g.pjev[k], hipEventDisableTiming));
-            }
-        }
-        HIPCK(hipEventRecord(g.pfev, s));
-        ps[0] = s;
-        for (int i = 1; i < L.np; i++) { ps[i] = g.ps[i - 1]; HIPCK(hipStreamWaitEvent(ps[i], g.pfev, 0)); }
-    }
-    RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, a, na, b, nb, nullptr, s, sync ? g.pev : nullptr, 0, nullptr,
-                           nullptr, L.par ? ps : nullptr, L.n));
-    if (L.par)
-        for (int i = 1; i < L.np; i++) { HIPCK(hipEventRecord(g.pjev[i - 1], ps[i])); HIPCK(hipStreamWaitEvent(s, g.pjev[i - 1], 0)); }
+    RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, L.par ? L.n : 0, a, na, b, nb, nullptr, s, sync ? g.pev : nullptr));
     if (sync) HIPCK(hipEventRecord(g.ev[2], s));
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.pl = A; hd.plane = L.n; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
@@ -801,7 +817,8 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     if (!sync) return 0;
     HIPCK(hipStreamSynchronize(s));
     float ms, tb = 0, t;
-    for (int i = 0; i < L.np; i++) { HIPCK(hipEventElapsedTime(&t, g.pev[2 * i], g.pev[2 * i + 1])); tb += t; }
+    for (int i = 0; i < (L.par ? 1 : L.np); i++) { HIPCK(hipEventElapsedTime(&t, g.pev[2 * i], g.pev[2 * i + 1])); tb += t; }
+    if (L.par) tb *= 0.5f;                                       /* the forward launches hold both operands */
     HIPCK(hipEventElapsedTime(&ms, g.ev[0], g.ev[2]));
     g.last_ms[0] = tb; g.last_ms[1] = ms - tb;
     HIPCK(hipEventElapsedTime(&ms, g.ev[2], g.ev[3])); g.last_ms[2] = ms;
@@ -841,11 +858,16 @@ int nttm_mul_cyclic(uint64_t *v, const uint64_t *a, size_t na, const uint64_t *b
     const size_t nc = L + 3;
     if (!na || !nb) { HIPCK(hipMemsetAsync(v, 0, nc * 8, s)); return flag ? 0 : nttm_hip_check(hipStreamSynchronize(s), "cyclic product"); }
     int np; RCK(choose_np(na < nb ? na : nb, &np));
-    const size_t planes_bytes = (size_t)(np + 1) * L * 8;
+    bool par = L <= g_par_points;
+    size_t planes_bytes = (size_t)(par ? 2 * np : np + 1) * L * 8;
+    const size_t crt_bytes = nttm_crt_scratch_words(nttm_crt_blocks(nc)) * 4 + 256;
+    if (par && g.cfg.workspace_bytes && align_up(planes_bytes, 256) + 256 + crt_bytes > g.cfg.workspace_bytes) {
+        par = false; planes_bytes = (size_t)(np + 1) * L * 8;
+    }
     const size_t off_desc = align_up(planes_bytes, 256), off_crt = off_desc + 256;
-    RCK(ws_need(off_crt + nttm_crt_scratch_words(nttm_crt_blocks(nc)) * 4 + 256));
+    RCK(ws_need(off_crt + crt_bytes));
     double *A = (double *)g.ws, *Bp = A + (size_t)np * L;
-    RCK(product_transforms(np, logn, r3, 1, A, Bp, a, na, b, nb, nullptr, s, nullptr));
+    RCK(product_transforms(np, logn, r3, 1, A, Bp, par ? L : 0, a, na, b, nb, nullptr, s, nullptr));
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.pl = A; hd.plane = L; hd.ncoef = L; hd.c = v; hd.nc = nc;
     char *hs = (char *)g.hpin;
@@ -1048,49 +1070,71 @@ struct GroupBuild {
     int r3 = 0, logn = 0, tile = 0, pts = 0;
     int crt_per = 8;                                             /* CRT limbs per thread: 1 when every product is small */
     uint64_t n = 0, cnt = 0, cnt_b = 0, nblk = 0;
-    bool share = false;
+    bool share = false, merged = false;
+    struct Chunk { uint64_t c0, cn, b0, cnb, blk0, nblk; double crt_bytes; };   /* products, distinct B operands, CRT blocks */
+    std::vector<Chunk> chunk;
     std::vector<CrtDesc> cd;
     std::vector<LoadDesc> ld, ldb;
     std::vector<uint32_t> bmap;
     size_t planes_bytes = 0;                                     /* (np cnt + cnt_b) n doubles */
     size_t off_cd = 0, off_ld = 0, off_ldb = 0, off_bmap = 0, off_ncn = 0, off_crt = 0, desc_bytes = 0;
-    double crt_bytes = 0;
 };
+/* products of a group that run together (a chunk), and whether all primes of a chunk share a launch per pass */
+static uint64_t chunk_products(uint64_t n) { return std::max<uint64_t>(1, g_chunk_points / n); }
+static bool chunk_merged(uint64_t n, uint64_t cn) { return n * cn <= std::max(g_chunk_points, g_par_points); }
+static size_t chunk_planes_bytes(int np, uint64_t n, uint64_t cnt)
+{
+    const uint64_t cn = std::min(cnt, chunk_products(n));
+    return (size_t)(chunk_merged(n, cn) ? 2 * np : np + 1) * cn * n * 8;
+}
 static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<size_t> &G, int np, int r3, int logn,
                         int tile, int pts)
 {
     gb.r3 = r3; gb.logn = logn; gb.tile = tile; gb.pts = pts;
     const uint64_t n = (uint64_t)(r3 ? 3 : 1) << logn, cnt = G.size();          /* points per product plane */
-    gb.n = n; gb.cnt = cnt; gb.nblk = 0; gb.crt_bytes = 0;
+    gb.n = n; gb.cnt = cnt; gb.nblk = 0; gb.cnt_b = 0; gb.planes_bytes = 0;
     gb.crt_per = n <= 1024 ? 1 : 8;                              /* products of at most n + 1 limbs: 256-limb blocks */
-    gb.cd.assign(cnt, CrtDesc()); gb.ld.assign(cnt, LoadDesc()); gb.ldb.clear(); gb.bmap.clear();
-    for (uint64_t j = 0; j < cnt; j++) {
-        const nttm_prod &q = P[G[j]];
-        LoadDesc &l = gb.ld[j];
-        CrtDesc &c = gb.cd[j];
-        l.a = q.a; l.na = q.na; l.b = q.b; l.nb = q.nb;
-        c.pl = nullptr; c.plane = cnt * n; c.ncoef = q.na + q.nb - 1; c.x = q.x; c.nx = q.x ? q.nx : 0;
-        c.c = q.c; c.nc = q.na + q.nb + (q.x ? 1 : 0); c.first_block = gb.nblk; c.trunc = 0;
-        gb.nblk += nttm_crt_blocks(c.nc, gb.crt_per);
-        gb.crt_bytes += 8.0 * np * c.ncoef + 8.0 * c.nc + 8.0 * c.nx;
+    gb.cd.assign(cnt, CrtDesc()); gb.ld.assign(cnt, LoadDesc()); gb.ldb.clear(); gb.bmap.clear(); gb.chunk.clear();
+    const uint64_t cmax = chunk_products(n);
+    gb.merged = chunk_merged(n, std::min(cnt, cmax));
+    for (uint64_t c0 = 0; c0 < cnt; c0 += cmax) gb.chunk.push_back({c0, std::min(cmax, cnt - c0), 0, 0, 0, 0, 0.0});
+    for (GroupBuild::Chunk &ch : gb.chunk) {
+        ch.blk0 = gb.nblk;
+        for (uint64_t j = ch.c0; j < ch.c0 + ch.cn; j++) {
+            const nttm_prod &q = P[G[j]];
+            LoadDesc &l = gb.ld[j];
+            CrtDesc &c = gb.cd[j];
+            l.a = q.a; l.na = q.na; l.b = q.b; l.nb = q.nb;
+            c.pl = nullptr; c.plane = ch.cn * n; c.ncoef = q.na + q.nb - 1; c.x = q.x; c.nx = q.x ? q.nx : 0;
+            c.c = q.c; c.nc = q.na + q.nb + (q.x ? 1 : 0); c.first_block = gb.nblk; c.trunc = 0;
+            gb.nblk += nttm_crt_blocks(c.nc, gb.crt_per);
+            ch.crt_bytes += 8.0 * np * c.ncoef + 8.0 * c.nc + 8.0 * c.nx;
+        }
+        ch.nblk = gb.nblk - ch.blk0;
     }
     /* products that share their B operand (the same b and nb: the binary-splitting tree's P1 Q2 + P2 and Q1 Q2,
-     * E/rns_mul.c:476-495) transform it once, where B has planes (a transform of more than one pass, or a radix-3
-     * length) and the double-fused tiles lie inside one transform */
+     * E/rns_mul.c:476-495) transform it once per chunk, where B has planes (a transform of more than one pass, or a
+     * radix-3 length) and the double-fused tiles lie inside one transform */
     std::vector<uint32_t> slot(cnt);
     Plan pq; product_plan(&pq, logn, r3 ? 3 * cnt : cnt, product_tile_log(logn, tile));
     const bool can = logn >= NTTM_FUSED_LOG && (pq.npass > 1 || r3);
-    std::map<std::pair<const uint64_t *, uint64_t>, uint32_t> seen;
-    for (uint64_t j = 0; j < cnt && can; j++) {
-        auto key = std::make_pair(gb.ld[j].b, gb.ld[j].nb);
-        auto it = seen.find(key);
-        if (it == seen.end()) {
-            it = seen.emplace(key, (uint32_t)gb.ldb.size()).first;
-            gb.ldb.push_back(gb.ld[j]);
+    if (can) gb.ldb.reserve(cnt);
+    for (GroupBuild::Chunk &ch : gb.chunk) {
+        std::map<std::pair<const uint64_t *, uint64_t>, uint32_t> seen;
+        ch.b0 = gb.ldb.size();
+        for (uint64_t j = ch.c0; j < ch.c0 + ch.cn && can; j++) {
+            auto key = std::make_pair(gb.ld[j].b, gb.ld[j].nb);
+            auto it = seen.find(key);
+            if (it == seen.end()) {
+                it = seen.emplace(key, (uint32_t)(gb.ldb.size() - ch.b0)).first;
+                gb.ldb.push_back(gb.ld[j]);
+            }
+            slot[j] = it->second;
         }
-        slot[j] = it->second;
+        ch.cnb = can ? gb.ldb.size() - ch.b0 : ch.cn;            /* no sharing: one B per product */
+        gb.cnt_b += ch.cnb;
+        gb.planes_bytes = std::max(gb.planes_bytes, ((size_t)np * ch.cn + (size_t)(gb.merged ? np : 1) * ch.cnb) * n * 8);
     }
-    gb.cnt_b = can ? gb.ldb.size() : cnt;                       /* no sharing: one B per product */
     gb.share = gb.cnt_b < cnt;
     if (!gb.share) gb.ldb.clear();
     const uint64_t tb = r3 ? 3 * cnt : cnt;
@@ -1098,7 +1142,6 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
         gb.bmap.resize(tb);
         for (uint64_t t = 0; t < tb; t++) gb.bmap[t] = r3 ? 3 * slot[t / 3] + (uint32_t)(t % 3) : slot[t];
     }
-    gb.planes_bytes = ((size_t)np * cnt + gb.cnt_b) * n * 8;
     gb.off_cd = 0;
     gb.off_ld = align_up(gb.off_cd + cnt * sizeof(CrtDesc), 256);
     gb.off_ldb = align_up(gb.off_ld + cnt * sizeof(LoadDesc), 256);
@@ -1113,7 +1156,8 @@ static int batch_pts(int logn) { return g.cfg.pts ? g.cfg.pts : logn <= 14 ? 8 :
 /* the group's descriptors as one host image (planes at A), to copy to the group's descriptor base */
 static void group_image(GroupBuild &gb, double *A, char *img)
 {
-    for (uint64_t j = 0; j < gb.cnt; j++) gb.cd[j].pl = A + j * gb.n;          /* (the alignment gaps stay unread) */
+    for (const GroupBuild::Chunk &ch : gb.chunk)                     /* (the alignment gaps stay unread) */
+        for (uint64_t j = 0; j < ch.cn; j++) gb.cd[ch.c0 + j].pl = A + j * gb.n;
     memcpy(img + gb.off_cd, gb.cd.data(), gb.cnt * sizeof(CrtDesc));
     memcpy(img + gb.off_ld, gb.ld.data(), gb.cnt * sizeof(LoadDesc));
     if (gb.share) {
@@ -1127,12 +1171,18 @@ static int group_launch(const GroupBuild &gb, int np, double *A, char *dbase, hi
 {
     const int tile0 = g.cfg.tile_log, pts0 = nttm_get_pts();
     g.cfg.tile_log = gb.tile; nttm_set_pts(gb.pts);
-    double *Bp = A + (size_t)np * gb.cnt * gb.n;
-    int rc = product_transforms(np, gb.logn, gb.r3, gb.cnt, A, Bp, nullptr, 0, nullptr, 0, (const LoadDesc *)(dbase + gb.off_ld),
-                                s, nullptr, gb.cnt_b, gb.share ? (const LoadDesc *)(dbase + gb.off_ldb) : nullptr,
-                                gb.share ? (const uint32_t *)(dbase + gb.off_bmap) : nullptr);
-    if (!rc) rc = nttm_crt_launch_batch(dbase + gb.off_cd, gb.cnt, gb.nblk, np, g.cc, (uint32_t *)(dbase + gb.off_crt), s,
-                                        gb.crt_bytes, gb.crt_per);
+    int rc = 0;
+    for (const GroupBuild::Chunk &ch : gb.chunk) {               /* chunk after chunk through the same planes */
+        double *Bp = A + (size_t)np * ch.cn * gb.n;
+        const LoadDesc *ld = (const LoadDesc *)(dbase + gb.off_ld) + ch.c0;
+        rc = product_transforms(np, gb.logn, gb.r3, ch.cn, A, Bp, gb.merged ? ch.cnb * gb.n : 0, nullptr, 0, nullptr, 0, ld, s,
+                                nullptr, ch.cnb, gb.share ? (const LoadDesc *)(dbase + gb.off_ldb) + ch.b0 : nullptr,
+                                gb.share ? (const uint32_t *)(dbase + gb.off_bmap) + (gb.r3 ? 3 : 1) * ch.c0 : nullptr);
+        if (!rc) rc = nttm_crt_launch_limbs((const CrtDesc *)(dbase + gb.off_cd) + ch.c0, ch.cn, ch.blk0, ch.nblk, np, g.cc,
+                                            (uint32_t *)(dbase + gb.off_crt), s, ch.crt_bytes, gb.crt_per);
+        if (rc) break;
+    }
+    if (!rc) rc = nttm_crt_launch_carry(dbase + gb.off_cd, gb.cnt, gb.nblk, (uint32_t *)(dbase + gb.off_crt), s, gb.crt_per);
     if (!rc && norm) rc = nttm_run_norm(dbase + gb.off_cd, gb.cnt, (uint64_t *)(dbase + gb.off_ncn), s);
     g.cfg.tile_log = tile0; nttm_set_pts(pts0);
     return rc;
@@ -1626,7 +1676,7 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
         int ki[4];
         RCK(prod_kinds(mm, q.a, q.na, q.b, q.nb, q.x, q.nx, q.c, nc, ki, i));
         if (any_host(ki)) return nttm_fail(NTTM_EINVAL, "nttm_mul_each_async: product %zu: host memory (device memory only)", i);
-        if (q.na && q.nb && fits_one(q.na, q.nb, nc)) {                /* (with the concurrent primes' B planes) */
+        if (q.na && q.nb && fits_one(q.na, q.nb, nc)) {                /* (with every prime's B plane) */
             CoreLayout L; RCK(core_layout(q.na, q.nb, q.x != nullptr, SIZE_MAX, &L, true));
             ws_max = std::max(ws_max, L.bytes);
         }
@@ -1777,7 +1827,7 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
             if (logn > NTTM_LOGN_MAX) return 1;
             for (uint64_t c0 = 0; c0 < cnt_all; c0 += TREE_CHUNK) {   /* the group's chunks (below) */
                 const uint64_t cn = std::min<uint64_t>(TREE_CHUNK, cnt_all - c0), tb = r3 ? 3 * cn : cn;
-                planes_max = std::max(planes_max, (size_t)(lev_np[k] + 1) * cn * npts * 8);
+                planes_max = std::max(planes_max, chunk_planes_bytes(lev_np[k], npts, cn));
                 const size_t img = align_up(cn * sizeof(CrtDesc), 256) + 2 * align_up(cn * sizeof(LoadDesc), 256) +
                                    align_up(tb * 4, 256) + 256;
                 img_total += img;
@@ -2069,7 +2119,9 @@ extern "C" int nttm_ntt_fwd3(int prime, uint64_t *x, int logk, size_t batch, voi
     hipStream_t s = (hipStream_t)stream;
     const uint64_t cnt = 3 * ((uint64_t)batch << logk);
     RCK(nttm_run_u64_to_f64((double *)x, cnt, s));
-    RCK(nttm_run_r3(false, (double *)x, batch, logk, g.pk[prime], g.twf[prime].b3, nullptr, 0, nullptr, 0, nullptr, s));
+    JobSet r; memset(&r, 0, sizeof r);
+    r.n = 1; r.j[0] = prime_job(prime, (double *)x, batch, false);
+    RCK(nttm_run_r3(false, logk, r, s));
     RCK(fwd_planes(prime, (double *)x, logk, 3 * (uint64_t)batch, s));
     return nttm_run_f64_to_canon((double *)x, cnt, g.pk[prime], s);
 }
@@ -2078,8 +2130,10 @@ static int inv3_planes(int prime, double *x, const double *y, int ymode, int log
 {
     const uint64_t p = NTTM_PRIMES[prime];
     RCK(inv_planes(prime, x, y, ymode, logk, 3 * batch, 1, s, 1));
-    const double2 third = h_shoup(h_inv(3, p), p);
-    return nttm_run_r3(true, x, batch, logk, g.pk[prime], g.twi[prime].b3, nullptr, 0, nullptr, 0, &third, s);
+    JobSet r; memset(&r, 0, sizeof r);
+    r.n = 1; r.j[0] = prime_job(prime, x, batch, true);
+    r.j[0].in_scale = h_shoup(h_inv(3, p), p); r.j[0].do_in_scale = 1;
+    return nttm_run_r3(true, logk, r, s);
 }
 extern "C" int nttm_ntt_inv3(int prime, uint64_t *x, int logk, size_t batch, void *stream)
 {

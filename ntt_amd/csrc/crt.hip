@@ -46,6 +46,7 @@ struct CrtArgs {
     const CrtDesc *desc; uint64_t nprod;
     uint32_t *status;                    /* one word per block (CRT_ST_*) */
     uint32_t *ctl;                       /* [1] error flags */
+    uint32_t block0;                     /* the launch's first block */
     CrtConst cc;
 };
 
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
     __shared__ uint32_t s_prod, s_err;
     __shared__ uint32_t s_wave[CRT_T / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t blk = blockIdx.x;
+    const uint32_t blk = a.block0 + blockIdx.x;
     if (tid == 0) {
         uint64_t lo = 0, hi = a.nprod - 1;                  /* the product whose block range holds blk */
         while (lo < hi) { const uint64_t mid = (lo + hi + 1) >> 1; if (a.desc[mid].first_block <= blk) lo = mid; else hi = mid - 1; }
@@ -443,41 +444,53 @@ uint64_t nttm_crt_blocks(uint64_t nc, int per) { const uint64_t ch = (uint64_t)C
 
 uint64_t nttm_crt_scratch_words(uint64_t nblocks) { return nblocks + CRT_CTL_WORDS; }
 
-/* desc_dev: nprod descriptors in device memory whose block ranges tile [0, nblocks); scratch: 16-byte aligned,
- * nttm_crt_scratch_words(nblocks) words, of which word 1 receives the error flags */
-int nttm_crt_launch_batch(const void *desc_dev, uint64_t nprod, uint64_t nblocks, int np, const CrtConst &cc,
+/* desc_dev: nprod descriptors in device memory whose block ranges tile [blk0, blk0 + nblk) of scratch's status words:
+ * their limbs for a carry into every block of 0, and the blocks' carry maps */
+int nttm_crt_launch_limbs(const void *desc_dev, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np, const CrtConst &cc,
                           uint32_t *scratch, hipStream_t s, double alg_bytes, int per)
 {
     if (per != 1 && per != CRT_WIDE) return nttm_fail(NTTM_EINVAL, "crt: %d limbs per thread", per);
     if (np < 3 || np > NTTM_MAX_PRIMES) return nttm_fail(NTTM_EINVAL, "crt: np = %d", np);
-    if (!nprod || !nblocks) return 0;
-    if (nblocks > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "crt: too many blocks");
+    if (!nprod || !nblk) return 0;
+    if (blk0 + nblk > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "crt: too many blocks");
     if ((uintptr_t)scratch & 15) return nttm_fail(NTTM_EINVAL, "crt: scratch not 16-byte aligned");
     CrtArgs a;
-    a.desc = (const CrtDesc *)desc_dev; a.nprod = nprod;
+    a.desc = (const CrtDesc *)desc_dev; a.nprod = nprod; a.block0 = (uint32_t)blk0;
     a.ctl = scratch; a.status = scratch + CRT_CTL_WORDS; a.cc = cc;
     prof_begin("k_crt", alg_bytes, s);
     if (per == 1) {
-        if (np == 3) hipLaunchKernelGGL((k_crt<3, 1>), dim3((unsigned)nblocks), dim3(CRT_T), 0, s, a);
-        else hipLaunchKernelGGL((k_crt<4, 1>), dim3((unsigned)nblocks), dim3(CRT_T), 0, s, a);
+        if (np == 3) hipLaunchKernelGGL((k_crt<3, 1>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
+        else hipLaunchKernelGGL((k_crt<4, 1>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
     } else {
-        if (np == 3) hipLaunchKernelGGL((k_crt<3, CRT_WIDE>), dim3((unsigned)nblocks), dim3(CRT_T), 0, s, a);
-        else hipLaunchKernelGGL((k_crt<4, CRT_WIDE>), dim3((unsigned)nblocks), dim3(CRT_T), 0, s, a);
+        if (np == 3) hipLaunchKernelGGL((k_crt<3, CRT_WIDE>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
+        else hipLaunchKernelGGL((k_crt<4, CRT_WIDE>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
     }
     prof_end(s);
-    int rc = nttm_hip_check(hipGetLastError(), "k_crt launch");
-    if (rc) return rc;
+    return nttm_hip_check(hipGetLastError(), "k_crt launch");
+}
+/* every block's carry in, and the limbs of the blocks that receive one; scratch's word 1 receives the error flags */
+int nttm_crt_launch_carry(const void *desc_dev, uint64_t nprod, uint64_t nblocks, uint32_t *scratch, hipStream_t s, int per)
+{
+    if (!nprod || !nblocks) return 0;
+    uint32_t *status = scratch + CRT_CTL_WORDS;
     prof_begin("k_crt_scan", 8.0 * (double)nblocks, s);
-    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, a.status, nblocks, a.ctl);
+    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, status, nblocks, scratch);
     prof_end(s);
-    rc = nttm_hip_check(hipGetLastError(), "k_crt_scan launch");
-    if (rc) return rc;
+    RCK(nttm_hip_check(hipGetLastError(), "k_crt_scan launch"));
     prof_begin("k_crt_fix", 4.0 * (double)nblocks, s);
     const dim3 gfix((unsigned)((nblocks + CRT_FIX_W - 1) / CRT_FIX_W));
-    if (per == 1) hipLaunchKernelGGL((k_crt_fix<1>), gfix, dim3(256), 0, s, a.desc, nprod, (const uint32_t *)a.status, nblocks);
-    else hipLaunchKernelGGL((k_crt_fix<CRT_WIDE>), gfix, dim3(256), 0, s, a.desc, nprod, (const uint32_t *)a.status, nblocks);
+    const CrtDesc *d = (const CrtDesc *)desc_dev;
+    if (per == 1) hipLaunchKernelGGL((k_crt_fix<1>), gfix, dim3(256), 0, s, d, nprod, (const uint32_t *)status, nblocks);
+    else hipLaunchKernelGGL((k_crt_fix<CRT_WIDE>), gfix, dim3(256), 0, s, d, nprod, (const uint32_t *)status, nblocks);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_crt_fix launch");
+}
+/* both for a whole launch of products: scratch 16-byte aligned, nttm_crt_scratch_words(nblocks) words */
+int nttm_crt_launch_batch(const void *desc_dev, uint64_t nprod, uint64_t nblocks, int np, const CrtConst &cc,
+                          uint32_t *scratch, hipStream_t s, double alg_bytes, int per)
+{
+    RCK(nttm_crt_launch_limbs(desc_dev, nprod, 0, nblocks, np, cc, scratch, s, alg_bytes, per));
+    return nttm_crt_launch_carry(desc_dev, nprod, nblocks, scratch, s, per);
 }
 
 /* ---- addition and subtraction of limb arrays, with the carry resolved like the CRT's -------------------------------

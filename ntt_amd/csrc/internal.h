@@ -59,6 +59,31 @@ struct PassArgs {
     double2 dfr_scale;
 };
 
+/* One launch can run a pass for several planes of one geometry (the primes of a product, both of its operands): block
+ * row blockIdx.y takes job blockIdx.y, whose fields replace the same ones of PassArgs */
+#define NTTM_MAX_JOBS (2 * NTTM_MAX_PRIMES)
+struct PassJob {
+    double *x;                      /* the plane */
+    const uint64_t *limbs; uint64_t nlimbs;
+    const LoadDesc *ldesc; int which;
+    int do_in_scale, dfr_do_scale;
+    uint64_t batch;                 /* transforms in this job's plane */
+    double p, pinv;
+    TwTables tw;
+    double2 in_scale;               /* of the limbs (do_in_scale) or of the deferred twiddles (dfr_do_scale) */
+};
+struct JobSet { int n; PassJob j[NTTM_MAX_JOBS]; };
+/* the double-fused pass's jobs: one per prime */
+struct FusedJob {
+    double *x, *xb;                 /* A's and B's planes */
+    double p, pinv;
+    const double2 *stage, *istage;  /* the forward and inverse stage tables */
+    double2 in_scale;               /* of B's limbs */
+};
+struct FusedSet { int n; FusedJob j[NTTM_MAX_PRIMES]; };
+/* B's operand of a single-pass transform (read here; the limbs or the descriptors), or the map of shared B transforms */
+struct FusedB { const uint64_t *limbs; uint64_t nlimbs; const LoadDesc *ldesc; const uint32_t *bmap; };
+
 struct Ctx;
 /* live kernel timing: when profiling is on, launches are bracketed by events (prof_begin before, prof_end after) */
 void prof_begin(const char *name, double alg_bytes, hipStream_t s);

@@ -338,9 +338,24 @@ __device__ __forceinline__ void bound_chain(double *v, const PassPos &pp, int lo
     }
 }
 
-template <int MODE, int PTS, int GM = -1, int GW = -1, int GH = -1>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_pass(PassArgs a)
+/* a uniform value held in scalar registers from here on: the compiler otherwise reads a job's fields again from the
+ * argument segment inside a persistent kernel's loop */
+template <typename T> __device__ __forceinline__ void hold(T &v) { asm volatile("" : "+s"(v)); }
+
+/* the fields of the block row's job (blockIdx.y) into the pass's arguments */
+__device__ __forceinline__ void apply_job(PassArgs &a, const JobSet &js)
 {
+    const PassJob &j = js.j[blockIdx.y];
+    a.x = j.x; a.limbs = j.limbs; a.nlimbs = j.nlimbs; a.ldesc = j.ldesc; a.which = j.which;
+    a.do_in_scale = j.do_in_scale; a.in_scale = j.in_scale; a.dfr_do_scale = j.dfr_do_scale; a.dfr_scale = j.in_scale;
+    a.batch = j.batch; a.pk.p = j.p; a.pk.pinv = j.pinv; a.tw = j.tw;
+}
+
+template <int MODE, int PTS, int GM = -1, int GW = -1, int GH = -1>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_pass(PassArgs a, JobSet js)
+{
+    apply_job(a, js);
+    if (blockIdx.x >= (a.batch << a.logn) >> (a.m + a.logw + a.logh)) return;   /* a job of fewer transforms */
     const int gm = GM >= 0 ? GM : a.m, gw = GW >= 0 ? GW : a.logw, gh = GH >= 0 ? GH : a.logh;
     constexpr bool INV = MODE >= PM_INV;
     extern __shared__ double lds_raw[];                         /* LDS_WORDS(T) doubles, sized at launch */
@@ -471,8 +486,11 @@ __device__ __forceinline__ void lds_barrier()
 
 
 template <int MODE, int GM, int GW>
-__global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, uint32_t ntiles)
+__global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
 {
+    apply_job(a, js);
+    hold(a.x); hold(a.pk.p); hold(a.pk.pinv);
+    const uint32_t ntiles = (uint32_t)((a.batch << a.logn) >> (GM + GW));
     constexpr bool INV = MODE == PM_INV, LIMB = MODE == PM_FWD_LIMB;
     constexpr int PTS = 16, T = 1 << (GM + GW), W = 1 << GW, NBQ = 4 << NTTM_BQ_LOG;
     static_assert(T == PTS * STREAM_T, "2^13-point tiles, 16 points per thread");
@@ -788,8 +806,15 @@ __device__ __forceinline__ void tile_forward(const PassArgs &q, const PassPos &p
 }
 
 template <int PTS, int GM = -1, int GH = -1, bool LIMBS = true>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_fused2(PassArgs a, PassArgs bq)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_fused2(PassArgs a, FusedB fb, FusedSet js)
 {
+    {   /* the block row's prime: planes and tables (the operands are the same for all) */
+        const FusedJob &j = js.j[blockIdx.y];
+        a.x = j.x; a.pk.p = j.p; a.pk.pinv = j.pinv; a.tw.stage = j.stage; a.twi.stage = j.istage;
+    }
+    PassArgs bq = a;
+    bq.x = js.j[blockIdx.y].xb; bq.limbs = fb.limbs; bq.nlimbs = fb.nlimbs; bq.ldesc = fb.ldesc; bq.which = 1;
+    bq.bmap = fb.bmap; bq.do_in_scale = 1; bq.in_scale = js.j[blockIdx.y].in_scale;
     __shared__ double xs_raw[LDS_WORDS(1 << FUSED_LOG)];
     /* the fixed shapes (4096-point tiles of 2^GM-point blocks, GM = 10, 11 or 12) keep the stage table's low entries in
      * LDS (the inverse mirrors them): the forward rounds after the first and the first two inverse rounds cover stages
@@ -936,6 +961,16 @@ struct R3Args {
     const LoadDesc *ldesc; int which;           /* ... or operand a / b of ldesc[t] */
     double2 scale; int do_scale;                /* multiply every output by scale */
 };
+/* the block row's layer (blockIdx.y): a job's plane, operand, tables of the layer's direction and scale */
+__device__ __forceinline__ R3Args r3_args(const JobSet &js, int logk)
+{
+    const PassJob &j = js.j[blockIdx.y];
+    R3Args a;
+    a.x = j.x; a.batch = j.batch; a.logk = logk; a.pk.p = j.p; a.pk.pinv = j.pinv; a.pk.pu = 0; a.b3 = j.tw.b3;
+    a.limbs = j.limbs; a.nlimbs = j.nlimbs; a.ldesc = j.ldesc; a.which = j.which;
+    a.scale = j.in_scale; a.do_scale = j.do_in_scale;
+    return a;
+}
 __device__ __forceinline__ double r3_input(const R3Args &a, uint64_t t, uint64_t k)
 {
     const uint64_t *src; uint64_t nl;
@@ -954,8 +989,9 @@ __device__ __forceinline__ void r3_twiddles(const R3Args &a, uint64_t j, double 
     *t1 = w1; *t2 = w2;
 }
 template <bool LIMB>
-__global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(R3Args a)
+__global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(int logk, JobSet js)
 {
+    const R3Args a = r3_args(js, logk);
     const uint64_t m = (uint64_t)1 << a.logk, total = a.batch << a.logk;
     const uint64_t stride = (uint64_t)gridDim.x * NTTM_THREADS;
     const double p = a.pk.p, pinv = a.pk.pinv;
@@ -977,8 +1013,9 @@ __global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(R3Args a)
         v[j + 2 * m] = mul_barrett(y2, t2, p, pinv);
     }
 }
-__global__ __launch_bounds__(NTTM_THREADS) void k_r3_inv(R3Args a)
+__global__ __launch_bounds__(NTTM_THREADS) void k_r3_inv(int logk, JobSet js)
 {
+    const R3Args a = r3_args(js, logk);
     const uint64_t m = (uint64_t)1 << a.logk, total = a.batch << a.logk;
     const uint64_t stride = (uint64_t)gridDim.x * NTTM_THREADS;
     const double p = a.pk.p, pinv = a.pk.pinv;
@@ -1038,18 +1075,39 @@ bool nttm_fwd_pass_streams(const PassArgs &a, const PassGeom &g)
     return fixed && g_stream && shape && g.lo >= g.logw && !a.do_scale &&
            (!limb || ((a.ldesc || a.batch == 1) && g.lo + g.m < 32));
 }
-int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s)
+/* the one job of a pass's own arguments */
+static JobSet job_of(const PassArgs &a)
 {
-    if (!pass_geom_ok(g, a.logn, a.batch)) return nttm_fail(NTTM_EINVAL, "internal: bad pass geometry");
-    const uint64_t tiles = plan_tiles(g, a.logn, a.batch);
+    JobSet js; memset(&js, 0, sizeof js);
+    js.n = 1;
+    PassJob &j = js.j[0];
+    j.x = a.x; j.limbs = a.limbs; j.nlimbs = a.nlimbs; j.ldesc = a.ldesc; j.which = a.which;
+    j.do_in_scale = a.do_in_scale; j.in_scale = a.in_scale;
+    j.batch = a.batch; j.p = a.pk.p; j.pinv = a.pk.pinv; j.tw = a.tw;
+    return js;
+}
+/* one pass over a's plane, or (js) over the plane of each job with a's geometry and flags: a.limbs / a.ldesc then only
+ * say whether the jobs read limbs */
+int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s, const JobSet *jobs)
+{
+    const JobSet js = jobs ? *jobs : job_of(a);
+    if (js.n < 1 || js.n > NTTM_MAX_JOBS) return nttm_fail(NTTM_EINVAL, "internal: %d jobs", js.n);
+    uint64_t tiles = 0;                                            /* of the largest job */
+    double pts = 0, lbytes = 0;
+    for (int k = 0; k < js.n; k++) {
+        if (!pass_geom_ok(g, a.logn, js.j[k].batch)) return nttm_fail(NTTM_EINVAL, "internal: bad pass geometry");
+        const uint64_t t = plan_tiles(g, a.logn, js.j[k].batch);
+        tiles = t > tiles ? t : tiles;
+        pts += (double)(js.j[k].batch << a.logn);
+        lbytes += 8.0 * (double)(js.j[k].ldesc ? 0 : js.j[k].nlimbs);
+    }
     if (tiles > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "internal: too many tiles");
     PassArgs b = a; b.lo = g.lo; b.m = g.m; b.logw = g.logw; b.logh = g.logh;
     const bool limb = !inv && (b.limbs || b.ldesc);
     const int mode = !inv ? (limb ? PM_FWD_LIMB : PM_FWD) : (b.y ? PM_INV_PW : PM_INV);
-    const double pts = (double)(a.batch << a.logn);
     /* algorithmic bytes: read and write the plane once (16 B per point), plus the y plane of a fused pointwise (8 B);
      * a limb-input pass reads the limbs (8 B per point of operand) instead of the plane */
-    const double bytes = mode == PM_FWD_LIMB ? pts * 8.0 + 8.0 * (double)(b.ldesc ? 0 : b.nlimbs)
+    const double bytes = mode == PM_FWD_LIMB ? pts * 8.0 + lbytes
                        : pts * (mode == PM_INV_PW ? 24.0 : 16.0);
     static const char *names[4] = {"k_pass<fwd>", "k_pass<fwd,limb>", "k_pass<inv>", "k_pass<inv,pw>"};
     prof_begin(names[mode], bytes, s);
@@ -1058,20 +1116,20 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s)
     const int ppt = (T >= 64 * g_pts && T <= 512 * g_pts) ? g_pts : PASS_PTS;
     const unsigned nthr = (unsigned)(T / ppt < 64 ? 64 : T / ppt);
     if (nthr > 512) return nttm_fail(NTTM_EINVAL, "internal: %u threads per tile", nthr);
-    const dim3 grid((unsigned)tiles), blk(nthr);
+    const dim3 grid((unsigned)tiles, (unsigned)js.n), blk(nthr);
     const size_t lds = (size_t)LDS_WORDS(T) * sizeof(double);
 #define NTTM_PASS_LAUNCH(P) \
     switch (mode) { \
-    case PM_FWD: hipLaunchKernelGGL((k_pass<PM_FWD, P>), grid, blk, lds, s, b); break; \
-    case PM_FWD_LIMB: hipLaunchKernelGGL((k_pass<PM_FWD_LIMB, P>), grid, blk, lds, s, b); break; \
-    case PM_INV: hipLaunchKernelGGL((k_pass<PM_INV, P>), grid, blk, lds, s, b); break; \
-    default: hipLaunchKernelGGL((k_pass<PM_INV_PW, P>), grid, blk, lds, s, b); break; }
+    case PM_FWD: hipLaunchKernelGGL((k_pass<PM_FWD, P>), grid, blk, lds, s, b, js); break; \
+    case PM_FWD_LIMB: hipLaunchKernelGGL((k_pass<PM_FWD_LIMB, P>), grid, blk, lds, s, b, js); break; \
+    case PM_INV: hipLaunchKernelGGL((k_pass<PM_INV, P>), grid, blk, lds, s, b, js); break; \
+    default: hipLaunchKernelGGL((k_pass<PM_INV_PW, P>), grid, blk, lds, s, b, js); break; }
 #define NTTM_PASS_LAUNCH_G(P, M, W, H) \
     switch (mode) { \
-    case PM_FWD: hipLaunchKernelGGL((k_pass<PM_FWD, P, M, W, H>), grid, blk, lds, s, b); break; \
-    case PM_FWD_LIMB: hipLaunchKernelGGL((k_pass<PM_FWD_LIMB, P, M, W, H>), grid, blk, lds, s, b); break; \
-    case PM_INV: hipLaunchKernelGGL((k_pass<PM_INV, P, M, W, H>), grid, blk, lds, s, b); break; \
-    default: hipLaunchKernelGGL((k_pass<PM_INV_PW, P, M, W, H>), grid, blk, lds, s, b); break; }
+    case PM_FWD: hipLaunchKernelGGL((k_pass<PM_FWD, P, M, W, H>), grid, blk, lds, s, b, js); break; \
+    case PM_FWD_LIMB: hipLaunchKernelGGL((k_pass<PM_FWD_LIMB, P, M, W, H>), grid, blk, lds, s, b, js); break; \
+    case PM_INV: hipLaunchKernelGGL((k_pass<PM_INV, P, M, W, H>), grid, blk, lds, s, b, js); break; \
+    default: hipLaunchKernelGGL((k_pass<PM_INV_PW, P, M, W, H>), grid, blk, lds, s, b, js); break; }
     /* the strided tile shapes of large transforms, compiled with their geometry fixed */
     const bool fixed = g_fixed_shapes && g.logh == 0 && T >= PASS_PTS;
     /* the streamed shapes: strided 2^13-point tiles of 1 to 9-bit rows (2^(13 - m) columns), limbs from one operand
@@ -1083,12 +1141,14 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s)
     if ((b.dfr_out && (!stream || mode != PM_FWD_LIMB)) || (b.dfr_in && (!stream || mode != PM_FWD || g.m < 4)))
         return nttm_fail(NTTM_EINVAL, "internal: deferred boundary twiddles on a pass that does not stream");
     if (stream) {
-        const unsigned nb = (unsigned)(tiles < (uint64_t)g_ncu ? tiles : (uint64_t)g_ncu);
-        const uint32_t nt = (uint32_t)tiles;
+        /* one block per CU in all (a block holds nearly all of its CU's LDS), shared between the jobs */
+        const unsigned per = (unsigned)(g_ncu > js.n ? g_ncu / js.n : 1);
+        const unsigned nb = (unsigned)(tiles < (uint64_t)per ? tiles : (uint64_t)per);
+        const dim3 sgrid(nb, (unsigned)js.n);
 #define NTTM_STREAM_LAUNCH(M, W) \
-        if (mode == PM_FWD) hipLaunchKernelGGL((k_pass_stream<PM_FWD, M, W>), dim3(nb), dim3(STREAM_T), 0, s, b, nt); \
-        else if (mode == PM_FWD_LIMB) hipLaunchKernelGGL((k_pass_stream<PM_FWD_LIMB, M, W>), dim3(nb), dim3(STREAM_T), 0, s, b, nt); \
-        else hipLaunchKernelGGL((k_pass_stream<PM_INV, M, W>), dim3(nb), dim3(STREAM_T), 0, s, b, nt);
+        if (mode == PM_FWD) hipLaunchKernelGGL((k_pass_stream<PM_FWD, M, W>), sgrid, dim3(STREAM_T), 0, s, b, js); \
+        else if (mode == PM_FWD_LIMB) hipLaunchKernelGGL((k_pass_stream<PM_FWD_LIMB, M, W>), sgrid, dim3(STREAM_T), 0, s, b, js); \
+        else hipLaunchKernelGGL((k_pass_stream<PM_INV, M, W>), sgrid, dim3(STREAM_T), 0, s, b, js);
         switch (g.m) {
         case 1: NTTM_STREAM_LAUNCH(1, 12) break;
         case 2: NTTM_STREAM_LAUNCH(2, 11) break;
@@ -1143,19 +1203,21 @@ int nttm_run_fused(const PassArgs &a, const PassGeom &g, hipStream_t s)
     return nttm_hip_check(hipGetLastError(), "k_fused launch");
 }
 
-/* the double-fused last pass: a = A's pass arguments (x = A's plane), bq = B's (x = B's plane before its last pass) */
-int nttm_run_fused2(const PassArgs &a, const PassArgs &bq, const PassGeom &g, hipStream_t s)
+/* the double-fused last pass of every prime of js: a = A's common arguments (its operand where a transform is a single
+ * pass: limbs or descriptors; a.ymode and a.scale unused), fb = B's */
+int nttm_run_fused2(const PassArgs &a, const FusedB &fb, const PassGeom &g, hipStream_t s, const FusedSet &js)
 {
+    if (js.n < 1 || js.n > NTTM_MAX_PRIMES) return nttm_fail(NTTM_EINVAL, "internal: %d primes in one pass", js.n);
+    for (int k = 0; k < js.n; k++)
+        if (!js.j[k].x || !js.j[k].xb) return nttm_fail(NTTM_EINVAL, "internal: double-fused pass without a plane");
     if (!pass_geom_ok(g, a.logn, a.batch) || g.lo != 0 || g.logw != 0 || g.m + g.logh > FUSED_LOG ||
-        g.m + g.logh < 4 || !bq.x || bq.logn != a.logn || bq.batch != a.batch || a.do_scale || a.bmap ||
-        (bq.bmap && (g.m + g.logh > a.logn || bq.limbs || bq.ldesc)))
+        g.m + g.logh < 4 || a.do_scale || a.bmap || (fb.bmap && (g.m + g.logh > a.logn || fb.limbs || fb.ldesc)))
         return nttm_fail(NTTM_EINVAL, "internal: bad double-fused pass geometry");
     const uint64_t tiles = plan_tiles(g, a.logn, a.batch);
     if (tiles > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "internal: too many tiles");
     PassArgs A = a; A.lo = 0; A.m = g.m; A.logw = 0; A.logh = g.logh;
-    PassArgs Bq = bq; Bq.lo = 0; Bq.m = g.m; Bq.logw = 0; Bq.logh = g.logh;
-    const double pts = (double)(a.batch << a.logn);
-    const bool alimb = A.limbs || A.ldesc, blimb = Bq.limbs || Bq.ldesc;
+    const double pts = (double)js.n * (double)(a.batch << a.logn);
+    const bool alimb = A.limbs || A.ldesc, blimb = fb.limbs || fb.ldesc;
     /* read A (or its limbs), read B (or its limbs), write A */
     prof_begin("k_fused2", pts * (24.0 - (alimb ? 8.0 : 0.0) - (blimb ? 8.0 : 0.0)), s);
     const int T = 1 << (g.m + g.logh);
@@ -1167,29 +1229,29 @@ int nttm_run_fused2(const PassArgs &a, const PassArgs &bq, const PassGeom &g, hi
      * transforms of 2^8 and 2^9 points from the limbs in tiles of 16 and 8 blocks (8 points per thread) */
     const bool fixed_shape = g_fixed_shapes && g.m + g.logh == FUSED_LOG && (g.m >= 10 || (g.m >= 8 && ppt == 8));
     const bool fixed = fixed_shape && !alimb && !blimb && g.m >= 10;
-    const dim3 grid((unsigned)tiles), blk(nthr);
+    const dim3 grid((unsigned)tiles, (unsigned)js.n), blk(nthr);
     if (fixed_shape && !fixed && (alimb || blimb)) {            /* a single-pass transform: both operands from limbs */
         if (ppt == 8) {
-            if (g.m == 12) hipLaunchKernelGGL((k_fused2<8, 12, 0, true>), grid, blk, 0, s, A, Bq);
-            else if (g.m == 11) hipLaunchKernelGGL((k_fused2<8, 11, 1, true>), grid, blk, 0, s, A, Bq);
-            else if (g.m == 10) hipLaunchKernelGGL((k_fused2<8, 10, 2, true>), grid, blk, 0, s, A, Bq);
-            else if (g.m == 9) hipLaunchKernelGGL((k_fused2<8, 9, 3, true>), grid, blk, 0, s, A, Bq);
-            else hipLaunchKernelGGL((k_fused2<8, 8, 4, true>), grid, blk, 0, s, A, Bq);
+            if (g.m == 12) hipLaunchKernelGGL((k_fused2<8, 12, 0, true>), grid, blk, 0, s, A, fb, js);
+            else if (g.m == 11) hipLaunchKernelGGL((k_fused2<8, 11, 1, true>), grid, blk, 0, s, A, fb, js);
+            else if (g.m == 10) hipLaunchKernelGGL((k_fused2<8, 10, 2, true>), grid, blk, 0, s, A, fb, js);
+            else if (g.m == 9) hipLaunchKernelGGL((k_fused2<8, 9, 3, true>), grid, blk, 0, s, A, fb, js);
+            else hipLaunchKernelGGL((k_fused2<8, 8, 4, true>), grid, blk, 0, s, A, fb, js);
         } else {
-            if (g.m == 12) hipLaunchKernelGGL((k_fused2<PASS_PTS, 12, 0, true>), grid, blk, 0, s, A, Bq);
-            else if (g.m == 11) hipLaunchKernelGGL((k_fused2<PASS_PTS, 11, 1, true>), grid, blk, 0, s, A, Bq);
-            else hipLaunchKernelGGL((k_fused2<PASS_PTS, 10, 2, true>), grid, blk, 0, s, A, Bq);
+            if (g.m == 12) hipLaunchKernelGGL((k_fused2<PASS_PTS, 12, 0, true>), grid, blk, 0, s, A, fb, js);
+            else if (g.m == 11) hipLaunchKernelGGL((k_fused2<PASS_PTS, 11, 1, true>), grid, blk, 0, s, A, fb, js);
+            else hipLaunchKernelGGL((k_fused2<PASS_PTS, 10, 2, true>), grid, blk, 0, s, A, fb, js);
         }
     } else if (fixed && ppt == 8) {
-        if (g.m == 12) hipLaunchKernelGGL((k_fused2<8, 12, 0, false>), grid, blk, 0, s, A, Bq);
-        else if (g.m == 11) hipLaunchKernelGGL((k_fused2<8, 11, 1, false>), grid, blk, 0, s, A, Bq);
-        else hipLaunchKernelGGL((k_fused2<8, 10, 2, false>), grid, blk, 0, s, A, Bq);
+        if (g.m == 12) hipLaunchKernelGGL((k_fused2<8, 12, 0, false>), grid, blk, 0, s, A, fb, js);
+        else if (g.m == 11) hipLaunchKernelGGL((k_fused2<8, 11, 1, false>), grid, blk, 0, s, A, fb, js);
+        else hipLaunchKernelGGL((k_fused2<8, 10, 2, false>), grid, blk, 0, s, A, fb, js);
     } else if (fixed) {
-        if (g.m == 12) hipLaunchKernelGGL((k_fused2<PASS_PTS, 12, 0, false>), grid, blk, 0, s, A, Bq);
-        else if (g.m == 11) hipLaunchKernelGGL((k_fused2<PASS_PTS, 11, 1, false>), grid, blk, 0, s, A, Bq);
-        else hipLaunchKernelGGL((k_fused2<PASS_PTS, 10, 2, false>), grid, blk, 0, s, A, Bq);
-    } else if (ppt == 8) hipLaunchKernelGGL((k_fused2<8>), grid, blk, 0, s, A, Bq);
-    else hipLaunchKernelGGL((k_fused2<PASS_PTS>), grid, blk, 0, s, A, Bq);
+        if (g.m == 12) hipLaunchKernelGGL((k_fused2<PASS_PTS, 12, 0, false>), grid, blk, 0, s, A, fb, js);
+        else if (g.m == 11) hipLaunchKernelGGL((k_fused2<PASS_PTS, 11, 1, false>), grid, blk, 0, s, A, fb, js);
+        else hipLaunchKernelGGL((k_fused2<PASS_PTS, 10, 2, false>), grid, blk, 0, s, A, fb, js);
+    } else if (ppt == 8) hipLaunchKernelGGL((k_fused2<8>), grid, blk, 0, s, A, fb, js);
+    else hipLaunchKernelGGL((k_fused2<PASS_PTS>), grid, blk, 0, s, A, fb, js);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_fused2 launch");
 }
@@ -1226,28 +1288,30 @@ int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_load launch");
 }
-/* the radix-3 layer of batch transforms of 3 2^logk points (logk >= 1): forward (from the plane or from limbs) or
- * inverse, in place */
-int nttm_run_r3(bool inv, double *x, uint64_t batch, int logk, const PrimeK &pk, const double2 *b3,
-                const uint64_t *limbs, uint64_t nlimbs, const LoadDesc *ldesc, int which, const double2 *scale,
-                hipStream_t s)
+/* the radix-3 layer of the jobs' transforms of 3 2^logk points (logk >= 1): forward (from the planes, or every job from
+ * limbs) or inverse, in place.  A job: x, batch (transforms of 3 2^logk points), its operand, pk, tw.b3 (the direction's
+ * table) and the scale of every output in in_scale */
+int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s)
 {
-    if (logk < 1 || logk > NTTM_LOGN_MAX || !batch) return nttm_fail(NTTM_EINVAL, "internal: radix-3 layer of 3 2^%d", logk);
-    if (inv && (limbs || ldesc)) return nttm_fail(NTTM_EINVAL, "internal: inverse radix-3 layer from limbs");
-    if (limbs && batch != 1) return nttm_fail(NTTM_EINVAL, "internal: one limb operand for %llu transforms",
-                                              (unsigned long long)batch);
-    R3Args a; memset(&a, 0, sizeof a);
-    a.x = x; a.batch = batch; a.logk = logk; a.pk = pk; a.b3 = b3;
-    a.limbs = limbs; a.nlimbs = nlimbs; a.ldesc = ldesc; a.which = which;
-    a.do_scale = scale != nullptr; a.scale = scale ? *scale : make_double2(1.0, 0.0);
-    const bool limb = limbs || ldesc;
-    const uint64_t pts = 3 * (batch << logk);
-    prof_begin(inv ? "k_r3_inv" : limb ? "k_r3_fwd<limb>" : "k_r3_fwd",
-               limb ? 8.0 * (double)pts + 8.0 * (double)(ldesc ? 0 : nlimbs) : 16.0 * (double)pts, s);
-    const unsigned grid = grid_for(batch << logk);
-    if (inv) hipLaunchKernelGGL(k_r3_inv, dim3(grid), dim3(NTTM_THREADS), 0, s, a);
-    else if (limb) hipLaunchKernelGGL(k_r3_fwd<true>, dim3(grid), dim3(NTTM_THREADS), 0, s, a);
-    else hipLaunchKernelGGL(k_r3_fwd<false>, dim3(grid), dim3(NTTM_THREADS), 0, s, a);
+    if (js.n < 1 || js.n > NTTM_MAX_JOBS || logk < 1 || logk > NTTM_LOGN_MAX) return nttm_fail(NTTM_EINVAL, "internal: radix-3 layer of 3 2^%d", logk);
+    const bool limb = js.j[0].limbs || js.j[0].ldesc;
+    uint64_t most = 0;
+    double bytes = 0;
+    for (int k = 0; k < js.n; k++) {
+        const PassJob &j = js.j[k];
+        if (!j.batch || (j.limbs || j.ldesc) != limb) return nttm_fail(NTTM_EINVAL, "internal: radix-3 layer's jobs");
+        if (inv && limb) return nttm_fail(NTTM_EINVAL, "internal: inverse radix-3 layer from limbs");
+        if (j.limbs && j.batch != 1) return nttm_fail(NTTM_EINVAL, "internal: one limb operand for %llu transforms",
+                                                      (unsigned long long)j.batch);
+        most = j.batch > most ? j.batch : most;
+        const double pts = 3.0 * (double)(j.batch << logk);
+        bytes += limb ? 8.0 * pts + 8.0 * (double)(j.ldesc ? 0 : j.nlimbs) : 16.0 * pts;
+    }
+    prof_begin(inv ? "k_r3_inv" : limb ? "k_r3_fwd<limb>" : "k_r3_fwd", bytes, s);
+    const dim3 grid(grid_for(most << logk), (unsigned)js.n);
+    if (inv) hipLaunchKernelGGL(k_r3_inv, grid, dim3(NTTM_THREADS), 0, s, logk, js);
+    else if (limb) hipLaunchKernelGGL(k_r3_fwd<true>, grid, dim3(NTTM_THREADS), 0, s, logk, js);
+    else hipLaunchKernelGGL(k_r3_fwd<false>, grid, dim3(NTTM_THREADS), 0, s, logk, js);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_r3 launch");
 }

@@ -1,0 +1,87 @@
+"""The launch schedules of a product give one result: every prime and both operands in one launch per pass, or prime
+after prime (NTTM_PAR_POINTS=0), and a batch group whole or in chunks through the same planes (NTTM_CHUNK_POINTS), with
+shared B operands inside a chunk and across chunks, radix-3 lengths and four primes.  Products are compared with the
+oracle, limb for limb."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle as O
+from gpu_util import dev, host, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def schedule(nttm):
+    import torch
+
+    def set_(par=None, chunk=None, **cfg):
+        for k, v in (("NTTM_PAR_POINTS", par), ("NTTM_CHUNK_POINTS", chunk)):
+            if v is None:
+                os.environ.pop(k, None)
+            else:
+                os.environ[k] = str(v)
+        torch.cuda.synchronize()
+        nttm.shutdown()
+        nttm.init(0, **cfg)
+        return nttm
+    yield set_
+    set_()
+
+
+# a single pass, two passes at the smallest strided rows, 9-bit rows, three passes with deferred twiddles, 3 2^k
+@pytest.mark.parametrize("na,nb", [(2049, 2047), (4097, 1), (5000, 3193), (700001, 300001), (1 << 21, 2097151)])
+@pytest.mark.parametrize("cfg", [dict(), dict(radix3=2), dict(nprimes=4), dict(tile_log=12, pts=8)])
+def test_product_schedules(schedule, na, nb, cfg):
+    a, s = O.gen_limbs(na, na + nb)
+    b, _ = O.gen_limbs(nb, s)
+    da, db = dev(a), dev(b)
+    say("schedules", na, nb, cfg)
+    together = host(schedule(**cfg).mul(da, db))
+    apart = host(schedule(par=0, **cfg).mul(da, db))
+    assert np.array_equal(together, apart)
+    if na * nb <= 20_000_000:
+        assert np.array_equal(together, O.mul_school(a, b))
+    else:
+        assert O.tref_res(a, b, together)
+
+
+@pytest.mark.parametrize("chunk", [1, 3 << 13, 1 << 15, 1 << 17])
+@pytest.mark.parametrize("cfg", [dict(), dict(radix3=2)])
+def test_group_chunks(schedule, chunk, cfg):
+    """11 products of about 2^14 points and 7 of about 2^12, most in pairs with one B: chunks of one product, of an odd
+    number of them (a pair split between two chunks) and of all"""
+    import torch
+    rng = np.random.default_rng(chunk)
+    ops, s = [], 99
+    for i in range(18):
+        lo, hi = (7000, 9000) if i < 11 else (1500, 2100)
+        a, s = O.gen_limbs(int(rng.integers(lo, hi)), s)
+        if i % 2 == 0:
+            b, s = O.gen_limbs(int(rng.integers(lo - 1000, hi - 1000)), s)
+            db = dev(b)
+        x = None
+        if i % 3 == 0:
+            x, s = O.gen_limbs(int(rng.integers(1, len(a) + len(b) + 1)), s)
+        ops.append((a, b, x, db))
+    say("chunks", chunk, cfg)
+    n = schedule(chunk=chunk, **cfg)
+    items = [(dev(a), db, None if x is None else dev(x),
+              torch.full((len(a) + len(b) + (x is not None),), -1, dtype=torch.int64, device="cuda"))
+             for a, b, x, db in ops]
+    prods = n.make_prods(items)
+    n.mul_batch(prods)
+    plan = n.BatchPlan(prods, autotune=False)
+    eager = [host(it[3]) for it in items]
+    for _ in range(2):
+        for it in items:
+            it[3].fill_(-1)
+        plan.run()
+        lens = plan.ncn()
+        for (a, b, x, _), it, c, ln, pr in zip(ops, items, eager, lens, prods):
+            want = O.mul_school(a, b, x)
+            assert np.array_equal(c, want) and np.array_equal(host(it[3]), want)
+            assert ln == pr.ncn == int(np.nonzero(want)[0][-1]) + 1
+    plan.close()
