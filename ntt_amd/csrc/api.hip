@@ -35,13 +35,14 @@ int nttm_run_load_planes(double *dst, uint64_t plane, const uint64_t *src, uint6
                          const PrimeK *pk, const double2 *scale, int out_u64, hipStream_t s);
 int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which, uint64_t count, int logn, int np,
                         const PrimeK *pk, const double2 *scale, hipStream_t s);
-int nttm_crt_launch_batch(const void *desc_dev, uint64_t nprod, uint64_t nblocks, int np, const CrtConst &cc,
-                          uint32_t *scratch, hipStream_t s, double alg_bytes, int per = 8);
-/* the two halves of nttm_crt_launch_batch: the limbs of products whose blocks are [blk0, blk0 + nblk) of the launch's
- * block numbering, for a carry in of 0; then every block's carry */
-int nttm_crt_launch_limbs(const void *desc_dev, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np, const CrtConst &cc,
-                          uint32_t *scratch, hipStream_t s, double alg_bytes, int per);
-int nttm_crt_launch_carry(const void *desc_dev, uint64_t nprod, uint64_t nblocks, uint32_t *scratch, hipStream_t s, int per);
+/* the CRT of products whose blocks are [blk0, blk0 + nblk) of the launch's block numbering (limbs for a carry in of 0),
+ * then every block's carry; nttm_crt_launch_one: both for one product */
+int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np,
+                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp = nullptr);
+int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t nblocks, uint32_t *scratch,
+                          uint32_t *ctl, hipStream_t s, int per, uint64_t *stamp = nullptr);
+int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtConst &cc, uint32_t *scratch, uint32_t *ctl,
+                        hipStream_t s, double alg_bytes, uint64_t *stamps = nullptr);
 uint64_t nttm_crt_blocks(uint64_t nc, int per = 8);      /* per: CRT limbs per thread, 8 (2048-limb blocks) or 1 (256) */
 uint64_t nttm_crt_scratch_words(uint64_t nblocks);
 int nttm_run_norm(const void *desc_dev, uint64_t nprod, uint64_t *ncn_dev, hipStream_t s);
@@ -49,7 +50,7 @@ int nttm_run_fill_x(const void *desc_dev, uint64_t nprod, hipStream_t s);
 int nttm_run_dft16_mfma(const uint64_t *x, double *y, int logn, uint64_t batch, const void *etab, const double *tlo,
                         const double *thi, const double *consts, double p, hipStream_t s);
 int nttm_run_add_carry(uint64_t *c, uint64_t n, const uint64_t *carry, hipStream_t s);
-int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s);
+int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *stamp = nullptr);
 
 /* ---- errors ----------------------------------------------------------------------------------------------------- */
 /* per host thread: the library's own helper threads (the e pipeline's download preparation) may fail too */
@@ -123,6 +124,7 @@ struct Ctx {
     hipEvent_t ev[4];
     hipEvent_t pev[2 * NTTM_MAX_PRIMES];      /* around B's transform of each prime (phase times of nttm_mul) */
     double last_ms[3];
+    uint64_t *stamps; int last_stamped;      /* pinned: the device clock at the last short product's phase boundaries */
 };
 static Ctx g;
 static uint64_t g_init_count;
@@ -422,6 +424,7 @@ extern "C" int nttm_init(int device, const nttm_config *cfg)
     for (int i = 0; i < 4; i++) HIPCK(hipEventCreate(&g.ev[i]));
     for (int i = 0; i < 2 * NTTM_MAX_PRIMES; i++) HIPCK(hipEventCreate(&g.pev[i]));
     RCK(hpin_need(1 << 16));
+    HIPCK(hipHostMalloc((void **)&g.stamps, 64, hipHostMallocDefault));
     {
         const char *e = getenv("NTTM_NO_DEFER");
         g_no_defer = e && e[0] == '1';
@@ -461,6 +464,7 @@ extern "C" void nttm_shutdown(void)
     if (g.tpin) (void)hipHostFree(g.tpin);
     if (g.tables) (void)hipFree(g.tables);
     if (g.hpin) (void)hipHostFree(g.hpin);
+    if (g.stamps) (void)hipHostFree(g.stamps);
     if (g.stage) (void)hipFree(g.stage);
     if (g.chk) (void)hipFree(g.chk);
     if (g.bounce) (void)hipHostFree(g.bounce);
@@ -512,16 +516,6 @@ static int inv_planes(int prime, double *x, const double *y, int ymode, int logn
 }
 
 /* ---- the product ------------------------------------------------------------------------------------------------------- */
-struct CrtDesc {                 /* must match crt.hip */
-    const double *pl; uint64_t plane;
-    uint64_t ncoef;
-    const uint64_t *x; uint64_t nx;
-    uint64_t *c; uint64_t nc;
-    uint64_t first_block;
-    uint64_t trunc;
-};
-static_assert(sizeof(CrtDesc) <= 96, "a product's pinned slot holds its CRT descriptor below byte 96");
-
 static int choose_np(size_t mn, int *np)
 {
     int want = g.cfg.nprimes;
@@ -575,7 +569,8 @@ static void product_plan(Plan *pl, int logn, uint64_t batch, int tile_log)
  * to back.  After it, A holds the cyclic convolutions mod each prime, natural order.
  * Shared B operands (bmap non-null): B's plane holds the cnt_b distinct operands of ldesc_b; A's engine transform t
  * pairs with B's engine transform bmap[t] in the double-fused pass.
- * pev (or null): 2 np events recorded around B's transform of each prime. */
+ * pev (or null): 2 np events recorded around B's transform of each prime.  stamps (or null): the device clock at the
+ * start of the first forward launch and of the double-fused pass. */
 /* the first forward pass (from limbs) leaves its boundary twiddles to the second when both are streamed strided
  * passes (a transform of three or more passes): the limb pass has no VALU to spare, the second pass, bound by HBM, has.
  * q: the first pass's arguments (limbs set, in_scale as the caller wants it applied) */
@@ -604,7 +599,7 @@ static PassJob prime_job(int i, double *x, uint64_t batch, bool inv)
 static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A, double *Bp, uint64_t bstride,
                               const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb, const LoadDesc *ldesc,
                               hipStream_t s, hipEvent_t *pev, uint64_t cnt_b = 0, const LoadDesc *ldesc_b = nullptr,
-                              const uint32_t *bmap = nullptr)
+                              const uint32_t *bmap = nullptr, uint64_t *stamps = nullptr)
 {
     if (!bmap) { cnt_b = cnt; ldesc_b = ldesc; }
     const uint64_t tb = r3 ? 3 * cnt : cnt, tbb = r3 ? 3 * cnt_b : cnt_b;   /* engine transforms of 2^logn points */
@@ -614,8 +609,8 @@ static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A,
     const int last = pl.npass - 1;
     if (bmap && (plb.npass != pl.npass || pl.p[last].m + pl.p[last].logh > logn || (last == 0 && !r3)))
         return nttm_fail(NTTM_EINVAL, "internal: shared B operands on this length");
-    /* both operands' strided passes in one launch where their geometry is the same (it differs only in the blocks a
-     * tile spans, by the powers of two in the two batch counts) */
+    /* both operands' strided passes in one launch where every prime is too, and where their geometry is the same (it
+     * differs only in the blocks a tile spans, by the powers of two in the two batch counts) */
     bool pair = bstride > 0;
     for (int j = 0; j < last; j++) if (memcmp(&pl.p[j], &plb.p[j], sizeof(PassGeom))) pair = false;
     const int step = bstride ? np : 1;
@@ -639,12 +634,13 @@ static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A,
         }
         /* the forward passes but the last, of the given jobs; the first reads the operand limbs (a radix-3 layer does
          * where there is one).  j0: the jobs as the caller set them up */
-        auto forward = [&](JobSet js, const Plan &q) -> int {
+        auto forward = [&](JobSet js, const Plan &q, uint64_t *stamp) -> int {
             auto limbs_done = [&]() { for (int k = 0; k < js.n; k++) { PassJob &j = js.j[k]; j.limbs = nullptr; j.ldesc = nullptr; j.do_in_scale = 0; } };
             if (r3) {
                 JobSet r = js;
                 for (int k = 0; k < r.n; k++) r.j[k].batch /= 3;
-                RCK(nttm_run_r3(false, logn, r, s));
+                RCK(nttm_run_r3(false, logn, r, s, stamp));
+                stamp = nullptr;
                 limbs_done();
             }
             PassArgs f = base_args(i0, js.j[0].x, logn, js.j[0].batch, false);
@@ -652,6 +648,7 @@ static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A,
             const bool dfr = !r3 && defer_ok(f, q, last);
             for (int j = 0; j < last; j++) {
                 defer_set(f, q, j, dfr);
+                f.stamp = j == 0 ? stamp : nullptr;
                 if (dfr && j == 0) for (int k = 0; k < js.n; k++) js.j[k].dfr_do_scale = js.j[k].do_in_scale;
                 RCK(nttm_run_pass(false, f, q.p[j], s, &js));
                 f.limbs = nullptr; f.ldesc = nullptr;
@@ -663,17 +660,18 @@ static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A,
             JobSet all = jb;
             for (int k = 0; k < step; k++) all.j[all.n++] = ja.j[k];
             if (pev) HIPCK(hipEventRecord(pev[2 * i0], s));
-            RCK(forward(all, pl));
+            RCK(forward(all, pl, stamps));
             if (pev) HIPCK(hipEventRecord(pev[2 * i0 + 1], s));
         } else {
             if (pev) HIPCK(hipEventRecord(pev[2 * i0], s));
-            if (last > 0 || r3) RCK(forward(jb, plb));
+            if (last > 0 || r3) RCK(forward(jb, plb, stamps));
             if (pev) HIPCK(hipEventRecord(pev[2 * i0 + 1], s));
-            if (last > 0 || r3) RCK(forward(ja, pl));
+            if (last > 0 || r3) RCK(forward(ja, pl, nullptr));
         }
         /* B's last forward pass, A's last forward pass, the pointwise product and A's first inverse pass */
         PassArgs fa = base_args(i0, jf.j[0].x, logn, tb, false);
         FusedB fb{nullptr, 0, nullptr, bmap};
+        fa.stamp = stamps ? stamps + 1 : nullptr;
         if (last == 0 && !r3) {                                  /* a single-pass transform reads both operands here */
             fa.limbs = ldesc ? nullptr : a; fa.nlimbs = na; fa.ldesc = ldesc; fa.which = 0;
             fb.limbs = ldesc ? nullptr : b; fb.nlimbs = nb; fb.ldesc = ldesc;
@@ -772,7 +770,10 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
 /* c = a b (+ x), device pointers.  wcut: write only the low wcut limbs of the result (the value mod B^wcut; no check of
  * what lies above).  ws: the workspace (null: the library's, grown to fit; else ws_cap bytes of the caller's).
  * sync = 1: returns after the stream has drained and the CRT's flags are checked; sync = 0: returns after the launches,
- * the flags copied to pinned slot `slot` (g.hpin + 128 slot + 64, read by the caller after a synchronization). */
+ * the flags in pinned slot `slot` (g.hpin + 128 slot + 96, read by the caller after a synchronization).
+ * Nothing is copied in either direction: the CRT's descriptor goes with its launches, and the carry scan writes the flags
+ * straight to the pinned slot.  The phase times of a product whose primes run together come from the device clock
+ * (stamps in pinned memory): an event costs 2.2 us of the call, a copy 3 us. */
 static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b, size_t nb, const uint64_t *x, size_t nx,
                     hipStream_t s, size_t wcut = SIZE_MAX, char *ws = nullptr, size_t ws_cap = 0, int sync = 1,
                     size_t slot = 0)
@@ -798,31 +799,34 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
         ws = g.ws;
     }
     double *A = (double *)ws, *Bp = A + (size_t)L.np * L.n;
-    CrtDesc *ddesc = (CrtDesc *)(ws + L.off_desc);
     uint32_t *crt_scr = (uint32_t *)(ws + L.off_crt);
-    char *hs = (char *)g.hpin + 128 * slot;                       /* pinned: the descriptor, then (at 96) the flags */
+    uint32_t *ctl = (uint32_t *)((char *)g.hpin + 128 * slot + 96);
+    const bool events = sync && !L.par;
+    uint64_t *stamps = sync && L.par ? g.stamps : nullptr;
+    if (stamps) stamps[0] = ~(uint64_t)0;                        /* (a transform of one pass has no forward launch) */
 
-    if (sync) HIPCK(hipEventRecord(g.ev[0], s));
-    RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, L.par ? L.n : 0, a, na, b, nb, nullptr, s, sync ? g.pev : nullptr));
-    if (sync) HIPCK(hipEventRecord(g.ev[2], s));
+    if (events) HIPCK(hipEventRecord(g.ev[0], s));
+    RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, L.par ? L.n : 0, a, na, b, nb, nullptr, s, events ? g.pev : nullptr, 0,
+                           nullptr, nullptr, stamps));
+    if (events) HIPCK(hipEventRecord(g.ev[2], s));
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.pl = A; hd.plane = L.n; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
     hd.trunc = nc < nc_full;
-    memcpy(hs, &hd, sizeof hd);
-    HIPCK(hipMemcpyAsync(ddesc, hs, sizeof hd, hipMemcpyHostToDevice, s));
-    RCK(nttm_crt_launch_batch(ddesc, 1, nttm_crt_blocks(nc), L.np, g.cc, crt_scr, s,
-                              8.0 * L.np * (double)L.ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? (nx < nc ? nx : nc) : 0)));
-    if (sync) HIPCK(hipEventRecord(g.ev[3], s));
-    HIPCK(hipMemcpyAsync(hs + 96, crt_scr, 8, hipMemcpyDeviceToHost, s));
+    RCK(nttm_crt_launch_one(hd, nttm_crt_blocks(nc), L.np, g.cc, crt_scr, ctl, s,
+                            8.0 * L.np * (double)L.ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? (nx < nc ? nx : nc) : 0),
+                            stamps ? stamps + 2 : nullptr));
+    if (events) HIPCK(hipEventRecord(g.ev[3], s));
     if (!sync) return 0;
     HIPCK(hipStreamSynchronize(s));
-    float ms, tb = 0, t;
-    for (int i = 0; i < (L.par ? 1 : L.np); i++) { HIPCK(hipEventElapsedTime(&t, g.pev[2 * i], g.pev[2 * i + 1])); tb += t; }
-    if (L.par) tb *= 0.5f;                                       /* the forward launches hold both operands */
-    HIPCK(hipEventElapsedTime(&ms, g.ev[0], g.ev[2]));
-    g.last_ms[0] = tb; g.last_ms[1] = ms - tb;
-    HIPCK(hipEventElapsedTime(&ms, g.ev[2], g.ev[3])); g.last_ms[2] = ms;
-    const uint32_t flags = ((const uint32_t *)(hs + 96))[1];
+    g.last_stamped = stamps != nullptr;
+    if (events) {
+        float ms, tb = 0, t;
+        for (int i = 0; i < L.np; i++) { HIPCK(hipEventElapsedTime(&t, g.pev[2 * i], g.pev[2 * i + 1])); tb += t; }
+        HIPCK(hipEventElapsedTime(&ms, g.ev[0], g.ev[2]));
+        g.last_ms[0] = tb; g.last_ms[1] = ms - tb;
+        HIPCK(hipEventElapsedTime(&ms, g.ev[2], g.ev[3])); g.last_ms[2] = ms;
+    }
+    const uint32_t flags = ctl[1];
     if (flags & 1) return nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond the top limb (wrong residues)");
     return 0;
 }
@@ -870,15 +874,11 @@ int nttm_mul_cyclic(uint64_t *v, const uint64_t *a, size_t na, const uint64_t *b
     RCK(product_transforms(np, logn, r3, 1, A, Bp, par ? L : 0, a, na, b, nb, nullptr, s, nullptr));
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.pl = A; hd.plane = L; hd.ncoef = L; hd.c = v; hd.nc = nc;
-    char *hs = (char *)g.hpin;
-    memcpy(hs, &hd, sizeof hd);
-    HIPCK(hipMemcpyAsync(g.ws + off_desc, hs, sizeof hd, hipMemcpyHostToDevice, s));
-    uint32_t *crt_scr = (uint32_t *)(g.ws + off_crt);
-    RCK(nttm_crt_launch_batch(g.ws + off_desc, 1, nttm_crt_blocks(nc), np, g.cc, crt_scr, s, 8.0 * np * L + 8.0 * nc));
-    HIPCK(hipMemcpyAsync(hs + 96, crt_scr, 8, hipMemcpyDeviceToHost, s));
-    if (flag) { *flag = (const uint32_t *)(hs + 96) + 1; return 0; }
+    uint32_t *ctl = (uint32_t *)((char *)g.hpin + 96);            /* the flags, written by the carry scan */
+    RCK(nttm_crt_launch_one(hd, nttm_crt_blocks(nc), np, g.cc, (uint32_t *)(g.ws + off_crt), ctl, s, 8.0 * np * L + 8.0 * nc));
+    if (flag) { *flag = ctl + 1; return 0; }
     HIPCK(hipStreamSynchronize(s));
-    if (((const uint32_t *)(hs + 96))[1] & 1) return nttm_fail(NTTM_ECHECK, "cyclic product: crt: non-zero carry beyond the top limb");
+    if (ctl[1] & 1) return nttm_fail(NTTM_ECHECK, "cyclic product: crt: non-zero carry beyond the top limb");
     return 0;
 }
 
@@ -1057,6 +1057,14 @@ int nttm_mul_launch(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
 
 extern "C" int nttm_last_phase_ms(double *f, double *i, double *c)
 {
+    if (g.last_stamped) {                                        /* a product whose primes ran together */
+        int khz = 0;
+        if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g.dev) != hipSuccess || khz <= 0) { (void)hipGetLastError(); khz = 100000; }
+        const uint64_t *t = g.stamps;
+        auto ms = [&](uint64_t a, uint64_t b) { return b > a ? (double)(b - a) / khz : 0.0; };
+        const double fwd = ms(t[0], t[1]);                       /* both operands' forward passes, one launch each */
+        g.last_ms[0] = 0.5 * fwd; g.last_ms[1] = 0.5 * fwd + ms(t[1], t[2]); g.last_ms[2] = ms(t[2], t[3]);
+    }
     if (f) *f = g.last_ms[0];
     if (i) *i = g.last_ms[1];
     if (c) *c = g.last_ms[2];
@@ -1178,11 +1186,12 @@ static int group_launch(const GroupBuild &gb, int np, double *A, char *dbase, hi
         rc = product_transforms(np, gb.logn, gb.r3, ch.cn, A, Bp, gb.merged ? ch.cnb * gb.n : 0, nullptr, 0, nullptr, 0, ld, s,
                                 nullptr, ch.cnb, gb.share ? (const LoadDesc *)(dbase + gb.off_ldb) + ch.b0 : nullptr,
                                 gb.share ? (const uint32_t *)(dbase + gb.off_bmap) + (gb.r3 ? 3 : 1) * ch.c0 : nullptr);
-        if (!rc) rc = nttm_crt_launch_limbs((const CrtDesc *)(dbase + gb.off_cd) + ch.c0, ch.cn, ch.blk0, ch.nblk, np, g.cc,
-                                            (uint32_t *)(dbase + gb.off_crt), s, ch.crt_bytes, gb.crt_per);
+        if (!rc) rc = nttm_crt_launch_limbs((const CrtDesc *)(dbase + gb.off_cd) + ch.c0, nullptr, ch.cn, ch.blk0, ch.nblk, np,
+                                            g.cc, (uint32_t *)(dbase + gb.off_crt), s, ch.crt_bytes, gb.crt_per);
         if (rc) break;
     }
-    if (!rc) rc = nttm_crt_launch_carry(dbase + gb.off_cd, gb.cnt, gb.nblk, (uint32_t *)(dbase + gb.off_crt), s, gb.crt_per);
+    uint32_t *scr = (uint32_t *)(dbase + gb.off_crt);
+    if (!rc) rc = nttm_crt_launch_carry((const CrtDesc *)(dbase + gb.off_cd), nullptr, gb.cnt, gb.nblk, scr, scr, s, gb.crt_per);
     if (!rc && norm) rc = nttm_run_norm(dbase + gb.off_cd, gb.cnt, (uint64_t *)(dbase + gb.off_ncn), s);
     g.cfg.tile_log = tile0; nttm_set_pts(pts0);
     return rc;
@@ -2199,16 +2208,11 @@ extern "C" int nttm_crt(uint64_t *c, size_t nc, const uint64_t *const *planes, i
     }
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.pl = pl; hd.plane = ncoef; hd.ncoef = ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
+    uint32_t *ctl = (uint32_t *)((char *)g.hpin + 96);
+    RCK(nttm_crt_launch_one(hd, nttm_crt_blocks(nc), np, g.cc, (uint32_t *)(g.ws + pbytes + 256), ctl, s,
+                            8.0 * np * (double)ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? nx : 0)));
     HIPCK(hipStreamSynchronize(s));
-    memcpy(g.hpin, &hd, sizeof hd);
-    CrtDesc *dd = (CrtDesc *)(g.ws + pbytes);
-    uint32_t *crt_scr = (uint32_t *)(g.ws + pbytes + 256);
-    HIPCK(hipMemcpyAsync(dd, g.hpin, sizeof hd, hipMemcpyHostToDevice, s));
-    RCK(nttm_crt_launch_batch(dd, 1, nttm_crt_blocks(nc), np, g.cc, crt_scr, s,
-                              8.0 * np * (double)ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? nx : 0)));
-    HIPCK(hipMemcpyAsync(g.hpin + 64, crt_scr, 8, hipMemcpyDeviceToHost, s));
-    HIPCK(hipStreamSynchronize(s));
-    const uint32_t flags = ((const uint32_t *)(g.hpin + 64))[1];
+    const uint32_t flags = ctl[1];
     if (flags & 1) return nttm_fail(NTTM_ECHECK, "crt: the value needs more than nc limbs");
     return 0;
 }

@@ -19,6 +19,7 @@
  * per stripe and merges the spills serially on the host or on one thread per product (E/rns_mul.c:452-470;
  * E/dbig.c:1007-1052).  The final carry beyond limb nc-1 must be zero; a non-zero one sets an error flag.
  */
+#include <string.h>
 #include "internal.h"
 
 #define CRT_T 256
@@ -34,19 +35,12 @@
 #define CRT_ST_FIRST (1u << 5)
 #define CRT_SCAN_T 1024
 
-struct CrtDesc {                         /* one product; must match api.hip */
-    const double *pl; uint64_t plane;    /* residues of prime j, coefficient k at pl[j * plane + k] */
-    uint64_t ncoef;
-    const uint64_t *x; uint64_t nx;
-    uint64_t *c; uint64_t nc;
-    uint64_t first_block;                /* the product's first block in the launch */
-    uint64_t trunc;                      /* nonzero: c is the value mod B^nc (nothing above it is checked) */
-};
 struct CrtArgs {
-    const CrtDesc *desc; uint64_t nprod;
+    const CrtDesc *desc; uint64_t nprod; /* null: the one product `one` */
+    CrtDesc one;
     uint32_t *status;                    /* one word per block (CRT_ST_*) */
-    uint32_t *ctl;                       /* [1] error flags */
     uint32_t block0;                     /* the launch's first block */
+    uint64_t *stamp;                     /* or null: the device clock at the launch's start */
     CrtConst cc;
 };
 
@@ -126,13 +120,16 @@ __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
     __shared__ uint32_t s_wave[CRT_T / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t blk = a.block0 + blockIdx.x;
-    if (tid == 0) {
+    stamp_clock(a.stamp);
+    if (tid == 0 && !a.desc) { s_prod = 0; s_err = 0; }
+    else if (tid == 0) {
         uint64_t lo = 0, hi = a.nprod - 1;                  /* the product whose block range holds blk */
         while (lo < hi) { const uint64_t mid = (lo + hi + 1) >> 1; if (a.desc[mid].first_block <= blk) lo = mid; else hi = mid - 1; }
         s_prod = (uint32_t)lo; s_err = 0;
     }
     __syncthreads();
-    const CrtDesc dsc = a.desc[s_prod];
+    CrtDesc dsc = a.one;                             /* (copied as values: see input_limb_raw) */
+    if (a.desc) dsc = a.desc[s_prod];
     const uint32_t first = (uint32_t)dsc.first_block, local = blk - first;
     const uint64_t k0 = (uint64_t)local * CH;
 
@@ -271,7 +268,7 @@ __device__ __forceinline__ uint32_t crt_step_map(uint32_t st)
     const uint32_t m = st & 3u;                                     /* a first block ignores the carry before it */
     return (st & CRT_ST_FIRST) ? (m & 1u) * 3u : m;
 }
-__global__ __launch_bounds__(CRT_SCAN_T) void k_crt_scan(uint32_t *status, uint64_t n, uint32_t *ctl)
+__global__ __launch_bounds__(CRT_SCAN_T) void k_crt_scan(uint32_t *status, uint64_t n, uint32_t *ctl, uint64_t *stamp)
 {
     __shared__ uint32_t s_map[CRT_SCAN_T / 64], s_err;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -351,6 +348,7 @@ __global__ __launch_bounds__(CRT_SCAN_T) void k_crt_scan(uint32_t *status, uint6
     if (__ballot(err != 0) && lane == 0) atomicOr(&s_err, 1u);
     __syncthreads();
     if (tid == 0) { ctl[0] = 0; ctl[1] = s_err; }
+    stamp_clock(stamp);
 }
 
 /* the limbs of a block whose carry in is 1: its stored limbs (for carry 0) plus one, i.e. the leading limbs equal to
@@ -358,7 +356,7 @@ __global__ __launch_bounds__(CRT_SCAN_T) void k_crt_scan(uint32_t *status, uint6
  * every 4th block found and rewrites it (CH / 64 limbs per lane, all loads in flight at once). */
 #define CRT_FIX_W 64
 template <int PER>
-__global__ __launch_bounds__(256) void k_crt_fix(const CrtDesc *desc, uint64_t nprod, const uint32_t *status, uint64_t n)
+__global__ __launch_bounds__(256) void k_crt_fix(const CrtDesc *desc, CrtDesc one, uint64_t nprod, const uint32_t *status, uint64_t n)
 {
     constexpr int CH = CRT_T * PER;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -370,9 +368,10 @@ __global__ __launch_bounds__(256) void k_crt_fix(const CrtDesc *desc, uint64_t n
         todo &= todo - 1;
         if ((r & 3) != wave) continue;
         const uint64_t blk = b0 + f;
-        uint64_t lo = 0, hi = nprod - 1;
+        uint64_t lo = 0, hi = desc ? nprod - 1 : 0;
         while (lo < hi) { const uint64_t mid = (lo + hi + 1) >> 1; if (desc[mid].first_block <= blk) lo = mid; else hi = mid - 1; }
-        const CrtDesc d = desc[lo];
+        CrtDesc d = one;
+        if (desc) d = desc[lo];
         const uint64_t k0 = (blk - d.first_block) * CH, end = k0 + CH < d.nc ? k0 + CH : d.nc;
         uint64_t v[CH / 64];
 #pragma unroll
@@ -444,19 +443,22 @@ uint64_t nttm_crt_blocks(uint64_t nc, int per) { const uint64_t ch = (uint64_t)C
 
 uint64_t nttm_crt_scratch_words(uint64_t nblocks) { return nblocks + CRT_CTL_WORDS; }
 
-/* desc_dev: nprod descriptors in device memory whose block ranges tile [blk0, blk0 + nblk) of scratch's status words:
- * their limbs for a carry into every block of 0, and the blocks' carry maps */
-int nttm_crt_launch_limbs(const void *desc_dev, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np, const CrtConst &cc,
-                          uint32_t *scratch, hipStream_t s, double alg_bytes, int per)
+/* desc_dev: nprod descriptors in device memory whose block ranges tile [blk0, blk0 + nblk) of scratch's status words
+ * (null: the one product `one`): their limbs for a carry into every block of 0, and the blocks' carry maps */
+int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np,
+                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp)
 {
     if (per != 1 && per != CRT_WIDE) return nttm_fail(NTTM_EINVAL, "crt: %d limbs per thread", per);
     if (np < 3 || np > NTTM_MAX_PRIMES) return nttm_fail(NTTM_EINVAL, "crt: np = %d", np);
     if (!nprod || !nblk) return 0;
+    if (!desc_dev && (!one || nprod != 1)) return nttm_fail(NTTM_EINVAL, "crt: no descriptors");
     if (blk0 + nblk > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "crt: too many blocks");
     if ((uintptr_t)scratch & 15) return nttm_fail(NTTM_EINVAL, "crt: scratch not 16-byte aligned");
     CrtArgs a;
-    a.desc = (const CrtDesc *)desc_dev; a.nprod = nprod; a.block0 = (uint32_t)blk0;
-    a.ctl = scratch; a.status = scratch + CRT_CTL_WORDS; a.cc = cc;
+    memset(&a.one, 0, sizeof a.one);
+    if (one) a.one = *one;
+    a.desc = desc_dev; a.nprod = nprod; a.block0 = (uint32_t)blk0; a.stamp = stamp;
+    a.status = scratch + CRT_CTL_WORDS; a.cc = cc;
     prof_begin("k_crt", alg_bytes, s);
     if (per == 1) {
         if (np == 3) hipLaunchKernelGGL((k_crt<3, 1>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
@@ -468,29 +470,33 @@ int nttm_crt_launch_limbs(const void *desc_dev, uint64_t nprod, uint64_t blk0, u
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_crt launch");
 }
-/* every block's carry in, and the limbs of the blocks that receive one; scratch's word 1 receives the error flags */
-int nttm_crt_launch_carry(const void *desc_dev, uint64_t nprod, uint64_t nblocks, uint32_t *scratch, hipStream_t s, int per)
+/* every block's carry in, and the limbs of the blocks that receive one; word 1 of ctl (scratch, or pinned host memory)
+ * receives the error flags */
+int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t nblocks, uint32_t *scratch,
+                          uint32_t *ctl, hipStream_t s, int per, uint64_t *stamp)
 {
     if (!nprod || !nblocks) return 0;
     uint32_t *status = scratch + CRT_CTL_WORDS;
+    CrtDesc d1; memset(&d1, 0, sizeof d1);
+    if (one) d1 = *one;
     prof_begin("k_crt_scan", 8.0 * (double)nblocks, s);
-    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, status, nblocks, scratch);
+    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, status, nblocks, ctl, stamp);
     prof_end(s);
     RCK(nttm_hip_check(hipGetLastError(), "k_crt_scan launch"));
     prof_begin("k_crt_fix", 4.0 * (double)nblocks, s);
     const dim3 gfix((unsigned)((nblocks + CRT_FIX_W - 1) / CRT_FIX_W));
-    const CrtDesc *d = (const CrtDesc *)desc_dev;
-    if (per == 1) hipLaunchKernelGGL((k_crt_fix<1>), gfix, dim3(256), 0, s, d, nprod, (const uint32_t *)status, nblocks);
-    else hipLaunchKernelGGL((k_crt_fix<CRT_WIDE>), gfix, dim3(256), 0, s, d, nprod, (const uint32_t *)status, nblocks);
+    if (per == 1) hipLaunchKernelGGL((k_crt_fix<1>), gfix, dim3(256), 0, s, desc_dev, d1, nprod, (const uint32_t *)status, nblocks);
+    else hipLaunchKernelGGL((k_crt_fix<CRT_WIDE>), gfix, dim3(256), 0, s, desc_dev, d1, nprod, (const uint32_t *)status, nblocks);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_crt_fix launch");
 }
-/* both for a whole launch of products: scratch 16-byte aligned, nttm_crt_scratch_words(nblocks) words */
-int nttm_crt_launch_batch(const void *desc_dev, uint64_t nprod, uint64_t nblocks, int np, const CrtConst &cc,
-                          uint32_t *scratch, hipStream_t s, double alg_bytes, int per)
+/* one product, its descriptor passed with the launches: scratch 16-byte aligned, nttm_crt_scratch_words(nblocks) words.
+ * stamps (or null): the device clock at the start and at the end of the carry scan */
+int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtConst &cc, uint32_t *scratch, uint32_t *ctl,
+                        hipStream_t s, double alg_bytes, uint64_t *stamps)
 {
-    RCK(nttm_crt_launch_limbs(desc_dev, nprod, 0, nblocks, np, cc, scratch, s, alg_bytes, per));
-    return nttm_crt_launch_carry(desc_dev, nprod, nblocks, scratch, s, per);
+    RCK(nttm_crt_launch_limbs(nullptr, &d, 1, 0, nblocks, np, cc, scratch, s, alg_bytes, CRT_WIDE, stamps));
+    return nttm_crt_launch_carry(nullptr, &d, 1, nblocks, scratch, ctl, s, CRT_WIDE, stamps ? stamps + 1 : nullptr);
 }
 
 /* ---- addition and subtraction of limb arrays, with the carry resolved like the CRT's -------------------------------
@@ -590,7 +596,7 @@ int nttm_run_addsub(uint64_t *r, uint64_t nout, const uint64_t *a, uint64_t na, 
     hipLaunchKernelGGL(k_addsub, dim3((unsigned)nblocks), dim3(CRT_T), 0, s, A);
     int rc = nttm_hip_check(hipGetLastError(), "k_addsub launch");
     if (rc) return rc;
-    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, A.status, nblocks, scratch);
+    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, A.status, nblocks, scratch, (uint64_t *)nullptr);
     if ((rc = nttm_hip_check(hipGetLastError(), "k_crt_scan launch"))) return rc;
     hipLaunchKernelGGL(k_addsub_fix, dim3((unsigned)nblocks), dim3(64), 0, s, r, nout, (const uint32_t *)A.status, nblocks);
     return nttm_hip_check(hipGetLastError(), "k_addsub_fix launch");

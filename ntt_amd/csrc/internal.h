@@ -30,6 +30,16 @@ struct LoadDesc {
     const uint64_t *b; uint64_t nb;
 };
 
+/* the CRT of one product */
+struct CrtDesc {
+    const double *pl; uint64_t plane;    /* residues of prime j, coefficient k at pl[j * plane + k] */
+    uint64_t ncoef;
+    const uint64_t *x; uint64_t nx;
+    uint64_t *c; uint64_t nc;
+    uint64_t first_block;                /* the product's first block in the launch */
+    uint64_t trunc;                      /* nonzero: c is the value mod B^nc (nothing above it is checked) */
+};
+
 /* one pass over bits [lo, lo + m) of every transform of 2^logn points in a batch; a tile holds W low columns x 2^m
  * rows x H high blocks (log2 of each below) */
 struct PassArgs {
@@ -57,7 +67,15 @@ struct PassArgs {
      * c1 < 2^(dfr_lom - dfr_gm) its column) by w_(2^dfr_lom)^(brev_dfr_gm(h) c1), times dfr_scale when dfr_do_scale */
     int dfr_out, dfr_in, dfr_lom, dfr_gm, dfr_do_scale;
     double2 dfr_scale;
+    uint64_t *stamp;                /* or null: the device clock at the launch's first block goes here (pinned host memory) */
 };
+/* the phase clock of short products: the device's constant-rate clock, stored by one thread of a launch */
+#if defined(__HIPCC__) || defined(__HIP__)
+__device__ __forceinline__ void stamp_clock(uint64_t *stamp)
+{
+    if (stamp && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *stamp = wall_clock64();
+}
+#endif
 
 /* One launch can run a pass for several planes of one geometry (the primes of a product, both of its operands): block
  * row blockIdx.y takes job blockIdx.y, whose fields replace the same ones of PassArgs */

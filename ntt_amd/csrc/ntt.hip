@@ -232,6 +232,11 @@ __device__ __forceinline__ void round_split(int m, int i, int *s_lo, int *logR, 
     case 2: { constexpr int LR = 2; __VA_ARGS__ } break; \
     default: { constexpr int LR = 1; __VA_ARGS__ } break; }
 
+/* limbs and planes as global-space pointers: an address read from memory is generic to the compiler, and a generic
+ * (flat) access counts against the LDS counter too */
+typedef const __attribute__((address_space(1))) uint64_t *GLimb;
+typedef __attribute__((address_space(1))) double *GPlane;
+
 /* the pass's input element: from the plane, or (the first forward pass) from the operand limbs, zero beyond them */
 __device__ __forceinline__ double input_limb_raw(const PassArgs &a, uint64_t gi, double p, double pinv)
 {
@@ -241,7 +246,7 @@ __device__ __forceinline__ double input_limb_raw(const PassArgs &a, uint64_t gi,
     const uint64_t *src; uint64_t nl;
     if (a.ldesc) { const LoadDesc d = a.ldesc[b]; src = a.which ? d.b : d.a; nl = a.which ? d.nb : d.na; }
     else { src = a.limbs; nl = a.nlimbs; }
-    return k < nl ? limb_to_res(src[k], p, pinv) : 0.0;
+    return k < nl ? limb_to_res(((GLimb)src)[k], p, pinv) : 0.0;
 }
 __device__ __forceinline__ double input_limb(const PassArgs &a, uint64_t gi, double p, double pinv)
 {
@@ -261,7 +266,7 @@ struct LimbCache {
             const uint64_t bb = gi >> a.logn;
             if (bb != b) { const LoadDesc d = a.ldesc[bb]; src = a.which ? d.b : d.a; nl = a.which ? d.nb : d.na; b = bb; }
         } else { src = a.limbs; nl = a.nlimbs; }
-        double x = k < nl ? limb_to_res(src[k], p, pinv) : 0.0;
+        double x = k < nl ? limb_to_res(((GLimb)src)[k], p, pinv) : 0.0;
         if (a.do_in_scale) x = mul_shoup(x, a.in_scale.x, a.in_scale.y, p);
         return x;
     }
@@ -355,6 +360,7 @@ template <int MODE, int PTS, int GM = -1, int GW = -1, int GH = -1>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_pass(PassArgs a, JobSet js)
 {
     apply_job(a, js);
+    stamp_clock(a.stamp);
     if (blockIdx.x >= (a.batch << a.logn) >> (a.m + a.logw + a.logh)) return;   /* a job of fewer transforms */
     const int gm = GM >= 0 ? GM : a.m, gw = GW >= 0 ? GW : a.logw, gh = GH >= 0 ? GH : a.logh;
     constexpr bool INV = MODE >= PM_INV;
@@ -388,7 +394,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     const bool scale_in_chain = MODE == PM_FWD_LIMB && a.lo > 0 && a.do_in_scale;
     auto limb_at = [&](uint32_t o) -> double {
         double x;
-        if (limb_one) { const uint64_t k = lk0 + o; x = k < lnl ? limb_to_res(lsrc[k], p, pinv) : 0.0; }
+        if (limb_one) { const uint64_t k = lk0 + o; x = k < lnl ? limb_to_res(((GLimb)lsrc)[k], p, pinv) : 0.0; }
         else x = input_limb_raw(a, gbase + o, p, pinv);
         if (a.do_in_scale && !scale_in_chain) x = mul_shoup(x, a.in_scale.x, a.in_scale.y, p);
         return x;
@@ -489,6 +495,7 @@ template <int MODE, int GM, int GW>
 __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
 {
     apply_job(a, js);
+    stamp_clock(a.stamp);
     hold(a.x); hold(a.pk.p); hold(a.pk.pinv);
     const uint32_t ntiles = (uint32_t)((a.batch << a.logn) >> (GM + GW));
     constexpr bool INV = MODE == PM_INV, LIMB = MODE == PM_FWD_LIMB;
@@ -570,7 +577,7 @@ __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
         if (tile + gridDim.x < ntiles) fetch(tile + gridDim.x, nxt);
         uint32_t colbase;
         const uint64_t gbase = tile_base(tile, &colbase);
-        double *xt = a.x + gbase;
+        const GPlane xt = (GPlane)(a.x + gbase);
 
         double v[PTS], w[PTS];
         const bool bound_out = !INV && !(LIMB && a.dfr_out);           /* the output's boundary twiddles here */
@@ -757,9 +764,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
  * STW_LOG read their twiddles there */
 #define STW_LOG 8
 /* LT: stw is the LDS copy of the stage table's low entries, for the rounds after the first */
-template <int PTS, int MAXR, bool LIMBS, bool LT>
+/* loaded(): called once the tile's loads have been issued */
+template <int PTS, int MAXR, bool LIMBS, bool LT, typename F>
 __device__ __forceinline__ void tile_forward(const PassArgs &q, const PassPos &pp, bool active, uint64_t gbase,
-                                             const SwzLds &xs, double *v, double p, double pinv, const double2 *stw)
+                                             const SwzLds &xs, double *v, double p, double pinv, const double2 *stw, F loaded)
 {
     const bool limb = LIMBS && (q.limbs || q.ldesc);
     /* a shared B: the tile (inside one transform) is read from the transform the map names */
@@ -773,6 +781,7 @@ __device__ __forceinline__ void tile_forward(const PassArgs &q, const PassPos &p
         if (active) ROUND_SWITCH(logR, for_slots<LR, PTS>(pp, s_lo, [&](int sl, uint32_t, uint32_t o, uint32_t,
                                                                        uint32_t) {
             v[sl] = limb ? lc.at(q, gbase + o, p, pinv) : xt[o]; });)
+        loaded();
     } else {
         if (active) {
 #pragma unroll
@@ -781,6 +790,7 @@ __device__ __forceinline__ void tile_forward(const PassArgs &q, const PassPos &p
                 xs[e] = limb ? lc.at(q, gbase + e, p, pinv) : xt[e];
             }
         }
+        loaded();
         __syncthreads();
         if (active) ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
                                                                        uint32_t) { v[sl] = xs.at(e); });)
@@ -825,10 +835,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     __shared__ double2 stw_lds[LT ? 1 << STW_LOG : 1];
     const SwzLds xs{xs_raw};
     constexpr int MAXR = PTS >= 16 ? 4 : 3;
-    if (LT) {
-        for (int i = threadIdx.x; i < (1 << STW_LOG); i += blockDim.x) stw_lds[i] = a.tw.stage[i];
-        /* visible to the rounds after the first round's barrier; the first round's stages lie above STW_LOG */
-    }
+    /* the table's entries are requested ahead of B's tile and stored once that is requested too (LT: 256 threads, one entry
+     * each): visible to the rounds after the first round's barrier; the first round's stages lie above STW_LOG */
+    static_assert(!LT || (1 << FUSED_LOG) / PTS == (1 << STW_LOG), "one stage table entry per thread");
+    double2 st;
+    if (LT) st = a.tw.stage[threadIdx.x];
     if (GM >= 0) { a.m = GM; bq.m = GM; }
     if (GH >= 0) { a.logh = GH; bq.logh = GH; }
     PassPos pp; pp.m = a.m; pp.logw = 0; pp.lo = 0;
@@ -843,9 +854,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     int s_lo, logR;
 
     const double2 *stw = LT ? (const double2 *)stw_lds : nullptr;
-    tile_forward<PTS, MAXR, LIMBS, LT>(bq, pp, active, gbase, xs, bv, p, pinv, stw);
+    tile_forward<PTS, MAXR, LIMBS, LT>(bq, pp, active, gbase, xs, bv, p, pinv, stw, [&]() {
+        if (LT) stw_lds[threadIdx.x] = st;
+        stamp_clock(a.stamp);
+    });
     __syncthreads();                                             /* B's last LDS reads before A's first writes */
-    tile_forward<PTS, MAXR, LIMBS, LT>(a, pp, active, gbase, xs, v, p, pinv, stw);
+    tile_forward<PTS, MAXR, LIMBS, LT>(a, pp, active, gbase, xs, v, p, pinv, stw, []() {});
     if (active) {
 #pragma unroll
         for (int sl = 0; sl < PTS; sl++) v[sl] = mul_barrett(v[sl], bv[sl], p, pinv);
@@ -976,7 +990,7 @@ __device__ __forceinline__ double r3_input(const R3Args &a, uint64_t t, uint64_t
     const uint64_t *src; uint64_t nl;
     if (a.ldesc) { const LoadDesc d = a.ldesc[t]; src = a.which ? d.b : d.a; nl = a.which ? d.nb : d.na; }
     else { src = a.limbs; nl = a.nlimbs; }
-    return k < nl ? limb_to_res(src[k], a.pk.p, a.pk.pinv) : 0.0;
+    return k < nl ? limb_to_res(((GLimb)src)[k], a.pk.p, a.pk.pinv) : 0.0;
 }
 /* w^j and w^(2j) (times the scale when given), |.| <= p */
 __device__ __forceinline__ void r3_twiddles(const R3Args &a, uint64_t j, double *t1, double *t2)
@@ -989,8 +1003,9 @@ __device__ __forceinline__ void r3_twiddles(const R3Args &a, uint64_t j, double 
     *t1 = w1; *t2 = w2;
 }
 template <bool LIMB>
-__global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(int logk, JobSet js)
+__global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(int logk, JobSet js, uint64_t *stamp)
 {
+    stamp_clock(stamp);
     const R3Args a = r3_args(js, logk);
     const uint64_t m = (uint64_t)1 << a.logk, total = a.batch << a.logk;
     const uint64_t stride = (uint64_t)gridDim.x * NTTM_THREADS;
@@ -1203,6 +1218,9 @@ int nttm_run_fused(const PassArgs &a, const PassGeom &g, hipStream_t s)
     return nttm_hip_check(hipGetLastError(), "k_fused launch");
 }
 
+/* Bound by vector issue (166 of 178 vector instructions a point are FP64).  A block's first loads wait for nothing but its
+ * arguments: the LDS table's entry is requested before B's tile and stored behind it, and limbs are read through
+ * global-space pointers (2.06 -> 1.97 ms per launch at 2^28 points). */
 /* the double-fused last pass of every prime of js: a = A's common arguments (its operand where a transform is a single
  * pass: limbs or descriptors; a.ymode and a.scale unused), fb = B's */
 int nttm_run_fused2(const PassArgs &a, const FusedB &fb, const PassGeom &g, hipStream_t s, const FusedSet &js)
@@ -1291,7 +1309,7 @@ int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which
 /* the radix-3 layer of the jobs' transforms of 3 2^logk points (logk >= 1): forward (from the planes, or every job from
  * limbs) or inverse, in place.  A job: x, batch (transforms of 3 2^logk points), its operand, pk, tw.b3 (the direction's
  * table) and the scale of every output in in_scale */
-int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s)
+int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *stamp)
 {
     if (js.n < 1 || js.n > NTTM_MAX_JOBS || logk < 1 || logk > NTTM_LOGN_MAX) return nttm_fail(NTTM_EINVAL, "internal: radix-3 layer of 3 2^%d", logk);
     const bool limb = js.j[0].limbs || js.j[0].ldesc;
@@ -1310,8 +1328,8 @@ int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s)
     prof_begin(inv ? "k_r3_inv" : limb ? "k_r3_fwd<limb>" : "k_r3_fwd", bytes, s);
     const dim3 grid(grid_for(most << logk), (unsigned)js.n);
     if (inv) hipLaunchKernelGGL(k_r3_inv, grid, dim3(NTTM_THREADS), 0, s, logk, js);
-    else if (limb) hipLaunchKernelGGL(k_r3_fwd<true>, grid, dim3(NTTM_THREADS), 0, s, logk, js);
-    else hipLaunchKernelGGL(k_r3_fwd<false>, grid, dim3(NTTM_THREADS), 0, s, logk, js);
+    else if (limb) hipLaunchKernelGGL(k_r3_fwd<true>, grid, dim3(NTTM_THREADS), 0, s, logk, js, stamp);
+    else hipLaunchKernelGGL(k_r3_fwd<false>, grid, dim3(NTTM_THREADS), 0, s, logk, js, stamp);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_r3 launch");
 }

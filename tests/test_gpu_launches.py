@@ -85,3 +85,24 @@ def test_group_chunks(schedule, chunk, cfg):
             assert np.array_equal(c, want) and np.array_equal(host(it[3]), want)
             assert ln == pr.ncn == int(np.nonzero(want)[0][-1]) + 1
     plan.close()
+
+
+@pytest.mark.parametrize("n", [100, 5000, 300000])
+@pytest.mark.parametrize("par", [None, 0])
+def test_phase_times(schedule, n, par):
+    """the phase times of a call are its own: none negative, together positive and within the call's wall time (plus
+    the 0.01 ms tick of the device clock per phase)"""
+    import time
+    import torch
+    lib = schedule(par=par)
+    a, s = O.gen_limbs(n, 3)
+    da, db = dev(a), dev(O.gen_limbs(n, s)[0])
+    lib.mul(da, db)
+    for _ in range(3):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        lib.mul(da, db)
+        wall = 1e3 * (time.perf_counter() - t0)
+        ph = lib.last_phase_ms()
+        say("phases", n, par, ph, wall)
+        assert all(p >= 0 for p in ph) and 0 < sum(ph) <= wall + 0.03
