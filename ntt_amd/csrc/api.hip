@@ -15,14 +15,13 @@
 #include "plan.h"
 
 int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s, const JobSet *jobs = nullptr);
-int nttm_run_fused(const PassArgs &a, const PassGeom &g, hipStream_t s);
 int nttm_run_fused2(const PassArgs &a, const FusedB &fb, const PassGeom &g, hipStream_t s, const FusedSet &js);
 bool nttm_fwd_pass_streams(const PassArgs &a, const PassGeom &g);
 void nttm_set_pts(int pts);
 int nttm_get_pts(void);
 void nttm_set_fixed_shapes(int on);
 void nttm_set_stream(int on, int ncu);
-#define NTTM_FUSED_LOG 12          /* tile of the fused forward + pointwise + inverse pass (k_fused) */
+#define NTTM_FUSED_LOG 12          /* tile of the fused forward + pointwise + inverse pass (k_fused2) */
 #define NTTM_TILE_LOG_DEFAULT 13   /* tile of the strided passes: 2^13 points (64 KiB of LDS), runs of 32 columns */
 #define NTTM_PRODUCT_LOGN_MIN 4    /* products use at least 2^4 points, so every fused tile has >= 16 */
 #define NTTM_STAGE_CHUNK ((size_t)1 << 30)   /* staged bytes per sub-batch of a batch with host operands (default) */
@@ -45,6 +44,10 @@ int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtCon
                         hipStream_t s, double alg_bytes, uint64_t *stamps = nullptr);
 uint64_t nttm_crt_blocks(uint64_t nc, int per = 8);      /* per: CRT limbs per thread, 8 (2048-limb blocks) or 1 (256) */
 uint64_t nttm_crt_scratch_words(uint64_t nblocks);
+int nttm_small_log(int logn);
+int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1,
+                   uint64_t cnt, uint64_t *ncn, uint32_t *ctl, const TwTables *fwd, const TwTables *inv, const double2 *ninv,
+                   const CrtConst &cc, hipStream_t s, double alg_bytes, uint64_t *stamps);
 int nttm_run_norm(const void *desc_dev, uint64_t nprod, uint64_t *ncn_dev, hipStream_t s);
 int nttm_run_fill_x(const void *desc_dev, uint64_t nprod, hipStream_t s);
 int nttm_run_dft16_mfma(const uint64_t *x, double *y, int logn, uint64_t batch, const void *etab, const double *tlo,
@@ -130,6 +133,7 @@ static Ctx g;
 static uint64_t g_init_count;
 static int g_prof_on;                        /* live kernel timing on (nttm_profile) */
 static int g_no_defer;                       /* NTTM_NO_DEFER=1: every pass applies its own boundary twiddles */
+static int g_no_small;                       /* NTTM_GENERIC_PASSES=1: no whole product in one kernel either */
 static int g_tree_levelwise;                 /* NTTM_TREE_LEVELWISE=1: the tree level by level (for comparison) */
 static int g_fused_bits_env;                 /* NTTM_FUSED_BITS=10|11|12: that last-pass width for every product
                                               * transform above it (for comparison measurements) */
@@ -400,6 +404,7 @@ extern "C" int nttm_init(int device, const nttm_config *cfg)
     {   /* NTTM_GENERIC_PASSES=1: runtime-geometry pass kernels only (for comparison) */
         const char *e = getenv("NTTM_GENERIC_PASSES");
         nttm_set_fixed_shapes(!(e && e[0] == '1'));
+        g_no_small = e && e[0] == '1';
     }
     int nd = 0;
     HIPCK(hipGetDeviceCount(&nd));
@@ -532,7 +537,7 @@ static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 /* the transforms of one length group of products (cnt transforms of 2^logn points per prime):
  *   B: forward, the first pass reading b's limbs (times n^-1, folded here once);
  *   A: forward up to its last pass, the first pass reading a's limbs;
- *   A: the fused last forward pass + pointwise product with B + first inverse pass (k_fused);
+ *   A: the fused last forward pass + pointwise product with B + first inverse pass (k_fused2);
  *   A: the remaining inverse passes.
  * Operand limbs come from (a, na, b, nb) when cnt == 1 and ldesc is null, else from the device descriptors ldesc.
  * Result: plane i of A holds the cyclic convolution mod p_i. */
@@ -767,6 +772,17 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
     return 0;
 }
 
+/* whether products of this transform length run as one kernel each (small.hip): 2^k points up to 2^12 */
+static bool small_len(int logn, int r3) { return !r3 && !g_no_small && nttm_small_log(logn) != 0; }
+static int run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1,
+                     uint64_t cnt, uint64_t *ncn, uint32_t *ctl, hipStream_t s, double bytes, uint64_t *stamps = nullptr)
+{
+    const int sl = nttm_small_log(logn);
+    double2 ninv[NTTM_MAX_PRIMES];
+    for (int i = 0; i < np; i++) { const uint64_t p = NTTM_PRIMES[i]; ninv[i] = h_shoup(h_inv((uint64_t)1 << sl, p), p); }
+    return nttm_run_small(np, sl, ld, cd, ld1, cd1, cnt, ncn, ctl, g.twf, g.twi, ninv, g.cc, s, bytes, stamps);
+}
+
 /* c = a b (+ x), device pointers.  wcut: write only the low wcut limbs of the result (the value mod B^wcut; no check of
  * what lies above).  ws: the workspace (null: the library's, grown to fit; else ws_cap bytes of the caller's).
  * sync = 1: returns after the stream has drained and the CRT's flags are checked; sync = 0: returns after the launches,
@@ -792,6 +808,19 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     }
     if (!nc) return 0;
     CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws));
+    uint32_t *ctl = (uint32_t *)((char *)g.hpin + 128 * slot + 96);
+    CrtDesc hd; memset(&hd, 0, sizeof hd);
+    hd.plane = L.n; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
+    hd.trunc = nc < nc_full;
+    if (small_len(L.logn, L.r3)) {
+        const LoadDesc ld{a, na, b, nb};
+        RCK(run_small(L.np, L.logn, nullptr, nullptr, &ld, &hd, 1, nullptr, ctl, s, 8.0 * (double)(na + nb + nc + hd.nx),
+                      sync ? g.stamps : nullptr));
+        if (!sync) return 0;
+        HIPCK(hipStreamSynchronize(s));
+        g.last_stamped = 1;
+        return ctl[1] & 1 ? nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond the top limb (wrong residues)") : 0;
+    }
     if (ws) {
         if (L.bytes > ws_cap) return nttm_fail(NTTM_EINVAL, "the product needs %zu bytes of workspace, above the %zu given", L.bytes, ws_cap);
     } else {
@@ -800,7 +829,6 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     }
     double *A = (double *)ws, *Bp = A + (size_t)L.np * L.n;
     uint32_t *crt_scr = (uint32_t *)(ws + L.off_crt);
-    uint32_t *ctl = (uint32_t *)((char *)g.hpin + 128 * slot + 96);
     const bool events = sync && !L.par;
     uint64_t *stamps = sync && L.par ? g.stamps : nullptr;
     if (stamps) stamps[0] = ~(uint64_t)0;                        /* (a transform of one pass has no forward launch) */
@@ -809,9 +837,7 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, L.par ? L.n : 0, a, na, b, nb, nullptr, s, events ? g.pev : nullptr, 0,
                            nullptr, nullptr, stamps));
     if (events) HIPCK(hipEventRecord(g.ev[2], s));
-    CrtDesc hd; memset(&hd, 0, sizeof hd);
-    hd.pl = A; hd.plane = L.n; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
-    hd.trunc = nc < nc_full;
+    hd.pl = A;
     RCK(nttm_crt_launch_one(hd, nttm_crt_blocks(nc), L.np, g.cc, crt_scr, ctl, s,
                             8.0 * L.np * (double)L.ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? (nx < nc ? nx : nc) : 0),
                             stamps ? stamps + 2 : nullptr));
@@ -1078,14 +1104,14 @@ struct GroupBuild {
     int r3 = 0, logn = 0, tile = 0, pts = 0;
     int crt_per = 8;                                             /* CRT limbs per thread: 1 when every product is small */
     uint64_t n = 0, cnt = 0, cnt_b = 0, nblk = 0;
-    bool share = false, merged = false;
+    bool share = false, merged = false, small = false;
     struct Chunk { uint64_t c0, cn, b0, cnb, blk0, nblk; double crt_bytes; };   /* products, distinct B operands, CRT blocks */
     std::vector<Chunk> chunk;
     std::vector<CrtDesc> cd;
     std::vector<LoadDesc> ld, ldb;
     std::vector<uint32_t> bmap;
     size_t planes_bytes = 0;                                     /* (np cnt + cnt_b) n doubles */
-    size_t off_cd = 0, off_ld = 0, off_ldb = 0, off_bmap = 0, off_ncn = 0, off_crt = 0, desc_bytes = 0;
+    size_t off_cd = 0, off_ld = 0, off_ldb = 0, off_bmap = 0, off_ctl = 0, off_ncn = 0, off_crt = 0, desc_bytes = 0;
 };
 /* products of a group that run together (a chunk), and whether all primes of a chunk share a launch per pass */
 static uint64_t chunk_products(uint64_t n) { return std::max<uint64_t>(1, g_chunk_points / n); }
@@ -1103,7 +1129,8 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
     gb.n = n; gb.cnt = cnt; gb.nblk = 0; gb.cnt_b = 0; gb.planes_bytes = 0;
     gb.crt_per = n <= 1024 ? 1 : 8;                              /* products of at most n + 1 limbs: 256-limb blocks */
     gb.cd.assign(cnt, CrtDesc()); gb.ld.assign(cnt, LoadDesc()); gb.ldb.clear(); gb.bmap.clear(); gb.chunk.clear();
-    const uint64_t cmax = chunk_products(n);
+    gb.small = small_len(logn, r3);                              /* one kernel, no planes and no CRT blocks */
+    const uint64_t cmax = gb.small ? cnt : chunk_products(n);
     gb.merged = chunk_merged(n, std::min(cnt, cmax));
     for (uint64_t c0 = 0; c0 < cnt; c0 += cmax) gb.chunk.push_back({c0, std::min(cmax, cnt - c0), 0, 0, 0, 0, 0.0});
     for (GroupBuild::Chunk &ch : gb.chunk) {
@@ -1115,8 +1142,8 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
             l.a = q.a; l.na = q.na; l.b = q.b; l.nb = q.nb;
             c.pl = nullptr; c.plane = ch.cn * n; c.ncoef = q.na + q.nb - 1; c.x = q.x; c.nx = q.x ? q.nx : 0;
             c.c = q.c; c.nc = q.na + q.nb + (q.x ? 1 : 0); c.first_block = gb.nblk; c.trunc = 0;
-            gb.nblk += nttm_crt_blocks(c.nc, gb.crt_per);
-            ch.crt_bytes += 8.0 * np * c.ncoef + 8.0 * c.nc + 8.0 * c.nx;
+            if (!gb.small) gb.nblk += nttm_crt_blocks(c.nc, gb.crt_per);
+            ch.crt_bytes += gb.small ? 8.0 * (q.na + q.nb) + 8.0 * c.nc + 8.0 * c.nx : 8.0 * np * c.ncoef + 8.0 * c.nc + 8.0 * c.nx;
         }
         ch.nblk = gb.nblk - ch.blk0;
     }
@@ -1125,7 +1152,7 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
      * radix-3 length) and the double-fused tiles lie inside one transform */
     std::vector<uint32_t> slot(cnt);
     Plan pq; product_plan(&pq, logn, r3 ? 3 * cnt : cnt, product_tile_log(logn, tile));
-    const bool can = logn >= NTTM_FUSED_LOG && (pq.npass > 1 || r3);
+    const bool can = !gb.small && logn >= NTTM_FUSED_LOG && (pq.npass > 1 || r3);
     if (can) gb.ldb.reserve(cnt);
     for (GroupBuild::Chunk &ch : gb.chunk) {
         std::map<std::pair<const uint64_t *, uint64_t>, uint32_t> seen;
@@ -1141,7 +1168,7 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
         }
         ch.cnb = can ? gb.ldb.size() - ch.b0 : ch.cn;            /* no sharing: one B per product */
         gb.cnt_b += ch.cnb;
-        gb.planes_bytes = std::max(gb.planes_bytes, ((size_t)np * ch.cn + (size_t)(gb.merged ? np : 1) * ch.cnb) * n * 8);
+        if (!gb.small) gb.planes_bytes = std::max(gb.planes_bytes, ((size_t)np * ch.cn + (size_t)(gb.merged ? np : 1) * ch.cnb) * n * 8);
     }
     gb.share = gb.cnt_b < cnt;
     if (!gb.share) gb.ldb.clear();
@@ -1154,7 +1181,8 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
     gb.off_ld = align_up(gb.off_cd + cnt * sizeof(CrtDesc), 256);
     gb.off_ldb = align_up(gb.off_ld + cnt * sizeof(LoadDesc), 256);
     gb.off_bmap = align_up(gb.off_ldb + gb.ldb.size() * sizeof(LoadDesc), 256);
-    gb.off_ncn = align_up(gb.off_bmap + gb.bmap.size() * 4, 256);
+    gb.off_ctl = align_up(gb.off_bmap + gb.bmap.size() * 4, 256);   /* a small group's flags, zeroed by the upload */
+    gb.off_ncn = gb.off_ctl + 256;
     gb.off_crt = align_up(gb.off_ncn + cnt * 8, 256);
     gb.desc_bytes = align_up(gb.off_crt + nttm_crt_scratch_words(gb.nblk) * 4, 256);
 }
@@ -1168,6 +1196,7 @@ static void group_image(GroupBuild &gb, double *A, char *img)
         for (uint64_t j = 0; j < ch.cn; j++) gb.cd[ch.c0 + j].pl = A + j * gb.n;
     memcpy(img + gb.off_cd, gb.cd.data(), gb.cnt * sizeof(CrtDesc));
     memcpy(img + gb.off_ld, gb.ld.data(), gb.cnt * sizeof(LoadDesc));
+    memset(img + gb.off_ctl, 0, 16);
     if (gb.share) {
         memcpy(img + gb.off_ldb, gb.ldb.data(), gb.ldb.size() * sizeof(LoadDesc));
         memcpy(img + gb.off_bmap, gb.bmap.data(), gb.bmap.size() * 4);
@@ -1177,6 +1206,9 @@ static void group_image(GroupBuild &gb, double *A, char *img)
  * per thread (the library's settings are restored afterwards) */
 static int group_launch(const GroupBuild &gb, int np, double *A, char *dbase, hipStream_t s, bool norm = true)
 {
+    if (gb.small)
+        return run_small(np, gb.logn, (const LoadDesc *)(dbase + gb.off_ld), (const CrtDesc *)(dbase + gb.off_cd), nullptr, nullptr,
+                         gb.cnt, (uint64_t *)(dbase + gb.off_ncn), (uint32_t *)(dbase + gb.off_ctl), s, gb.chunk[0].crt_bytes);
     const int tile0 = g.cfg.tile_log, pts0 = nttm_get_pts();
     g.cfg.tile_log = gb.tile; nttm_set_pts(gb.pts);
     int rc = 0;
@@ -1195,6 +1227,18 @@ static int group_launch(const GroupBuild &gb, int np, double *A, char *dbase, hi
     if (!rc && norm) rc = nttm_run_norm(dbase + gb.off_cd, gb.cnt, (uint64_t *)(dbase + gb.off_ncn), s);
     g.cfg.tile_log = tile0; nttm_set_pts(pts0);
     return rc;
+}
+
+/* a group's lengths (device words read back) to put(j, n); true when a CRT's carry ran beyond a top limb.  A small group's
+ * lengths carry their product's flag in bit 63; the others' flags are ctl's */
+template <typename F> static bool group_lengths(const GroupBuild &gb, const uint64_t *ncn, const uint32_t *ctl, F put)
+{
+    bool bad = !gb.small && (ctl[1] & 1);
+    for (uint64_t j = 0; j < gb.cnt; j++) {
+        if (gb.small && ncn[j] >> 63) bad = true;
+        put(j, ncn[j] & ~((uint64_t)1 << 63));
+    }
+    return bad;
 }
 
 /* the batch on device memory (every pointer of P classed MEM_DEV) */
@@ -1240,11 +1284,10 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
         HIPCK(hipMemcpyAsync(g.ws + off_d, hp, gb.off_ncn, hipMemcpyHostToDevice, s));   /* descriptors up to ncn */
         RCK(group_launch(gb, np, (double *)g.ws, g.ws + off_d, s));
         HIPCK(hipMemcpyAsync(hp, g.ws + off_d + gb.off_ncn, gb.cnt * 8, hipMemcpyDeviceToHost, s));
-        HIPCK(hipMemcpyAsync(hp + gb.cnt * 8, g.ws + off_d + gb.off_crt, 8, hipMemcpyDeviceToHost, s));
+        HIPCK(hipMemcpyAsync(hp + gb.cnt * 8, g.ws + off_d + (gb.small ? gb.off_ctl : gb.off_crt), 8, hipMemcpyDeviceToHost, s));
         HIPCK(hipStreamSynchronize(s));
-        const uint32_t flags = ((const uint32_t *)(hp + gb.cnt * 8))[1];
-        if (flags & 1) return nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond a top limb (wrong residues)");
-        for (uint64_t j = 0; j < gb.cnt; j++) P[G[j]].ncn = ((const uint64_t *)hp)[j];
+        if (group_lengths(gb, (const uint64_t *)hp, (const uint32_t *)(hp + gb.cnt * 8), [&](uint64_t j, uint64_t n) { P[G[j]].ncn = n; }))
+            return nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond a top limb (wrong residues)");
     }
     /* zero-operand products: normalized length of x */
     for (size_t i = 0; i < N; i++) {
@@ -1836,9 +1879,9 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
             if (logn > NTTM_LOGN_MAX) return 1;
             for (uint64_t c0 = 0; c0 < cnt_all; c0 += TREE_CHUNK) {   /* the group's chunks (below) */
                 const uint64_t cn = std::min<uint64_t>(TREE_CHUNK, cnt_all - c0), tb = r3 ? 3 * cn : cn;
-                planes_max = std::max(planes_max, chunk_planes_bytes(lev_np[k], npts, cn));
+                if (!small_len(logn, r3)) planes_max = std::max(planes_max, chunk_planes_bytes(lev_np[k], npts, cn));
                 const size_t img = align_up(cn * sizeof(CrtDesc), 256) + 2 * align_up(cn * sizeof(LoadDesc), 256) +
-                                   align_up(tb * 4, 256) + 256;
+                                   align_up(tb * 4, 256) + 256 + 256;
                 img_total += img;
                 desc_total += img + align_up(cn * 8, 256) + align_up(nttm_crt_scratch_words(blk[key]) * 4, 256) + 256;
                 ngroups++;
@@ -1932,7 +1975,7 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
                 HIPCK(hipEventRecord(ev, g.tcs));
                 HIPCK(hipStreamWaitEvent(s, ev, 0));
                 RCK(group_launch(gb, lev_np[k], (double *)g.ws, dbase, s, false));
-                flag_at.push_back(dbase + gb.off_crt + 4);
+                flag_at.push_back(dbase + (gb.small ? gb.off_ctl : gb.off_crt) + 4);
                 ipos = align_up(ipos + gb.off_ncn, 256);
                 dpos = align_up(dpos + gb.desc_bytes, 256);
             }
@@ -2556,16 +2599,15 @@ extern "C" int nttm_batch_plan_ncn(nttm_batch_plan *pl, size_t *ncn, void *strea
         at[i] = w;
         HIPCK(hipMemcpyAsync(h + w, pl->blob + pl->goff[i] + x.off_ncn, x.cnt * 8, hipMemcpyDeviceToHost, s));
         w += x.cnt;
-        HIPCK(hipMemcpyAsync(h + w, pl->blob + pl->goff[i] + x.off_crt, 8, hipMemcpyDeviceToHost, s));
+        HIPCK(hipMemcpyAsync(h + w, pl->blob + pl->goff[i] + (x.small ? x.off_ctl : x.off_crt), 8, hipMemcpyDeviceToHost, s));
         w += 2;
     }
     if (!pl->zidx.empty()) HIPCK(hipMemcpyAsync(h + w, pl->blob + pl->off_zncn, pl->zidx.size() * 8, hipMemcpyDeviceToHost, s));
     HIPCK(hipStreamSynchronize(s));
     for (size_t i = 0; i < pl->gb.size(); i++) {
         const GroupBuild &x = pl->gb[i];
-        const uint32_t flags = ((const uint32_t *)(h + at[i] + x.cnt))[1];
-        if (flags & 1) return nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond a top limb (wrong residues)");
-        for (uint64_t j = 0; j < x.cnt; j++) ncn[pl->gidx[i][j]] = h[at[i] + j];
+        if (group_lengths(x, h + at[i], (const uint32_t *)(h + at[i] + x.cnt), [&](uint64_t j, uint64_t n) { ncn[pl->gidx[i][j]] = n; }))
+            return nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond a top limb (wrong residues)");
     }
     for (size_t z = 0; z < pl->zidx.size(); z++) ncn[pl->zidx[z]] = h[w + z];
     return 0;

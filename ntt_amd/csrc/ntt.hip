@@ -8,234 +8,10 @@
 #include <string.h>
 #include "internal.h"
 #include "plan.h"
+#include "rounds.h"
 /* the round loops carry an unroll request that applies to the fixed-shape instantiations only */
 #pragma clang diagnostic ignored "-Wpass-failed"
 
-
-/* ---- the pass kernel -------------------------------------------------------------------------------------------------
- * A tile of T = W x 2^m x H points (T <= 2^13) is handled by T / 16 threads holding 16 points each in registers.  The m
- * stages run in rounds of up to 4 stages (radix 2..16 in registers); between rounds the tile goes through LDS once.
- * In a round over row bits [s_lo, s_lo + logR) (L = logw + s_lo), thread t owns G = 16 / R groups of R points; group g
- * has the base element
- *     eb = (tau mod 2^L) | (tau div 2^L) << (L + logR),   tau = g * nthr + t,
- * and point j of the group is element eb + j 2^L.  For every point the lanes of a wave touch consecutive LDS words
- * (and, in the first and last round, consecutive global addresses of a row).  Since the round's bits lie inside the
- * row field, point j sits at global offset ob + j 2^(s_lo + lo) and at bit-reversed row kb + brev(j) 2^(m - s_lo - logR):
- * addresses and boundary-twiddle exponents of a group are a base plus compile-time multiples.  Each thread reads and
- * writes exactly the elements of its groups within a round, so one barrier separates consecutive rounds.
- * Lazy reduction (bounds of arith.h): the DIF reduces its sum path at odd levels and at a round's last level (values
- * entering a butterfly stay within [-2p, 2p]); the DIT reduces both outputs at a round's last level only (after levels
- * 0..3 the outputs are within 1.75p, 2.5p, 3.5p, 4.5p + 2, and every mul_shoup input within 4p; with the trivial
- * first level of a lowest-bits round, 2p, 2.75p + 1, 3.75p + 2, 4.75p + 3, mul_shoup inputs within 3.75p + 2).
- * Where the round's low row bits are known to be zero at compile time, twiddles w^0 = 1 are not multiplied: the DIF
- * difference then follows the sum path's rule, the DIT skips them at its first level (where all of them are 1). */
-#define PASS_PTS 16               /* points per thread of full tiles; tiles below 16 points use one thread */
-
-template <int BITS>
-__device__ __forceinline__ constexpr uint32_t brev_c(uint32_t j)
-{
-    uint32_t r = 0;
-    for (int i = 0; i < BITS; i++) r |= ((j >> i) & 1u) << (BITS - 1 - i);
-    return r;
-}
-
-/* rlow == 0 known at compile time (the round over the lowest bits of a fixed-shape tile): the butterflies with
- * jj = 0 then have the twiddle w^0 = 1 */
-#define NTTM_TRIVIAL_W(rlow, jj) ((jj) == 0 && __builtin_constant_p(rlow) && (rlow) == 0)
-
-/* a stage table in global memory, read through a buffer resource: the table's base in scalar registers, the lane's
- * part of an index as the 32-bit vector offset and its compile-time part as the scalar offset, so a twiddle's address
- * costs no vector instruction (a 64-bit pointer sum costs two, in kernels bound by vector issue) */
-struct GTab {
-    __amdgpu_buffer_rsrc_t r;
-    __device__ __forceinline__ explicit GTab(const double2 *p)
-        : r(__builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, 0x7fffffff, 0x00020000)) {}
-};
-/* a stage table in LDS (or any pointer): restrict, so that its loads move freely around the tile's LDS stores */
-typedef const double2 *__restrict__ LTab;
-/* entry lane + fixed of a stage table (lane: the part that varies across lanes; fixed: a compile-time part) */
-__device__ __forceinline__ double2 tw_at(LTab tw, uint32_t lane, uint32_t fixed) { return tw[lane + fixed]; }
-__device__ __forceinline__ double2 tw_at(const GTab &tw, uint32_t lane, uint32_t fixed)
-{
-    typedef int v4i __attribute__((ext_vector_type(4)));
-    const v4i x = __builtin_amdgcn_raw_buffer_load_b128(tw.r, (int)(lane * 16u), (int)(fixed * 16u), 0);
-    double2 d;
-    __builtin_memcpy(&d, &x, 16);
-    return d;
-}
-
-template <int LOGR, typename TW>
-__device__ __forceinline__ void dif_group(double *v, int s_lo, uint32_t rlow, TW tw, double p, double pinv)
-{
-    constexpr int R = 1 << LOGR;
-#pragma unroll
-    for (int lev = 0; lev < LOGR; lev++) {
-        const int k = LOGR - 1 - lev, h = 1 << k;
-        const bool red = (lev & 1) || lev == LOGR - 1;
-#pragma unroll
-        for (int jj = 0; jj < h; jj++) {
-            /* a trivial twiddle: the difference follows the sum path's bound and reduction rule */
-            const bool one = NTTM_TRIVIAL_W(rlow, jj);
-            const double2 w = one ? make_double2(1.0, 0.0) : tw_at(tw, rlow, (1u << (s_lo + k)) + ((uint32_t)jj << s_lo));
-#pragma unroll
-            for (int j = jj; j < R; j += 2 * h) {
-                const double u = v[j], x = v[j + h];
-                const double sm = u + x, df = u - x;
-                v[j] = red ? reduce(sm, p, pinv) : sm;
-                v[j + h] = one ? (red ? reduce(df, p, pinv) : df) : mul_shoup(df, w.x, w.y, p);
-            }
-        }
-    }
-}
-
-template <int LOGR, typename TW>
-__device__ __forceinline__ void dit_group(double *v, int s_lo, uint32_t rlow, TW tw, double p, double pinv)
-{
-    constexpr int R = 1 << LOGR;
-#pragma unroll
-    for (int lev = 0; lev < LOGR; lev++) {
-        const int k = lev, h = 1 << k;
-        const bool red = lev == LOGR - 1;
-#pragma unroll
-        for (int jj = 0; jj < h; jj++) {
-            /* a trivial twiddle at the first level only (inputs within p: outputs within 2p, and the later bounds
-             * below hold with 0.25p to spare) */
-            const bool one = lev == 0 && NTTM_TRIVIAL_W(rlow, jj);
-            const double2 w = one ? make_double2(1.0, 0.0) : tw_at(tw, rlow, (1u << (s_lo + k)) + ((uint32_t)jj << s_lo));
-#pragma unroll
-            for (int j = jj; j < R; j += 2 * h) {
-                const double u = v[j], x = one ? v[j + h] : mul_shoup(v[j + h], w.x, w.y, p);
-                const double s1 = u + x, s2 = u - x;
-                v[j] = red ? reduce(s1, p, pinv) : s1;
-                v[j + h] = red ? reduce(s2, p, pinv) : s2;
-            }
-        }
-    }
-}
-
-/* geometry of the pass seen by one thread */
-struct PassPos {
-    int m, logw, lo, nthr, t;
-};
-
-/* f(slot, e, o, c, k) for every slot of a round: e the LDS index, o the global offset in the tile, c the column inside
- * the tile, k the bit-reversed row */
-/* PAD: e is the padded LDS index (SwzLds below) of the element; eb and the slot offsets j 2^L have disjoint bits, so
- * pad(eb + j 2^L) = pad(eb) + pad(j 2^L), the second term a compile-time constant in the fixed-shape kernels */
-template <int LOGR, int PTS, bool PAD = false, typename F>
-__device__ __forceinline__ void for_slots(const PassPos &pp, int s_lo, F f)
-{
-    constexpr int R = 1 << LOGR, G = PTS / R;
-    const int L = pp.logw + s_lo;
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        const uint32_t tau = (uint32_t)(g * pp.nthr + pp.t);
-        const uint32_t eb = (tau & ((1u << L) - 1)) | ((tau >> L) << (L + LOGR));
-        const uint32_t pe = PAD ? eb + (eb >> 5) : eb;
-        const uint32_t c = eb & ((1u << pp.logw) - 1), r = (eb >> pp.logw) & ((1u << pp.m) - 1);
-        const uint32_t h = eb >> (pp.logw + pp.m);
-        /* h << (lo + m) in 64 bits: a tile of the first pass of a 2^32-point transform has lo + m = 32 (and h = 0) */
-        const uint32_t ob = (uint32_t)((uint64_t)h << (pp.lo + pp.m)) + (r << pp.lo) + c;
-        const uint32_t kb = pp.m ? (__brev(r) >> (32 - pp.m)) : 0u;
-        const int ksh = pp.m - s_lo - LOGR;
-#pragma unroll
-        for (int j = 0; j < R; j++) {
-            const uint32_t dj = (uint32_t)j << L;
-            f(g * R + j, pe + (PAD ? dj + (dj >> 5) : dj), ob + ((uint32_t)j << (s_lo + pp.lo)), c,
-              kb + (brev_c<LOGR>(j) << ksh));
-        }
-    }
-}
-
-/* the radix step of one round on all PTS slots: PTS / R groups of R points */
-/* TW: GTab (a global stage table) or LTab (a table in LDS, named explicitly so that it stays restrict) */
-template <int LOGR, bool INV, int PTS, typename TW>
-__device__ __forceinline__ void round_compute(double *v, const PassPos &pp, int s_lo, TW tw, double p, double pinv)
-{
-    constexpr int R = 1 << LOGR, G = PTS / R;
-    const int L = pp.logw + s_lo;
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        const uint32_t tau = (uint32_t)(g * pp.nthr + pp.t);
-        const uint32_t rlow = (tau & ((1u << L) - 1)) >> pp.logw;      /* row bits below s_lo */
-        if (INV) dit_group<LOGR, TW>(v + g * R, s_lo, rlow, tw, p, pinv);
-        else dif_group<LOGR, TW>(v + g * R, s_lo, rlow, tw, p, pinv);
-    }
-}
-
-/* dit_group with the inverse twiddles taken from the FORWARD stage table: w^-j of stage s is the mirrored forward entry
- * negated, w^-j = -w^(2^s - j) (w^(2^s) = -1), the negation folded into the butterfly (the product's sign flipped), and
- * w^0 = 1 taken from entry 1 (stage 0).  Lets a kernel keep one small table in LDS for both directions. */
-template <int LOGR>
-__device__ __forceinline__ void dit_group_mirror(double *v, int s_lo, uint32_t rlow, const double2 *tw, double p,
-                                                 double pinv)
-{
-    constexpr int R = 1 << LOGR;
-#pragma unroll
-    for (int lev = 0; lev < LOGR; lev++) {
-        const int k = lev, h = 1 << k, s = s_lo + k;
-        const bool red = lev == LOGR - 1;
-#pragma unroll
-        for (int jj = 0; jj < h; jj++) {
-            const bool one = lev == 0 && NTTM_TRIVIAL_W(rlow, jj);
-            const uint32_t j = rlow + ((uint32_t)jj << s_lo);
-            double2 w;                                   /* (w, wq) negated for a mirrored entry */
-            if (jj == 0) {
-                const bool z = rlow == 0;
-                const double2 t = tw[z ? 1u : (2u << s) - j];
-                w = z ? t : make_double2(-t.x, -t.y);
-            } else {
-                const double2 t = tw[(2u << s) - j];
-                w = make_double2(-t.x, -t.y);
-            }
-#pragma unroll
-            for (int i = jj; i < R; i += 2 * h) {
-                const double u = v[i], x = one ? v[i + h] : mul_shoup(v[i + h], w.x, w.y, p);
-                const double s1 = u + x, s2 = u - x;
-                v[i] = red ? reduce(s1, p, pinv) : s1;
-                v[i + h] = red ? reduce(s2, p, pinv) : s2;
-            }
-        }
-    }
-}
-template <int LOGR, int PTS>
-__device__ __forceinline__ void round_compute_mirror(double *v, const PassPos &pp, int s_lo, const double2 *tw, double p,
-                                                     double pinv)
-{
-    constexpr int R = 1 << LOGR, G = PTS / R;
-    const int L = pp.logw + s_lo;
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        const uint32_t tau = (uint32_t)(g * pp.nthr + pp.t);
-        const uint32_t rlow = (tau & ((1u << L) - 1)) >> pp.logw;
-        dit_group_mirror<LOGR>(v + g * R, s_lo, rlow, tw, p, pinv);
-    }
-}
-
-/* rounds of a pass: sizes of at most maxr bits (the log2 of the points per thread, at most 4), balanced; forward from
- * the top bits down, inverse from bit 0 up */
-__device__ __forceinline__ int round_count(int m, int maxr) { return (m + maxr - 1) / maxr; }
-__device__ __forceinline__ void round_split(int m, int i, int *s_lo, int *logR, bool inv, int maxr)
-{
-    const int nr = round_count(m, maxr), q = m / nr, rem = m % nr;
-    int lo = 0;                                     /* rounds in ascending bit order: sizes q+1 first (rem of them) */
-    int k = inv ? i : nr - 1 - i;
-    for (int r = 0; r < k; r++) lo += q + (r < rem ? 1 : 0);
-    *s_lo = lo; *logR = q + (k < rem ? 1 : 0);
-}
-
-/* call body.template operator()<LOGR>() with the runtime round size */
-#define ROUND_SWITCH(logR, ...) \
-    switch (logR) { \
-    case 4: { constexpr int LR = 4; __VA_ARGS__ } break; \
-    case 3: { constexpr int LR = 3; __VA_ARGS__ } break; \
-    case 2: { constexpr int LR = 2; __VA_ARGS__ } break; \
-    default: { constexpr int LR = 1; __VA_ARGS__ } break; }
-
-/* limbs and planes as global-space pointers: an address read from memory is generic to the compiler, and a generic
- * (flat) access counts against the LDS counter too */
-typedef const __attribute__((address_space(1))) uint64_t *GLimb;
-typedef __attribute__((address_space(1))) double *GPlane;
 
 /* the pass's input element: from the plane, or (the first forward pass) from the operand limbs, zero beyond them */
 __device__ __forceinline__ double input_limb_raw(const PassArgs &a, uint64_t gi, double p, double pinv)
@@ -282,18 +58,6 @@ __device__ __forceinline__ uint64_t y_index(const PassArgs &a, uint64_t gi)
     return a.ymode == NTTM_Y_FULL ? gi : a.ymode == NTTM_Y_BCAST ? (gi & nmask)
                                        : ((((gi >> a.logn) >> 1) << a.logn) | (gi & nmask));
 }
-
-/* The tile in LDS, padded: element e at word e + e / 32 (LDS_WORDS(T) words for T elements).  A round over the lowest
- * row bits of a contiguous tile has lanes 16 elements apart, which unpadded all hit the same bank pair; padded, every
- * round, the linear staging and the strided tiles' rounds spread over all banks.  For a group's slots
- * e = eb + j 2^L the padded index is pad(eb) + a compile-time multiple of j (L >= 5, or the slot bits below bit 5 with
- * eb's bits clear), so the offsets stay immediate. */
-#define LDS_WORDS(T) ((T) + ((T) >> 5))
-struct SwzLds {
-    double *p;
-    __device__ __forceinline__ double &operator[](uint32_t e) const { return p[e + (e >> 5)]; }
-    __device__ __forceinline__ double &at(uint32_t pe) const { return p[pe]; }   /* an index padded already */
-};
 
 enum { PM_FWD = 0, PM_FWD_LIMB = 1, PM_INV = 2, PM_INV_PW = 3 };
 
@@ -667,102 +431,15 @@ __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
     __builtin_amdgcn_s_waitcnt(0);                                     /* no LDS fetch in flight past the block's end */
 }
 
-/* ---- the fused last forward pass + pointwise product + first inverse pass ------------------------------------------------
- * For the contiguous low-bit pass (lo = 0, m + logh <= 12): the DIF rounds of the forward transform, the product with
- * y in a linear pass over LDS (y read coalesced), the DIT rounds of the inverse, one read and one write of x.
- * LIMB: x comes from the operand limbs (a transform that is a single pass). */
-#define FUSED_LOG 12
-template <bool LIMB, int PTS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_fused(PassArgs a)
-{
-    __shared__ double xs_raw[LDS_WORDS(1 << FUSED_LOG)];
-    const SwzLds xs{xs_raw};
-    constexpr int MAXR = PTS >= 16 ? 4 : 3;
-    PassPos pp; pp.m = a.m; pp.logw = 0; pp.lo = 0;
-    const int T = 1 << (a.m + a.logh);
-    pp.nthr = T / PTS; pp.t = threadIdx.x;
-    const bool active = pp.t < pp.nthr;
-    const double p = a.pk.p, pinv = a.pk.pinv;
-    const uint64_t gbase = (uint64_t)blockIdx.x << (a.m + a.logh);  /* lo = 0, W = 1: the tile is contiguous */
-    double *xt = a.x + gbase;
-    const double *yt = a.y + gbase;                                   /* FULL layout (the product path) */
-    const int nr = round_count(a.m, MAXR);
-    double v[PTS];
-    int s_lo, logR;
-    auto in_at = [&](uint32_t o) -> double { return LIMB ? input_limb(a, gbase + o, p, pinv) : xt[o]; };
-
-    round_split(a.m, 0, &s_lo, &logR, false, MAXR);
-    if (s_lo >= 4) {
-        if (active) ROUND_SWITCH(logR, for_slots<LR, PTS>(pp, s_lo, [&](int sl, uint32_t, uint32_t o, uint32_t,
-                                                                            uint32_t) { v[sl] = in_at(o); });)
-    } else {
-        if (active) {
-#pragma unroll
-            for (int sl = 0; sl < PTS; sl++) { const uint32_t e = sl * pp.nthr + pp.t; xs[e] = in_at(e); }
-        }
-        __syncthreads();
-        if (active) ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
-                                                                            uint32_t) { v[sl] = xs.at(e); });)
-    }
-    for (int i = 0; i < nr; i++) {                               /* forward, top bits first */
-        round_split(a.m, i, &s_lo, &logR, false, MAXR);
-        if (i > 0) {
-            __syncthreads();
-            if (active) ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t,
-                                                                                uint32_t, uint32_t) { v[sl] = xs.at(e); });)
-        }
-        if (active) ROUND_SWITCH(logR, round_compute<LR, false, PTS>(v, pp, s_lo, GTab(a.tw.stage), p, pinv);)
-        if (active) ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
-                                                                            uint32_t) { xs.at(e) = v[sl]; });)
-    }
-    __syncthreads();
-    if (active) {                                                /* the pointwise product, linear: y read coalesced */
-#pragma unroll
-        for (int sl = 0; sl < PTS; sl++) {
-            const uint32_t e = sl * pp.nthr + pp.t;
-            xs[e] = mul_barrett(xs[e], yt[e], p, pinv);
-        }
-    }
-    for (int i = 0; i < nr; i++) {                               /* inverse, bit 0 first */
-        round_split(a.m, i, &s_lo, &logR, true, MAXR);
-        __syncthreads();
-        if (active) ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
-                                                                            uint32_t) { v[sl] = xs.at(e); });)
-        if (active) ROUND_SWITCH(logR, round_compute<LR, true, PTS>(v, pp, s_lo, GTab(a.twi.stage), p, pinv);)
-        if (i + 1 < nr && active)
-            ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
-                                                                    uint32_t) { xs.at(e) = v[sl]; });)
-    }
-    if (s_lo >= 4) {
-        if (active) ROUND_SWITCH(logR, for_slots<LR, PTS>(pp, s_lo, [&](int sl, uint32_t, uint32_t o, uint32_t,
-                                                                            uint32_t) {
-            double x = v[sl];
-            if (a.do_scale) x = mul_shoup(x, a.scale.x, a.scale.y, p);
-            xt[o] = x; });)
-    } else {
-        if (active) ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
-                                                                            uint32_t) { xs.at(e) = v[sl]; });)
-        __syncthreads();
-        if (active) {
-#pragma unroll
-            for (int sl = 0; sl < PTS; sl++) {
-                const uint32_t e = sl * pp.nthr + pp.t;
-                double x = xs[e];
-                if (a.do_scale) x = mul_shoup(x, a.scale.x, a.scale.y, p);
-                xt[e] = x;
-            }
-        }
-    }
-}
-
 /* ---- the double-fused last pass: B's last forward pass + A's last forward pass + pointwise + A's first inverse pass ---
- * Same geometry as k_fused (lo = 0, m + logh <= 12).  The forward's last round and the inverse's first round cover the
+ * For the contiguous low-bit pass (lo = 0, m + logh <= 12).  The forward's last round and the inverse's first round cover the
  * same bits [0, logR) with the same slot layout, so B's transformed tile stays in registers (bv) and is never written;
  * the product v * bv and the first inverse round follow A's last forward round without an LDS round trip.
  * One read of A (or its limbs), one read of B (or its limbs), one write of A. */
 /* stw: the forward stage table's first 2^STW_LOG entries in LDS (nullptr: none); rounds whose stages all lie below
  * STW_LOG read their twiddles there */
 #define STW_LOG 8
+#define FUSED_LOG 12
 /* LT: stw is the LDS copy of the stage table's low entries, for the rounds after the first */
 /* loaded(): called once the tile's loads have been issued */
 template <int PTS, int MAXR, bool LIMBS, bool LT, typename F>
@@ -1187,35 +864,6 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
 #undef NTTM_PASS_LAUNCH_G
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_pass launch");
-}
-
-/* the fused last forward pass + pointwise + first inverse pass; g must be a contiguous pass (lo = 0) of at most 2^12
- * points per tile and at least 16 */
-int nttm_run_fused(const PassArgs &a, const PassGeom &g, hipStream_t s)
-{
-    if (!pass_geom_ok(g, a.logn, a.batch) || g.lo != 0 || g.logw != 0 || g.m + g.logh > FUSED_LOG ||
-        g.m + g.logh < 4 || !a.y || a.ymode != NTTM_Y_FULL)
-        return nttm_fail(NTTM_EINVAL, "internal: bad fused pass geometry");
-    const uint64_t tiles = plan_tiles(g, a.logn, a.batch);
-    if (tiles > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "internal: too many tiles");
-    PassArgs b = a; b.lo = 0; b.m = g.m; b.logw = 0; b.logh = g.logh;
-    const bool limb = b.limbs || b.ldesc;
-    const double pts = (double)(a.batch << a.logn);
-    /* read x (or its limbs), read y, write x */
-    prof_begin(limb ? "k_fused<limb>" : "k_fused", pts * (limb ? 16.0 : 24.0), s);
-    const int T = 1 << (g.m + g.logh);
-    const int ppt = (T >= 64 * g_pts && T <= 512 * g_pts) ? g_pts : PASS_PTS;
-    const unsigned nthr = (unsigned)(T / ppt < 64 ? 64 : T / ppt);
-    if (nthr > 512) return nttm_fail(NTTM_EINVAL, "internal: %u threads per tile", nthr);
-    if (ppt == 8) {
-        if (limb) hipLaunchKernelGGL((k_fused<true, 8>), dim3((unsigned)tiles), dim3(nthr), 0, s, b);
-        else hipLaunchKernelGGL((k_fused<false, 8>), dim3((unsigned)tiles), dim3(nthr), 0, s, b);
-    } else {
-        if (limb) hipLaunchKernelGGL((k_fused<true, PASS_PTS>), dim3((unsigned)tiles), dim3(nthr), 0, s, b);
-        else hipLaunchKernelGGL((k_fused<false, PASS_PTS>), dim3((unsigned)tiles), dim3(nthr), 0, s, b);
-    }
-    prof_end(s);
-    return nttm_hip_check(hipGetLastError(), "k_fused launch");
 }
 
 /* Bound by vector issue (166 of 178 vector instructions a point are FP64).  A block's first loads wait for nothing but its

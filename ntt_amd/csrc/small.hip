@@ -1,0 +1,308 @@
+/* small.hip - whole products in one kernel: every transform of up to 2^12 points, the pointwise product, the CRT and
+ * the carries of a product inside one workgroup.
+ *
+ * A product of up to 4096 coefficients is three transforms per prime over at most 32 KiB of LDS per prime: the residues
+ * of every prime fit a workgroup's LDS at once, so nothing but the operands' limbs and the product's own limbs crosses
+ * HBM and no other launch follows.  (In separate launches a product of this size took three: the double-fused pass,
+ * the CRT with its planes through HBM, the carry scan and its fix.)
+ *
+ * A block holds a tile of T = max(n, 1024) points per prime, H = T / n products of n points, 16 points per thread: T / 16
+ * threads per prime, so a wave works for one prime (T = 1024: exactly one, whose rounds then need no barrier).
+ *   - transforms: the rounds of k_fused2 on each prime's tile; B's transform stays in registers; the inverse ends in LDS in
+ *     natural order;
+ *   - digits: each coefficient's residues are replaced in place by its base-10^18 digits (crt_digits);
+ *   - limbs: words of 64 limbs, one per wave and step.  Product limbs run to n + 2 (n coefficients, two digits more), so
+ *     a product has W = n / 64 + 1 words and a block at most 65.  A word's carry chain is one addition of its ballot
+ *     masks (crt.hip), and the chain over the words the same once more: lane l holds word l's carry out for either
+ *     carry in, a product's last word passes nothing on.
+ * Bound by vector issue as k_fused2 is: 2846 vector instructions per wave and prime at n = 4096 and about 160 per
+ * coefficient for the digits. */
+#include <string.h>
+#include "internal.h"
+#include "rounds.h"
+#include "crt_dev.h"
+
+#define SMALL_LOG_MIN 7
+#define SMALL_LOG_MAX 12
+
+struct SmallArgs {
+    const LoadDesc *ld; const CrtDesc *cd;      /* cnt products in device memory, or null: the one product below */
+    LoadDesc ld1; CrtDesc cd1;
+    uint64_t cnt;
+    uint64_t *ncn;                              /* or null: the normalized lengths, bit 63 set for a carry beyond the top */
+    uint32_t *ctl;                              /* one product: words 0, 1 written (1: the error); else word 1 gets it or-ed in */
+    uint64_t *stamps;                           /* or null: the device clock at the four phase boundaries */
+    const double2 *stage[NTTM_MAX_PRIMES], *istage[NTTM_MAX_PRIMES];
+    double2 ninv[NTTM_MAX_PRIMES];
+    CrtConst cc;
+};
+
+/* a barrier between the threads of one prime: the whole block's, or (one wave per prime) none but the compiler's, since a
+ * wave's LDS operations complete in order */
+template <bool WAVE> __device__ __forceinline__ void prime_barrier()
+{
+    if (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else __syncthreads();
+}
+
+template <int LOGN, int NP>
+__global__ __launch_bounds__(NP << ((LOGN > 10 ? LOGN : 10) - 4)) void k_small(SmallArgs a)
+{
+    constexpr int TL = LOGN > 10 ? LOGN : 10, T = 1 << TL, N = 1 << LOGN, H = T / N, PTS = 16;
+    constexpr int NT = T / PTS, NTH = NP * NT, NW = NTH / 64;        /* threads per prime and block, waves */
+    constexpr int SW = LOGN < 8 ? LOGN : 8;                          /* stages whose twiddles are kept in LDS */
+    constexpr int WPP = N / 64 + 1, NWORD = H * WPP, IT = (NWORD + NW - 1) / NW;
+    constexpr bool WAVE = NT == 64;
+    constexpr int NR = (LOGN + 3) / 4;
+    static_assert(NWORD <= 65, "the word chain is one 64-bit addition and its carry out");
+    typedef __attribute__((address_space(1))) uint64_t *GOut;
+    struct Prod { const uint64_t *a, *b, *x; uint64_t *c; uint32_t na, nb, nx, nc, ncoef, trunc; };
+    __shared__ double pl[NP][LDS_WORDS(T)];
+    __shared__ double2 stw[NP][1 << SW];
+    __shared__ Prod sp[H];
+    __shared__ uint64_t sgx[NWORD], sgy[NWORD];
+    __shared__ uint32_t slen[H], serr[H];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t pi = __builtin_amdgcn_readfirstlane((uint32_t)tid / NT);
+    const int t = tid & (NT - 1);
+    const uint64_t prod0 = (uint64_t)blockIdx.x * H;
+    if (a.stamps) stamp_clock(a.stamps);
+
+    const double2 *gst = a.stage[pi];
+#pragma unroll
+    for (int i = 0; i < ((1 << SW) + NT - 1) / NT; i++) {
+        const int e = i * NT + t;
+        if (e < (1 << SW)) stw[pi][e] = gst[e];
+    }
+    if (tid < H) {
+        Prod q; q.a = q.b = q.x = (const uint64_t *)gst; q.c = nullptr;      /* a dead product reads no limb: any address */
+        q.na = q.nb = q.nx = q.nc = q.ncoef = q.trunc = 0;
+        const uint64_t i = prod0 + tid;
+        if (i < a.cnt) {
+            LoadDesc l = a.ld1; CrtDesc c = a.cd1;
+            if (a.ld) { l = a.ld[i]; c = a.cd[i]; }
+            q.a = l.a; q.b = l.b; q.na = (uint32_t)l.na; q.nb = (uint32_t)l.nb;
+            if (c.x && c.nx) { q.x = c.x; q.nx = (uint32_t)c.nx; }
+            q.c = c.c; q.nc = (uint32_t)c.nc; q.ncoef = (uint32_t)c.ncoef; q.trunc = c.trunc != 0;
+        }
+        sp[tid] = q; slen[tid] = 0; serr[tid] = 0;
+    }
+    __syncthreads();
+
+    /* ---- the cyclic convolution modulo this wave's prime, into pl[pi] in natural order */
+    const double p = a.cc.pk[pi].p, pinv = a.cc.pk[pi].pinv;
+    {
+        const SwzLds xs{pl[pi]};
+        const double2 *lt = stw[pi];
+        const GTab gf(a.stage[pi]), gi(a.istage[pi]);
+        PassPos pp; pp.m = LOGN; pp.logw = 0; pp.lo = 0; pp.nthr = NT; pp.t = t;
+        int s_lo, logR;
+        round_split(LOGN, 0, &s_lo, &logR, false, 4);
+        uint64_t raw[2][PTS];
+        uint32_t in[2] = {0, 0};                                     /* bit sl: the slot lies inside the operand */
+#pragma unroll
+        for (int w = 0; w < 2; w++)                                  /* B's limbs, then A's: all requested at once */
+            ROUND_SWITCH(logR, for_slots<LR, PTS>(pp, s_lo, [&](int sl, uint32_t, uint32_t o, uint32_t, uint32_t) {
+                const Prod &q = sp[H > 1 ? o >> LOGN : 0];
+                const uint32_t k = o & (N - 1), nl = w ? q.na : q.nb;
+                const bool inside = k < nl;
+                raw[w][sl] = ((GLimb)(w ? q.a : q.b))[inside ? k : 0];
+                in[w] |= (uint32_t)inside << sl;
+            });)
+        double v[PTS], bv[PTS];
+        const double2 ninv = a.ninv[pi];
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+            if (w) prime_barrier<WAVE>();                            /* B's last LDS reads before A's first writes */
+#pragma unroll
+            for (int sl = 0; sl < PTS; sl++) {
+                double x = (in[w] >> sl) & 1 ? limb_to_res(raw[w][sl], p, pinv) : 0.0;
+                if (w == 0) x = mul_shoup(x, ninv.x, ninv.y, p);
+                v[sl] = x;
+            }
+#pragma unroll
+            for (int i = 0; i < NR; i++) {                           /* top bits first; the last round stays in registers */
+                round_split(LOGN, i, &s_lo, &logR, false, 4);
+                if (i > 0) {
+                    prime_barrier<WAVE>();
+                    ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
+                        v[sl] = xs.at(e); });)
+                }
+                if (i == 0 && LOGN > SW) { ROUND_SWITCH(logR, round_compute<LR, false, PTS>(v, pp, s_lo, gf, p, pinv);) }
+                else { ROUND_SWITCH(logR, round_compute<LR, false, PTS, LTab>(v, pp, s_lo, lt, p, pinv);) }
+                if (i + 1 < NR)
+                    ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
+                        xs.at(e) = v[sl]; });)
+            }
+            if (w == 0) {
+#pragma unroll
+                for (int sl = 0; sl < PTS; sl++) bv[sl] = v[sl];
+            }
+        }
+        if (a.stamps) stamp_clock(a.stamps + 1);
+#pragma unroll
+        for (int sl = 0; sl < PTS; sl++) v[sl] = mul_barrett(v[sl], bv[sl], p, pinv);
+#pragma unroll
+        for (int i = 0; i < NR; i++) {                               /* bit 0 first; round 0 has the layout in v */
+            round_split(LOGN, i, &s_lo, &logR, true, 4);
+            if (i > 0) {
+                prime_barrier<WAVE>();
+                ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
+                    v[sl] = xs.at(e); });)
+            }
+            if (i == NR - 1 && LOGN > SW) { ROUND_SWITCH(logR, round_compute<LR, true, PTS>(v, pp, s_lo, gi, p, pinv);) }
+            else { ROUND_SWITCH(logR, round_compute_mirror<LR, PTS>(v, pp, s_lo, lt, p, pinv);) }
+            ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
+                xs.at(e) = v[sl]; });)
+        }
+    }
+
+    /* ---- the product's x limbs are requested; the residues become digits in place */
+    uint64_t xk[IT], xp[IT];
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+        const int w = wave + i * NW;
+        const int h = w / WPP;
+        const uint32_t k = (uint32_t)(w - h * WPP) * 64 + lane;
+        xk[i] = xp[i] = 0;
+        if (w < NWORD) {
+            const Prod &q = sp[h];
+            if (k < q.nx && k < q.nc) xk[i] = ((GLimb)q.x)[k];
+            if (lane == 0 && k >= 1 && k - 1 < q.nx) xp[i] = ((GLimb)q.x)[k - 1];
+        }
+    }
+    __syncthreads();
+    if (a.stamps) stamp_clock(a.stamps + 2);
+    for (int e = tid; e < T; e += NTH) {
+        const bool live = (uint32_t)(e & (N - 1)) < sp[H > 1 ? e >> LOGN : 0].ncoef;
+        double r[NP];
+        uint64_t d[NP];
+#pragma unroll
+        for (int j = 0; j < NP; j++) r[j] = live ? pl[j][e + (e >> 5)] : 0.0;
+        crt_digits<NP>(a.cc, r, d);
+#pragma unroll
+        for (int j = 0; j < NP; j++) pl[j][e + (e >> 5)] = __longlong_as_double((long long)d[j]);
+    }
+    __syncthreads();
+
+    /* ---- limbs: v_k = sum_j d_j[k - j] + x_k < NP B + 2^31, w_k = v_k - q_k B + q_(k-1) */
+    auto digit = [&](int h, int j, int k) -> uint64_t {              /* d_j of coefficient k of product h */
+        const int e = h * N + k;
+        return k >= 0 && k < N ? (uint64_t)__double_as_longlong(pl[j][e + (e >> 5)]) : 0;
+    };
+    auto vsum = [&](int h, int k, uint64_t x) -> uint64_t {
+        uint64_t v = x;
+#pragma unroll
+        for (int j = 0; j < NP; j++) v += digit(h, j, k - j);
+        return v;
+    };
+    auto quot = [](uint64_t v) -> uint32_t {
+        uint32_t q = 0;
+#pragma unroll
+        for (int c = 1; c <= NP; c++) q += v >= (uint64_t)c * NTTM_B;
+        return q;
+    };
+    uint64_t wv[IT], GX[IT], GY[IT];
+    uint32_t ql[IT];
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+        const int w = wave + i * NW;
+        wv[i] = GX[i] = GY[i] = 0; ql[i] = 0;
+        if (w < NWORD) {
+            const int h = w / WPP, k = (w - h * WPP) * 64 + lane;
+            const int nc = (int)sp[h].nc;
+            const uint64_t v = k < nc ? vsum(h, k, xk[i]) : 0;
+            const uint32_t q = quot(v);
+            uint32_t qp = __shfl_up(q, 1, 64);
+            if (lane == 0) qp = k >= 1 && k <= nc ? quot(vsum(h, k - 1, xp[i])) : 0u;
+            wv[i] = v - (uint64_t)q * NTTM_B + qp;
+            if (k >= nc) wv[i] = 0;
+            ql[i] = q;
+            const uint64_t g = __ballot(wv[i] >= NTTM_B), pr = __ballot(wv[i] == NTTM_B - 1);
+            GX[i] = g; GY[i] = g | pr;
+            if (lane == 0) { sgx[w] = g; sgy[w] = g | pr; }
+        }
+    }
+    __syncthreads();
+    /* the carry into every word of the block: bit w of CI (word 64: cout) */
+    uint64_t CI; uint32_t cout64;
+    {
+        uint32_t f0 = 0, f1 = 0;
+        if (lane < NWORD && lane % WPP != WPP - 1) {
+            f0 = add_cout(sgx[lane], sgy[lane], 0); f1 = add_cout(sgx[lane], sgy[lane], 1);
+        }
+        const uint64_t G = __ballot(f0 != 0), GP = __ballot(f1 != 0), S = G + GP;
+        CI = S ^ G ^ GP; cout64 = S < G;
+    }
+#pragma unroll
+    for (int i = 0; i < IT; i++) {
+        const int w = wave + i * NW;
+        if (w < NWORD) {
+            const int h = w / WPP, k = (w - h * WPP) * 64 + lane;
+            const int nc = (int)sp[h].nc;
+            const uint32_t c = w < 64 ? (uint32_t)(CI >> w) & 1u : cout64;
+            const uint64_t S = GX[i] + GY[i] + c, CB = S ^ GX[i] ^ GY[i];      /* bit b: the carry into bit b */
+            const uint32_t oin = (uint32_t)(CB >> lane) & 1u;
+            const uint32_t oout = lane == 63 ? add_cout(GX[i], GY[i], c) : (uint32_t)(CB >> (lane + 1)) & 1u;
+            const uint64_t limb = wv[i] + oin - (oout ? NTTM_B : 0);
+            if (k < nc) ((GOut)sp[h].c)[k] = limb;
+            const uint64_t nz = __ballot(k < nc && limb != 0);
+            if (nz && lane == 0) atomicMax(&slen[h], (uint32_t)(k + 64 - __clzll((long long)nz)));
+            if (k + 1 == nc && !sp[h].trunc) {                       /* the last limb: nothing may remain beyond it */
+                uint64_t extra = ql[i] + oout;
+#pragma unroll
+                for (int e = 1; e < NP; e++)
+#pragma unroll
+                    for (int j = e; j < NP; j++) extra += digit(h, j, k + e - j);
+                serr[h] = extra != 0;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < H && prod0 + tid < a.cnt) {
+        const uint32_t err = serr[tid];
+        if (a.ncn) a.ncn[prod0 + tid] = slen[tid] | (uint64_t)err << 63;
+        if (!a.ld) { a.ctl[0] = 0; a.ctl[1] = err; }
+        else if (err && a.ctl) atomicOr(a.ctl + 1, 1u);
+    }
+    if (a.stamps) stamp_clock(a.stamps + 3);
+}
+
+/* the points of the kernel for a transform of 2^logn points (0: too long) */
+int nttm_small_log(int logn) { return logn > SMALL_LOG_MAX ? 0 : logn < SMALL_LOG_MIN ? SMALL_LOG_MIN : logn; }
+
+/* cnt products of at most 2^logn coefficients (logn from nttm_small_log), from device descriptors, or (ld null) the one
+ * product ld1, cd1, whose flags go to ctl's two words (device or pinned host memory).  stage / istage: the forward and
+ * inverse stage tables of the np primes; ninv: 2^-logn modulo each */
+int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1,
+                   uint64_t cnt, uint64_t *ncn, uint32_t *ctl, const TwTables *fwd, const TwTables *inv, const double2 *ninv,
+                   const CrtConst &cc, hipStream_t s, double alg_bytes, uint64_t *stamps)
+{
+    if (np < 3 || np > NTTM_MAX_PRIMES || logn < SMALL_LOG_MIN || logn > SMALL_LOG_MAX || !cnt || (!ld != !cd) ||
+        (!ld && (!ld1 || !cd1 || cnt != 1 || !ctl)))
+        return nttm_fail(NTTM_EINVAL, "internal: small products");
+    SmallArgs a; memset(&a, 0, sizeof a);
+    a.ld = ld; a.cd = cd; a.cnt = cnt; a.ncn = ncn; a.ctl = ctl; a.stamps = stamps; a.cc = cc;
+    if (ld1) a.ld1 = *ld1;
+    if (cd1) a.cd1 = *cd1;
+    for (int i = 0; i < np; i++) { a.stage[i] = fwd[i].stage; a.istage[i] = inv[i].stage; a.ninv[i] = ninv[i]; }
+    const int tl = logn > 10 ? logn : 10, h = 1 << (tl - logn);
+    const uint64_t blocks = (cnt + h - 1) / h;
+    if (blocks > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "internal: too many small products");
+    const dim3 grid((unsigned)blocks), blk((unsigned)(np << (tl - 4)));
+    prof_begin("k_small", alg_bytes, s);
+#define SMALL_LAUNCH(L) \
+    case L: \
+        if (np == 3) hipLaunchKernelGGL((k_small<L, 3>), grid, blk, 0, s, a); \
+        else hipLaunchKernelGGL((k_small<L, 4>), grid, blk, 0, s, a); \
+        break;
+    switch (logn) {
+    SMALL_LAUNCH(7) SMALL_LAUNCH(8) SMALL_LAUNCH(9) SMALL_LAUNCH(10) SMALL_LAUNCH(11)
+    default: SMALL_LAUNCH(12)
+    }
+#undef SMALL_LAUNCH
+    prof_end(s);
+    return nttm_hip_check(hipGetLastError(), "k_small launch");
+}

@@ -106,3 +106,56 @@ def test_phase_times(schedule, n, par):
         ph = lib.last_phase_ms()
         say("phases", n, par, ph, wall)
         assert all(p >= 0 for p in ph) and 0 < sum(ph) <= wall + 0.03
+
+
+def _limbs(kind, n, s):
+    if kind == "max":
+        return np.full(n, O.B - 1, dtype=np.uint64), s
+    if kind == "zero":
+        return np.zeros(n, dtype=np.uint64), s
+    return O.gen_limbs(n, s)
+
+
+# around every length of the one-kernel products (2^7 .. 2^12 points) and just above the longest
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 128, 129, 255, 256, 257, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097])
+@pytest.mark.parametrize("nprimes", [0, 4])
+def test_one_kernel_products(schedule, n, nprimes):
+    """c = a b and c = a b + x with n coefficients: random limbs, all limbs B - 1 (carry chains through every word),
+    zeros, x of every length class, the low limbs alone (a cut), c over a; singly and as one batch with neighbours of
+    the same kernel, an incomplete last block among them"""
+    import torch
+    lib = schedule(nprimes=nprimes)
+    ops, s = [], n
+    for kind in ("random", "max", "zero"):
+        for na in sorted({1, (n + 1) // 2, n}):
+            nb = n + 1 - na
+            a, s = _limbs(kind, na, s)
+            b, s = _limbs("random" if kind == "zero" else kind, nb, s)
+            for nx in (None, 1, n, n + 1):
+                x = None if nx is None else _limbs("random" if kind == "random" else "max", nx, s)[0]
+                ops.append((a, b, x))
+    say("one kernel", n, nprimes)
+    want = [O.mul_school(a, b, x) for a, b, x in ops]
+    items = [(dev(a), dev(b), None if x is None else dev(x),
+              torch.full((len(w),), -1, dtype=torch.int64, device="cuda")) for (a, b, x), w in zip(ops, want)]
+    prods = lib.make_prods(items)
+    lib.mul_batch(prods)
+    plan = lib.BatchPlan(prods, autotune=False)
+    for run in (lambda: None, plan.run):
+        run()
+        for it, w, pr in zip(items, want, prods):
+            nz = np.nonzero(w)[0]
+            assert np.array_equal(host(it[3]), w) and pr.ncn == (int(nz[-1]) + 1 if len(nz) else 0)
+            it[3].fill_(-1)
+    assert plan.ncn() == [pr.ncn for pr in prods]
+    plan.close()
+    for (a, b, x), it, w in list(zip(ops, items, want))[::3]:
+        got = lib.mul(it[0], it[1]) if x is None else lib.mul_add(it[0], it[1], it[2])
+        assert np.array_equal(host(got), w)
+    a, b, w = ops[0][0], ops[0][1], want[0]
+    for cut in sorted({1, (n + 1) // 2, n}):
+        assert np.array_equal(host(lib.mul_cut(items[0][0], items[0][1], w=cut)), w[:cut])
+    over = torch.full((len(w),), -1, dtype=torch.int64, device="cuda")
+    over[:len(a)] = items[0][0]
+    lib.mul(over[:len(a)], items[0][1], out=over)
+    assert np.array_equal(host(over), w)
