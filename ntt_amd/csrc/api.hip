@@ -26,7 +26,6 @@ void nttm_set_stream(int on, int ncu);
 #define NTTM_PRODUCT_LOGN_MIN 4    /* products use at least 2^4 points, so every fused tile has >= 16 */
 #define NTTM_STAGE_CHUNK ((size_t)1 << 30)   /* staged bytes per sub-batch of a batch with host operands (default) */
 struct LoadArgs;
-int nttm_run_u64_to_f64(double *x, uint64_t count, hipStream_t s);
 int nttm_run_cvt_u64_f64(double *dst, const uint64_t *src, uint64_t count, hipStream_t s);
 int nttm_run_f64_to_canon(double *x, uint64_t count, const PrimeK &pk, hipStream_t s);
 int nttm_run_pw_u64(uint64_t *x, const uint64_t *y, uint64_t count, const PrimeK &pk, hipStream_t s);
@@ -37,11 +36,12 @@ int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which
 /* the CRT of products whose blocks are [blk0, blk0 + nblk) of the launch's block numbering (limbs for a carry in of 0),
  * then every block's carry; nttm_crt_launch_one: both for one product */
 int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np,
-                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp = nullptr);
+                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp = nullptr,
+                          const uint64_t *const *res = nullptr);
 int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t nblocks, uint32_t *scratch,
                           uint32_t *ctl, hipStream_t s, int per, uint64_t *stamp = nullptr);
 int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtConst &cc, uint32_t *scratch, uint32_t *ctl,
-                        hipStream_t s, double alg_bytes, uint64_t *stamps = nullptr);
+                        hipStream_t s, double alg_bytes, uint64_t *stamps = nullptr, const uint64_t *const *res = nullptr);
 uint64_t nttm_crt_blocks(uint64_t nc, int per = 8);      /* per: CRT limbs per thread, 8 (2048-limb blocks) or 1 (256) */
 uint64_t nttm_crt_scratch_words(uint64_t nblocks);
 int nttm_small_log(int logn);
@@ -53,7 +53,7 @@ int nttm_run_fill_x(const void *desc_dev, uint64_t nprod, hipStream_t s);
 int nttm_run_dft16_mfma(const uint64_t *x, double *y, int logn, uint64_t batch, const void *etab, const double *tlo,
                         const double *thi, const double *consts, double p, hipStream_t s);
 int nttm_run_add_carry(uint64_t *c, uint64_t n, const uint64_t *carry, hipStream_t s);
-int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *stamp = nullptr);
+int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *stamp = nullptr, bool u64 = false);
 
 /* ---- errors ----------------------------------------------------------------------------------------------------- */
 /* per host thread: the library's own helper threads (the e pipeline's download preparation) may fail too */
@@ -494,23 +494,29 @@ static PassArgs base_args(int prime, double *x, int logn, uint64_t batch, bool i
     a.pk = g.pk[prime]; a.tw = inv ? g.twi[prime] : g.twf[prime]; a.twi = g.twi[prime];
     return a;
 }
-static int fwd_planes(int prime, double *x, int logn, uint64_t batch, hipStream_t s)
+/* in_u64 / out_u64: the plane holds canonical uint64 residues before / after the transform (converted in its first and
+ * last pass) */
+static int fwd_planes(int prime, double *x, int logn, uint64_t batch, hipStream_t s, int in_u64 = 0, int out_u64 = 0)
 {
     Plan pl; plan_make(&pl, logn, batch, g.cfg.tile_log);
-    PassArgs a = base_args(prime, x, logn, batch, false);
-    for (int i = 0; i < pl.npass; i++) RCK(nttm_run_pass(false, a, pl.p[i], s));
+    for (int i = 0; i < pl.npass; i++) {
+        PassArgs a = base_args(prime, x, logn, batch, false);
+        a.in_u64 = in_u64 && i == 0; a.out_u64 = out_u64 && i == pl.npass - 1;
+        RCK(nttm_run_pass(false, a, pl.p[i], s));
+    }
     return 0;
 }
 /* inverse with the pointwise product by y (ymode layout) fused into the first pass; scale by n^-1 in the last pass.
  * r3y: the batch is the thirds of transforms of 3 2^logn points, y holds whole such transforms */
 static int inv_planes(int prime, double *x, const double *y, int ymode, int logn, uint64_t batch, int scale, hipStream_t s,
-                      int r3y = 0)
+                      int r3y = 0, int in_u64 = 0, int y_u64 = 0, int out_u64 = 0)
 {
     Plan pl; plan_make(&pl, logn, batch, g.cfg.tile_log);
     PassArgs a = base_args(prime, x, logn, batch, true);
     for (int i = pl.npass - 1; i >= 0; i--) {
         PassArgs b = a;
-        if (i == pl.npass - 1) { b.y = y; b.ymode = ymode; b.r3y = r3y; }
+        if (i == pl.npass - 1) { b.y = y; b.ymode = ymode; b.r3y = r3y; b.in_u64 = in_u64; b.y_u64 = y && y_u64; }
+        if (i == 0) b.out_u64 = out_u64;
         if (i == 0 && scale) {
             const uint64_t p = NTTM_PRIMES[prime];
             b.scale = h_shoup(h_inv(((uint64_t)1 << logn) % p, p), p); b.do_scale = 1;
@@ -2087,23 +2093,29 @@ static int prim_check(int prime, const void *x, int logn, size_t batch, int r3 =
     DEVCK(x, ((uint64_t)batch << logn) * (r3 ? 3 : 1) * 8, "x");
     return 0;
 }
+/* the residues are converted in a transform's first and last pass: passes of their own (16 B a point each) took 40% of a
+ * product formed from the primitives at 2^22 points */
 extern "C" int nttm_ntt_fwd(int prime, uint64_t *x, int logn, size_t batch, void *stream)
 {
     RCK(prim_check(prime, x, logn, batch));
-    hipStream_t s = (hipStream_t)stream;
-    const uint64_t cnt = (uint64_t)batch << logn;
-    RCK(nttm_run_u64_to_f64((double *)x, cnt, s));
-    RCK(fwd_planes(prime, (double *)x, logn, batch, s));
-    return nttm_run_f64_to_canon((double *)x, cnt, g.pk[prime], s);
+    return fwd_planes(prime, (double *)x, logn, batch, (hipStream_t)stream, 1, 1);
 }
 extern "C" int nttm_ntt_inv(int prime, uint64_t *x, int logn, size_t batch, void *stream)
 {
     RCK(prim_check(prime, x, logn, batch));
-    hipStream_t s = (hipStream_t)stream;
-    const uint64_t cnt = (uint64_t)batch << logn;
-    RCK(nttm_run_u64_to_f64((double *)x, cnt, s));
-    RCK(inv_planes(prime, (double *)x, nullptr, NTTM_Y_FULL, logn, batch, 1, s));
-    return nttm_run_f64_to_canon((double *)x, cnt, g.pk[prime], s);
+    return inv_planes(prime, (double *)x, nullptr, NTTM_Y_FULL, logn, batch, 1, (hipStream_t)stream, 0, 1, 0, 1);
+}
+/* y as the fused inverse reads it: in place (canonical residues), or, where it shares memory with x other than element for
+ * element, an FP64 copy made first (the inverse's first pass overwrites x tile by tile) */
+static int pw_operand(const uint64_t *x, uint64_t cnt, const uint64_t *y, uint64_t ycnt, int ymode, hipStream_t s,
+                      const double **yp, int *y_u64)
+{
+    *yp = (const double *)y; *y_u64 = 1;
+    if (!(x < y + ycnt && y < x + cnt) || (ymode == NTTM_Y_FULL && x == y)) return 0;
+    RCK(ws_need(ycnt * 8));
+    RCK(nttm_run_cvt_u64_f64((double *)g.ws, y, ycnt, s));
+    *yp = (const double *)g.ws; *y_u64 = 0;
+    return 0;
 }
 extern "C" int nttm_ntt_inv_pw(int prime, uint64_t *x, const uint64_t *y, int ymode, int logn, size_t batch, void *stream)
 {
@@ -2115,11 +2127,9 @@ extern "C" int nttm_ntt_inv_pw(int prime, uint64_t *x, const uint64_t *y, int ym
     const uint64_t ycnt = ymode == NTTM_Y_FULL ? cnt : ymode == NTTM_Y_BCAST ? ((uint64_t)1 << logn)
                                                      : ((uint64_t)((batch + 1) / 2) << logn);
     DEVCK(y, ycnt * 8, "y");
-    RCK(ws_need(ycnt * 8));
-    RCK(nttm_run_cvt_u64_f64((double *)g.ws, y, ycnt, s));
-    RCK(nttm_run_u64_to_f64((double *)x, cnt, s));
-    RCK(inv_planes(prime, (double *)x, (const double *)g.ws, ymode, logn, batch, 1, s));
-    return nttm_run_f64_to_canon((double *)x, cnt, g.pk[prime], s);
+    const double *yp; int y_u64;
+    RCK(pw_operand(x, cnt, y, ycnt, ymode, s, &yp, &y_u64));
+    return inv_planes(prime, (double *)x, yp, ymode, logn, batch, 1, s, 0, 1, y_u64, 1);
 }
 
 /* the forward transform with its first four levels as one radix-16 stage on INT8 matrix cores (mfma.hip), the
@@ -2169,32 +2179,25 @@ extern "C" int nttm_ntt_fwd3(int prime, uint64_t *x, int logk, size_t batch, voi
 {
     RCK(prim_check(prime, x, logk, batch, 1));
     hipStream_t s = (hipStream_t)stream;
-    const uint64_t cnt = 3 * ((uint64_t)batch << logk);
-    RCK(nttm_run_u64_to_f64((double *)x, cnt, s));
     JobSet r; memset(&r, 0, sizeof r);
     r.n = 1; r.j[0] = prime_job(prime, (double *)x, batch, false);
-    RCK(nttm_run_r3(false, logk, r, s));
-    RCK(fwd_planes(prime, (double *)x, logk, 3 * (uint64_t)batch, s));
-    return nttm_run_f64_to_canon((double *)x, cnt, g.pk[prime], s);
+    RCK(nttm_run_r3(false, logk, r, s, nullptr, true));
+    return fwd_planes(prime, (double *)x, logk, 3 * (uint64_t)batch, s, 0, 1);
 }
 /* the inverse: the engine's inverses scale by 2^-logk, the radix-3 layer by 3^-1 */
-static int inv3_planes(int prime, double *x, const double *y, int ymode, int logk, uint64_t batch, hipStream_t s)
+static int inv3_planes(int prime, double *x, const double *y, int y_u64, int ymode, int logk, uint64_t batch, hipStream_t s)
 {
     const uint64_t p = NTTM_PRIMES[prime];
-    RCK(inv_planes(prime, x, y, ymode, logk, 3 * batch, 1, s, 1));
+    RCK(inv_planes(prime, x, y, ymode, logk, 3 * batch, 1, s, 1, 1, y_u64, 0));
     JobSet r; memset(&r, 0, sizeof r);
     r.n = 1; r.j[0] = prime_job(prime, x, batch, true);
     r.j[0].in_scale = h_shoup(h_inv(3, p), p); r.j[0].do_in_scale = 1;
-    return nttm_run_r3(true, logk, r, s);
+    return nttm_run_r3(true, logk, r, s, nullptr, true);
 }
 extern "C" int nttm_ntt_inv3(int prime, uint64_t *x, int logk, size_t batch, void *stream)
 {
     RCK(prim_check(prime, x, logk, batch, 1));
-    hipStream_t s = (hipStream_t)stream;
-    const uint64_t cnt = 3 * ((uint64_t)batch << logk);
-    RCK(nttm_run_u64_to_f64((double *)x, cnt, s));
-    RCK(inv3_planes(prime, (double *)x, nullptr, NTTM_Y_FULL, logk, batch, s));
-    return nttm_run_f64_to_canon((double *)x, cnt, g.pk[prime], s);
+    return inv3_planes(prime, (double *)x, nullptr, 0, NTTM_Y_FULL, logk, batch, (hipStream_t)stream);
 }
 extern "C" int nttm_ntt_inv3_pw(int prime, uint64_t *x, const uint64_t *y, int ymode, int logk, size_t batch, void *stream)
 {
@@ -2205,11 +2208,9 @@ extern "C" int nttm_ntt_inv3_pw(int prime, uint64_t *x, const uint64_t *y, int y
     const uint64_t n3 = (uint64_t)3 << logk, cnt = n3 * batch;
     const uint64_t ycnt = ymode == NTTM_Y_FULL ? cnt : ymode == NTTM_Y_BCAST ? n3 : (uint64_t)((batch + 1) / 2) * n3;
     DEVCK(y, ycnt * 8, "y");
-    RCK(ws_need(ycnt * 8));
-    RCK(nttm_run_cvt_u64_f64((double *)g.ws, y, ycnt, s));
-    RCK(nttm_run_u64_to_f64((double *)x, cnt, s));
-    RCK(inv3_planes(prime, (double *)x, (const double *)g.ws, ymode, logk, batch, s));
-    return nttm_run_f64_to_canon((double *)x, cnt, g.pk[prime], s);
+    const double *yp; int y_u64;
+    RCK(pw_operand(x, cnt, y, ycnt, ymode, s, &yp, &y_u64));
+    return inv3_planes(prime, (double *)x, yp, y_u64, ymode, logk, batch, s);
 }
 extern "C" int nttm_pw(int prime, uint64_t *x, const uint64_t *y, size_t count, void *stream)
 {
@@ -2241,19 +2242,25 @@ extern "C" int nttm_crt(uint64_t *c, size_t nc, const uint64_t *const *planes, i
     DEVCK(x, nx * 8, "x");
     for (int i = 0; i < np; i++) DEVCK(planes[i], ncoef * 8, "plane");
     hipStream_t s = (hipStream_t)stream;
-    const size_t pbytes = align_up((size_t)np * ncoef * 8, 256);
+    for (int i = 0; i < np; i++) if (!planes[i] && ncoef) return nttm_fail(NTTM_EINVAL, "null plane %d", i);
+    /* the planes are read in place as canonical residues, unless c shares memory with one of them (the CRT's blocks write
+     * c while others still read): then through FP64 copies */
+    bool copy = false;
+    for (int i = 0; i < np; i++) copy = copy || (ncoef && c < planes[i] + ncoef && planes[i] < c + nc);
+    const size_t pbytes = copy ? align_up((size_t)np * ncoef * 8, 256) : 0;
     const size_t crt_words = nttm_crt_scratch_words(nttm_crt_blocks(nc));
     RCK(ws_need(pbytes + 256 + crt_words * 4 + 256));
-    double *pl = (double *)g.ws;
-    for (int i = 0; i < np; i++) {
-        if (!planes[i] && ncoef) return nttm_fail(NTTM_EINVAL, "null plane %d", i);
-        if (ncoef) RCK(nttm_run_cvt_u64_f64(pl + (size_t)i * ncoef, planes[i], ncoef, s));
-    }
     CrtDesc hd; memset(&hd, 0, sizeof hd);
-    hd.pl = pl; hd.plane = ncoef; hd.ncoef = ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
+    hd.ncoef = ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
+    if (copy) {
+        double *pl = (double *)g.ws;
+        hd.pl = pl; hd.plane = ncoef;
+        for (int i = 0; i < np; i++) RCK(nttm_run_cvt_u64_f64(pl + (size_t)i * ncoef, planes[i], ncoef, s));
+    }
     uint32_t *ctl = (uint32_t *)((char *)g.hpin + 96);
     RCK(nttm_crt_launch_one(hd, nttm_crt_blocks(nc), np, g.cc, (uint32_t *)(g.ws + pbytes + 256), ctl, s,
-                            8.0 * np * (double)ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? nx : 0)));
+                            8.0 * np * (double)ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? nx : 0), nullptr,
+                            copy ? nullptr : planes));
     HIPCK(hipStreamSynchronize(s));
     const uint32_t flags = ctl[1];
     if (flags & 1) return nttm_fail(NTTM_ECHECK, "crt: the value needs more than nc limbs");

@@ -42,10 +42,12 @@ struct CrtArgs {
     uint32_t *status;                    /* one word per block (CRT_ST_*) */
     uint32_t block0;                     /* the launch's first block */
     uint64_t *stamp;                     /* or null: the device clock at the launch's start */
+    const uint64_t *res[NTTM_MAX_PRIMES];/* the planes of a k_crt<.., U>: canonical residues, one array per prime */
     CrtConst cc;
 };
 
-template <int NP, int PER>
+/* U: the residues are canonical uint64 in a.res[prime] (the primitive's planes) instead of the product's FP64 planes */
+template <int NP, int PER, bool U = false>
 __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
 {
     constexpr int CH = CRT_T * PER;                                  /* limbs per block */
@@ -76,17 +78,21 @@ __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
          * limit of 15 outstanding operations would serialize the prefetch */
         const __attribute__((address_space(1))) double *pl = (const __attribute__((address_space(1))) double *)dsc.pl;
         const __attribute__((address_space(1))) uint64_t *xg = (const __attribute__((address_space(1))) uint64_t *)dsc.x;
+        auto residue = [&](int j, uint64_t kk) -> double {
+            if (U) return u64_to_res(((const __attribute__((address_space(1))) uint64_t *)a.res[j])[kk]);
+            return pl[j * dsc.plane + kk];
+        };
         double rr[PER + 1][NP];
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const uint64_t kk = k0 + i * CRT_T + tid;
 #pragma unroll
-            for (int j = 0; j < NP; j++) rr[i][j] = kk < dsc.ncoef ? pl[j * dsc.plane + kk] : 0.0;
+            for (int j = 0; j < NP; j++) rr[i][j] = kk < dsc.ncoef ? residue(j, kk) : 0.0;
         }
         {
             const uint64_t kk = k0 + tid - CRT_HALO;
 #pragma unroll
-            for (int j = 0; j < NP; j++) rr[PER][j] = halo && kk < dsc.ncoef ? pl[j * dsc.plane + kk] : 0.0;
+            for (int j = 0; j < NP; j++) rr[PER][j] = halo && kk < dsc.ncoef ? residue(j, kk) : 0.0;
         }
 #pragma unroll
         for (int i = 0; i < PER; i++) {                          /* x at the limbs of the limb phase below */
@@ -380,7 +386,8 @@ uint64_t nttm_crt_scratch_words(uint64_t nblocks) { return nblocks + CRT_CTL_WOR
 /* desc_dev: nprod descriptors in device memory whose block ranges tile [blk0, blk0 + nblk) of scratch's status words
  * (null: the one product `one`): their limbs for a carry into every block of 0, and the blocks' carry maps */
 int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np,
-                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp)
+                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp,
+                          const uint64_t *const *res)
 {
     if (per != 1 && per != CRT_WIDE) return nttm_fail(NTTM_EINVAL, "crt: %d limbs per thread", per);
     if (np < 3 || np > NTTM_MAX_PRIMES) return nttm_fail(NTTM_EINVAL, "crt: np = %d", np);
@@ -393,8 +400,13 @@ int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t 
     if (one) a.one = *one;
     a.desc = desc_dev; a.nprod = nprod; a.block0 = (uint32_t)blk0; a.stamp = stamp;
     a.status = scratch + CRT_CTL_WORDS; a.cc = cc;
+    for (int j = 0; j < NTTM_MAX_PRIMES; j++) a.res[j] = res && j < np ? res[j] : nullptr;
+    if (res && per == 1) return nttm_fail(NTTM_EINVAL, "crt: residue planes take the wide blocks");
     prof_begin("k_crt", alg_bytes, s);
-    if (per == 1) {
+    if (res) {
+        if (np == 3) hipLaunchKernelGGL((k_crt<3, CRT_WIDE, true>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
+        else hipLaunchKernelGGL((k_crt<4, CRT_WIDE, true>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
+    } else if (per == 1) {
         if (np == 3) hipLaunchKernelGGL((k_crt<3, 1>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
         else hipLaunchKernelGGL((k_crt<4, 1>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
     } else {
@@ -425,11 +437,12 @@ int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t 
     return nttm_hip_check(hipGetLastError(), "k_crt_fix launch");
 }
 /* one product, its descriptor passed with the launches: scratch 16-byte aligned, nttm_crt_scratch_words(nblocks) words.
- * stamps (or null): the device clock at the start and at the end of the carry scan */
+ * stamps (or null): the device clock at the start and at the end of the carry scan.  res (or null): the np planes as
+ * arrays of canonical residues, in place of d's */
 int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtConst &cc, uint32_t *scratch, uint32_t *ctl,
-                        hipStream_t s, double alg_bytes, uint64_t *stamps)
+                        hipStream_t s, double alg_bytes, uint64_t *stamps, const uint64_t *const *res)
 {
-    RCK(nttm_crt_launch_limbs(nullptr, &d, 1, 0, nblocks, np, cc, scratch, s, alg_bytes, CRT_WIDE, stamps));
+    RCK(nttm_crt_launch_limbs(nullptr, &d, 1, 0, nblocks, np, cc, scratch, s, alg_bytes, CRT_WIDE, stamps, res));
     return nttm_crt_launch_carry(nullptr, &d, 1, nblocks, scratch, ctl, s, CRT_WIDE, stamps ? stamps + 1 : nullptr);
 }
 

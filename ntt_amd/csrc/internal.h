@@ -67,6 +67,8 @@ struct PassArgs {
      * c1 < 2^(dfr_lom - dfr_gm) its column) by w_(2^dfr_lom)^(brev_dfr_gm(h) c1), times dfr_scale when dfr_do_scale */
     int dfr_out, dfr_in, dfr_lom, dfr_gm, dfr_do_scale;
     double2 dfr_scale;
+    int in_u64, out_u64;            /* the plane holds canonical uint64 residues before / after this pass (transform primitives) */
+    int y_u64;                      /* y too */
     uint64_t *stamp;                /* or null: the device clock at the launch's first block goes here (pinned host memory) */
 };
 /* the phase clock of short products: the device's constant-rate clock, stored by one thread of a launch */

@@ -120,7 +120,21 @@ __device__ __forceinline__ void apply_job(PassArgs &a, const JobSet &js)
     a.batch = j.batch; a.pk.p = j.p; a.pk.pinv = j.pinv; a.tw = j.tw;
 }
 
-template <int MODE, int PTS, int GM = -1, int GW = -1, int GH = -1>
+#define STW_LOG 8                 /* entries (log2) of the stage table that fixed contiguous tiles keep in LDS */
+
+/* canonical residues as the transform primitives take them, and the FP64 values of the passes */
+__device__ __forceinline__ double res_load(double raw, int u64)
+{
+    return u64 ? u64_to_res((uint64_t)__double_as_longlong(raw)) : raw;
+}
+__device__ __forceinline__ double res_store(double x, int u64, double p, double pinv)
+{
+    return u64 ? __longlong_as_double((long long)res_canon(x, p, pinv)) : x;
+}
+
+/* U: the plane may hold canonical uint64 residues on the pass's input or output side (a.in_u64, a.out_u64, a.y_u64), so
+ * that a transform primitive converts in its first and last pass instead of in passes of their own */
+template <int MODE, int PTS, int GM = -1, int GW = -1, int GH = -1, bool U = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_pass(PassArgs a, JobSet js)
 {
     apply_job(a, js);
@@ -137,6 +151,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     const double p = a.pk.p, pinv = a.pk.pinv;
     const GTab gtw(a.tw.stage);
     constexpr int MAXR = PTS >= 16 ? 4 : PTS == 8 ? 3 : PTS == 4 ? 2 : 1;
+    /* fixed contiguous tiles: the stage table's first 2^STW_LOG entries in LDS, for the rounds whose stages all lie below */
+    constexpr bool LT = GM >= 10 && GW == 0 && PTS == 16;
+    __shared__ double2 stw[LT ? 1 << STW_LOG : 1];
+    if (LT && threadIdx.x < (1 << STW_LOG)) stw[threadIdx.x] = a.tw.stage[threadIdx.x];
     const int lom = a.lo + gm, nr = round_count(gm, MAXR);
     /* the tile: column block cb (W columns below bit lo) of block group hb (H blocks of 2^lom points) */
     const uint64_t tile = blockIdx.x;
@@ -166,13 +184,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 
     /* the boundary twiddles of a strided pass (lo > 0) go with the round over row bits [0, logR) -- the last forward
      * round, the first inverse one -- as base * step^i chains (bound_chain), applied to v between load and round */
+    /* y of a tile inside one transform (or laid out like x): one base for the tile */
+    const bool y_one = MODE == PM_INV_PW && (a.ymode == NTTM_Y_FULL || a.lo + gm + gh <= a.logn);
+    const double *yt = y_one ? a.y + y_index(a, gbase) : a.y;
     auto load_at = [&](uint32_t o, uint32_t, uint32_t) -> double {
         double x = MODE == PM_FWD_LIMB ? limb_at(o) : xt[o];
-        if (MODE == PM_INV_PW) x = mul_barrett(x, a.y[y_index(a, gbase + o)], p, pinv);
+        if (U) x = res_load(x, a.in_u64);
+        if (MODE == PM_INV_PW) {
+            double y = y_one ? yt[o] : a.y[y_index(a, gbase + o)];
+            if (U) y = res_load(y, a.y_u64);
+            x = mul_barrett(x, y, p, pinv);
+        }
         return x;
     };
     auto store_at = [&](uint32_t o, uint32_t, uint32_t, double x) {
         if (a.do_scale) x = mul_shoup(x, a.scale.x, a.scale.y, p);
+        if (U) x = res_store(x, a.out_u64, p, pinv);
         xt[o] = x;
     };
 
@@ -202,7 +229,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
             if (active) ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
                                                                            uint32_t) { v[sl] = lds.at(e); });)
         }
-        if (active) ROUND_SWITCH(logR, round_compute<LR, INV, PTS>(v, pp, s_lo, gtw, p, pinv);)
+        if (LT && s_lo + logR <= STW_LOG) {
+            if (i == 0 && !(gw + s_lo < 4)) __syncthreads();        /* (no barrier has passed since the table was stored) */
+            if (active) ROUND_SWITCH(logR, round_compute<LR, INV, PTS, LTab>(v, pp, s_lo, stw, p, pinv);)
+        } else {
+            if (active) ROUND_SWITCH(logR, round_compute<LR, INV, PTS>(v, pp, s_lo, gtw, p, pinv);)
+        }
         if (i + 1 < nr && active)
             ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
                                                                uint32_t) { lds.at(e) = v[sl]; });)
@@ -255,7 +287,7 @@ __device__ __forceinline__ void lds_barrier()
 }
 
 
-template <int MODE, int GM, int GW>
+template <int MODE, int GM, int GW, bool U = false>
 __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
 {
     apply_job(a, js);
@@ -379,6 +411,10 @@ __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
             } else
                 ROUND_SWITCH(logR, for_slots<LR, PTS>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
                     v[sl] = cur[e]; });)
+            if (U && i == 0) {
+#pragma unroll
+                for (int j = 0; j < PTS; j++) v[j] = res_load(v[j], a.in_u64);
+            }
             if (INV && i == 0) {
                 if (GM == 8) {
 #pragma unroll
@@ -425,6 +461,10 @@ __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
 #pragma unroll
             for (int j = 0; j < PTS; j++) v[j] = mul_shoup(v[j], a.scale.x, a.scale.y, p);
         }
+        if (U) {
+#pragma unroll
+            for (int j = 0; j < PTS; j++) v[j] = res_store(v[j], a.out_u64, p, pinv);
+        }
         ROUND_SWITCH(logR, for_slots<LR, PTS>(pp, s_lo, [&](int sl, uint32_t, uint32_t o, uint32_t, uint32_t) {
             xt[o] = v[sl]; });)
     }
@@ -438,7 +478,6 @@ __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
  * One read of A (or its limbs), one read of B (or its limbs), one write of A. */
 /* stw: the forward stage table's first 2^STW_LOG entries in LDS (nullptr: none); rounds whose stages all lie below
  * STW_LOG read their twiddles there */
-#define STW_LOG 8
 #define FUSED_LOG 12
 /* LT: stw is the LDS copy of the stage table's low entries, for the rounds after the first */
 /* loaded(): called once the tile's loads have been issued */
@@ -679,7 +718,8 @@ __device__ __forceinline__ void r3_twiddles(const R3Args &a, uint64_t j, double 
     if (a.do_scale) { w1 = mul_shoup(w1, a.scale.x, a.scale.y, p); w2 = mul_shoup(w2, a.scale.x, a.scale.y, p); }
     *t1 = w1; *t2 = w2;
 }
-template <bool LIMB>
+/* LIMB: from operand limbs; U: the plane holds canonical uint64 residues (before the forward, after the inverse layer) */
+template <bool LIMB, bool U>
 __global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(int logk, JobSet js, uint64_t *stamp)
 {
     stamp_clock(stamp);
@@ -693,7 +733,7 @@ __global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(int logk, JobSet js, ui
         double *v = a.x + t * 3 * m;
         double x0, x1, x2;
         if (LIMB) { x0 = r3_input(a, t, j); x1 = r3_input(a, t, j + m); x2 = r3_input(a, t, j + 2 * m); }
-        else { x0 = v[j]; x1 = v[j + m]; x2 = v[j + 2 * m]; }       /* |x| <= p */
+        else { x0 = res_load(v[j], U); x1 = res_load(v[j + m], U); x2 = res_load(v[j + 2 * m], U); }       /* |x| <= p */
         const double u = mul_shoup(x1 - x2, w3.x, w3.y, p);         /* |u| <= 5p/8 */
         double y0 = reduce(x0 + x1 + x2, p, pinv);
         const double y1 = reduce((x0 - x2) + u, p, pinv), y2 = reduce((x0 - x1) - u, p, pinv);
@@ -705,6 +745,7 @@ __global__ __launch_bounds__(NTTM_THREADS) void k_r3_fwd(int logk, JobSet js, ui
         v[j + 2 * m] = mul_barrett(y2, t2, p, pinv);
     }
 }
+template <bool U>
 __global__ __launch_bounds__(NTTM_THREADS) void k_r3_inv(int logk, JobSet js)
 {
     const R3Args a = r3_args(js, logk);
@@ -721,9 +762,9 @@ __global__ __launch_bounds__(NTTM_THREADS) void k_r3_inv(int logk, JobSet js)
         if (a.do_scale) y0 = mul_shoup(y0, a.scale.x, a.scale.y, p);
         const double y1 = mul_barrett(v[j + m], t1, p, pinv), y2 = mul_barrett(v[j + 2 * m], t2, p, pinv);
         const double u = mul_shoup(y2 - y1, w3.x, w3.y, p);         /* |u| <= 5p/8 */
-        v[j] = reduce(y0 + y1 + y2, p, pinv);
-        v[j + m] = reduce((y0 - y1) + u, p, pinv);
-        v[j + 2 * m] = reduce((y0 - y2) - u, p, pinv);
+        v[j] = res_store(reduce(y0 + y1 + y2, p, pinv), U, p, pinv);
+        v[j + m] = res_store(reduce((y0 - y1) + u, p, pinv), U, p, pinv);
+        v[j + 2 * m] = res_store(reduce((y0 - y2) - u, p, pinv), U, p, pinv);
     }
 }
 
@@ -822,6 +863,13 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
     case PM_FWD_LIMB: hipLaunchKernelGGL((k_pass<PM_FWD_LIMB, P, M, W, H>), grid, blk, lds, s, b, js); break; \
     case PM_INV: hipLaunchKernelGGL((k_pass<PM_INV, P, M, W, H>), grid, blk, lds, s, b, js); break; \
     default: hipLaunchKernelGGL((k_pass<PM_INV_PW, P, M, W, H>), grid, blk, lds, s, b, js); break; }
+#define NTTM_PASS_LAUNCH_U(...) \
+    switch (mode) { \
+    case PM_FWD: hipLaunchKernelGGL((k_pass<PM_FWD, __VA_ARGS__, true>), grid, blk, lds, s, b, js); break; \
+    case PM_INV: hipLaunchKernelGGL((k_pass<PM_INV, __VA_ARGS__, true>), grid, blk, lds, s, b, js); break; \
+    default: hipLaunchKernelGGL((k_pass<PM_INV_PW, __VA_ARGS__, true>), grid, blk, lds, s, b, js); break; }
+    const bool u = b.in_u64 || b.out_u64 || b.y_u64;             /* a transform primitive's first or last pass */
+    if (u && (limb || b.dfr_in || b.dfr_out)) return nttm_fail(NTTM_EINVAL, "internal: residues in a product's pass");
     /* the strided tile shapes of large transforms, compiled with their geometry fixed */
     const bool fixed = g_fixed_shapes && g.logh == 0 && T >= PASS_PTS;
     /* the streamed shapes: strided 2^13-point tiles of 1 to 9-bit rows (2^(13 - m) columns), limbs from one operand
@@ -838,7 +886,9 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
         const unsigned nb = (unsigned)(tiles < (uint64_t)per ? tiles : (uint64_t)per);
         const dim3 sgrid(nb, (unsigned)js.n);
 #define NTTM_STREAM_LAUNCH(M, W) \
-        if (mode == PM_FWD) hipLaunchKernelGGL((k_pass_stream<PM_FWD, M, W>), sgrid, dim3(STREAM_T), 0, s, b, js); \
+        if (u && mode == PM_FWD) hipLaunchKernelGGL((k_pass_stream<PM_FWD, M, W, true>), sgrid, dim3(STREAM_T), 0, s, b, js); \
+        else if (u) hipLaunchKernelGGL((k_pass_stream<PM_INV, M, W, true>), sgrid, dim3(STREAM_T), 0, s, b, js); \
+        else if (mode == PM_FWD) hipLaunchKernelGGL((k_pass_stream<PM_FWD, M, W>), sgrid, dim3(STREAM_T), 0, s, b, js); \
         else if (mode == PM_FWD_LIMB) hipLaunchKernelGGL((k_pass_stream<PM_FWD_LIMB, M, W>), sgrid, dim3(STREAM_T), 0, s, b, js); \
         else hipLaunchKernelGGL((k_pass_stream<PM_INV, M, W>), sgrid, dim3(STREAM_T), 0, s, b, js);
         switch (g.m) {
@@ -854,6 +904,18 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
         }
 #undef NTTM_STREAM_LAUNCH
     }
+    else if (u) {                                                  /* (the contiguous 2^13- and 2^12-point tiles fixed) */
+        if (g_fixed_shapes && ppt == PASS_PTS && g.lo == 0 && g.m == 13) { NTTM_PASS_LAUNCH_U(PASS_PTS, 13, 0, 0) }
+        else if (g_fixed_shapes && ppt == PASS_PTS && g.lo == 0 && g.m == 12 && g.logh == 1) { NTTM_PASS_LAUNCH_U(PASS_PTS, 12, 0, 1) }
+        else if (g_fixed_shapes && ppt == PASS_PTS && g.lo == 0 && g.m == 12 && g.logh == 0) { NTTM_PASS_LAUNCH_U(PASS_PTS, 12, 0, 0) }
+        else if (g_fixed_shapes && ppt == PASS_PTS && g.lo == 0 && g.m == 11 && g.logh == 2) { NTTM_PASS_LAUNCH_U(PASS_PTS, 11, 0, 2) }
+        else if (g_fixed_shapes && ppt == PASS_PTS && g.lo == 0 && g.m == 10 && g.logh == 3) { NTTM_PASS_LAUNCH_U(PASS_PTS, 10, 0, 3) }
+        else if (T >= PASS_PTS && ppt == 8) { NTTM_PASS_LAUNCH_U(8, -1, -1, -1) }
+        else if (T >= PASS_PTS) { NTTM_PASS_LAUNCH_U(PASS_PTS, -1, -1, -1) }
+        else if (T == 8) { NTTM_PASS_LAUNCH_U(8, -1, -1, -1) }
+        else if (T == 4) { NTTM_PASS_LAUNCH_U(4, -1, -1, -1) }
+        else { NTTM_PASS_LAUNCH_U(2, -1, -1, -1) }
+    }
     else if (fixed && ppt == PASS_PTS && g.m == 8 && g.logw == 5) { NTTM_PASS_LAUNCH_G(PASS_PTS, 8, 5, 0) }
     else if (T >= PASS_PTS && ppt == 8) { NTTM_PASS_LAUNCH(8) }
     else if (T >= PASS_PTS) { NTTM_PASS_LAUNCH(PASS_PTS) }
@@ -862,6 +924,7 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
     else { NTTM_PASS_LAUNCH(2) }
 #undef NTTM_PASS_LAUNCH
 #undef NTTM_PASS_LAUNCH_G
+#undef NTTM_PASS_LAUNCH_U
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_pass launch");
 }
@@ -890,25 +953,11 @@ int nttm_run_fused2(const PassArgs &a, const FusedB &fb, const PassGeom &g, hipS
     const int ppt = (T >= 64 * g_pts && T <= 512 * g_pts) ? g_pts : PASS_PTS;
     const unsigned nthr = (unsigned)(T / ppt < 64 ? 64 : T / ppt);
     if (nthr > 512) return nttm_fail(NTTM_EINVAL, "internal: %u threads per tile", nthr);
-    /* the fixed shapes: 4096-point tiles of 2^12-point blocks, or of 4 x 2^10 and 2 x 2^11 (the last pass of a
-     * transform of more than one pass, or a whole transform of 2^10 to 2^12 points, which reads the limbs); whole
-     * transforms of 2^8 and 2^9 points from the limbs in tiles of 16 and 8 blocks (8 points per thread) */
-    const bool fixed_shape = g_fixed_shapes && g.m + g.logh == FUSED_LOG && (g.m >= 10 || (g.m >= 8 && ppt == 8));
-    const bool fixed = fixed_shape && !alimb && !blimb && g.m >= 10;
+    /* the fixed shapes: 4096-point tiles of 2^12-point blocks, or of 4 x 2^10 and 2 x 2^11 (the last pass of a transform of
+     * more than one pass; whole transforms of up to 2^12 points are small.hip's, but for the cyclic products) */
+    const bool fixed = g_fixed_shapes && g.m + g.logh == FUSED_LOG && g.m >= 10 && !alimb && !blimb;
     const dim3 grid((unsigned)tiles, (unsigned)js.n), blk(nthr);
-    if (fixed_shape && !fixed && (alimb || blimb)) {            /* a single-pass transform: both operands from limbs */
-        if (ppt == 8) {
-            if (g.m == 12) hipLaunchKernelGGL((k_fused2<8, 12, 0, true>), grid, blk, 0, s, A, fb, js);
-            else if (g.m == 11) hipLaunchKernelGGL((k_fused2<8, 11, 1, true>), grid, blk, 0, s, A, fb, js);
-            else if (g.m == 10) hipLaunchKernelGGL((k_fused2<8, 10, 2, true>), grid, blk, 0, s, A, fb, js);
-            else if (g.m == 9) hipLaunchKernelGGL((k_fused2<8, 9, 3, true>), grid, blk, 0, s, A, fb, js);
-            else hipLaunchKernelGGL((k_fused2<8, 8, 4, true>), grid, blk, 0, s, A, fb, js);
-        } else {
-            if (g.m == 12) hipLaunchKernelGGL((k_fused2<PASS_PTS, 12, 0, true>), grid, blk, 0, s, A, fb, js);
-            else if (g.m == 11) hipLaunchKernelGGL((k_fused2<PASS_PTS, 11, 1, true>), grid, blk, 0, s, A, fb, js);
-            else hipLaunchKernelGGL((k_fused2<PASS_PTS, 10, 2, true>), grid, blk, 0, s, A, fb, js);
-        }
-    } else if (fixed && ppt == 8) {
+    if (fixed && ppt == 8) {
         if (g.m == 12) hipLaunchKernelGGL((k_fused2<8, 12, 0, false>), grid, blk, 0, s, A, fb, js);
         else if (g.m == 11) hipLaunchKernelGGL((k_fused2<8, 11, 1, false>), grid, blk, 0, s, A, fb, js);
         else hipLaunchKernelGGL((k_fused2<8, 10, 2, false>), grid, blk, 0, s, A, fb, js);
@@ -956,8 +1005,9 @@ int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which
 }
 /* the radix-3 layer of the jobs' transforms of 3 2^logk points (logk >= 1): forward (from the planes, or every job from
  * limbs) or inverse, in place.  A job: x, batch (transforms of 3 2^logk points), its operand, pk, tw.b3 (the direction's
- * table) and the scale of every output in in_scale */
-int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *stamp)
+ * table) and the scale of every output in in_scale.  u64: a forward layer's input or an inverse layer's output is
+ * canonical uint64 residues */
+int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *stamp, bool u64)
 {
     if (js.n < 1 || js.n > NTTM_MAX_JOBS || logk < 1 || logk > NTTM_LOGN_MAX) return nttm_fail(NTTM_EINVAL, "internal: radix-3 layer of 3 2^%d", logk);
     const bool limb = js.j[0].limbs || js.j[0].ldesc;
@@ -966,6 +1016,7 @@ int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *s
     for (int k = 0; k < js.n; k++) {
         const PassJob &j = js.j[k];
         if (!j.batch || (j.limbs || j.ldesc) != limb) return nttm_fail(NTTM_EINVAL, "internal: radix-3 layer's jobs");
+        if (u64 && limb) return nttm_fail(NTTM_EINVAL, "internal: radix-3 layer from limbs and residues");
         if (inv && limb) return nttm_fail(NTTM_EINVAL, "internal: inverse radix-3 layer from limbs");
         if (j.limbs && j.batch != 1) return nttm_fail(NTTM_EINVAL, "internal: one limb operand for %llu transforms",
                                                       (unsigned long long)j.batch);
@@ -975,16 +1026,13 @@ int nttm_run_r3(bool inv, int logk, const JobSet &js, hipStream_t s, uint64_t *s
     }
     prof_begin(inv ? "k_r3_inv" : limb ? "k_r3_fwd<limb>" : "k_r3_fwd", bytes, s);
     const dim3 grid(grid_for(most << logk), (unsigned)js.n);
-    if (inv) hipLaunchKernelGGL(k_r3_inv, grid, dim3(NTTM_THREADS), 0, s, logk, js);
-    else if (limb) hipLaunchKernelGGL(k_r3_fwd<true>, grid, dim3(NTTM_THREADS), 0, s, logk, js, stamp);
-    else hipLaunchKernelGGL(k_r3_fwd<false>, grid, dim3(NTTM_THREADS), 0, s, logk, js, stamp);
+    if (inv && u64) hipLaunchKernelGGL(k_r3_inv<true>, grid, dim3(NTTM_THREADS), 0, s, logk, js);
+    else if (inv) hipLaunchKernelGGL(k_r3_inv<false>, grid, dim3(NTTM_THREADS), 0, s, logk, js);
+    else if (u64) hipLaunchKernelGGL((k_r3_fwd<false, true>), grid, dim3(NTTM_THREADS), 0, s, logk, js, stamp);
+    else if (limb) hipLaunchKernelGGL((k_r3_fwd<true, false>), grid, dim3(NTTM_THREADS), 0, s, logk, js, stamp);
+    else hipLaunchKernelGGL((k_r3_fwd<false, false>), grid, dim3(NTTM_THREADS), 0, s, logk, js, stamp);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_r3 launch");
-}
-int nttm_run_u64_to_f64(double *x, uint64_t count, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_cvt_u64_f64, dim3(grid_for(count)), dim3(NTTM_THREADS), 0, s, x, (const uint64_t *)x, count);
-    return nttm_hip_check(hipGetLastError(), "k_cvt_u64_f64 launch");
 }
 int nttm_run_cvt_u64_f64(double *dst, const uint64_t *src, uint64_t count, hipStream_t s)
 {
