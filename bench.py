@@ -358,8 +358,7 @@ def bench_binsplit(nttm, reps, nodes=256, lo=12000, hi=16000, seed=0x5EED0007):
 
 
 PROF_NAMES = (("k_fused2", "k_fused2"), ("k_pass_stream<0", "k_pass<fwd>"), ("k_pass_stream<1", "k_pass<fwd,limb>"),
-              ("k_pass_stream<2", "k_pass<inv>"), ("k_crt<", "k_crt"), ("k_crt_scan", "k_crt_scan"),
-              ("k_crt_fix", "k_crt_fix"))
+              ("k_pass_stream<2", "k_pass<inv>"), ("k_crt<", "k_crt"), ("k_carry", "k_carry"), ("k_small", "k_small"))
 
 
 def bench_config4(nttm, da, db, reps=3):

@@ -36,8 +36,8 @@ int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which
 /* the CRT of products whose blocks are [blk0, blk0 + nblk) of the launch's block numbering (limbs for a carry in of 0),
  * then every block's carry; nttm_crt_launch_one: both for one product */
 int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np,
-                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp = nullptr,
-                          const uint64_t *const *res = nullptr);
+                          const CrtConst &cc, uint32_t *scratch, uint32_t *ctl, hipStream_t s, double alg_bytes, int per,
+                          uint64_t *stamp = nullptr, const uint64_t *const *res = nullptr);
 int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t nblocks, uint32_t *scratch,
                           uint32_t *ctl, hipStream_t s, int per, uint64_t *stamp = nullptr);
 int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtConst &cc, uint32_t *scratch, uint32_t *ctl,
@@ -1225,7 +1225,7 @@ static int group_launch(const GroupBuild &gb, int np, double *A, char *dbase, hi
                                 nullptr, ch.cnb, gb.share ? (const LoadDesc *)(dbase + gb.off_ldb) + ch.b0 : nullptr,
                                 gb.share ? (const uint32_t *)(dbase + gb.off_bmap) + (gb.r3 ? 3 : 1) * ch.c0 : nullptr);
         if (!rc) rc = nttm_crt_launch_limbs((const CrtDesc *)(dbase + gb.off_cd) + ch.c0, nullptr, ch.cn, ch.blk0, ch.nblk, np,
-                                            g.cc, (uint32_t *)(dbase + gb.off_crt), s, ch.crt_bytes, gb.crt_per);
+                                            g.cc, (uint32_t *)(dbase + gb.off_crt), (uint32_t *)(dbase + gb.off_crt), s, ch.crt_bytes, gb.crt_per);
         if (rc) break;
     }
     uint32_t *scr = (uint32_t *)(dbase + gb.off_crt);

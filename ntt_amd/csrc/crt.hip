@@ -11,10 +11,9 @@
  * carry-lookahead chain.  For 64 consecutive limbs it is resolved by one 64-bit addition of the ballot masks
  * X = G, Y = G | P (the carries into the bits of X + Y + cin are the o's, the textbook adder identity).  Words chain
  * inside a wave and waves inside a block; each block then stores its limbs for a carry in of 0 together with its
- * (cin -> cout) map of one bit.  One workgroup scans the maps of all blocks (restarting at every product's first
- * block) into each block's carry in, and a last pass adds 1 to the limbs of the blocks that receive a carry: the
- * limbs for cin = 1 are those for cin = 0 plus one, a ripple through the leading limbs equal to B - 1.  No block
- * waits on another, and the scan reads one word per 2048 limbs.
+ * (cin -> cout) map of one bit.  A second launch (k_carry) finds each block's carry in from the maps before it and adds
+ * 1 to the limbs of the blocks that receive one: the limbs for cin = 1 are those for cin = 0 plus one, a ripple through
+ * the leading limbs equal to B - 1.  No block waits on another.
  * The reference instead ripples each 256-coefficient chunk on one thread of a wave64 ballot scan, writes a 4-limb spill
  * per stripe and merges the spills serially on the host or on one thread per product (E/rns_mul.c:452-470;
  * E/dbig.c:1007-1052).  The final carry beyond limb nc-1 must be zero; a non-zero one sets an error flag.
@@ -29,18 +28,17 @@
 #define CRT_HALO 4                       /* digits of coefficients k0-4 .. k0-1: v_{k0-1} with four primes */
 #define CRT_ID_MAP 0x2u                  /* one-bit carry maps: bit c = cout(cin = c); the identity is 0b10 */
 #define CRT_CTL_WORDS 4                  /* control words before the block status words (16-byte aligned) */
-/* block status word: map (2 bits) | error for cin 0 << 2 | error for cin 1 << 3 | carry in << 4 | first of product << 5 */
+/* block status word: map (2 bits) | error for cin 0 << 2 | error for cin 1 << 3 | first of product << 5 */
 #define CRT_ST_E0 (1u << 2)
 #define CRT_ST_E1 (1u << 3)
-#define CRT_ST_CIN (1u << 4)
 #define CRT_ST_FIRST (1u << 5)
-#define CRT_SCAN_T 1024
 
 struct CrtArgs {
     const CrtDesc *desc; uint64_t nprod; /* null: the one product `one` */
     CrtDesc one;
     uint32_t *status;                    /* one word per block (CRT_ST_*) */
     uint32_t block0;                     /* the launch's first block */
+    uint32_t *ctl;                       /* words 0 and 1 cleared by block 0 (k_carry sets word 1 on an error) */
     uint64_t *stamp;                     /* or null: the device clock at the launch's start */
     const uint64_t *res[NTTM_MAX_PRIMES];/* the planes of a k_crt<.., U>: canonical residues, one array per prime */
     CrtConst cc;
@@ -57,6 +55,7 @@ __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t blk = a.block0 + blockIdx.x;
     stamp_clock(a.stamp);
+    if (tid == 0 && blk == 0) { a.ctl[0] = 0; a.ctl[1] = 0; }
     if (tid == 0 && !a.desc) { s_prod = 0; s_err = 0; }
     else if (tid == 0) {
         uint64_t lo = 0, hi = a.nprod - 1;                  /* the product whose block range holds blk */
@@ -200,109 +199,55 @@ __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
     if (tid == 0) a.status[blk] = A | s_err | (local == 0 ? CRT_ST_FIRST : 0u);
 }
 
-/* carry in of every block: maps composed in block order, restarting at each product's first block.  One workgroup of
- * 16 waves, each over a contiguous run of the status words (four per lane and load); the error flag of a product's
- * last block is taken for its actual carry in. */
+/* a block's map as the next block sees it: a product's first block ignores the carry before it.  Monotone: constant 0
+ * (0b00), identity (0b10) or constant 1 (0b11) */
 __device__ __forceinline__ uint32_t crt_step_map(uint32_t st)
 {
-    const uint32_t m = st & 3u;                                     /* a first block ignores the carry before it */
+    const uint32_t m = st & 3u;
     return (st & CRT_ST_FIRST) ? (m & 1u) * 3u : m;
 }
-__global__ __launch_bounds__(CRT_SCAN_T) void k_crt_scan(uint32_t *status, uint64_t n, uint32_t *ctl, uint64_t *stamp)
-{
-    __shared__ uint32_t s_map[CRT_SCAN_T / 64], s_err;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int NW = CRT_SCAN_T / 64, U = 4;                      /* waves; loads of 4 words in flight per lane */
-    if (tid == 0) s_err = 0;
-    const uint64_t per = ((n + NW - 1) / NW + 256 * U - 1) / (256 * U) * (256 * U);
-    const uint64_t lo = (uint64_t)wave * per, hi = lo + per < n ? lo + per : n;
-    auto load4 = [&](uint64_t i, uint32_t *w) {                     /* words i..i+3 (i a multiple of 4) */
-        if (i + 4 <= hi) {
-            const uint4 v = *(const uint4 *)(status + i);
-            w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 4; j++) w[j] = i + j < hi ? status[i + j] : CRT_ID_MAP;
-        }
-    };
-    /* pass 1: the map of the wave's run */
-    uint32_t F = CRT_ID_MAP;
-    for (uint64_t b = lo; b < hi; b += 256 * U) {
-        uint32_t w[U][4];
-#pragma unroll
-        for (int u = 0; u < U; u++) load4(b + u * 256 + lane * 4, w[u]);
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            uint32_t m = CRT_ID_MAP;
-#pragma unroll
-            for (int j = 0; j < 4; j++) m = map_compose(crt_step_map(w[u][j]), m);
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {                      /* lane 0: m_63 o ... o m_0 */
-                const uint32_t o = __shfl_down(m, d, 64);
-                if ((lane & (2 * d - 1)) == 0) m = map_compose(o, m);
-            }
-            F = map_compose(__builtin_amdgcn_readfirstlane(m), F);
-        }
-    }
-    if (lane == 0) s_map[wave] = F;
-    __syncthreads();
-    uint32_t cw = 0;                                                /* the carry into the wave's run */
-    for (int v = 0; v < wave; v++) cw = map_apply(s_map[v], cw);
-    /* pass 2: carries into the blocks */
-    uint32_t err = 0;
-    for (uint64_t b = lo; b < hi; b += 256 * U) {
-        uint32_t w[U][4];
-#pragma unroll
-        for (int u = 0; u < U; u++) load4(b + u * 256 + lane * 4, w[u]);
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            uint32_t m = CRT_ID_MAP;
-#pragma unroll
-            for (int j = 0; j < 4; j++) m = map_compose(crt_step_map(w[u][j]), m);
-            uint32_t inc = m;                                       /* inclusive scan over the lanes */
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const uint32_t o = __shfl_up(inc, d, 64);
-                if (lane >= d) inc = map_compose(inc, o);
-            }
-            uint32_t ex = __shfl_up(inc, 1, 64);
-            if (lane == 0) ex = CRT_ID_MAP;
-            uint32_t ci = map_apply(ex, cw);
-            const uint64_t i0 = b + u * 256 + lane * 4;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t st = w[u][j];
-                if (st & CRT_ST_FIRST) ci = 0;
-                err |= st & (ci ? CRT_ST_E1 : CRT_ST_E0);
-                w[u][j] = (st & ~CRT_ST_CIN) | (ci ? CRT_ST_CIN : 0u);
-                ci = map_apply(st & 3u, ci);
-            }
-            if (i0 + 4 <= hi) *(uint4 *)(status + i0) = make_uint4(w[u][0], w[u][1], w[u][2], w[u][3]);
-            else {
-#pragma unroll
-                for (int j = 0; j < 4; j++) if (i0 + j < hi) status[i0 + j] = w[u][j];
-            }
-            cw = map_apply(__builtin_amdgcn_readlane(inc, 63), cw);
-        }
-    }
-    if (__ballot(err != 0) && lane == 0) atomicOr(&s_err, 1u);
-    __syncthreads();
-    if (tid == 0) { ctl[0] = 0; ctl[1] = s_err; }
-    stamp_clock(stamp);
-}
-
-/* the limbs of a block whose carry in is 1: its stored limbs (for carry 0) plus one, i.e. the leading limbs equal to
- * B - 1 become 0 and the first other one grows by 1.  A workgroup scouts 64 status words; each of its 4 waves takes
- * every 4th block found and rewrites it (CH / 64 limbs per lane, all loads in flight at once). */
-#define CRT_FIX_W 64
+/* The carry into every block, the limbs of the blocks that receive one, and the error flags.  A workgroup takes 64 blocks.
+ * The carry into its first is the value of the nearest block before it whose map is not the identity (a map that
+ * passes a carry through needs 2048 limbs equal to B - 1, so the block just before almost always decides; otherwise the
+ * workgroup goes on looking, 256 words at a time).  Among its own 64 blocks the carries are one addition of the ballot
+ * masks of the maps.  The limbs of a block whose carry in is 1 are its stored limbs (for carry 0) plus one, i.e. the
+ * leading limbs equal to B - 1 become 0 and the first other one grows by 1: each of the 4 waves takes every 4th such block
+ * and rewrites it (CH / 64 limbs per lane, all loads in flight at once).  A product's last block has its error flag taken
+ * for its actual carry in; k_crt has cleared ctl.
+ * (Two launches before, one workgroup scanning the maps of all blocks and the fix: 57 + 6 us at 131072 blocks, 5 + 4 at
+ * few.) */
+#define CRT_CARRY_W 64
 template <int PER>
-__global__ __launch_bounds__(256) void k_crt_fix(const CrtDesc *desc, CrtDesc one, uint64_t nprod, const uint32_t *status, uint64_t n)
+__global__ __launch_bounds__(256) void k_carry(const CrtDesc *desc, CrtDesc one, uint64_t nprod, const uint32_t *status,
+                                               uint64_t n, uint32_t *ctl, uint64_t *stamp)
 {
     constexpr int CH = CRT_T * PER;
+    stamp_clock(stamp);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t b0 = (uint64_t)blockIdx.x * CRT_FIX_W;
-    const uint32_t st = b0 + lane < n ? status[b0 + lane] : 0u;
-    uint64_t todo = __ballot((st & CRT_ST_CIN) != 0);
+    const uint64_t b0 = (uint64_t)blockIdx.x * CRT_CARRY_W;
+    const bool own = b0 + lane < n;
+    const uint32_t st = own ? status[b0 + lane] : 0u;
+    uint32_t cin = 0;                                            /* the carry into block b0 */
+    for (uint64_t pos = b0; pos; pos -= pos < 256 ? pos : 256) { /* words [pos - 256, pos), nearest first */
+        uint32_t w[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint64_t back = (uint64_t)u * 64 + 64 - lane;  /* word pos - back */
+            w[u] = back <= pos ? crt_step_map(status[pos - back]) : 0u;   /* nothing before the first block: constant 0 */
+        }
+        bool found = false;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint64_t dec = __ballot(w[u] != CRT_ID_MAP), val = __ballot((w[u] & 1u) != 0);
+            if (!found && dec) { cin = (uint32_t)(val >> (63 - __clzll((long long)dec))) & 1u; found = true; }
+        }
+        if (found) break;
+    }
+    const uint32_t m = own ? crt_step_map(st) : 0u;
+    const uint64_t X = __ballot(m == 3u), Y = X | __ballot(m == CRT_ID_MAP), CI = (X + Y + cin) ^ X ^ Y;
+    const uint32_t ci = (st & CRT_ST_FIRST) ? 0u : (uint32_t)(CI >> lane) & 1u;
+    if (__ballot(own && (st & (ci ? CRT_ST_E1 : CRT_ST_E0)) != 0) && threadIdx.x == 0) ctl[1] = 1;
+    uint64_t todo = __ballot(own && ci);
     for (int r = 0; todo; r++) {
         const int f = __ffsll((long long)todo) - 1;
         todo &= todo - 1;
@@ -386,8 +331,8 @@ uint64_t nttm_crt_scratch_words(uint64_t nblocks) { return nblocks + CRT_CTL_WOR
 /* desc_dev: nprod descriptors in device memory whose block ranges tile [blk0, blk0 + nblk) of scratch's status words
  * (null: the one product `one`): their limbs for a carry into every block of 0, and the blocks' carry maps */
 int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np,
-                          const CrtConst &cc, uint32_t *scratch, hipStream_t s, double alg_bytes, int per, uint64_t *stamp,
-                          const uint64_t *const *res)
+                          const CrtConst &cc, uint32_t *scratch, uint32_t *ctl, hipStream_t s, double alg_bytes, int per,
+                          uint64_t *stamp, const uint64_t *const *res)
 {
     if (per != 1 && per != CRT_WIDE) return nttm_fail(NTTM_EINVAL, "crt: %d limbs per thread", per);
     if (np < 3 || np > NTTM_MAX_PRIMES) return nttm_fail(NTTM_EINVAL, "crt: np = %d", np);
@@ -398,7 +343,7 @@ int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t 
     CrtArgs a;
     memset(&a.one, 0, sizeof a.one);
     if (one) a.one = *one;
-    a.desc = desc_dev; a.nprod = nprod; a.block0 = (uint32_t)blk0; a.stamp = stamp;
+    a.desc = desc_dev; a.nprod = nprod; a.block0 = (uint32_t)blk0; a.stamp = stamp; a.ctl = ctl;
     a.status = scratch + CRT_CTL_WORDS; a.cc = cc;
     for (int j = 0; j < NTTM_MAX_PRIMES; j++) a.res[j] = res && j < np ? res[j] : nullptr;
     if (res && per == 1) return nttm_fail(NTTM_EINVAL, "crt: residue planes take the wide blocks");
@@ -417,32 +362,28 @@ int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t 
     return nttm_hip_check(hipGetLastError(), "k_crt launch");
 }
 /* every block's carry in, and the limbs of the blocks that receive one; word 1 of ctl (scratch, or pinned host memory)
- * receives the error flags */
+ * receives the error flag */
 int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t nblocks, uint32_t *scratch,
                           uint32_t *ctl, hipStream_t s, int per, uint64_t *stamp)
 {
     if (!nprod || !nblocks) return 0;
-    uint32_t *status = scratch + CRT_CTL_WORDS;
+    const uint32_t *status = scratch + CRT_CTL_WORDS;
     CrtDesc d1; memset(&d1, 0, sizeof d1);
     if (one) d1 = *one;
-    prof_begin("k_crt_scan", 8.0 * (double)nblocks, s);
-    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, status, nblocks, ctl, stamp);
+    prof_begin("k_carry", 4.0 * (double)nblocks, s);
+    const dim3 grid((unsigned)((nblocks + CRT_CARRY_W - 1) / CRT_CARRY_W));
+    if (per == 1) hipLaunchKernelGGL((k_carry<1>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
+    else hipLaunchKernelGGL((k_carry<CRT_WIDE>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
     prof_end(s);
-    RCK(nttm_hip_check(hipGetLastError(), "k_crt_scan launch"));
-    prof_begin("k_crt_fix", 4.0 * (double)nblocks, s);
-    const dim3 gfix((unsigned)((nblocks + CRT_FIX_W - 1) / CRT_FIX_W));
-    if (per == 1) hipLaunchKernelGGL((k_crt_fix<1>), gfix, dim3(256), 0, s, desc_dev, d1, nprod, (const uint32_t *)status, nblocks);
-    else hipLaunchKernelGGL((k_crt_fix<CRT_WIDE>), gfix, dim3(256), 0, s, desc_dev, d1, nprod, (const uint32_t *)status, nblocks);
-    prof_end(s);
-    return nttm_hip_check(hipGetLastError(), "k_crt_fix launch");
+    return nttm_hip_check(hipGetLastError(), "k_carry launch");
 }
 /* one product, its descriptor passed with the launches: scratch 16-byte aligned, nttm_crt_scratch_words(nblocks) words.
- * stamps (or null): the device clock at the start and at the end of the carry scan.  res (or null): the np planes as
+ * stamps (or null): the device clock at the start of both launches.  res (or null): the np planes as
  * arrays of canonical residues, in place of d's */
 int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtConst &cc, uint32_t *scratch, uint32_t *ctl,
                         hipStream_t s, double alg_bytes, uint64_t *stamps, const uint64_t *const *res)
 {
-    RCK(nttm_crt_launch_limbs(nullptr, &d, 1, 0, nblocks, np, cc, scratch, s, alg_bytes, CRT_WIDE, stamps, res));
+    RCK(nttm_crt_launch_limbs(nullptr, &d, 1, 0, nblocks, np, cc, scratch, ctl, s, alg_bytes, CRT_WIDE, stamps, res));
     return nttm_crt_launch_carry(nullptr, &d, 1, nblocks, scratch, ctl, s, CRT_WIDE, stamps ? stamps + 1 : nullptr);
 }
 
@@ -450,8 +391,8 @@ int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtCon
  * r[0 .. nout) = a B^sa + b B^sb, or a B^sa - b B^sb computed as a B^sa + (B^nout - 1 - b B^sb) + 1 (b's limbs
  * complemented, 1 added at limb 0): its carry out of limb nout - 1 is 1 exactly when the difference is >= 0.
  * b may instead be B^bpow (bpow >= 0).  Each 2048-limb block writes its limbs for a carry in of 0 and its one-bit
- * carry map, with the same status words as k_crt; k_crt_scan then gives every block its carry in (and, from the last
- * block's error bits, the final carry out) and k_addsub_fix adds the carries.  Limbs past nout count as B - 1 so that
+ * carry map, with the same status words as k_crt; k_carry then adds every block's carry (and, from the last block's error
+ * bits, gives the final carry out).  Limbs past nout count as B - 1 so that
  * the last block's map is the carry out of limb nout - 1. */
 struct AddArgs {
     const uint64_t *a; uint64_t na, sa;
@@ -459,7 +400,7 @@ struct AddArgs {
     int64_t apow, bpow;
     uint64_t *r; uint64_t nout, nblocks;
     int sub;
-    uint32_t *status;
+    uint32_t *status, *ctl;
 };
 __device__ __forceinline__ uint64_t add_limb(const uint64_t *p, uint64_t n, uint64_t s, uint64_t k)
 {
@@ -471,6 +412,7 @@ __global__ __launch_bounds__(CRT_T) void k_addsub(AddArgs a)
     __shared__ uint32_t s_wave[CRT_T / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint64_t blk = blockIdx.x, k0 = blk * CH;
+    if (tid == 0 && blk == 0) { a.ctl[0] = 0; a.ctl[1] = 0; }
     uint64_t wv[PER], GX[PER], GY[PER];
 #pragma unroll
     for (int i = 0; i < PER; i++) {
@@ -513,23 +455,6 @@ __global__ __launch_bounds__(CRT_T) void k_addsub(AddArgs a)
         a.status[blk] = st;
     }
 }
-/* the blocks whose carry in is 1: their limbs plus one (a ripple through the leading limbs equal to B - 1) */
-__global__ __launch_bounds__(64) void k_addsub_fix(uint64_t *r, uint64_t nout, const uint32_t *status, uint64_t nblocks)
-{
-    constexpr int CH = CRT_T * CRT_WIDE;
-    const int lane = threadIdx.x;
-    const uint64_t blk = blockIdx.x;
-    if (blk >= nblocks || !(status[blk] & CRT_ST_CIN)) return;
-    const uint64_t k0 = blk * CH, end = k0 + CH < nout ? k0 + CH : nout;
-    for (uint64_t base = k0; base < end; base += 64) {
-        const uint64_t k = base + lane;
-        const uint64_t v = k < end ? r[k] : 0;
-        const uint64_t ne = __ballot(k < end && v != NTTM_B - 1);
-        const int f = ne ? __ffsll((long long)ne) - 1 : 64;                    /* first limb below B - 1 */
-        if (k < end && lane <= f) r[k] = lane < f ? 0 : v + 1;
-        if (ne) return;
-    }
-}
 int nttm_run_addsub(uint64_t *r, uint64_t nout, const uint64_t *a, uint64_t na, uint64_t sa, int64_t apow, const uint64_t *b,
                     uint64_t nb, uint64_t sb, int64_t bpow, int sub, uint32_t *scratch, hipStream_t s)
 {
@@ -540,13 +465,13 @@ int nttm_run_addsub(uint64_t *r, uint64_t nout, const uint64_t *a, uint64_t na, 
     AddArgs A;
     A.a = a; A.na = a ? na : 0; A.sa = sa; A.apow = apow; A.b = b; A.nb = b ? nb : 0; A.sb = sb; A.bpow = bpow;
     A.r = r; A.nout = nout; A.nblocks = nblocks; A.sub = sub; A.status = scratch + CRT_CTL_WORDS;
+    A.ctl = scratch;
     hipLaunchKernelGGL(k_addsub, dim3((unsigned)nblocks), dim3(CRT_T), 0, s, A);
     int rc = nttm_hip_check(hipGetLastError(), "k_addsub launch");
     if (rc) return rc;
-    hipLaunchKernelGGL(k_crt_scan, dim3(1), dim3(CRT_SCAN_T), 0, s, A.status, nblocks, scratch, (uint64_t *)nullptr);
-    if ((rc = nttm_hip_check(hipGetLastError(), "k_crt_scan launch"))) return rc;
-    hipLaunchKernelGGL(k_addsub_fix, dim3((unsigned)nblocks), dim3(64), 0, s, r, nout, (const uint32_t *)A.status, nblocks);
-    return nttm_hip_check(hipGetLastError(), "k_addsub_fix launch");
+    CrtDesc d; memset(&d, 0, sizeof d);
+    d.c = r; d.nc = nout;
+    return nttm_crt_launch_carry(nullptr, &d, 1, nblocks, scratch, scratch, s, CRT_WIDE, nullptr);
 }
 
 /* the normalized length of x[0 .. n): one more than the index of the highest nonzero limb */

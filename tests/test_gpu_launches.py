@@ -159,3 +159,39 @@ def test_one_kernel_products(schedule, n, nprimes):
     over[:len(a)] = items[0][0]
     lib.mul(over[:len(a)], items[0][1], out=over)
     assert np.array_equal(host(over), w)
+
+
+# blocks of 2048 limbs: within one workgroup's 64, across workgroups, beyond one look of 256 words, an odd end
+@pytest.mark.parametrize("blocks,extra", [(1, 0), (63, 5), (64, 0), (65, 1), (129, 2047), (320, 0), (900, 77)])
+def test_carry_through_blocks(nttm, blocks, extra):
+    """1 (B^n - 1) + x: with x = 1 the carry out of the first limb runs through every block to the top, with x = 0 (and
+    with x = 1 placed one limb below a limb that stops it) it does not; the same by the device addition and, for the
+    sign, the subtraction"""
+    import torch
+    n = 2048 * blocks + extra
+    one = dev(np.array([1], dtype=np.uint64))
+    nines = torch.full((n,), O.B - 1, dtype=torch.int64, device="cuda")
+    say("carry through", blocks, extra)
+    c = nttm.mul_add(one, nines, one)
+    assert int(c[n]) == 1 and int(c.count_nonzero()) == 1
+    c = nttm.mul_add(one, nines, torch.zeros(1, dtype=torch.int64, device="cuda"))
+    assert bool((c[:n] == O.B - 1).all()) and not bool(c[n:].any())
+    for stop in {0, n // 2, n - 1}:
+        b = nines.clone()
+        b[stop] = 5
+        b[n - 1].clamp_(min=1)
+        c = nttm.mul_add(one, b, one)
+        want = b.clone()
+        want[:stop] = 0
+        want[stop] = 6
+        assert torch.equal(c[:n], want) and not bool(c[n:].any())
+    r, carry = nttm.debug_addsub(nines, one, n)
+    assert carry and not bool(r.any())
+    r, carry = nttm.debug_addsub(nines, one, n + 1)
+    assert not carry and int(r[n]) == 1 and int(r.count_nonzero()) == 1
+    top = torch.zeros(n + 1, dtype=torch.int64, device="cuda")
+    top[n] = 1
+    r, ge = nttm.debug_addsub(top, one, n + 1, sub=True)
+    assert ge and bool((r[:n] == O.B - 1).all()) and int(r[n]) == 0
+    r, ge = nttm.debug_addsub(one, top, n + 1, sub=True)
+    assert not ge
