@@ -35,7 +35,8 @@ int nttm_run_addsub(uint64_t *r, uint64_t nout, const uint64_t *a, uint64_t na, 
                     uint64_t nb, uint64_t sb, int64_t bpow, int sub, uint32_t *scratch, hipStream_t s);
 int nttm_run_top_nonzero(const uint64_t *x, uint64_t n, uint64_t *out_dev, hipStream_t s);
 int nttm_copy_to_host(void *dst, const void *src, size_t bytes, hipStream_t s);
-int nttm_copy_to_host_prepare(void);
+int nttm_copy_to_host_prepare(size_t bytes);
+size_t nttm_copy_to_host_min(void);
 int nttm_mul_cyclic(uint64_t *v, const uint64_t *a, size_t na, const uint64_t *b, size_t nb, size_t L, hipStream_t s,
                     const uint32_t **flag);
 int nttm_mul_launch(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b, size_t nb, hipStream_t s,
@@ -515,19 +516,19 @@ extern "C" int nttm_e_fraction(uint64_t *out, size_t m, void *stream)
     size_t N = 2;
     while (lgamma((double)N + 1.0) < need) N += N / 2 + 1;
     { size_t lo = N / 2, hi = N; while (lo + 1 < hi) { size_t md = (lo + hi) / 2; if (lgamma((double)md + 1.0) < need) lo = md; else hi = md; } N = hi; }
-    /* the download's pinned buffers (a fraction above 64 MiB goes through them), allocated and first touched on
+    /* the download's pinned buffers (a fraction above 1 MiB goes through them), allocated and first touched on
      * another host thread while the device forms the series (inside the copy, their first use cost about 7 ms at
      * 10^9 digits) */
     struct Prep {
         std::thread t;
-        explicit Prep(bool on)
+        Prep(bool on, size_t bytes)
         {
             int dev = 0;
             if (on && hipGetDevice(&dev) == hipSuccess)         /* a new thread starts on device 0: the caller's device */
-                t = std::thread([dev]() { if (hipSetDevice(dev) == hipSuccess) (void)nttm_copy_to_host_prepare(); });
+                t = std::thread([dev, bytes]() { if (hipSetDevice(dev) == hipSuccess) (void)nttm_copy_to_host_prepare(bytes); });
         }
         ~Prep() { if (t.joinable()) t.join(); }
-    } prep(m * 8 > ((size_t)64 << 20));
+    } prep(m * 8 > nttm_copy_to_host_min(), m * 8);
     DevOps o;
     /* the arena: the series' leaves (about 2 m limbs per schoolbook level) and root, the Newton levels' numbers
      * (their products, wrapped products of L + 3 limbs and differences: about 12 m limbs over all levels) and the
@@ -554,7 +555,7 @@ extern "C" int nttm_e_fraction(uint64_t *out, size_t m, void *stream)
         }
         void join() { for (std::thread &x : t) if (x.joinable()) x.join(); }
         ~Touch() { join(); }
-    } touch(m * 8 > ((size_t)64 << 20), (char *)out, m * 8);
+    } touch(m * 8 > nttm_copy_to_host_min(), (char *)out, m * 8);
     bool ge;
     RCK(o.addsub(A, P, 0, Q, 0, true, &ge));                      /* e - 2 ~ A / Q, 0 <= A < Q */
     if (!ge || !A.n) return nttm_fail(NTTM_ECHECK, "e pipeline: P <= Q");
