@@ -22,6 +22,7 @@ void nttm_set_pts(int pts);
 int nttm_get_pts(void);
 void nttm_set_fixed_shapes(int on);
 void nttm_set_stream(int on, int ncu);
+#define NTTM_CRT_RUNS 0            /* the carry launch's blocks are k_inv_crt's runs */
 #define NTTM_FUSED_LOG 12          /* tile of the fused forward + pointwise + inverse pass (k_fused2) */
 #define NTTM_TILE_LOG_DEFAULT 13   /* tile of the strided passes: 2^13 points (64 KiB of LDS), runs of 32 columns */
 #define NTTM_PRODUCT_LOGN_MIN 4    /* products use at least 2^4 points, so every fused tile has >= 16 */
@@ -45,6 +46,11 @@ int nttm_crt_launch_one(const CrtDesc &d, uint64_t nblocks, int np, const CrtCon
                         hipStream_t s, double alg_bytes, uint64_t *stamps = nullptr, const uint64_t *const *res = nullptr);
 uint64_t nttm_crt_blocks(uint64_t nc, int per = 8);      /* per: CRT limbs per thread, 8 (2048-limb blocks) or 1 (256) */
 uint64_t nttm_crt_scratch_words(uint64_t nblocks);
+int nttm_inv_crt_ok(int logn, int lo, int m);
+uint64_t nttm_inv_crt_blocks(int m);
+int nttm_run_inv_crt(int np, int m, const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, const TwTables *inv,
+                     const CrtConst &cc, uint32_t *scratch, uint32_t *ctl, int first, hipStream_t s, double alg_bytes,
+                     uint64_t *stamp);
 int nttm_small_log(int logn);
 int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1,
                    uint64_t cnt, uint64_t *ncn, uint32_t *ctl, const TwTables *fwd, const TwTables *inv, const double2 *ninv,
@@ -151,6 +157,7 @@ static uint64_t g_par_points = (uint64_t)1 << 24;
  * the 4096 leaves' replay takes 5.83 ms at 2^24 points, 5.91 at 2^22, 6.71 at 2^21, 8.41 at 2^20 (four more launches
  * per chunk).  NTTM_CHUNK_POINTS overrides it. */
 static uint64_t g_chunk_points = (uint64_t)1 << 24;
+static uint64_t g_inv_crt_points = (uint64_t)1 << 22;   /* the last inverse pass with the CRT (inv_crt_bits) */
 
 /* the workspace of nttm_mul_noalloc: a file-scope device array, one copy per GPU, held until the process ends.  Host
  * code never uses its name as an address (on the host it is a stand-in, not the device address): nttm_init looks up
@@ -233,8 +240,8 @@ static void build_crt_const(CrtConst &cc)
 static int build_tables(void)
 {
     const size_t nst = (size_t)1 << NTTM_STAGE_LOG;
-    const size_t nbq = (size_t)4 << NTTM_BQ_LOG, nb3 = nbq + 1;
-    const size_t per_dir = nst + nbq + nb3, total = (size_t)NTTM_MAX_PRIMES * 2 * per_dir;
+    const size_t nbq = (size_t)4 << NTTM_BQ_LOG, nb3 = nbq + 1, ncol = (size_t)2 << 12;
+    const size_t per_dir = nst + nbq + nb3 + ncol, total = (size_t)NTTM_MAX_PRIMES * 2 * per_dir;
     std::vector<double2> h(total);
     for (int i = 0; i < NTTM_MAX_PRIMES; i++) {
         const uint64_t p = NTTM_PRIMES[i];
@@ -254,6 +261,12 @@ static int build_tables(void)
                 }
             }
             b3[nbq] = h_shoup(h_powmod(g.root3x32[i], (uint64_t)1 << 32, p), p);   /* the forward cube root */
+            double2 *co = b3 + nb3;
+            for (int m = 3; m <= 4; m++) {                               /* (unused in the forward direction) */
+                const uint64_t wm = h_powmod(w32, (uint64_t)1 << (32 - 12 - m), p);
+                uint64_t v = 1;
+                for (size_t c = 0; c < ((size_t)1 << 12); c++) { co[((size_t)(m - 3) << 12) + c] = h_shoup(v, p); v = h_mulmod(v, wm, p); }
+            }
             st[0] = h_shoup(1, p);
             for (int s = 0; s + 1 < NTTM_STAGE_LOG + 1 && ((size_t)1 << s) < nst; s++) {
                 const uint64_t ws = h_powmod(w32, (uint64_t)1 << (32 - (s + 1)), p);   /* order 2^(s+1) */
@@ -275,7 +288,7 @@ static int build_tables(void)
         for (int dir = 0; dir < 2; dir++) {
             const double2 *st = g.tables + ((size_t)i * 2 + dir) * per_dir;
             TwTables t; t.stage = st; t.bq = st + nst;
-            t.b3 = t.bq + nbq;
+            t.b3 = t.bq + nbq; t.col = t.b3 + nb3;
             if (dir) g.twi[i] = t; else g.twf[i] = t;
         }
     return 0;
@@ -436,9 +449,10 @@ extern "C" int nttm_init(int device, const nttm_config *cfg)
         g_no_defer = e && e[0] == '1';
     }
     {
-        const char *e = getenv("NTTM_PAR_POINTS"), *c = getenv("NTTM_CHUNK_POINTS");
+        const char *e = getenv("NTTM_PAR_POINTS"), *c = getenv("NTTM_CHUNK_POINTS"), *v = getenv("NTTM_INV_CRT_POINTS");
         g_par_points = e ? strtoull(e, nullptr, 0) : (uint64_t)1 << 24;
         g_chunk_points = c && strtoull(c, nullptr, 0) ? strtoull(c, nullptr, 0) : (uint64_t)1 << 24;
+        g_inv_crt_points = v && strtoull(v, nullptr, 0) ? strtoull(v, nullptr, 0) : (uint64_t)1 << 22;
     }
     {
         const char *e = getenv("NTTM_TREE_LEVELWISE");
@@ -575,6 +589,23 @@ static void product_plan(Plan *pl, int logn, uint64_t batch, int tile_log)
 {
     plan_make3(pl, logn, batch, tile_log, fused_bits(logn, tile_log), NTTM_FUSED_LOG);
 }
+/* the bits of a product transform's last inverse pass where it runs fused with the CRT (k_inv_crt: transforms of 2^13 to
+ * 2^16 points, whose one strided pass has at most 16 rows), else 0.  With 2 and 4 rows always: a batch of equal products
+ * against the two kernels, us, 2^13: 1 of them 53 / 59, 16 55 / 62, 256 138 / 162; 2^14: 52 / 55, 63 / 68, 215 / 250.
+ * With 8 and 16 a wave is long (120 to 250 registers) and few of them are slower than the two kernels that spread the same
+ * work wider: from 2^22 points.  2^15: 1 60 / 55, 64 152 / 153, 128 237 / 243, 256 441 / 464; 2^16: 1 63 / 57, 32 154 / 151,
+ * 64 242 / 244, 128 445 / 461, 256 839 / 894.  NTTM_INV_CRT_POINTS overrides that line. */
+static int inv_crt_bits(int logn, int r3, uint64_t cnt)
+{
+    if (r3 || g_no_small || g_fused_bits_env || logn <= NTTM_FUSED_LOG || logn > NTTM_FUSED_LOG + 4) return 0;
+    return logn <= NTTM_FUSED_LOG + 2 || (cnt << logn) >= g_inv_crt_points ? logn - NTTM_FUSED_LOG : 0;
+}
+/* the most blocks of the CRT of a product of nc limbs from a 2^logn (3 2^logn) point transform of n points */
+static uint64_t prod_crt_blocks(int logn, int r3, uint64_t n, uint64_t nc)
+{
+    const int m = inv_crt_bits(logn, r3, (uint64_t)1 << 32);
+    return std::max(m ? nttm_inv_crt_blocks(m) : 0, nttm_crt_blocks(nc, n <= 1024 ? 1 : 8));
+}
 
 /* the transforms of cnt products of one length: 2^logn points (r3 = 0), or 3 2^logn points (r3 = 1: a radix-3 layer,
  * reading the limbs, and the 2^logn engine on the 3 cnt thirds).  Plane i of A holds the cnt transforms of prime i back
@@ -582,7 +613,7 @@ static void product_plan(Plan *pl, int logn, uint64_t batch, int tile_log)
  * Shared B operands (bmap non-null): B's plane holds the cnt_b distinct operands of ldesc_b; A's engine transform t
  * pairs with B's engine transform bmap[t] in the double-fused pass.
  * pev (or null): 2 np events recorded around B's transform of each prime.  stamps (or null): the device clock at the
- * start of the first forward launch and of the double-fused pass. */
+ * start of the first forward launch and of the double-fused pass.  inv_crt: A's last inverse pass is left to k_inv_crt. */
 /* the first forward pass (from limbs) leaves its boundary twiddles to the second when both are streamed strided
  * passes (a transform of three or more passes): the limb pass has no VALU to spare, the second pass, bound by HBM, has.
  * q: the first pass's arguments (limbs set, in_scale as the caller wants it applied) */
@@ -611,7 +642,7 @@ static PassJob prime_job(int i, double *x, uint64_t batch, bool inv)
 static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A, double *Bp, uint64_t bstride,
                               const uint64_t *a, uint64_t na, const uint64_t *b, uint64_t nb, const LoadDesc *ldesc,
                               hipStream_t s, hipEvent_t *pev, uint64_t cnt_b = 0, const LoadDesc *ldesc_b = nullptr,
-                              const uint32_t *bmap = nullptr, uint64_t *stamps = nullptr)
+                              const uint32_t *bmap = nullptr, uint64_t *stamps = nullptr, bool inv_crt = false)
 {
     if (!bmap) { cnt_b = cnt; ldesc_b = ldesc; }
     const uint64_t tb = r3 ? 3 * cnt : cnt, tbb = r3 ? 3 * cnt_b : cnt_b;   /* engine transforms of 2^logn points */
@@ -621,6 +652,8 @@ static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A,
     const int last = pl.npass - 1;
     if (bmap && (plb.npass != pl.npass || pl.p[last].m + pl.p[last].logh > logn || (last == 0 && !r3)))
         return nttm_fail(NTTM_EINVAL, "internal: shared B operands on this length");
+    if (inv_crt && (last != 1 || !nttm_inv_crt_ok(logn, pl.p[0].lo, pl.p[0].m)))
+        return nttm_fail(NTTM_EINVAL, "internal: no CRT with the inverse pass at this length");
     /* both operands' strided passes in one launch where every prime is too, and where their geometry is the same (it
      * differs only in the blocks a tile spans, by the powers of two in the two batch counts) */
     bool pair = bstride > 0;
@@ -690,7 +723,7 @@ static int product_transforms(int np, int logn, int r3, uint64_t cnt, double *A,
         }
         RCK(nttm_run_fused2(fa, fb, pl.p[last], s, jf));
         PassArgs ia = base_args(i0, ji.j[0].x, logn, tb, true);
-        for (int j = last - 1; j >= 0; j--) RCK(nttm_run_pass(true, ia, pl.p[j], s, &ji));
+        for (int j = last - 1; j >= (inv_crt ? 1 : 0); j--) RCK(nttm_run_pass(true, ia, pl.p[j], s, &ji));
         if (r3) {
             for (int k = 0; k < step; k++) ji.j[k].batch = cnt;
             RCK(nttm_run_r3(true, logn, ji, s));
@@ -744,7 +777,7 @@ static int one_plan(size_t na, size_t nb, size_t nc, OnePlan *o)
     if (o->logn > NTTM_LOGN_MAX) return 1;
     o->n = (uint64_t)(o->r3 ? 3 : 1) << o->logn;
     o->planes_bytes = (size_t)(o->np + 1) * o->n * 8;
-    o->crt_words = nttm_crt_scratch_words(nttm_crt_blocks(nc));
+    o->crt_words = nttm_crt_scratch_words(std::max(nttm_crt_blocks(nc), prod_crt_blocks(o->logn, o->r3, o->n, nc)));
     o->ws_bytes = align_up(o->planes_bytes, 256) + 256 + o->crt_words * 4 + 256;
     return 0;
 }
@@ -768,7 +801,7 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
     L->n = (uint64_t)(L->r3 ? 3 : 1) << L->logn;                  /* points per plane */
     /* np planes of A and one of B: B's transform of each prime is made just before A's of that prime; primes in one
      * launch take a B plane each */
-    const size_t crt_words = nttm_crt_scratch_words(nttm_crt_blocks(L->nc));
+    const size_t crt_words = nttm_crt_scratch_words(std::max(nttm_crt_blocks(L->nc), prod_crt_blocks(L->logn, L->r3, L->n, L->nc)));
     for (int par = allow_par && L->np > 1 && L->n <= g_par_points; par >= 0; par--) {
         const size_t planes_bytes = (size_t)(par ? 2 * L->np : L->np + 1) * L->n * 8;
         L->par = par;
@@ -841,13 +874,17 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     if (stamps) stamps[0] = ~(uint64_t)0;                        /* (a transform of one pass has no forward launch) */
 
     if (events) HIPCK(hipEventRecord(g.ev[0], s));
+    const int im = inv_crt_bits(L.logn, L.r3, 1);
     RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, L.par ? L.n : 0, a, na, b, nb, nullptr, s, events ? g.pev : nullptr, 0,
-                           nullptr, nullptr, stamps));
+                           nullptr, nullptr, stamps, im != 0));
     if (events) HIPCK(hipEventRecord(g.ev[2], s));
     hd.pl = A;
-    RCK(nttm_crt_launch_one(hd, nttm_crt_blocks(nc), L.np, g.cc, crt_scr, ctl, s,
-                            8.0 * L.np * (double)L.ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? (nx < nc ? nx : nc) : 0),
-                            stamps ? stamps + 2 : nullptr));
+    const double crt_bytes = 8.0 * L.np * (double)L.ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? (nx < nc ? nx : nc) : 0);
+    if (im) {
+        RCK(nttm_run_inv_crt(L.np, im, nullptr, &hd, 1, g.twi, g.cc, crt_scr, ctl, 1, s, crt_bytes, stamps ? stamps + 2 : nullptr));
+        RCK(nttm_crt_launch_carry(nullptr, &hd, 1, nttm_inv_crt_blocks(im), crt_scr, ctl, s, NTTM_CRT_RUNS, stamps ? stamps + 3 : nullptr));
+    } else
+        RCK(nttm_crt_launch_one(hd, nttm_crt_blocks(nc), L.np, g.cc, crt_scr, ctl, s, crt_bytes, stamps ? stamps + 2 : nullptr));
     if (events) HIPCK(hipEventRecord(g.ev[3], s));
     if (!sync) return 0;
     HIPCK(hipStreamSynchronize(s));
@@ -1110,6 +1147,7 @@ extern "C" int nttm_last_phase_ms(double *f, double *i, double *c)
 struct GroupBuild {
     int r3 = 0, logn = 0, tile = 0, pts = 0;
     int crt_per = 8;                                             /* CRT limbs per thread: 1 when every product is small */
+    int inv_m = 0;                                               /* the last inverse pass's bits where the CRT runs it */
     uint64_t n = 0, cnt = 0, cnt_b = 0, nblk = 0;
     bool share = false, merged = false, small = false;
     struct Chunk { uint64_t c0, cn, b0, cnb, blk0, nblk; double crt_bytes; };   /* products, distinct B operands, CRT blocks */
@@ -1134,7 +1172,8 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
     gb.r3 = r3; gb.logn = logn; gb.tile = tile; gb.pts = pts;
     const uint64_t n = (uint64_t)(r3 ? 3 : 1) << logn, cnt = G.size();          /* points per product plane */
     gb.n = n; gb.cnt = cnt; gb.nblk = 0; gb.cnt_b = 0; gb.planes_bytes = 0;
-    gb.crt_per = n <= 1024 ? 1 : 8;                              /* products of at most n + 1 limbs: 256-limb blocks */
+    gb.inv_m = inv_crt_bits(logn, r3, cnt);
+    gb.crt_per = gb.inv_m ? NTTM_CRT_RUNS : n <= 1024 ? 1 : 8;    /* (products of at most n + 1 limbs: 256-limb blocks) */
     gb.cd.assign(cnt, CrtDesc()); gb.ld.assign(cnt, LoadDesc()); gb.ldb.clear(); gb.bmap.clear(); gb.chunk.clear();
     gb.small = small_len(logn, r3);                              /* one kernel, no planes and no CRT blocks */
     const uint64_t cmax = gb.small ? cnt : chunk_products(n);
@@ -1149,7 +1188,7 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
             l.a = q.a; l.na = q.na; l.b = q.b; l.nb = q.nb;
             c.pl = nullptr; c.plane = ch.cn * n; c.ncoef = q.na + q.nb - 1; c.x = q.x; c.nx = q.x ? q.nx : 0;
             c.c = q.c; c.nc = q.na + q.nb + (q.x ? 1 : 0); c.first_block = gb.nblk; c.trunc = 0;
-            if (!gb.small) gb.nblk += nttm_crt_blocks(c.nc, gb.crt_per);
+            if (!gb.small) gb.nblk += gb.inv_m ? nttm_inv_crt_blocks(gb.inv_m) : nttm_crt_blocks(c.nc, gb.crt_per);
             ch.crt_bytes += gb.small ? 8.0 * (q.na + q.nb) + 8.0 * c.nc + 8.0 * c.nx : 8.0 * np * c.ncoef + 8.0 * c.nc + 8.0 * c.nx;
         }
         ch.nblk = gb.nblk - ch.blk0;
@@ -1229,8 +1268,12 @@ static int group_launch(const GroupBuild &gb, int np, double *A, char *dbase, hi
         const LoadDesc *ld = (const LoadDesc *)(dbase + gb.off_ld) + ch.c0;
         rc = product_transforms(np, gb.logn, gb.r3, ch.cn, A, Bp, gb.merged ? ch.cnb * gb.n : 0, nullptr, 0, nullptr, 0, ld, s,
                                 nullptr, ch.cnb, gb.share ? (const LoadDesc *)(dbase + gb.off_ldb) + ch.b0 : nullptr,
-                                gb.share ? (const uint32_t *)(dbase + gb.off_bmap) + (gb.r3 ? 3 : 1) * ch.c0 : nullptr);
-        if (!rc) rc = nttm_crt_launch_limbs((const CrtDesc *)(dbase + gb.off_cd) + ch.c0, nullptr, ch.cn, ch.blk0, ch.nblk, np,
+                                gb.share ? (const uint32_t *)(dbase + gb.off_bmap) + (gb.r3 ? 3 : 1) * ch.c0 : nullptr, nullptr,
+                                gb.inv_m != 0);
+        if (!rc && gb.inv_m)
+            rc = nttm_run_inv_crt(np, gb.inv_m, (const CrtDesc *)(dbase + gb.off_cd) + ch.c0, nullptr, ch.cn, g.twi, g.cc,
+                                  (uint32_t *)(dbase + gb.off_crt), ctl, ch.c0 == 0, s, ch.crt_bytes, nullptr);
+        else if (!rc) rc = nttm_crt_launch_limbs((const CrtDesc *)(dbase + gb.off_cd) + ch.c0, nullptr, ch.cn, ch.blk0, ch.nblk, np,
                                             g.cc, (uint32_t *)(dbase + gb.off_crt), ctl, s, ch.crt_bytes, gb.crt_per);
         if (rc) break;
     }
@@ -1312,7 +1355,7 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
         const int r3 = gi > NTTM_LOGN_MAX, logn = (int)(gi % (NTTM_LOGN_MAX + 1));
         const uint64_t n = pts(gi), cnt = G.size();
         uint64_t blk = 0;
-        for (size_t i : G) blk += nttm_crt_blocks(P[i].na + P[i].nb + (P[i].x ? 1 : 0), n <= 1024 ? 1 : 8);
+        for (size_t i : G) blk += prod_crt_blocks(logn, r3, n, P[i].na + P[i].nb + (P[i].x ? 1 : 0));
         if (!small_len(logn, r3)) planes = std::max(planes, chunk_planes_bytes(np, n, cnt));
         const size_t im = align_up(cnt * sizeof(CrtDesc), 256) + 2 * align_up(cnt * sizeof(LoadDesc), 256) +
                           align_up((r3 ? 3 : 1) * cnt * 4, 256) + 512;
@@ -2010,7 +2053,7 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
                 const uint64_t npts = (uint64_t)(r3 ? 3 : 1) << logn;
                 kk[2 * i + t] = (int8_t)key;
                 cnt[key]++;
-                blk[key] += nttm_crt_blocks(na + nb + (t == 0 ? 1 : 0), npts <= 1024 ? 1 : 8);
+                blk[key] += prod_crt_blocks(logn, r3, npts, na + nb + (t == 0 ? 1 : 0));
             }
         }
         RCK(choose_np(mn_max, &lev_np[k]));

@@ -21,10 +21,12 @@
 #include <string.h>
 #include "internal.h"
 #include "crt_dev.h"
+#include "rounds.h"
 
 #define CRT_T 256
 #define CRT_WIDE 8                       /* limbs per thread of a block (2048-limb blocks); groups of small products
                                             use 1 (256-limb blocks, less of a block idle past a product's end) */
+#define CRT_RUNS 0                       /* in place of the limbs per thread: the blocks are k_inv_crt's runs */
 #define CRT_HALO 4                       /* digits of coefficients k0-4 .. k0-1: v_{k0-1} with four primes */
 #define CRT_ID_MAP 0x2u                  /* one-bit carry maps: bit c = cout(cin = c); the identity is 0b10 */
 #define CRT_CTL_WORDS 4                  /* control words before the block status words (16-byte aligned) */
@@ -217,11 +219,18 @@ __device__ __forceinline__ uint32_t crt_step_map(uint32_t st)
  * (Two launches before, one workgroup scanning the maps of all blocks and the fix: 57 + 6 us at 131072 blocks, 5 + 4 at
  * few.) */
 #define CRT_CARRY_W 64
-template <int PER>
+/* the runs of k_inv_crt: a product of 2^m rows of 2^RUN_LO limbs has RUN_BLOCKS runs per row, RUN_LEN limbs each (the last
+ * shorter), and one more for the limbs beyond the transform */
+#define RUN_LO 12
+#define RUN_LEN 60
+#define RUN_GROUPS(m) ((m) == 4 ? 1 : 2)        /* runs per row and wave */
+#define RUN_BLOCKS (((1 << RUN_LO) + RUN_LEN - 1) / RUN_LEN)
+/* RUNS: the blocks are k_inv_crt's runs of limbs instead of PER 256 limbs each */
+template <int PER, bool RUNS = false>
 __global__ __launch_bounds__(256) void k_carry(const CrtDesc *desc, CrtDesc one, uint64_t nprod, const uint32_t *status,
                                                uint64_t n, uint32_t *ctl, uint64_t *stamp)
 {
-    constexpr int CH = CRT_T * PER;
+    constexpr int CH = RUNS ? 64 : CRT_T * PER;
     stamp_clock(stamp);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t b0 = (uint64_t)blockIdx.x * CRT_CARRY_W;
@@ -257,7 +266,13 @@ __global__ __launch_bounds__(256) void k_carry(const CrtDesc *desc, CrtDesc one,
         while (lo < hi) { const uint64_t mid = (lo + hi + 1) >> 1; if (desc[mid].first_block <= blk) lo = mid; else hi = mid - 1; }
         CrtDesc d = one;
         if (desc) d = desc[lo];
-        const uint64_t k0 = (blk - d.first_block) * CH, end = k0 + CH < d.nc ? k0 + CH : d.nc;
+        const uint64_t bl = blk - d.first_block;
+        uint64_t k0 = bl * CH, end = k0 + CH;
+        if (RUNS) {
+            const uint64_t row = bl / RUN_BLOCKS, ch = bl - row * RUN_BLOCKS;
+            k0 = (row << RUN_LO) + ch * RUN_LEN; end = ch + 1 < RUN_BLOCKS ? k0 + RUN_LEN : (row + 1) << RUN_LO;
+        }
+        end = end < d.nc ? end : d.nc;
         uint64_t v[CH / 64];
 #pragma unroll
         for (int j = 0; j < CH / 64; j++) { const uint64_t k = k0 + j * 64 + lane; v[j] = k < end ? d.c[k] : 0; }
@@ -274,6 +289,157 @@ __global__ __launch_bounds__(256) void k_carry(const CrtDesc *desc, CrtDesc one,
             if (k < end && o <= first_ne) d.c[k] = o < first_ne ? 0 : v[j] + 1;
         }
     }
+}
+
+/* ---- the last inverse pass and the CRT in one kernel ------------------------------------------------------------------
+ * For transforms of 2^m rows of 2^12 points, m = 1 .. 4 (one strided pass): a lane takes one column of the plane of each
+ * prime, all 2^m rows of it in registers, multiplies in the boundary twiddles w^-(c brev(j)) (powers of the column's table entry),
+ * runs the 2^m-point DIT and has the residues of 2^m coefficients of every prime, which it turns into digits and
+ * limbs as k_crt does.  Nothing is exchanged but between neighbouring lanes: a wave covers 60 columns and, in its first
+ * four lanes, the four before them (a row's first run takes the last four columns and their previous row), so
+ * every limb's lower digits and the quotient before the first limb come by shuffles.  A wave's run of 60 limbs is
+ * one ballot word and one block of the carry launch.  For m < 4 a wave takes two runs, every load requested at once.
+ * It replaces a pass over the planes (16 B read and written per point and prime) and the CRT's reads (8 B): bound by
+ * vector issue, about 290 instructions per coefficient, of which 1 in 16 is spent on the four repeated columns, at 2 to 5
+ * waves per SIMD.  4096 products of 64 to 65536 limbs: 1.15 ms against 0.64 (inverse pass) + 0.65 (k_crt). */
+struct InvCrtArgs {
+    const CrtDesc *desc; uint64_t nprod;        /* null: the one product `one` */
+    CrtDesc one;
+    uint32_t *status, *ctl;
+    int first;                                  /* the launch that clears ctl */
+    uint64_t *stamp;
+    const double2 *stage[NTTM_MAX_PRIMES];      /* inverse stage tables */
+    const double2 *step[NTTM_MAX_PRIMES];       /* (w, wq) of w_(2^(12 + m))^-c, c < 2^12 */
+    CrtConst cc;
+};
+__device__ __forceinline__ uint64_t shfl_up64(uint64_t v, int d) { return (uint64_t)__shfl_up((unsigned long long)v, d, 64); }
+
+template <int M, int NP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_inv_crt(InvCrtArgs a)
+{
+    constexpr int R = 1 << M, G = RUN_GROUPS(M), COLS = 1 << RUN_LO, WPP = (RUN_BLOCKS + G - 1) / G;
+    typedef const __attribute__((address_space(1))) double *GRes;
+    typedef const __attribute__((address_space(1))) uint64_t *GIn;
+    typedef __attribute__((address_space(1))) uint64_t *GOut;
+    typedef const __attribute__((address_space(1))) char *GByte;
+    typedef __attribute__((address_space(1))) char *GByteW;
+    stamp_clock(a.stamp);
+    if (a.first && blockIdx.x == 0 && threadIdx.x == 0) { a.ctl[0] = 0; a.ctl[1] = 0; }
+    const int lane = threadIdx.x & 63;
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const uint32_t prod = wid / WPP, ch0 = (wid - prod * WPP) * G;
+    if (prod >= a.nprod) return;
+    CrtDesc d = a.one;
+    if (a.desc) d = a.desc[prod];
+    /* (products of at most 2^16 + 2 limbs) */
+    const int ncoef = (int)d.ncoef, nc = (int)d.nc, nx = (int)(d.nx < d.nc ? d.nx : d.nc);
+
+    /* uniform bases and 32-bit lane offsets: a load's address costs no vector registers of its own */
+    double r[NP][G][R];
+    int col[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        col[g] = (int)(ch0 + g) * RUN_LEN + lane - 4;            /* a row's first run: -4 .. -1 are the previous row's end */
+        const uint32_t off = 8u * (uint32_t)(col[g] < 0 ? col[g] + COLS : col[g] < COLS ? col[g] : COLS - 1);
+#pragma unroll
+        for (int p = 0; p < NP; p++)
+#pragma unroll
+            for (int j = 0; j < R; j++)
+                r[p][g][j] = *(GRes)((GByte)(d.pl + p * d.plane + ((uint32_t)j << RUN_LO)) + off);
+    }
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const double P = a.cc.pk[p].p, PI = a.cc.pk[p].pinv;
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            const uint32_t c = (uint32_t)(col[g] < 0 ? col[g] + COLS : col[g] < COLS ? col[g] : COLS - 1);
+            typedef double v2d __attribute__((ext_vector_type(2)));
+            const v2d step = *(const __attribute__((address_space(1))) v2d *)((GByte)a.step[p] + 16u * c);
+            double w = step[0];
+            r[p][g][R / 2] = mul_shoup(r[p][g][R / 2], step[0], step[1], P);     /* brev(R / 2) = 1 */
+#pragma unroll
+            for (int i = 2; i < R; i++) {
+                w = mul_shoup(w, step[0], step[1], P);
+                r[p][g][brev_c<M>(i)] = mul_barrett(r[p][g][brev_c<M>(i)], w, P, PI);
+            }
+            dit_group<M, CTab>(r[p][g], 0, 0u, CTab(a.stage[p]), P, PI);
+            __builtin_amdgcn_sched_barrier(0);                   /* one column at a time: the registers hold the residues */
+        }
+    }
+    auto quot = [](uint64_t v) -> uint32_t {
+        uint32_t q = 0;
+#pragma unroll
+        for (int c = 1; c <= NP; c++) q += v >= (uint64_t)c * NTTM_B;
+        return q;
+    };
+    /* the limbs and the carry map of the run of row `row` from the lane's digits and x limb */
+    auto finish = [&](int g, int row, const uint64_t *dg, uint64_t x) {
+        const bool in = col[g] < COLS;
+        const int k = (row << RUN_LO) + col[g];
+        const bool limb = in && k >= 0 && k < nc, act = lane >= 4 && in;
+        uint64_t v = dg[0] + x;
+#pragma unroll
+        for (int j = 1; j < NP; j++) v += shfl_up64(dg[j], j);       /* (lanes below 3: unused) */
+        v = limb ? v : 0;
+        const uint32_t q = quot(v), qp = __shfl_up(q, 1, 64);
+        const uint64_t w = v - (uint64_t)q * NTTM_B + qp;
+        const uint64_t live = __ballot(act) >> 4;
+        const uint64_t X = __ballot(act && limb && w >= NTTM_B) >> 4;
+        const uint64_t Y = X | (__ballot(act && limb && w == NTTM_B - 1) >> 4) | ~live;   /* past the run: passed on */
+        const uint64_t CI = (X + Y) ^ X ^ Y;
+        const uint32_t oin = (uint32_t)(CI >> (lane - 4)) & 1u, oout = (uint32_t)(CI >> (lane - 3)) & 1u;
+        if (act && k < nc) *(GOut)((GByteW)d.c + 8u * (uint32_t)k) = w + oin - (oout ? NTTM_B : 0);
+        uint32_t st = add_cout(X, Y, 0) | (add_cout(X, Y, 1) << 1);
+        const uint64_t top = __ballot(act && k + 1 == nc);
+        if (top && !d.trunc) {                                   /* the last limb: nothing may remain beyond it */
+            uint64_t extra = q;
+#pragma unroll
+            for (int e = 1; e < NP; e++)
+#pragma unroll
+                for (int j = e; j < NP; j++) extra += j == e ? dg[j] : shfl_up64(dg[j], j - e);
+            const uint64_t C1 = (X + Y + 1) ^ X ^ Y;
+            const uint32_t o1 = (uint32_t)(C1 >> (lane - 3)) & 1u;
+            const int l = __ffsll((long long)top) - 1;
+            if ((__ballot(extra + oout != 0) >> l) & 1) st |= CRT_ST_E0;
+            if ((__ballot(extra + o1 != 0) >> l) & 1) st |= CRT_ST_E1;
+        }
+        const uint32_t b = (uint32_t)row * RUN_BLOCKS + ch0 + g;
+        if (lane == 0) a.status[d.first_block + b] = st | (b == 0 ? CRT_ST_FIRST : 0u);
+    };
+    /* CNT rows from row0 on: their x limbs requested, their digits side by side (one coefficient's are a serial chain) */
+#define RUN_ROWS(CNT, ROW0) { \
+        uint64_t xv[CNT], dg[CNT][NP]; \
+        _Pragma("unroll") \
+        for (int u = 0; u < CNT; u++) { \
+            const int k = (((ROW0) + u) << RUN_LO) + col[g]; \
+            xv[u] = 0; \
+            if (nx && col[g] < COLS && k >= 0 && k < nx) xv[u] = *(GIn)((GByte)d.x + 8u * (uint32_t)k); \
+        } \
+        _Pragma("unroll") \
+        for (int u = 0; u < CNT; u++) { \
+            const int rw = (ROW0) + u, k = (rw << RUN_LO) + col[g]; \
+            const bool coef = col[g] < COLS && k >= 0 && k < ncoef; \
+            double rz[NP]; \
+            _Pragma("unroll") \
+            for (int p = 0; p < NP; p++) { \
+                const double here = rw < R ? r[p][g][rw < R ? rw : 0] : 0.0, prev = rw ? r[p][g][rw ? rw - 1 : 0] : 0.0; \
+                rz[p] = coef ? (wrap ? prev : here) : 0.0; \
+            } \
+            crt_digits<NP>(a.cc, rz, dg[u]); \
+        } \
+        _Pragma("unroll") \
+        for (int u = 0; u < CNT; u++) finish(g, (ROW0) + u, dg[u], xv[u]); \
+    }
+    constexpr int U = R < 1 ? R : 1;
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        if (ch0 + g >= RUN_BLOCKS) break;
+        const bool wrap = col[g] < 0;
+#pragma unroll
+        for (int row = 0; row < R; row += U) RUN_ROWS(U, row)
+        if (ch0 + g == 0) RUN_ROWS(1, R)                         /* the limbs from 2^logn on: the last coefficients' upper digits */
+    }
+#undef RUN_ROWS
 }
 
 /* c[0 .. n) += *carry (0 or 1), the carry rippling through the leading limbs equal to B - 1 (one workgroup, 2048
@@ -372,10 +538,44 @@ int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t 
     if (one) d1 = *one;
     prof_begin("k_carry", 4.0 * (double)nblocks, s);
     const dim3 grid((unsigned)((nblocks + CRT_CARRY_W - 1) / CRT_CARRY_W));
-    if (per == 1) hipLaunchKernelGGL((k_carry<1>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
+    if (per == CRT_RUNS) hipLaunchKernelGGL((k_carry<1, true>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
+    else if (per == 1) hipLaunchKernelGGL((k_carry<1>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
     else hipLaunchKernelGGL((k_carry<CRT_WIDE>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_carry launch");
+}
+/* whether the last inverse pass of a 2^logn-point transform (bits [lo, lo + m) of the index) runs fused with the CRT */
+int nttm_inv_crt_ok(int logn, int lo, int m) { return lo == RUN_LO && m >= 1 && m <= 4 && lo + m == logn; }
+/* a product's blocks there (runs) */
+uint64_t nttm_inv_crt_blocks(int m) { return ((uint64_t)RUN_BLOCKS << m) + 1; }
+/* the last inverse pass and the CRT of nprod products of 2^(12 + m) points, from device descriptors (null: `one`), with
+ * nttm_inv_crt_blocks(m) blocks each from its descriptor's first_block on; first: the launch that clears ctl */
+int nttm_run_inv_crt(int np, int m, const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, const TwTables *inv,
+                     const CrtConst &cc, uint32_t *scratch, uint32_t *ctl, int first, hipStream_t s, double alg_bytes,
+                     uint64_t *stamp)
+{
+    if (np < 3 || np > NTTM_MAX_PRIMES || m < 1 || m > 4 || !nprod || (!desc_dev && (!one || nprod != 1)))
+        return nttm_fail(NTTM_EINVAL, "internal: inverse pass with the CRT");
+    InvCrtArgs a; memset(&a, 0, sizeof a);
+    a.desc = desc_dev; a.nprod = nprod; a.status = scratch + CRT_CTL_WORDS; a.ctl = ctl; a.first = first; a.stamp = stamp; a.cc = cc;
+    if (one) a.one = *one;
+    for (int i = 0; i < np; i++) { a.stage[i] = inv[i].stage; a.step[i] = m <= 2 ? inv[i].stage + ((size_t)1 << (RUN_LO - 1 + m)) : inv[i].col + ((size_t)(m - 3) << RUN_LO); }
+    const uint64_t g = RUN_GROUPS(m), waves = nprod * ((RUN_BLOCKS + g - 1) / g), blocks = (waves + 3) / 4;
+    if (blocks > 0x3fffffffULL || nprod * nttm_inv_crt_blocks(m) > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "internal: too many products");
+    const dim3 grid((unsigned)blocks);
+    prof_begin("k_inv_crt", alg_bytes, s);
+#define INV_CRT_LAUNCH(L) \
+    if (np == 3) hipLaunchKernelGGL((k_inv_crt<L, 3>), grid, dim3(256), 0, s, a); \
+    else hipLaunchKernelGGL((k_inv_crt<L, 4>), grid, dim3(256), 0, s, a);
+    switch (m) {
+    case 1: INV_CRT_LAUNCH(1) break;
+    case 2: INV_CRT_LAUNCH(2) break;
+    case 3: INV_CRT_LAUNCH(3) break;
+    default: INV_CRT_LAUNCH(4) break;
+    }
+#undef INV_CRT_LAUNCH
+    prof_end(s);
+    return nttm_hip_check(hipGetLastError(), "k_inv_crt launch");
 }
 /* one product, its descriptor passed with the launches: scratch 16-byte aligned, nttm_crt_scratch_words(nblocks) words.
  * stamps (or null): the device clock at the start of both launches.  res (or null): the np planes as

@@ -22,6 +22,7 @@ struct TwTables {                   /* device pointers, one set per prime and di
     const double2 *bq;              /* four-level boundary table: bq[k 2^8 + x] = w32^(x 2^(8k)), k < 4 (16 KiB) */
     const double2 *b3;              /* the same for the root W3 of order 3 2^32: b3[k 2^8 + x] = W3^(x 2^(8k)); entry
                                      * 4 2^8 is the FORWARD cube root of unity w3 = W3^(2^32) in both directions */
+    const double2 *col;             /* inverse tables only: col[(m - 3) 2^12 + c] = w_(2^(12 + m))^c, m = 3, 4 */
 };
 
 /* operand limbs of the products of a batch (device array, one per transform) */

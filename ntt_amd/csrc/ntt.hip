@@ -63,21 +63,6 @@ enum { PM_FWD = 0, PM_FWD_LIMB = 1, PM_INV = 2, PM_INV_PW = 3 };
 
 /* GM, GW, GH >= 0 fix the tile shape (m, logw, logh) at compile time: round splits, LDS strides and shifts fold to
  * constants; -1 takes them from the arguments */
-/* w^E for a 32-bit exponent fraction E from the four-level table (bq[k 2^8 + x] = w32^(x 2^(8k))), balanced
- * (|result| <= p/2 + 1) */
-__device__ __forceinline__ double bq_twiddle(const double2 *bq, uint32_t E, double p, double pinv)
-{
-    constexpr uint32_t M = (1u << NTTM_BQ_LOG) - 1;
-    double x = bq[(3 << NTTM_BQ_LOG) + (E >> 24)].x;
-    const double2 t2 = bq[(2 << NTTM_BQ_LOG) + ((E >> 16) & M)];
-    const double2 t1 = bq[(1 << NTTM_BQ_LOG) + ((E >> 8) & M)];
-    const double2 t0 = bq[E & M];
-    x = mul_shoup(x, t2.x, t2.y, p);
-    x = mul_shoup(x, t1.x, t1.y, p);
-    x = mul_shoup(x, t0.x, t0.y, p);
-    return reduce(x, p, pinv);
-}
-
 /* the boundary twiddles w_N^(col k) (N = 2^lom) of the round over row bits [0, LOGR) (s_lo = 0), multiplied into v:
  * group g of a thread has column c and bit-reversed rows k_j = kb + brev(j) 2^(m - LOGR), so its twiddles are
  * base * step^brev(j) with base = w^(c kb), step = w^(c 2^(m - LOGR)) -- two table twiddles and a chain of Shoup

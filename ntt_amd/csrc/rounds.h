@@ -56,6 +56,18 @@ __device__ __forceinline__ double2 tw_at(const GTab &tw, uint32_t lane, uint32_t
     return d;
 }
 
+/* a stage table read at compile-time indices only (uniform): through the scalar unit */
+struct CTab {
+    const __attribute__((address_space(4))) double2 *p;
+    __device__ __forceinline__ explicit CTab(const double2 *q) : p((const __attribute__((address_space(4))) double2 *)q) {}
+};
+__device__ __forceinline__ double2 tw_at(const CTab &tw, uint32_t, uint32_t fixed)
+{
+    typedef double v2d __attribute__((ext_vector_type(2)));
+    const v2d x = ((const __attribute__((address_space(4))) v2d *)tw.p)[fixed];
+    return make_double2(x[0], x[1]);
+}
+
 template <int LOGR, typename TW>
 __device__ __forceinline__ void dif_group(double *v, int s_lo, uint32_t rlow, TW tw, double p, double pinv)
 {
@@ -240,4 +252,19 @@ struct SwzLds {
     __device__ __forceinline__ double &operator[](uint32_t e) const { return p[e + (e >> 5)]; }
     __device__ __forceinline__ double &at(uint32_t pe) const { return p[pe]; }   /* an index padded already */
 };
+
+/* w^E for a 32-bit exponent fraction E from the four-level table (bq[k 2^8 + x] = w32^(x 2^(8k))), balanced
+ * (|result| <= p/2 + 1) */
+__device__ __forceinline__ double bq_twiddle(const double2 *bq, uint32_t E, double p, double pinv)
+{
+    constexpr uint32_t M = (1u << NTTM_BQ_LOG) - 1;
+    double x = bq[(3 << NTTM_BQ_LOG) + (E >> 24)].x;
+    const double2 t2 = bq[(2 << NTTM_BQ_LOG) + ((E >> 16) & M)];
+    const double2 t1 = bq[(1 << NTTM_BQ_LOG) + ((E >> 8) & M)];
+    const double2 t0 = bq[E & M];
+    x = mul_shoup(x, t2.x, t2.y, p);
+    x = mul_shoup(x, t1.x, t1.y, p);
+    x = mul_shoup(x, t0.x, t0.y, p);
+    return reduce(x, p, pinv);
+}
 #endif

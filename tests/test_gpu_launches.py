@@ -17,8 +17,8 @@ pytestmark = pytest.mark.gpu
 def schedule(nttm):
     import torch
 
-    def set_(par=None, chunk=None, **cfg):
-        for k, v in (("NTTM_PAR_POINTS", par), ("NTTM_CHUNK_POINTS", chunk)):
+    def set_(par=None, chunk=None, inv_crt=None, **cfg):
+        for k, v in (("NTTM_PAR_POINTS", par), ("NTTM_CHUNK_POINTS", chunk), ("NTTM_INV_CRT_POINTS", inv_crt)):
             if v is None:
                 os.environ.pop(k, None)
             else:
@@ -195,3 +195,45 @@ def test_carry_through_blocks(nttm, blocks, extra):
     assert ge and bool((r[:n] == O.B - 1).all()) and int(r[n]) == 0
     r, ge = nttm.debug_addsub(one, top, n + 1, sub=True)
     assert not ge
+
+
+# transforms of 2^13 .. 2^16 points: the last inverse pass runs with the CRT, in runs of 60 limbs of rows of 4096
+@pytest.mark.parametrize("n", [4097, 8191, 8192, 8193, 12289, 16384, 16385, 20481, 32767, 32768, 32769, 40961, 65535, 65536])
+@pytest.mark.parametrize("nprimes", [0, 4])
+def test_inverse_with_crt(schedule, n, nprimes):
+    """n coefficients, random and all limbs B - 1 (carries through every run and row), + x up to the transform's last limbs
+    and beyond, single, batched (chunks of one product among them) and planned; against the path without it"""
+    import torch
+    ops, s = [], n
+    for kind in ("random", "max"):
+        for na in sorted({1, n // 3 + 1, (n + 1) // 2}):
+            nb = n + 1 - na
+            a, s = _limbs(kind, na, s)
+            b, s = _limbs(kind, nb, s)
+            for nx in (None, 1, n + 1):
+                ops.append((a, b, None if nx is None else _limbs("max" if kind == "max" or nx == 1 else "random", nx, s)[0]))
+    ops.append((np.array([1], dtype=np.uint64), np.full(n, O.B - 1, dtype=np.uint64), np.array([1], dtype=np.uint64)))
+    say("inverse with crt", n, nprimes)
+    lib = schedule(nprimes=nprimes, inv_crt=1)
+    ps = [lib.prime(i) for i in range(4 if nprimes else 3)]
+    want = [O.mul_ntt(a, b, ps, x) for a, b, x in ops]
+    assert int(want[-1][n]) == 1 and not want[-1][:n].any()
+    items = [(dev(a), dev(b), None if x is None else dev(x),
+              torch.full((len(w),), -1, dtype=torch.int64, device="cuda")) for (a, b, x), w in zip(ops, want)]
+    for chunk in (None, 1, 3 << 16):
+        lib = schedule(nprimes=nprimes, chunk=chunk, inv_crt=1 if chunk else None)
+        prods = lib.make_prods(items)
+        lib.mul_batch(prods)
+        for it, w, pr in zip(items, want, prods):
+            assert np.array_equal(host(it[3]), w) and pr.ncn == int(np.nonzero(w)[0][-1]) + 1
+            it[3].fill_(-1)
+    plan = lib.BatchPlan(prods, autotune=False)
+    plan.run()
+    assert plan.ncn() == [pr.ncn for pr in prods]
+    assert all(np.array_equal(host(it[3]), w) for it, w in zip(items, want))
+    plan.close()
+    for it, w in list(zip(items, want))[::2]:
+        got = lib.mul(it[0], it[1]) if it[2] is None else lib.mul_add(it[0], it[1], it[2])
+        assert np.array_equal(host(got), w)
+    for cut in sorted({1, 60, 4096, 4097, n // 2, n}):
+        assert np.array_equal(host(lib.mul_cut(items[3][0], items[3][1], w=cut)), want[3][:cut])
