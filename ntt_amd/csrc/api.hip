@@ -157,6 +157,7 @@ static uint64_t g_par_points = (uint64_t)1 << 24;
  * the 4096 leaves' replay takes 5.83 ms at 2^24 points, 5.91 at 2^22, 6.71 at 2^21, 8.41 at 2^20 (four more launches
  * per chunk).  NTTM_CHUNK_POINTS overrides it. */
 static uint64_t g_chunk_points = (uint64_t)1 << 24;
+static int64_t g_pieces_points = -1;         /* NTTM_PIECES: 0 never in pieces, else pieces of that many points */
 static uint64_t g_inv_crt_points = (uint64_t)1 << 22;   /* the last inverse pass with the CRT (inv_crt_bits) */
 
 /* the workspace of nttm_mul_noalloc: a file-scope device array, one copy per GPU, held until the process ends.  Host
@@ -452,6 +453,8 @@ extern "C" int nttm_init(int device, const nttm_config *cfg)
         const char *e = getenv("NTTM_PAR_POINTS"), *c = getenv("NTTM_CHUNK_POINTS"), *v = getenv("NTTM_INV_CRT_POINTS");
         g_par_points = e ? strtoull(e, nullptr, 0) : (uint64_t)1 << 24;
         g_chunk_points = c && strtoull(c, nullptr, 0) ? strtoull(c, nullptr, 0) : (uint64_t)1 << 24;
+        const char *pp = getenv("NTTM_PIECES");
+        g_pieces_points = pp ? (int64_t)strtoull(pp, nullptr, 0) : -1;
         g_inv_crt_points = v && strtoull(v, nullptr, 0) ? strtoull(v, nullptr, 0) : (uint64_t)1 << 22;
     }
     {
@@ -787,8 +790,68 @@ static bool fits_one(size_t na, size_t nb, size_t nc)
     return !one_plan(na, nb, nc, &o) && (!g.cfg.workspace_bytes || o.ws_bytes <= g.cfg.workspace_bytes);
 }
 
-/* the workspace of a one-transform product: the planes, its CRT descriptor and the CRT's scratch (bytes from ws) */
-struct CoreLayout { int np, logn, r3, par; uint64_t n, ncoef; size_t nc, nc_full, off_desc, off_crt, bytes; };
+/* ---- uneven products -----------------------------------------------------------------------------------------------------
+ * A product of a long operand (alen limbs) by a shorter one (blen) need not take one transform that holds both: the long one is
+ * cut into cnt pieces of `step` limbs, each piece times the short operand fits a transform of n >= 2 blen points, all
+ * pieces run as one batch that shares the short operand's transform, and the CRT adds the overlap of neighbouring pieces
+ * (the first blen - 1 coefficients of a piece to the last ones of the piece before: sums of residues of one convolution,
+ * so the bound of its coefficients is the whole product's).  It saves the short operand's forward transform at full
+ * length, a pass where the pieces take two and the whole product three, and padding.  Per call, us, whole / in pieces:
+ * 300000 x 300 limbs 87 / 70, 1000000 x 100000 176 / 147, 5000003 x 300007 568 / 374, 5000003 x 2000 545 / 305,
+ * 20000000 x 1000000 2650 / 1950, 100000000 x 300 10500 / 5200; the rest of the plane lies where the model below sees less
+ * than its error: 30011 x 2100 56 / 57, 5000003 x 1500000 681 / 700. */
+struct Pieces { int logn, r3; uint64_t n, cnt, step; };      /* cnt = 0: the product whole */
+/* a product's time by its passes, us: 4 per launch and, per point and prime, 2.4 ps for the limb pass and 1.6 more where it
+ * reads limbs, 3.6 a forward and 3.3 an inverse strided pass, 3.0 (and the limbs) and 2.6 the radix-3 layers, 7.6 the double-fused pass; the
+ * CRT 2.5 per coefficient, 3.3 from pieces (kernel times of products of 2^20 to 2^28 points) */
+static double passes_us(int np, int logn, int r3, uint64_t cnt, uint64_t alen, uint64_t blen)
+{
+    Plan pl; product_plan(&pl, logn, 1, product_tile_log(logn));
+    const int st = pl.npass - 1;
+    const double n = (double)(r3 ? 3 : 1) * ldexp(1.0, logn), ca = (double)cnt * n;
+    const double fwd = r3 ? 3.0 + 3.6 * st : st ? 2.4 + 3.6 * (st - 1) : 0.0, inv = 3.3 * st + (r3 ? 2.6 : 0.0);
+    return 4.0 * (2 * st + (r3 ? 2 : 0) + 3) +
+           1e-6 * np * (ca * (fwd + 7.6 + inv) + n * fwd + 1.6 * (double)(alen + blen) + (cnt > 1 ? 3.3 : 2.5) * (double)(alen + blen));
+}
+static Pieces choose_pieces(int np, size_t alen, size_t blen, int logn, int r3)
+{
+    Pieces best{0, 0, 0, 0, 0};
+    const uint64_t whole = (uint64_t)(r3 ? 3 : 1) << logn;
+    if (alen < 2 * blen || g_pieces_points == 0) return best;    /* (two pieces of at least blen limbs) */
+    /* in pieces where the model saves 10 us and 15 %: its error is up to 8 % either way, the descriptors take 4 us */
+    double most = passes_us(np, logn, r3, 1, alen, blen);
+    most = std::min(0.85 * most, most - 10.0);
+    for (int l = 12; l <= 26; l++)
+        for (int t = l == 12; t < 2; t++) {                      /* 2^l points from 2^13, 3 2^l from 3 2^12 */
+            const uint64_t n = (uint64_t)(t ? 3 : 1) << l;
+            if (n >= whole || n < 2 * (uint64_t)blen || (t && g.cfg.radix3 == NTTM_R3_NEVER)) continue;
+            const uint64_t step = (n - blen + 1) & ~(uint64_t)31;        /* (aligned as the operand is) */
+            if (step < 2048 || step < blen) continue;
+            const uint64_t cnt = (alen + step - 1) / step;
+            if (cnt < 2 || cnt > 0x100000) continue;
+            const double us = passes_us(np, l, t, cnt, alen, blen);
+            if (g_pieces_points < 0 ? us < most : n == (uint64_t)g_pieces_points) { most = us; best = Pieces{l, t, n, cnt, step}; }
+        }
+    return best;
+}
+/* the descriptors of the pieces and the map to their one B operand: written by a kernel, since nothing on the host would
+ * live until a copy of them has run in a call that does not wait */
+__global__ __launch_bounds__(256) void k_pieces(LoadDesc *ld, uint32_t *bmap, const uint64_t *a, uint64_t alen, uint64_t step,
+                                                uint32_t cnt, const uint64_t *b, uint64_t blen, int r3)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= cnt) return;
+    const uint64_t o = i * step;
+    LoadDesc d; d.a = a + o; d.na = alen - o < step ? alen - o : step; d.b = b; d.nb = blen;
+    ld[i] = d;
+    if (!i) ld[cnt] = d;
+    if (r3) { for (int j = 0; j < 3; j++) bmap[3 * i + j] = (uint32_t)j; }
+    else bmap[i] = 0;
+}
+
+/* the workspace of a one-transform product: the planes, its CRT descriptor (the pieces' descriptors) and the CRT's scratch
+ * (bytes from ws).  n: points of the transforms, plane: of one prime's plane of A */
+struct CoreLayout { int np, logn, r3, par; uint64_t n, plane, ncoef, cnt, step; size_t nc, nc_full, off_desc, off_bmap, off_crt, bytes; };
 /* allow_par: one launch per pass for all primes, each with its own B plane (in the library's workspace) */
 static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout *L, bool allow_par = false)
 {
@@ -798,7 +861,25 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
     L->ncoef = ncoef_full < L->nc ? ncoef_full : L->nc;           /* coefficients read */
     choose_len(ncoef_full, &L->logn, &L->r3);
     if (L->logn > NTTM_LOGN_MAX) return nttm_fail(NTTM_EBOUND, "transform length 2^%d above 2^%d", L->logn, NTTM_LOGN_MAX);
-    L->n = (uint64_t)(L->r3 ? 3 : 1) << L->logn;                  /* points per plane */
+    L->n = L->plane = (uint64_t)(L->r3 ? 3 : 1) << L->logn;       /* points per plane */
+    L->cnt = L->step = 0; L->off_bmap = 0;
+    if (allow_par) {                                             /* (the library's own workspace) */
+        const size_t alen = std::max(na, nb), blen = std::min(na, nb);
+        const Pieces q = choose_pieces(L->np, alen, blen, L->logn, L->r3);
+        if (q.cnt) {
+            const uint64_t plane = q.cnt * q.n;
+            const int par = L->np > 1 && plane <= g_par_points;
+            const size_t off_desc = align_up((size_t)(L->np * plane + (par ? L->np : 1) * q.n) * 8, 256);
+            const size_t off_bmap = off_desc + align_up((q.cnt + 1) * sizeof(LoadDesc), 256);
+            const size_t off_crt = off_bmap + align_up((q.r3 ? 3 : 1) * q.cnt * 4, 256);
+            const size_t bytes = off_crt + nttm_crt_scratch_words(nttm_crt_blocks(L->nc)) * 4 + 256;
+            if (!g.cfg.workspace_bytes || bytes <= g.cfg.workspace_bytes) {
+                L->logn = q.logn; L->r3 = q.r3; L->n = q.n; L->plane = plane; L->cnt = q.cnt; L->step = q.step; L->par = par;
+                L->off_desc = off_desc; L->off_bmap = off_bmap; L->off_crt = off_crt; L->bytes = bytes;
+                return 0;
+            }
+        }
+    }
     /* np planes of A and one of B: B's transform of each prime is made just before A's of that prime; primes in one
      * launch take a B plane each */
     const size_t crt_words = nttm_crt_scratch_words(std::max(nttm_crt_blocks(L->nc), prod_crt_blocks(L->logn, L->r3, L->n, L->nc)));
@@ -850,9 +931,9 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws));
     uint32_t *ctl = (uint32_t *)((char *)g.hpin + 128 * slot + 96);
     CrtDesc hd; memset(&hd, 0, sizeof hd);
-    hd.plane = L.n; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
+    hd.plane = L.plane; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
     hd.trunc = nc < nc_full;
-    if (small_len(L.logn, L.r3)) {
+    if (!L.cnt && small_len(L.logn, L.r3)) {
         const LoadDesc ld{a, na, b, nb};
         RCK(run_small(L.np, L.logn, nullptr, nullptr, &ld, &hd, 1, nullptr, ctl, s, 8.0 * (double)(na + nb + nc + hd.nx),
                       sync ? g.stamps : nullptr));
@@ -867,16 +948,28 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
         RCK(ws_need(L.bytes));
         ws = g.ws;
     }
-    double *A = (double *)ws, *Bp = A + (size_t)L.np * L.n;
+    double *A = (double *)ws, *Bp = A + (size_t)L.np * L.plane;
     uint32_t *crt_scr = (uint32_t *)(ws + L.off_crt);
     const bool events = sync && !L.par;
     uint64_t *stamps = sync && L.par ? g.stamps : nullptr;
     if (stamps) stamps[0] = ~(uint64_t)0;                        /* (a transform of one pass has no forward launch) */
 
     if (events) HIPCK(hipEventRecord(g.ev[0], s));
-    const int im = inv_crt_bits(L.logn, L.r3, 1);
-    RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, L.par ? L.n : 0, a, na, b, nb, nullptr, s, events ? g.pev : nullptr, 0,
-                           nullptr, nullptr, stamps, im != 0));
+    const int im = L.cnt ? 0 : inv_crt_bits(L.logn, L.r3, 1);
+    if (L.cnt) {
+        const bool sw = na < nb;
+        const uint64_t alen = sw ? nb : na, blen = sw ? na : nb;
+        LoadDesc *ld = (LoadDesc *)(ws + L.off_desc);
+        uint32_t *bmap = (uint32_t *)(ws + L.off_bmap);
+        hipLaunchKernelGGL(k_pieces, dim3((unsigned)((L.cnt + 255) / 256)), dim3(256), 0, s, ld, bmap, sw ? b : a, alen, L.step,
+                           (uint32_t)L.cnt, sw ? a : b, blen, L.r3);
+        RCK(nttm_hip_check(hipGetLastError(), "k_pieces launch"));
+        RCK(product_transforms(L.np, L.logn, L.r3, L.cnt, A, Bp, L.par ? L.n : 0, nullptr, 0, nullptr, 0, ld, s,
+                               events ? g.pev : nullptr, 1, ld + L.cnt, bmap, stamps));
+        hd.step = L.step; hd.tn = L.n; hd.over = blen - 1; hd.alen = alen;
+    } else
+        RCK(product_transforms(L.np, L.logn, L.r3, 1, A, Bp, L.par ? L.n : 0, a, na, b, nb, nullptr, s, events ? g.pev : nullptr, 0,
+                               nullptr, nullptr, stamps, im != 0));
     if (events) HIPCK(hipEventRecord(g.ev[2], s));
     hd.pl = A;
     const double crt_bytes = 8.0 * L.np * (double)L.ncoef + 8.0 * (double)nc + 8.0 * (double)(x ? (nx < nc ? nx : nc) : 0);

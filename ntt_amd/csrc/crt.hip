@@ -46,8 +46,10 @@ struct CrtArgs {
     CrtConst cc;
 };
 
-/* U: the residues are canonical uint64 in a.res[prime] (the primitive's planes) instead of the product's FP64 planes */
-template <int NP, int PER, bool U = false>
+/* U: the residues are canonical uint64 in a.res[prime] (the primitive's planes) instead of the product's FP64 planes.
+ * ST: the product of a descriptor with a step: coefficient kk = i step + pos (pos < step, at least the block's limbs, so that
+ * a block meets at most two pieces) is piece i's residue at pos plus, below `over`, piece i - 1's at step + pos. */
+template <int NP, int PER, bool U = false, bool ST = false>
 __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
 {
     constexpr int CH = CRT_T * PER;                                  /* limbs per block */
@@ -84,13 +86,36 @@ __global__ __launch_bounds__(CRT_T) void k_crt(CrtArgs a)
             return pl[j * dsc.plane + kk];
         };
         double rr[PER + 1][NP];
+        if (ST) {
+            /* the piece of the block's first limb; each coefficient's own by one comparison (the halo's: the piece before) */
+            const uint64_t i0 = k0 / dsc.step, s0 = i0 * dsc.step;
+            double pv[PER + 1][NP];
 #pragma unroll
-        for (int i = 0; i < PER; i++) {
-            const uint64_t kk = k0 + i * CRT_T + tid;
+            for (int i = 0; i <= PER; i++) {
+                const uint64_t kk = i < PER ? k0 + i * CRT_T + tid : k0 + tid - CRT_HALO;
+                const bool live = (i < PER || halo) && kk < dsc.ncoef;
+                uint64_t pc = i0, pos = kk - s0;
+                if (i == PER && pos > kk) { pc--; pos += dsc.step; }         /* (kk below s0: the difference wrapped) */
+                if (i < PER && pos >= dsc.step) { pc++; pos -= dsc.step; }
+                const uint64_t at = pc * dsc.tn + pos;
+                const bool own = live && pc * dsc.step < dsc.alen, prev = live && pc && pos < dsc.over;
 #pragma unroll
-            for (int j = 0; j < NP; j++) rr[i][j] = kk < dsc.ncoef ? residue(j, kk) : 0.0;
-        }
-        {
+                for (int j = 0; j < NP; j++) {
+                    rr[i][j] = own ? residue(j, at) : 0.0;
+                    pv[i][j] = prev ? residue(j, at - dsc.tn + dsc.step) : 0.0;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i <= PER; i++)
+#pragma unroll
+                for (int j = 0; j < NP; j++) rr[i][j] = reduce(rr[i][j] + pv[i][j], a.cc.pk[j].p, a.cc.pk[j].pinv);
+        } else {
+#pragma unroll
+            for (int i = 0; i < PER; i++) {
+                const uint64_t kk = k0 + i * CRT_T + tid;
+#pragma unroll
+                for (int j = 0; j < NP; j++) rr[i][j] = kk < dsc.ncoef ? residue(j, kk) : 0.0;
+            }
             const uint64_t kk = k0 + tid - CRT_HALO;
 #pragma unroll
             for (int j = 0; j < NP; j++) rr[PER][j] = halo && kk < dsc.ncoef ? residue(j, kk) : 0.0;
@@ -512,11 +537,16 @@ int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t 
     a.desc = desc_dev; a.nprod = nprod; a.block0 = (uint32_t)blk0; a.stamp = stamp; a.ctl = ctl;
     a.status = scratch + CRT_CTL_WORDS; a.cc = cc;
     for (int j = 0; j < NTTM_MAX_PRIMES; j++) a.res[j] = res && j < np ? res[j] : nullptr;
+    if (one && one->step && (per == 1 || res || one->step < CRT_T * CRT_WIDE || one->over > one->step || !one->tn))
+        return nttm_fail(NTTM_EINVAL, "crt: pieces of %llu limbs", (unsigned long long)one->step);
     if (res && per == 1) return nttm_fail(NTTM_EINVAL, "crt: residue planes take the wide blocks");
     prof_begin("k_crt", alg_bytes, s);
     if (res) {
         if (np == 3) hipLaunchKernelGGL((k_crt<3, CRT_WIDE, true>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
         else hipLaunchKernelGGL((k_crt<4, CRT_WIDE, true>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
+    } else if (one && one->step) {
+        if (np == 3) hipLaunchKernelGGL((k_crt<3, CRT_WIDE, false, true>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
+        else hipLaunchKernelGGL((k_crt<4, CRT_WIDE, false, true>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
     } else if (per == 1) {
         if (np == 3) hipLaunchKernelGGL((k_crt<3, 1>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);
         else hipLaunchKernelGGL((k_crt<4, 1>), dim3((unsigned)nblk), dim3(CRT_T), 0, s, a);

@@ -39,6 +39,9 @@ struct CrtDesc {
     uint64_t *c; uint64_t nc;
     uint64_t first_block;                /* the product's first block in the launch */
     uint64_t trunc;                      /* nonzero: c is the value mod B^nc (nothing above it is checked) */
+    /* a product formed in pieces of its longer operand (step limbs each; 0: whole): piece i's coefficients at plane offset
+     * i tn, tn points each; the first `over` of piece i + 1 add to piece i's from `step` on */
+    uint64_t step, tn, over, alen;       /* alen: the longer operand's limbs */
 };
 
 /* one pass over bits [lo, lo + m) of every transform of 2^logn points in a batch; a tile holds W low columns x 2^m
@@ -89,6 +92,7 @@ struct PassJob {
     const LoadDesc *ldesc; int which;
     int do_in_scale, dfr_do_scale;
     uint64_t batch;                 /* transforms in this job's plane */
+    uint32_t block0, blocks;        /* a streamed pass: the job's blocks in the launch */
     double p, pinv;
     TwTables tw;
     double2 in_scale;               /* of the limbs (do_in_scale) or of the deferred twiddles (dfr_do_scale) */

@@ -6,6 +6,7 @@
  * k_load replaces k_scatter4 / k_lload / ntt_load (E/rns_mul.c:430-443,1051-1055; E/ntt.c:376-380,624-628).
  */
 #include <string.h>
+#include <algorithm>
 #include "internal.h"
 #include "plan.h"
 #include "rounds.h"
@@ -96,10 +97,10 @@ __device__ __forceinline__ void bound_chain(double *v, const PassPos &pp, int lo
  * argument segment inside a persistent kernel's loop */
 template <typename T> __device__ __forceinline__ void hold(T &v) { asm volatile("" : "+s"(v)); }
 
-/* the fields of the block row's job (blockIdx.y) into the pass's arguments */
-__device__ __forceinline__ void apply_job(PassArgs &a, const JobSet &js)
+/* the fields of a job into the pass's arguments */
+__device__ __forceinline__ void apply_job(PassArgs &a, const JobSet &js, uint32_t job)
 {
-    const PassJob &j = js.j[blockIdx.y];
+    const PassJob &j = js.j[job];
     a.x = j.x; a.limbs = j.limbs; a.nlimbs = j.nlimbs; a.ldesc = j.ldesc; a.which = j.which;
     a.do_in_scale = j.do_in_scale; a.in_scale = j.in_scale; a.dfr_do_scale = j.dfr_do_scale; a.dfr_scale = j.in_scale;
     a.batch = j.batch; a.pk.p = j.p; a.pk.pinv = j.pinv; a.tw = j.tw;
@@ -122,7 +123,7 @@ __device__ __forceinline__ double res_store(double x, int u64, double p, double 
 template <int MODE, int PTS, int GM = -1, int GW = -1, int GH = -1, bool U = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k_pass(PassArgs a, JobSet js)
 {
-    apply_job(a, js);
+    apply_job(a, js, blockIdx.y);
     stamp_clock(a.stamp);
     if (blockIdx.x >= (a.batch << a.logn) >> (a.m + a.logw + a.logh)) return;   /* a job of fewer transforms */
     const int gm = GM >= 0 ? GM : a.m, gw = GW >= 0 ? GW : a.logw, gh = GH >= 0 ? GH : a.logh;
@@ -244,7 +245,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
 /* ---- the streaming strided pass ---------------------------------------------------------------------------------------
  * Strided passes (lo >= GW) of the fixed tile shapes 2^GM rows x 2^GW columns, GM + GW = 13 with GM = 5 .. 9 (H = 1,
  * 2^13 points, 16 per thread; 9-bit rows are 128-byte runs in three rounds of 3 bits, the others two rounds): one
- * block per CU walks the tiles blockIdx.x, + gridDim.x, ...  The next tile is fetched straight into the other of two
+ * block per CU walks its job's tiles.  The next tile is fetched straight into the other of two
  * LDS buffers (global_load_lds, 16 bytes per lane, the tile in natural row-major order) while the current one is
  * transformed, so HBM streams during the butterflies.  Vector-memory operations of a wave complete in issue order, so
  * the loop issues no global load it must wait on besides the fetch:
@@ -275,8 +276,11 @@ __device__ __forceinline__ void lds_barrier()
 template <int MODE, int GM, int GW, bool U = false>
 __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
 {
-    apply_job(a, js);
+    uint32_t job = 0;
+    while ((int)job + 1 < js.n && blockIdx.x >= js.j[job + 1].block0) job++;
+    apply_job(a, js, job);
     stamp_clock(a.stamp);
+    const uint32_t blk = blockIdx.x - js.j[job].block0, nblk = js.j[job].blocks;
     hold(a.x); hold(a.pk.p); hold(a.pk.pinv);
     const uint32_t ntiles = (uint32_t)((a.batch << a.logn) >> (GM + GW));
     constexpr bool INV = MODE == PM_INV, LIMB = MODE == PM_FWD_LIMB;
@@ -346,16 +350,16 @@ __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
 
     if (t < (1 << GM)) stw[t] = a.tw.stage[t];
     for (int i = t; i < NBQ; i += STREAM_T) bqs[i] = a.tw.bq[i];
-    uint32_t tile = blockIdx.x;
+    uint32_t tile = blk;
     if (tile < ntiles) fetch(tile, buf0);
     __builtin_amdgcn_s_waitcnt(0);                                     /* vmcnt(0) expcnt(0) lgkmcnt(0) */
-    for (uint32_t it = 0; tile < ntiles; it++, tile += gridDim.x) {
+    for (uint32_t it = 0; tile < ntiles; it++, tile += nblk) {
         double *cur = (it & 1) ? buf1 : buf0, *nxt = (it & 1) ? buf0 : buf1;
         /* this tile's fetch has landed (only the previous tile's 16 stores may be outstanding); every thread is past
          * the previous tile's LDS reads of nxt */
         __builtin_amdgcn_s_waitcnt(0x4F70);                             /* vmcnt(16) */
         __syncthreads();
-        if (tile + gridDim.x < ntiles) fetch(tile + gridDim.x, nxt);
+        if (tile + nblk < ntiles) fetch(tile + nblk, nxt);
         uint32_t colbase;
         const uint64_t gbase = tile_base(tile, &colbase);
         const GPlane xt = (GPlane)(a.x + gbase);
@@ -808,14 +812,14 @@ static JobSet job_of(const PassArgs &a)
  * say whether the jobs read limbs */
 int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s, const JobSet *jobs)
 {
-    const JobSet js = jobs ? *jobs : job_of(a);
+    JobSet js = jobs ? *jobs : job_of(a);
     if (js.n < 1 || js.n > NTTM_MAX_JOBS) return nttm_fail(NTTM_EINVAL, "internal: %d jobs", js.n);
-    uint64_t tiles = 0;                                            /* of the largest job */
+    uint64_t tiles = 0, all = 0;                                            /* of the largest job */
     double pts = 0, lbytes = 0;
     for (int k = 0; k < js.n; k++) {
         if (!pass_geom_ok(g, a.logn, js.j[k].batch)) return nttm_fail(NTTM_EINVAL, "internal: bad pass geometry");
         const uint64_t t = plan_tiles(g, a.logn, js.j[k].batch);
-        tiles = t > tiles ? t : tiles;
+        tiles = t > tiles ? t : tiles; all += t;
         pts += (double)(js.j[k].batch << a.logn);
         lbytes += 8.0 * (double)(js.j[k].ldesc ? 0 : js.j[k].nlimbs);
     }
@@ -866,10 +870,17 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
     if ((b.dfr_out && (!stream || mode != PM_FWD_LIMB)) || (b.dfr_in && (!stream || mode != PM_FWD || g.m < 4)))
         return nttm_fail(NTTM_EINVAL, "internal: deferred boundary twiddles on a pass that does not stream");
     if (stream) {
-        /* one block per CU in all (a block holds nearly all of its CU's LDS), shared between the jobs */
-        const unsigned per = (unsigned)(g_ncu > js.n ? g_ncu / js.n : 1);
-        const unsigned nb = (unsigned)(tiles < (uint64_t)per ? tiles : (uint64_t)per);
-        const dim3 sgrid(nb, (unsigned)js.n);
+        /* one block per CU in all (a block holds nearly all of its CU's LDS), shared between the jobs by their tiles: in
+         * equal shares the pieces of an uneven product (768 tiles a job) kept their CUs three times as long as their one B
+         * operand (256) did its own, 163 us for the limb pass of 5000003 x 300007 limbs against 113.  The jobs' blocks are
+         * numbered through, so that no XCD is given more of them than it has CUs (as block rows of unequal jobs: 192 us) */
+        uint32_t nb = 0;
+        for (int k = 0; k < js.n; k++) {
+            const uint64_t t = plan_tiles(g, a.logn, js.j[k].batch), share = std::max<uint64_t>(1, (uint64_t)g_ncu * t / all);
+            js.j[k].block0 = nb; js.j[k].blocks = (uint32_t)std::min(t, share);
+            nb += js.j[k].blocks;
+        }
+        const dim3 sgrid(nb);
 #define NTTM_STREAM_LAUNCH(M, W) \
         if (u && mode == PM_FWD) hipLaunchKernelGGL((k_pass_stream<PM_FWD, M, W, true>), sgrid, dim3(STREAM_T), 0, s, b, js); \
         else if (u) hipLaunchKernelGGL((k_pass_stream<PM_INV, M, W, true>), sgrid, dim3(STREAM_T), 0, s, b, js); \
