@@ -802,14 +802,15 @@ static bool fits_one(size_t na, size_t nb, size_t nc)
  * than its error: 30011 x 2100 56 / 57, 5000003 x 1500000 681 / 700. */
 struct Pieces { int logn, r3; uint64_t n, cnt, step; };      /* cnt = 0: the product whole */
 /* a product's time by its passes, us: 4 per launch and, per point and prime, 2.4 ps for the limb pass and 1.6 more where it
- * reads limbs, 3.6 a forward and 3.3 an inverse strided pass, 3.0 (and the limbs) and 2.6 the radix-3 layers, 7.6 the double-fused pass; the
- * CRT 2.5 per coefficient, 3.3 from pieces (kernel times of products of 2^20 to 2^28 points) */
+ * reads limbs, 3.6 a forward and 3.3 an inverse strided pass (9-bit rows 1.0 and 0.8 more), 3.8 (and the limbs) and 3.0 the radix-3 layers, 7.6
+ * the double-fused pass; the CRT 2.5 per coefficient, 3.3 from pieces (kernel times of products of 2^20 to 2^28 points) */
 static double passes_us(int np, int logn, int r3, uint64_t cnt, uint64_t alen, uint64_t blen)
 {
     Plan pl; product_plan(&pl, logn, 1, product_tile_log(logn));
     const int st = pl.npass - 1;
     const double n = (double)(r3 ? 3 : 1) * ldexp(1.0, logn), ca = (double)cnt * n;
-    const double fwd = r3 ? 3.0 + 3.6 * st : st ? 2.4 + 3.6 * (st - 1) : 0.0, inv = 3.3 * st + (r3 ? 2.6 : 0.0);
+    double fwd = r3 ? 3.8 + 3.6 * st : st ? 2.4 + 3.6 * (st - 1) : 0.0, inv = 3.3 * st + (r3 ? 3.0 : 0.0);
+    for (int j = 0; j < st; j++) if (pl.p[j].m == 9) { fwd += 1.0; inv += 0.8; }
     return 4.0 * (2 * st + (r3 ? 2 : 0) + 3) +
            1e-6 * np * (ca * (fwd + 7.6 + inv) + n * fwd + 1.6 * (double)(alen + blen) + (cnt > 1 ? 3.3 : 2.5) * (double)(alen + blen));
 }
@@ -818,9 +819,9 @@ static Pieces choose_pieces(int np, size_t alen, size_t blen, int logn, int r3)
     Pieces best{0, 0, 0, 0, 0};
     const uint64_t whole = (uint64_t)(r3 ? 3 : 1) << logn;
     if (alen < 2 * blen || g_pieces_points == 0) return best;    /* (two pieces of at least blen limbs) */
-    /* in pieces where the model saves 10 us and 15 %: its error is up to 8 % either way, the descriptors take 4 us */
+    /* in pieces where the model saves 8 us and a tenth: its error is up to 8 % either way, the descriptors take 4 us */
     double most = passes_us(np, logn, r3, 1, alen, blen);
-    most = std::min(0.85 * most, most - 10.0);
+    most = std::min(0.9 * most, most - 8.0);
     for (int l = 12; l <= 26; l++)
         for (int t = l == 12; t < 2; t++) {                      /* 2^l points from 2^13, 3 2^l from 3 2^12 */
             const uint64_t n = (uint64_t)(t ? 3 : 1) << l;
