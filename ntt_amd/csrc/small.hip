@@ -6,8 +6,8 @@
  * HBM and no other launch follows.  (In separate launches a product of this size took three: the double-fused pass,
  * the CRT with its planes through HBM, the carry scan and its fix.)
  *
- * A block holds a tile of T = max(n, 1024) points per prime, H = T / n products of n points, 16 points per thread: T / 16
- * threads per prime, so a wave works for one prime (T = 1024: exactly one, whose rounds then need no barrier).
+ * A block holds a tile of T points per prime, H = T / n products of n points, PTS points per thread: T / PTS threads per
+ * prime, at least 64, so a wave works for one prime (64: exactly one, whose rounds then need no barrier).
  *   - transforms: the rounds of k_fused2 on each prime's tile; B's transform stays in registers; the inverse ends in LDS in
  *     natural order;
  *   - digits: each coefficient's residues are replaced in place by its base-10^18 digits (crt_digits);
@@ -47,16 +47,20 @@ template <bool WAVE> __device__ __forceinline__ void prime_barrier()
     } else __syncthreads();
 }
 
-template <int LOGN, int NP>
-__global__ __launch_bounds__(NP << ((LOGN > 10 ? LOGN : 10) - 4)) void k_small(SmallArgs a)
+template <int LOGN, int NP, int TL = (LOGN > 10 ? LOGN : 10), int PTS = 16>
+__global__ __launch_bounds__((NP << TL) / PTS) void k_small(SmallArgs a)
 {
-    constexpr int TL = LOGN > 10 ? LOGN : 10, T = 1 << TL, N = 1 << LOGN, H = T / N, PTS = 16;
+    constexpr int T = 1 << TL, N = 1 << LOGN, H = T / N;
     constexpr int NT = T / PTS, NTH = NP * NT, NW = NTH / 64;        /* threads per prime and block, waves */
-    constexpr int SW = LOGN < 8 ? LOGN : 8;                          /* stages whose twiddles are kept in LDS */
+    constexpr int SW = LOGN < 8 ? LOGN : LOGN == 11 && PTS == 8 ? 9 : 8;   /* stages whose twiddles are kept in LDS */
     constexpr int WPP = N / 64 + 1, NWORD = H * WPP, IT = (NWORD + NW - 1) / NW;
     constexpr bool WAVE = NT == 64;
-    constexpr int NR = (LOGN + 3) / 4;
-    static_assert(NWORD <= 65, "the word chain is one 64-bit addition and its carry out");
+    constexpr int MAXR = PTS == 16 ? 4 : PTS == 8 ? 3 : 2, NR = (LOGN + MAXR - 1) / MAXR;   /* rounds, of at most MAXR bits */
+    constexpr int CH = NWORD <= 65 ? 1 : H;                          /* word chains: all products in one, or one each */
+    static_assert(NWORD <= 65 || WPP <= 65, "a word chain is one 64-bit addition and its carry out");
+    static_assert(PTS == 16 || PTS == 8 || PTS == 4, "rounds of 4, 3 or 2 bits");
+    static_assert(LOGN <= SW || LOGN - LOGN / NR <= SW, "only the top round's stages lie above the LDS table");
+    static_assert(NT % 64 == 0, "a wave works for one prime");
     typedef __attribute__((address_space(1))) uint64_t *GOut;
     struct Prod { const uint64_t *a, *b, *x; uint64_t *c; uint32_t na, nb, nx, nc, ncoef, trunc; };
     __shared__ double pl[NP][LDS_WORDS(T)];
@@ -99,7 +103,7 @@ __global__ __launch_bounds__(NP << ((LOGN > 10 ? LOGN : 10) - 4)) void k_small(S
         const GTab gf(a.stage[pi]), gi(a.istage[pi]);
         PassPos pp; pp.m = LOGN; pp.logw = 0; pp.lo = 0; pp.nthr = NT; pp.t = t;
         int s_lo, logR;
-        round_split(LOGN, 0, &s_lo, &logR, false, 4);
+        round_split(LOGN, 0, &s_lo, &logR, false, MAXR);
         uint64_t raw[2][PTS];
         uint32_t in[2] = {0, 0};                                     /* bit sl: the slot lies inside the operand */
 #pragma unroll
@@ -124,7 +128,7 @@ __global__ __launch_bounds__(NP << ((LOGN > 10 ? LOGN : 10) - 4)) void k_small(S
             }
 #pragma unroll
             for (int i = 0; i < NR; i++) {                           /* top bits first; the last round stays in registers */
-                round_split(LOGN, i, &s_lo, &logR, false, 4);
+                round_split(LOGN, i, &s_lo, &logR, false, MAXR);
                 if (i > 0) {
                     prime_barrier<WAVE>();
                     ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
@@ -146,7 +150,7 @@ __global__ __launch_bounds__(NP << ((LOGN > 10 ? LOGN : 10) - 4)) void k_small(S
         for (int sl = 0; sl < PTS; sl++) v[sl] = mul_barrett(v[sl], bv[sl], p, pinv);
 #pragma unroll
         for (int i = 0; i < NR; i++) {                               /* bit 0 first; round 0 has the layout in v */
-            round_split(LOGN, i, &s_lo, &logR, true, 4);
+            round_split(LOGN, i, &s_lo, &logR, true, MAXR);
             if (i > 0) {
                 prime_barrier<WAVE>();
                 ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
@@ -226,15 +230,17 @@ __global__ __launch_bounds__(NP << ((LOGN > 10 ? LOGN : 10) - 4)) void k_small(S
         }
     }
     __syncthreads();
-    /* the carry into every word of the block: bit w of CI (word 64: cout) */
-    uint64_t CI; uint32_t cout64;
-    {
+    /* the carry into every word of the block: bit w of its chain's CI (word 64: cout) */
+    uint64_t CI[CH]; uint32_t cout64[CH];
+#pragma unroll
+    for (int h = 0; h < CH; h++) {
+        constexpr int CW = CH == 1 ? NWORD : WPP;                    /* words of a chain */
         uint32_t f0 = 0, f1 = 0;
-        if (lane < NWORD && lane % WPP != WPP - 1) {
-            f0 = add_cout(sgx[lane], sgy[lane], 0); f1 = add_cout(sgx[lane], sgy[lane], 1);
+        if (lane < CW && lane % WPP != WPP - 1) {
+            f0 = add_cout(sgx[h * CW + lane], sgy[h * CW + lane], 0); f1 = add_cout(sgx[h * CW + lane], sgy[h * CW + lane], 1);
         }
         const uint64_t G = __ballot(f0 != 0), GP = __ballot(f1 != 0), S = G + GP;
-        CI = S ^ G ^ GP; cout64 = S < G;
+        CI[h] = S ^ G ^ GP; cout64[h] = S < G;
     }
 #pragma unroll
     for (int i = 0; i < IT; i++) {
@@ -242,7 +248,11 @@ __global__ __launch_bounds__(NP << ((LOGN > 10 ? LOGN : 10) - 4)) void k_small(S
         if (w < NWORD) {
             const int h = w / WPP, k = (w - h * WPP) * 64 + lane;
             const int nc = (int)sp[h].nc;
-            const uint32_t c = w < 64 ? (uint32_t)(CI >> w) & 1u : cout64;
+            uint64_t ci = CI[0]; uint32_t co = cout64[0];
+#pragma unroll
+            for (int j = 1; j < CH; j++) if (h == j) { ci = CI[j]; co = cout64[j]; }
+            const int cw = CH == 1 ? w : w - h * WPP;
+            const uint32_t c = cw < 64 ? (uint32_t)(ci >> cw) & 1u : co;
             const uint64_t S = GX[i] + GY[i] + c, CB = S ^ GX[i] ^ GY[i];      /* bit b: the carry into bit b */
             const uint32_t oin = (uint32_t)(CB >> lane) & 1u;
             const uint32_t oout = lane == 63 ? add_cout(GX[i], GY[i], c) : (uint32_t)(CB >> (lane + 1)) & 1u;
@@ -288,20 +298,27 @@ int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, cons
     if (ld1) a.ld1 = *ld1;
     if (cd1) a.cd1 = *cd1;
     for (int i = 0; i < np; i++) { a.stage[i] = fwd[i].stage; a.istage[i] = inv[i].stage; a.ninv[i] = ninv[i]; }
-    const int tl = logn > 10 ? logn : 10, h = 1 << (tl - logn);
+    /* Few products: a block each and 4 or 8 points a thread, so that more waves share a product's chain of rounds; many:
+     * 16 points, and at least a wave per prime (12 waves a block at 2^11 points, whose 6 of one product leave room for no
+     * second block: waves of 144 registers start on the same SIMDs).  The line is 2^19 points, one block a CU at 2^11.
+     * A plan's replay, us, many / few: 2^7 points 1 product 22 / 18, 4096 32 / 27, 8192 42 / 43; 2^9 256 26 / 22, 2048 44 / 44;
+     * 2^10 1 24 / 21, 512 33 / 31, 1024 45 / 62; 2^11 1 38 / 26, 256 43 / 29, 512 46 / 52, 8192 572 / 668 (6 waves of
+     * 16 points: 789).  One 64 x 64 limb call 35 -> 27 us, 1000 x 1000 46 -> 40. */
+    const bool few = cnt <= ((uint64_t)1 << 19) >> logn;
+    const int tl = few ? (logn < 8 ? 8 : logn) : logn == 11 ? 12 : logn > 10 ? logn : 10, h = 1 << (tl - logn);
+    const int pts = !few ? 16 : tl <= 8 ? 4 : tl <= 11 ? 8 : 16;
     const uint64_t blocks = (cnt + h - 1) / h;
     if (blocks > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "internal: too many small products");
-    const dim3 grid((unsigned)blocks), blk((unsigned)(np << (tl - 4)));
+    const dim3 grid((unsigned)blocks), blk((unsigned)((np << tl) / pts));
     prof_begin("k_small", alg_bytes, s);
-#define SMALL_LAUNCH(L) \
-    case L: \
-        if (np == 3) hipLaunchKernelGGL((k_small<L, 3>), grid, blk, 0, s, a); \
-        else hipLaunchKernelGGL((k_small<L, 4>), grid, blk, 0, s, a); \
-        break;
-    switch (logn) {
-    SMALL_LAUNCH(7) SMALL_LAUNCH(8) SMALL_LAUNCH(9) SMALL_LAUNCH(10) SMALL_LAUNCH(11)
-    default: SMALL_LAUNCH(12)
+#define SMALL_LAUNCH(L, TL, P) \
+    if (logn == L && tl == TL && pts == P) { \
+        if (np == 3) hipLaunchKernelGGL((k_small<L, 3, TL, P>), grid, blk, 0, s, a); \
+        else hipLaunchKernelGGL((k_small<L, 4, TL, P>), grid, blk, 0, s, a); \
     }
+    SMALL_LAUNCH(7, 8, 4) SMALL_LAUNCH(8, 8, 4) SMALL_LAUNCH(9, 9, 8) SMALL_LAUNCH(10, 10, 8) SMALL_LAUNCH(11, 11, 8)
+    SMALL_LAUNCH(12, 12, 16)
+    SMALL_LAUNCH(10, 10, 16) SMALL_LAUNCH(7, 10, 16) SMALL_LAUNCH(8, 10, 16) SMALL_LAUNCH(9, 10, 16) SMALL_LAUNCH(11, 12, 16)
 #undef SMALL_LAUNCH
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_small launch");

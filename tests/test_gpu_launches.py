@@ -237,3 +237,38 @@ def test_inverse_with_crt(schedule, n, nprimes):
         assert np.array_equal(host(got), w)
     for cut in sorted({1, 60, 4096, 4097, n // 2, n}):
         assert np.array_equal(host(lib.mul_cut(items[3][0], items[3][1], w=cut)), want[3][:cut])
+
+
+@pytest.mark.parametrize("logn", [7, 8, 9, 10, 11])
+@pytest.mark.parametrize("over", [-1, 0, 1])
+@pytest.mark.parametrize("np_", [3, 4])
+def test_small_products_few_and_many(schedule, logn, over, np_):
+    """batches of the largest count that takes a block per product (2^19 points), one less and one more, in ragged lengths"""
+    import torch
+    cnt = ((1 << 19) >> logn) + over
+    rng = np.random.default_rng(logn * 10 + over)
+    n = 1 << logn
+    say("few and many", logn, cnt, np_)
+    lib = schedule(nprimes=np_)
+    flat, _ = O.gen_limbs(cnt * (n + 1), logn)
+    df = dev(flat)
+    out = torch.full((cnt * (n + 1),), -1, dtype=torch.int64, device="cuda")
+    items, shape = [], []
+    for i in range(cnt):
+        total = int(rng.integers((n >> 1) + 2 if logn > 7 else 2, n + 2))       # na + nb - 1 coefficients of this length
+        na = int(rng.integers(1, total))
+        o = i * (n + 1)
+        items.append((df[o:o + na], df[o + na:o + total], None, out[o:o + total]))
+        shape.append((o, na, total))
+    prods = lib.make_prods(items)
+    lib.mul_batch(prods)
+    got = host(out)
+    for i in list(range(0, cnt, max(1, cnt // 300))) + [cnt - 1]:
+        o, na, total = shape[i]
+        want = O.mul_school(flat[o:o + na], flat[o + na:o + total])
+        assert np.array_equal(got[o:o + total], want), (i, na, total)
+        assert prods[i].ncn == int(np.nonzero(want)[0][-1]) + 1
+    rest = np.ones(len(got), dtype=bool)
+    for o, _, total in shape:
+        rest[o:o + total] = False
+    assert (got[rest] == np.uint64(2 ** 64 - 1)).all()
