@@ -22,7 +22,8 @@ void nttm_set_pts(int pts);
 int nttm_get_pts(void);
 void nttm_set_fixed_shapes(int on);
 void nttm_set_stream(int on, int ncu);
-#define NTTM_CRT_RUNS 0            /* the carry launch's blocks are k_inv_crt's runs */
+#define NTTM_CRT_RUNS 0            /* the carry launch's blocks are k_inv_crt's runs, */
+#define NTTM_CRT_SEGS (-1)         /* or k_segments' segments */
 #define NTTM_FUSED_LOG 12          /* tile of the fused forward + pointwise + inverse pass (k_fused2) */
 #define NTTM_TILE_LOG_DEFAULT 13   /* tile of the strided passes: 2^13 points (64 KiB of LDS), runs of 32 columns */
 #define NTTM_PRODUCT_LOGN_MIN 4    /* products use at least 2^4 points, so every fused tile has >= 16 */
@@ -55,6 +56,10 @@ int nttm_small_log(int logn);
 int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1,
                    uint64_t cnt, uint64_t *ncn, uint32_t *ctl, const TwTables *fwd, const TwTables *inv, const double2 *ninv,
                    const CrtConst &cc, hipStream_t s, double alg_bytes, uint64_t *stamps);
+uint64_t nttm_seg_len(uint64_t nb);
+int nttm_run_segments(int np, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1, uint64_t nprod,
+                      uint64_t groups, const TwTables *fwd, const TwTables *inv, const double2 *ninv,
+                      const CrtConst &cc, uint32_t *scratch, uint32_t *ctl, hipStream_t s, double alg_bytes, uint64_t *stamps);
 int nttm_run_norm(const void *desc_dev, uint64_t nprod, uint64_t *ncn_dev, hipStream_t s);
 int nttm_run_fill_x(const void *desc_dev, uint64_t nprod, hipStream_t s);
 int nttm_run_dft16_mfma(const uint64_t *x, double *y, int logn, uint64_t batch, const void *etab, const double *tlo,
@@ -800,8 +805,8 @@ static bool fits_one(size_t na, size_t nb, size_t nc)
  * 300000 x 300 limbs 87 / 70, 1000000 x 100000 176 / 147, 5000003 x 300007 568 / 374, 5000003 x 2000 545 / 305,
  * 20000000 x 1000000 2650 / 1950, 100000000 x 300 10500 / 5200; the rest of the plane lies where the model below sees less
  * than its error: 30011 x 2100 56 / 57, 5000003 x 1500000 681 / 700. */
-struct Pieces { int logn, r3; uint64_t n, cnt, step; };      /* cnt = 0: the product whole */
-/* a product's time by its passes, us: 4 per launch and, per point and prime, 2.4 ps for the limb pass and 1.6 more where it
+struct Pieces { int logn, r3; uint64_t n, cnt, step; double us; };   /* cnt = 0: the product whole; us: the time to beat */
+/* a product's time by its passes, us: 12 for the call, 7 per launch (its own and its first and last tiles') and, per point and prime, 2.4 ps for the limb pass and 1.6 more where it
  * reads limbs, 3.6 a forward and 3.3 an inverse strided pass (9-bit rows 1.0 and 0.8 more), 3.8 (and the limbs) and 3.0 the radix-3 layers, 7.6
  * the double-fused pass; the CRT 2.5 per coefficient, 3.3 from pieces (kernel times of products of 2^20 to 2^28 points) */
 static double passes_us(int np, int logn, int r3, uint64_t cnt, uint64_t alen, uint64_t blen)
@@ -811,17 +816,17 @@ static double passes_us(int np, int logn, int r3, uint64_t cnt, uint64_t alen, u
     const double n = (double)(r3 ? 3 : 1) * ldexp(1.0, logn), ca = (double)cnt * n;
     double fwd = r3 ? 3.8 + 3.6 * st : st ? 2.4 + 3.6 * (st - 1) : 0.0, inv = 3.3 * st + (r3 ? 3.0 : 0.0);
     for (int j = 0; j < st; j++) if (pl.p[j].m == 9) { fwd += 1.0; inv += 0.8; }
-    return 4.0 * (2 * st + (r3 ? 2 : 0) + 3) +
+    return 12.0 + 7.0 * (2 * st + (r3 ? 2 : 0) + 3) + (cnt > 1 ? 4.0 : 0.0) +
            1e-6 * np * (ca * (fwd + 7.6 + inv) + n * fwd + 1.6 * (double)(alen + blen) + (cnt > 1 ? 3.3 : 2.5) * (double)(alen + blen));
 }
 static Pieces choose_pieces(int np, size_t alen, size_t blen, int logn, int r3)
 {
-    Pieces best{0, 0, 0, 0, 0};
+    Pieces best{0, 0, 0, 0, 0, 0.0};
     const uint64_t whole = (uint64_t)(r3 ? 3 : 1) << logn;
-    if (alen < 2 * blen || g_pieces_points == 0) return best;    /* (two pieces of at least blen limbs) */
     /* in pieces where the model saves 8 us and a tenth: its error is up to 8 % either way, the descriptors take 4 us */
     double most = passes_us(np, logn, r3, 1, alen, blen);
-    most = std::min(0.9 * most, most - 8.0);
+    best.us = most = std::min(0.9 * most, most - 8.0);
+    if (alen < 2 * blen || g_pieces_points == 0) return best;    /* (two pieces of at least blen limbs) */
     for (int l = 12; l <= 26; l++)
         for (int t = l == 12; t < 2; t++) {                      /* 2^l points from 2^13, 3 2^l from 3 2^12 */
             const uint64_t n = (uint64_t)(t ? 3 : 1) << l;
@@ -831,9 +836,49 @@ static Pieces choose_pieces(int np, size_t alen, size_t blen, int logn, int r3)
             const uint64_t cnt = (alen + step - 1) / step;
             if (cnt < 2 || cnt > 0x100000) continue;
             const double us = passes_us(np, l, t, cnt, alen, blen);
-            if (g_pieces_points < 0 ? us < most : n == (uint64_t)g_pieces_points) { most = us; best = Pieces{l, t, n, cnt, step}; }
+            if (g_pieces_points < 0 ? us < most : n == (uint64_t)g_pieces_points) { most = us; best = Pieces{l, t, n, cnt, step, us}; }
         }
     return best;
+}
+/* whether products of this transform length run as one kernel each (small.hip): 2^k points up to 2^12 */
+static bool small_len(int logn, int r3) { return !r3 && !g_no_small && nttm_small_log(logn) != 0; }
+/* ---- products in segments of the result (k_segments): short operands of up to some 2000 limbs -------------------------------- */
+#define SEG_B_US 13.0              /* a workgroup (a CU has room for one): the short operand's transforms, ... */
+static double seg_us(uint64_t S) { return 21.0 + 10.0 * (double)S / 4096; }   /* ... and each segment of S limbs */
+/* the launch's time in workgroups of `per` segments, n workgroups in all */
+static double seg_launch_us(uint64_t n, uint32_t per, uint64_t S)
+{
+    const double r = (double)n / 256;
+    return (r <= 4 ? ceil(r) : r + 0.5) * (SEG_B_US + seg_us(S) * per);
+}
+static bool seg_forced(void) { return g_pieces_points == 1 << 12; }
+static bool seg_allowed(uint64_t S) { return S && !g_no_small && (g_pieces_points < 0 || seg_forced()); }
+/* one product: the segments of a workgroup that give it the least time, if that is below `most`; else 0 */
+static uint32_t choose_segments(size_t nc, size_t blen, double most)
+{
+    const uint64_t S = nttm_seg_len(blen);
+    if (!seg_allowed(S)) return 0;
+    const uint64_t segs = (nc + S - 1) / S;
+    if (segs > 0x7fffffffULL) return 0;
+    uint32_t best = 0;
+    for (uint32_t per = 1; per <= 8; per++) {
+        const double us = 17.0 + seg_launch_us((segs + per - 1) / per, per, S);
+        if (us < most || (seg_forced() && !best)) { most = us; best = per; }
+    }
+    return best;
+}
+/* a product of a batch, whose launches fill the device either way: segments against the passes and the CRT of its own length
+ * at 17 ps a point and prime from 2^16 points, 1.5 more for each bit below (measured 17.3 there, 19 at 2^15, 21 at 2^14) */
+static bool batch_segments(size_t na, size_t nb, int logn, int r3)
+{
+    const size_t alen = std::max(na, nb), blen = std::min(na, nb);
+    const uint64_t S = nttm_seg_len(blen);
+    if (!seg_allowed(S) || (uint64_t)na + nb > 0xffffffffULL) return false;
+    if (seg_forced()) return true;
+    if (small_len(logn, r3) || alen < 2 * blen) return false;
+    const double segs = ceil((double)(na + nb) / (double)S);
+    const double ps = 17.0 + 1.5 * std::max(0, 16 - logn - (r3 ? 1 : 0));
+    return (segs * seg_us(S) + SEG_B_US * ceil(segs / 6)) / 256 < 0.95 * ps * 3e-6 * (double)((uint64_t)(r3 ? 3 : 1) << logn);
 }
 /* the descriptors of the pieces and the map to their one B operand: written by a kernel, since nothing on the host would
  * live until a copy of them has run in a call that does not wait */
@@ -852,7 +897,7 @@ __global__ __launch_bounds__(256) void k_pieces(LoadDesc *ld, uint32_t *bmap, co
 
 /* the workspace of a one-transform product: the planes, its CRT descriptor (the pieces' descriptors) and the CRT's scratch
  * (bytes from ws).  n: points of the transforms, plane: of one prime's plane of A */
-struct CoreLayout { int np, logn, r3, par; uint64_t n, plane, ncoef, cnt, step; size_t nc, nc_full, off_desc, off_bmap, off_crt, bytes; };
+struct CoreLayout { int np, logn, r3, par; uint32_t seg_per; uint64_t n, plane, ncoef, cnt, step; size_t nc, nc_full, off_desc, off_bmap, off_crt, bytes; };
 /* allow_par: one launch per pass for all primes, each with its own B plane (in the library's workspace) */
 static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout *L, bool allow_par = false)
 {
@@ -863,10 +908,16 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
     choose_len(ncoef_full, &L->logn, &L->r3);
     if (L->logn > NTTM_LOGN_MAX) return nttm_fail(NTTM_EBOUND, "transform length 2^%d above 2^%d", L->logn, NTTM_LOGN_MAX);
     L->n = L->plane = (uint64_t)(L->r3 ? 3 : 1) << L->logn;       /* points per plane */
-    L->cnt = L->step = 0; L->off_bmap = 0;
+    L->cnt = L->step = 0; L->off_bmap = 0; L->seg_per = 0;
     if (allow_par) {                                             /* (the library's own workspace) */
         const size_t alen = std::max(na, nb), blen = std::min(na, nb);
         const Pieces q = choose_pieces(L->np, alen, blen, L->logn, L->r3);
+        if (!small_len(L->logn, L->r3) && (L->seg_per = choose_segments(L->nc, blen, q.us))) {
+            L->step = nttm_seg_len(blen); L->cnt = (L->nc + L->step - 1) / L->step; L->par = 1;
+            L->off_desc = L->off_crt = 0;
+            L->bytes = nttm_crt_scratch_words(L->cnt) * 4 + 256;
+            return 0;
+        }
         if (q.cnt) {
             const uint64_t plane = q.cnt * q.n;
             const int par = L->np > 1 && plane <= g_par_points;
@@ -894,8 +945,6 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
     return 0;
 }
 
-/* whether products of this transform length run as one kernel each (small.hip): 2^k points up to 2^12 */
-static bool small_len(int logn, int r3) { return !r3 && !g_no_small && nttm_small_log(logn) != 0; }
 static int run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1,
                      uint64_t cnt, uint64_t *ncn, uint32_t *ctl, hipStream_t s, double bytes, uint64_t *stamps = nullptr)
 {
@@ -905,6 +954,13 @@ static int run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, co
     return nttm_run_small(np, sl, ld, cd, ld1, cd1, cnt, ncn, ctl, g.twf, g.twi, ninv, g.cc, s, bytes, stamps);
 }
 
+static int run_segments(int np, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1, uint64_t nprod,
+                        uint64_t groups, uint32_t *scratch, uint32_t *ctl, hipStream_t s, double bytes, uint64_t *stamps = nullptr)
+{
+    double2 ninv[NTTM_MAX_PRIMES];
+    for (int i = 0; i < np; i++) { const uint64_t p = NTTM_PRIMES[i]; ninv[i] = h_shoup(h_inv((uint64_t)1 << 12, p), p); }
+    return nttm_run_segments(np, ld, cd, ld1, cd1, nprod, groups, g.twf, g.twi, ninv, g.cc, scratch, ctl, s, bytes, stamps);
+}
 /* c = a b (+ x), device pointers.  wcut: write only the low wcut limbs of the result (the value mod B^wcut; no check of
  * what lies above).  ws: the workspace (null: the library's, grown to fit; else ws_cap bytes of the caller's).
  * sync = 1: returns after the stream has drained and the CRT's flags are checked; sync = 0: returns after the launches,
@@ -948,6 +1004,21 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     } else {
         RCK(ws_need(L.bytes));
         ws = g.ws;
+    }
+    if (L.seg_per) {
+        const bool sw = na < nb;
+        const LoadDesc ld{sw ? b : a, sw ? nb : na, sw ? a : b, sw ? na : nb};
+        hd.step = L.step; hd.over = L.seg_per;
+        uint64_t *st = sync ? g.stamps : nullptr;
+        if (st) st[0] = ~(uint64_t)0;
+        RCK(run_segments(L.np, nullptr, nullptr, &ld, &hd, 1, (L.cnt + L.seg_per - 1) / L.seg_per, (uint32_t *)ws, ctl, s,
+                         8.0 * (double)(na + nb + nc + hd.nx), st ? st + 1 : nullptr));
+        RCK(nttm_crt_launch_carry(nullptr, &hd, 1, L.cnt, (uint32_t *)ws, ctl, s, NTTM_CRT_SEGS, st ? st + 2 : nullptr));
+        if (st) st[3] = 0;
+        if (!sync) return 0;
+        HIPCK(hipStreamSynchronize(s));
+        g.last_stamped = 1;
+        return ctl[1] & 1 ? nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond the top limb (wrong residues)") : 0;
     }
     double *A = (double *)ws, *Bp = A + (size_t)L.np * L.plane;
     uint32_t *crt_scr = (uint32_t *)(ws + L.off_crt);
@@ -1244,6 +1315,8 @@ struct GroupBuild {
     int inv_m = 0;                                               /* the last inverse pass's bits where the CRT runs it */
     uint64_t n = 0, cnt = 0, cnt_b = 0, nblk = 0;
     bool share = false, merged = false, small = false;
+    uint32_t seg_per = 0;                                        /* r3 = 2: products in segments, this many a workgroup */
+    uint64_t seg_groups = 0;
     struct Chunk { uint64_t c0, cn, b0, cnb, blk0, nblk; double crt_bytes; };   /* products, distinct B operands, CRT blocks */
     std::vector<Chunk> chunk;
     std::vector<CrtDesc> cd;
@@ -1260,10 +1333,59 @@ static size_t chunk_planes_bytes(int np, uint64_t n, uint64_t cnt)
     const uint64_t cn = std::min(cnt, chunk_products(n));
     return (size_t)(chunk_merged(n, cn) ? 2 * np : np + 1) * cn * n * 8;
 }
+#define SEG_CLASS (2 * (NTTM_LOGN_MAX + 1) + 12)   /* the group class of products in segments of 2^12 points (r3 = 2) */
+static uint64_t seg_blocks(const nttm_prod &q)
+{
+    const uint64_t S = nttm_seg_len(std::min(q.na, q.nb)), nc = q.na + q.nb + (q.x ? 1 : 0);
+    return (nc + S - 1) / S;
+}
+static void group_offsets(GroupBuild &gb)
+{
+    gb.off_cd = 0;
+    gb.off_ld = align_up(gb.off_cd + gb.cnt * sizeof(CrtDesc), 256);
+    gb.off_ldb = align_up(gb.off_ld + gb.cnt * sizeof(LoadDesc), 256);
+    gb.off_bmap = align_up(gb.off_ldb + gb.ldb.size() * sizeof(LoadDesc), 256);
+    gb.off_ctl = align_up(gb.off_bmap + gb.bmap.size() * 4, 256);   /* a small group's flags, zeroed by the upload */
+    gb.off_ncn = gb.off_ctl + 256;
+    gb.off_crt = align_up(gb.off_ncn + gb.cnt * 8, 256);
+    gb.desc_bytes = align_up(gb.off_crt + nttm_crt_scratch_words(gb.nblk) * 4, 256);
+}
+static void group_build_segments(GroupBuild &gb, const nttm_prod *P, const std::vector<size_t> &G)
+{
+    const uint64_t cnt = G.size();
+    gb.n = (uint64_t)1 << gb.logn; gb.cnt = gb.cnt_b = cnt; gb.nblk = 0; gb.planes_bytes = 0; gb.inv_m = 0;
+    gb.crt_per = NTTM_CRT_SEGS; gb.small = gb.share = false; gb.merged = true;
+    gb.cd.assign(cnt, CrtDesc()); gb.ld.assign(cnt, LoadDesc()); gb.ldb.clear(); gb.bmap.clear();
+    gb.chunk.assign(1, GroupBuild::Chunk{0, cnt, 0, cnt, 0, 0, 0.0});
+    double least = 0;
+    for (uint32_t per = 1; per <= 8; per++) {                    /* (the longest segments' time: all alike in the comparison) */
+        uint64_t n = 0;
+        for (size_t i : G) n += (seg_blocks(P[i]) + per - 1) / per;
+        const double us = seg_launch_us(n, per, 4032);
+        if (per == 1 || us < least) { least = us; gb.seg_per = per; }
+    }
+    gb.seg_groups = 0;
+    for (uint64_t j = 0; j < cnt; j++) {
+        const nttm_prod &q = P[G[j]];
+        const bool sw = q.na < q.nb;
+        gb.ld[j] = LoadDesc{sw ? q.b : q.a, sw ? q.nb : q.na, sw ? q.a : q.b, sw ? q.na : q.nb};
+        CrtDesc &c = gb.cd[j];
+        c.ncoef = q.na + q.nb - 1; c.x = q.x; c.nx = q.x ? q.nx : 0; c.c = q.c; c.nc = q.na + q.nb + (q.x ? 1 : 0);
+        c.first_block = gb.nblk; c.step = nttm_seg_len(gb.ld[j].nb); c.tn = gb.seg_groups;
+        const uint64_t sb = seg_blocks(q);
+        const uint64_t groups = (sb + gb.seg_per - 1) / gb.seg_per;
+        c.over = (sb + groups - 1) / groups;                     /* (evenly) */
+        gb.nblk += sb; gb.seg_groups += groups;
+        gb.chunk[0].crt_bytes += 8.0 * (double)(q.na + q.nb + c.nc + c.nx);
+    }
+    gb.chunk[0].nblk = gb.nblk;
+    group_offsets(gb);
+}
 static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<size_t> &G, int np, int r3, int logn,
                         int tile, int pts)
 {
     gb.r3 = r3; gb.logn = logn; gb.tile = tile; gb.pts = pts;
+    if (r3 == 2) { group_build_segments(gb, P, G); return; }
     const uint64_t n = (uint64_t)(r3 ? 3 : 1) << logn, cnt = G.size();          /* points per product plane */
     gb.n = n; gb.cnt = cnt; gb.nblk = 0; gb.cnt_b = 0; gb.planes_bytes = 0;
     gb.inv_m = inv_crt_bits(logn, r3, cnt);
@@ -1321,14 +1443,7 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
         gb.bmap.resize(tb);
         for (uint64_t t = 0; t < tb; t++) gb.bmap[t] = r3 ? 3 * slot[t / 3] + (uint32_t)(t % 3) : slot[t];
     }
-    gb.off_cd = 0;
-    gb.off_ld = align_up(gb.off_cd + cnt * sizeof(CrtDesc), 256);
-    gb.off_ldb = align_up(gb.off_ld + cnt * sizeof(LoadDesc), 256);
-    gb.off_bmap = align_up(gb.off_ldb + gb.ldb.size() * sizeof(LoadDesc), 256);
-    gb.off_ctl = align_up(gb.off_bmap + gb.bmap.size() * 4, 256);   /* a small group's flags, zeroed by the upload */
-    gb.off_ncn = gb.off_ctl + 256;
-    gb.off_crt = align_up(gb.off_ncn + cnt * 8, 256);
-    gb.desc_bytes = align_up(gb.off_crt + nttm_crt_scratch_words(gb.nblk) * 4, 256);
+    group_offsets(gb);
 }
 /* points per thread of a batch group's passes: the configured value, else 8 up to 2^14 points and 16 above (what the
  * batch plans' autotuner chose for every such group of the 4096-leaf workload) */
@@ -1354,6 +1469,14 @@ static int group_launch(const GroupBuild &gb, int np, double *A, char *dbase, hi
     if (gb.small)
         return run_small(np, gb.logn, (const LoadDesc *)(dbase + gb.off_ld), (const CrtDesc *)(dbase + gb.off_cd), nullptr, nullptr,
                          gb.cnt, ncn, ncn ? nullptr : ctl, s, gb.chunk[0].crt_bytes);
+    if (gb.seg_per) {
+        uint32_t *scr = (uint32_t *)(dbase + gb.off_crt);
+        const CrtDesc *cd = (const CrtDesc *)(dbase + gb.off_cd);
+        RCK(run_segments(np, (const LoadDesc *)(dbase + gb.off_ld), cd, nullptr, nullptr, gb.cnt, gb.seg_groups, scr, ctl, s,
+                         gb.chunk[0].crt_bytes));
+        RCK(nttm_crt_launch_carry(cd, nullptr, gb.cnt, gb.nblk, scr, ctl, s, NTTM_CRT_SEGS));
+        return ncn ? nttm_run_norm(cd, gb.cnt, ncn, s) : 0;
+    }
     const int tile0 = g.cfg.tile_log, pts0 = nttm_get_pts();
     g.cfg.tile_log = gb.tile; nttm_set_pts(gb.pts);
     int rc = 0;
@@ -1415,7 +1538,7 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
     /* validate; zero-operand products are written directly */
     size_t mn_max = 0;
     /* groups by transform length: 2^logn at [logn], 3 2^logn at [NTTM_LOGN_MAX + 1 + logn] */
-    std::vector<std::vector<size_t>> groups(2 * (NTTM_LOGN_MAX + 1));
+    std::vector<std::vector<size_t>> groups(SEG_CLASS + 1);      /* and the products in segments at SEG_CLASS */
     for (size_t i = 0; i < N; i++) {
         const nttm_prod &q = P[i];
         if (q.x && q.nx > q.na + q.nb) return nttm_fail(NTTM_EINVAL, "product %zu: nx exceeds na + nb", i);
@@ -1425,7 +1548,7 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
         int logn, r3;
         choose_len(q.na + q.nb - 1, &logn, &r3);
         if (logn > NTTM_LOGN_MAX) return nttm_fail(NTTM_EBOUND, "product %zu: transform above 2^%d", i, NTTM_LOGN_MAX);
-        groups[r3 * (NTTM_LOGN_MAX + 1) + logn].push_back(i);
+        groups[batch_segments(q.na, q.nb, logn, r3) ? SEG_CLASS : r3 * (NTTM_LOGN_MAX + 1) + logn].push_back(i);
     }
     int np; RCK(choose_np(mn_max ? mn_max : 1, &np));
     for (size_t i = 0; i < N; i++) {
@@ -1441,16 +1564,17 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
      * synchronization at the end.  (Waiting per group left the device idle for 0.9 of the 4096 leaves' 6.6 ms.) */
     std::vector<size_t> order;
     size_t planes = 256, desc = 0, img = 0, words = 0;
-    auto pts = [&](size_t gi) { return (uint64_t)(gi > NTTM_LOGN_MAX ? 3 : 1) << (gi % (NTTM_LOGN_MAX + 1)); };
+    auto radix = [](size_t gi) { return (int)(gi / (NTTM_LOGN_MAX + 1)); };
+    auto pts = [&](size_t gi) { return (uint64_t)(radix(gi) == 1 ? 3 : radix(gi) ? 8 : 1) << (gi % (NTTM_LOGN_MAX + 1)); };   /* (about 8 segments) */
     for (size_t gi = 0; gi < groups.size(); gi++) {
         const std::vector<size_t> &G = groups[gi];
         if (G.empty()) continue;
         order.push_back(gi);
-        const int r3 = gi > NTTM_LOGN_MAX, logn = (int)(gi % (NTTM_LOGN_MAX + 1));
+        const int r3 = radix(gi), logn = (int)(gi % (NTTM_LOGN_MAX + 1));
         const uint64_t n = pts(gi), cnt = G.size();
         uint64_t blk = 0;
-        for (size_t i : G) blk += prod_crt_blocks(logn, r3, n, P[i].na + P[i].nb + (P[i].x ? 1 : 0));
-        if (!small_len(logn, r3)) planes = std::max(planes, chunk_planes_bytes(np, n, cnt));
+        for (size_t i : G) blk += r3 == 2 ? seg_blocks(P[i]) : prod_crt_blocks(logn, r3, n, P[i].na + P[i].nb + (P[i].x ? 1 : 0));
+        if (r3 != 2 && !small_len(logn, r3)) planes = std::max(planes, chunk_planes_bytes(np, n, cnt));
         const size_t im = align_up(cnt * sizeof(CrtDesc), 256) + 2 * align_up(cnt * sizeof(LoadDesc), 256) +
                           align_up((r3 ? 3 : 1) * cnt * 4, 256) + 512;
         img += im;
@@ -1476,7 +1600,7 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
             const std::vector<size_t> &G = groups[order[k]];
             GroupBuild &gb = gbs[k];
             const int logn = (int)(order[k] % (NTTM_LOGN_MAX + 1));
-            group_build(gb, P, G, np, order[k] > NTTM_LOGN_MAX, logn, g.cfg.tile_log, batch_pts(logn));
+            group_build(gb, P, G, np, radix(order[k]), logn, g.cfg.tile_log, batch_pts(logn));
             if (dpos + gb.desc_bytes > g.tdesc_bytes || ipos + gb.off_ncn > img || gb.planes_bytes > g.ws_bytes)
                 return nttm_fail(NTTM_EINVAL, "internal: a batch group exceeds its sizing");
             char *dbase = g.tdesc + dpos;
@@ -2756,6 +2880,7 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
     /* validate and class the products by their 2^k length */
     size_t mn_max = 0;
     std::vector<std::vector<size_t>> cls(NTTM_LOGN_MAX + 1);
+    std::vector<size_t> segs;
     for (size_t i = 0; i < N; i++) {
         const nttm_prod &q = P[i];
         if (q.x && q.nx > q.na + q.nb) return fail(nttm_fail(NTTM_EINVAL, "product %zu: nx exceeds na + nb", i));
@@ -2765,7 +2890,10 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
         int logn, r3;
         choose_len(q.na + q.nb - 1, NTTM_R3_NEVER, g.cfg.tile_log, &logn, &r3);
         if (logn > NTTM_LOGN_MAX) return fail(nttm_fail(NTTM_EBOUND, "product %zu: transform above 2^%d", i, NTTM_LOGN_MAX));
-        cls[logn].push_back(i);
+        int ln, r3b;
+        choose_len(q.na + q.nb - 1, &ln, &r3b);
+        if (batch_segments(q.na, q.nb, ln, r3b)) segs.push_back(i);
+        else cls[logn].push_back(i);
     }
     int rc = choose_np(mn_max ? mn_max : 1, &pl->np);
     if (rc) return fail(rc);
@@ -2804,6 +2932,11 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
         }
         pl->gb.push_back(std::move(b3)); pl->gidx.push_back(S3); pl->gms.push_back(t3);
         if (!S2.empty()) { pl->gb.push_back(std::move(b2)); pl->gidx.push_back(S2); pl->gms.push_back(t2); }
+    }
+    if (!segs.empty()) {
+        GroupBuild b;
+        group_build(b, P, segs, np, 2, SEG_CLASS % (NTTM_LOGN_MAX + 1), g.cfg.tile_log, 16);
+        pl->gb.push_back(std::move(b)); pl->gidx.push_back(segs); pl->gms.push_back(0);
     }
     pl->tune_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
     /* one device blob: the planes (the largest group's; groups run one after another), then every descriptor */

@@ -26,14 +26,10 @@
 #define CRT_T 256
 #define CRT_WIDE 8                       /* limbs per thread of a block (2048-limb blocks); groups of small products
                                             use 1 (256-limb blocks, less of a block idle past a product's end) */
-#define CRT_RUNS 0                       /* in place of the limbs per thread: the blocks are k_inv_crt's runs */
+#define CRT_RUNS 0                       /* in place of the limbs per thread: the blocks are k_inv_crt's runs, */
+#define CRT_SEGS (-1)                    /* or k_segments' segments */
 #define CRT_HALO 4                       /* digits of coefficients k0-4 .. k0-1: v_{k0-1} with four primes */
 #define CRT_ID_MAP 0x2u                  /* one-bit carry maps: bit c = cout(cin = c); the identity is 0b10 */
-#define CRT_CTL_WORDS 4                  /* control words before the block status words (16-byte aligned) */
-/* block status word: map (2 bits) | error for cin 0 << 2 | error for cin 1 << 3 | first of product << 5 */
-#define CRT_ST_E0 (1u << 2)
-#define CRT_ST_E1 (1u << 3)
-#define CRT_ST_FIRST (1u << 5)
 
 struct CrtArgs {
     const CrtDesc *desc; uint64_t nprod; /* null: the one product `one` */
@@ -250,12 +246,13 @@ __device__ __forceinline__ uint32_t crt_step_map(uint32_t st)
 #define RUN_LEN 60
 #define RUN_GROUPS(m) ((m) == 4 ? 1 : 2)        /* runs per row and wave */
 #define RUN_BLOCKS (((1 << RUN_LO) + RUN_LEN - 1) / RUN_LEN)
-/* RUNS: the blocks are k_inv_crt's runs of limbs instead of PER 256 limbs each */
-template <int PER, bool RUNS = false>
+/* PER = CRT_RUNS, CRT_SEGS: the blocks are k_inv_crt's runs of limbs, or step limbs of each product, instead of PER 256 */
+template <int PER>
 __global__ __launch_bounds__(256) void k_carry(const CrtDesc *desc, CrtDesc one, uint64_t nprod, const uint32_t *status,
                                                uint64_t n, uint32_t *ctl, uint64_t *stamp)
 {
-    constexpr int CH = RUNS ? 64 : CRT_T * PER;
+    constexpr bool RUNS = PER == CRT_RUNS, SEGS = PER == CRT_SEGS;
+    constexpr int CH = RUNS || SEGS ? 64 : CRT_T * PER;             /* limbs rewritten at a time */
     stamp_clock(stamp);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t b0 = (uint64_t)blockIdx.x * CRT_CARRY_W;
@@ -297,7 +294,18 @@ __global__ __launch_bounds__(256) void k_carry(const CrtDesc *desc, CrtDesc one,
             const uint64_t row = bl / RUN_BLOCKS, ch = bl - row * RUN_BLOCKS;
             k0 = (row << RUN_LO) + ch * RUN_LEN; end = ch + 1 < RUN_BLOCKS ? k0 + RUN_LEN : (row + 1) << RUN_LO;
         }
+        if (SEGS) { k0 = bl * d.step; end = k0 + d.step; }
         end = end < d.nc ? end : d.nc;
+        if (SEGS) {                                             /* word by word: nearly always the first is the last */
+            for (; k0 < end; k0 += 64) {
+                const uint64_t k = k0 + lane, x = k < end ? d.c[k] : 0;
+                const uint64_t ne = __ballot(k < end && x != NTTM_B - 1);
+                const int at = ne ? __ffsll((long long)ne) - 1 : 64;
+                if (k < end && lane <= at) d.c[k] = lane < at ? 0 : x + 1;
+                if (ne) break;
+            }
+            continue;
+        }
         uint64_t v[CH / 64];
 #pragma unroll
         for (int j = 0; j < CH / 64; j++) { const uint64_t k = k0 + j * 64 + lane; v[j] = k < end ? d.c[k] : 0; }
@@ -568,7 +576,8 @@ int nttm_crt_launch_carry(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t 
     if (one) d1 = *one;
     prof_begin("k_carry", 4.0 * (double)nblocks, s);
     const dim3 grid((unsigned)((nblocks + CRT_CARRY_W - 1) / CRT_CARRY_W));
-    if (per == CRT_RUNS) hipLaunchKernelGGL((k_carry<1, true>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
+    if (per == CRT_RUNS) hipLaunchKernelGGL((k_carry<CRT_RUNS>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
+    else if (per == CRT_SEGS) hipLaunchKernelGGL((k_carry<CRT_SEGS>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
     else if (per == 1) hipLaunchKernelGGL((k_carry<1>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
     else hipLaunchKernelGGL((k_carry<CRT_WIDE>), grid, dim3(256), 0, s, desc_dev, d1, nprod, status, nblocks, ctl, stamp);
     prof_end(s);

@@ -4,6 +4,12 @@
 #define NTTM_CRT_DEV_H
 #include "internal.h"
 
+#define CRT_CTL_WORDS 4                  /* control words before the block status words (16-byte aligned) */
+/* block status word: map (2 bits) | error for cin 0 << 2 | error for cin 1 << 3 | first of product << 5 */
+#define CRT_ST_E0 (1u << 2)
+#define CRT_ST_E1 (1u << 3)
+#define CRT_ST_FIRST (1u << 5)
+
 __device__ __forceinline__ uint32_t map_apply(uint32_t f, uint32_t c) { return (f >> c) & 1u; }
 /* (g o f)(c) = g(f(c)) for maps {0,1} -> {0,1} */
 __device__ __forceinline__ uint32_t map_compose(uint32_t g, uint32_t f)

@@ -323,3 +323,252 @@ int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, cons
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_small launch");
 }
+
+/* ---- uneven products in segments of the result ------------------------------------------------------------------------------
+ * A product of a long operand by one of blen limbs, 2^12 points at a time: limbs [s, s + S) of the result need coefficients
+ * s - 4 .. s + S - 1 (three digits below, and one limb more for the quotient), which are coefficients blen - 1 .. of the
+ * cyclic convolution of the short operand with the long one's limbs from s - 4 - (blen - 1) on, S = 4093 - blen rounded down
+ * to whole words.  A workgroup keeps the short operand's transforms in registers and walks several (the descriptor's
+ * `over`) consecutive segments:
+ * forward, pointwise product and inverse of every prime, digits and limbs as in k_small, so that nothing but operand and
+ * result limbs crosses memory.  A segment is one block of the carry launch.  The overlapping limbs are transformed twice:
+ * the rules that choose it (choose_segments, batch_segments) weigh that.
+ * Bound by vector issue and latency at one workgroup a CU (12 waves, 115 KiB of LDS): 13 us for the short operand and 26 to 31
+ * for a segment of 2048 to 4032 limbs.  Through passes of 2^13 points and more, us, before / now: 500 products of
+ * 8000 x 500 limbs 458 / 210, of 60000 x 1000 1743 / 1178, 8 of 60000 x 300 72 / 50; one of 1000000 x 1000 116 / 88,
+ * of 20000000 x 300 2660 / 625 (in pieces 1080). */
+struct SegArgs {
+    const LoadDesc *ld; const CrtDesc *cd;      /* nprod products in device memory, or null: the one product below */
+    LoadDesc ld1; CrtDesc cd1;
+    uint64_t nprod;
+    uint32_t *status, *ctl;
+    uint64_t *stamps;
+    const double2 *stage[NTTM_MAX_PRIMES], *istage[NTTM_MAX_PRIMES];
+    double2 ninv[NTTM_MAX_PRIMES];
+    CrtConst cc;
+};
+template <int NP>
+__global__ __launch_bounds__(NP * 256) void k_segments(SegArgs a)
+{
+    constexpr int LOGN = SMALL_LOG_MAX, N = 1 << LOGN, PTS = 16, NT = N / PTS, NTH = NP * NT, NW = NTH / 64, SW = 8, NR = 3;
+    constexpr int IT = (63 + NW - 1) / NW;                           /* words of a wave */
+    typedef __attribute__((address_space(1))) uint64_t *GOut;
+    __shared__ double pl[NP][LDS_WORDS(N)];
+    __shared__ double2 stw[NP][1 << SW];
+    __shared__ uint64_t sgx[64], sgy[64];
+    __shared__ uint32_t s_prod, s_err;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t pi = __builtin_amdgcn_readfirstlane((uint32_t)tid / NT);
+    const int t = tid & (NT - 1);
+    if (a.stamps) stamp_clock(a.stamps);
+    if (blockIdx.x == 0 && tid == 0) { a.ctl[0] = 0; a.ctl[1] = 0; }
+    stw[pi][t] = a.stage[pi][t];                                     /* (256 threads and entries a prime) */
+    if (tid == 0) {
+        uint64_t lo = 0, hi = a.cd ? a.nprod - 1 : 0;                /* the product whose workgroups hold this one */
+        while (lo < hi) { const uint64_t mid = (lo + hi + 1) >> 1; if (a.cd[mid].tn <= blockIdx.x) lo = mid; else hi = mid - 1; }
+        s_prod = (uint32_t)lo;
+    }
+    __syncthreads();
+    LoadDesc l = a.ld1; CrtDesc d = a.cd1;
+    if (a.ld) { const uint32_t prod = __builtin_amdgcn_readfirstlane(s_prod); l = a.ld[prod]; d = a.cd[prod]; }
+    const int nb = (int)l.nb, S = (int)d.step, nw = S >> 6;
+    const uint32_t per = (uint32_t)d.over, nseg = (uint32_t)((d.nc + S - 1) / S), seg0 = (blockIdx.x - (uint32_t)d.tn) * per;
+    const uint32_t seg1 = seg0 + per < nseg ? seg0 + per : nseg;
+
+    const double p = a.cc.pk[pi].p, pinv = a.cc.pk[pi].pinv;
+    const SwzLds xs{pl[pi]};
+    const double2 *lt = stw[pi];
+    const GTab gf(a.stage[pi]), gi(a.istage[pi]);
+    PassPos pp; pp.m = LOGN; pp.logw = 0; pp.lo = 0; pp.nthr = NT; pp.t = t;
+    int s_lo, logR;
+    double v[PTS], bv[PTS];
+    uint64_t raw[PTS];
+    uint32_t in = 0;                                                 /* bit sl: the slot lies inside the operand */
+    auto request = [&](const uint64_t *src, uint64_t n, int64_t base) {
+        in = 0;
+        for_slots<4, PTS>(pp, 8, [&](int sl, uint32_t, uint32_t o, uint32_t, uint32_t) {
+            const uint64_t k = (uint64_t)(base + o);                 /* (before the first limb: beyond any length) */
+            const bool inside = k < n;
+            raw[sl] = ((GLimb)src)[inside ? k : 0];
+            in |= (uint32_t)inside << sl;
+        });
+    };
+    auto forward = [&]() {                                           /* of raw, into v in the last round's layout */
+#pragma unroll
+        for (int sl = 0; sl < PTS; sl++) v[sl] = (in >> sl) & 1 ? limb_to_res(raw[sl], p, pinv) : 0.0;
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            round_split(LOGN, i, &s_lo, &logR, false, 4);
+            if (i > 0) {
+                __syncthreads();
+                for_slots<4, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) { v[sl] = xs.at(e); });
+            }
+            if (i == 0) round_compute<4, false, PTS>(v, pp, s_lo, gf, p, pinv);
+            else round_compute<4, false, PTS, LTab>(v, pp, s_lo, lt, p, pinv);
+            if (i + 1 < NR) for_slots<4, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) { xs.at(e) = v[sl]; });
+        }
+    };
+    auto first = [&](uint32_t seg) { return (int64_t)seg * S - 4 - (nb - 1); };   /* the coefficient of the window's element 0 */
+    request(l.b, l.nb, 0);
+    forward();
+    const double2 ninv = a.ninv[pi];
+#pragma unroll
+    for (int sl = 0; sl < PTS; sl++) bv[sl] = mul_shoup(v[sl], ninv.x, ninv.y, p);
+
+    __syncthreads();                                                 /* B's last LDS reads before A's first writes */
+    for (uint32_t seg = seg0; seg < seg1; seg++) {
+        /* opaque to the compiler, which otherwise keeps every twiddle and address of the loop in registers it has not got */
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63;
+        pp.t = tid & (NT - 1);
+        request(l.a, l.na, first(seg));
+        forward();
+#pragma unroll
+        for (int sl = 0; sl < PTS; sl++) v[sl] = mul_barrett(v[sl], bv[sl], p, pinv);
+#pragma unroll
+        for (int i = 0; i < NR; i++) {                               /* bit 0 first; round 0 has the layout in v */
+            round_split(LOGN, i, &s_lo, &logR, true, 4);
+            if (i > 0) {
+                __syncthreads();
+                for_slots<4, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) { v[sl] = xs.at(e); });
+            }
+            if (i == NR - 1) round_compute<4, true, PTS>(v, pp, s_lo, gi, p, pinv);
+            else round_compute_mirror<4, PTS>(v, pp, s_lo, lt, p, pinv);
+            for_slots<4, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) { xs.at(e) = v[sl]; });
+        }
+        /* the segment's x limbs are requested, the next one's operand limbs drawn into the L2 (a word of every line; in registers
+         * they would be spilled); residues become digits in place */
+        const uint64_t s0 = (uint64_t)seg * S;
+        uint64_t xk[IT], xp[IT];
+#pragma unroll
+        for (int i = 0; i < IT; i++) {
+            const int w = wave + i * NW;
+            const uint64_t k = s0 + (uint64_t)w * 64 + lane;
+            xk[i] = xp[i] = 0;
+            if (w < nw) {
+                if (k < d.nx && k < d.nc) xk[i] = ((GLimb)d.x)[k];
+                if (lane == 0 && k >= 1 && k - 1 < d.nx) xp[i] = ((GLimb)d.x)[k - 1];
+            }
+        }
+
+        uint64_t touch = 0;
+        if (pi == 0 && seg + 1 < seg1) {
+            const uint64_t k = (uint64_t)(first(seg + 1) + 16 * tid);
+            touch = ((GLimb)l.a)[k < l.na ? k : 0];
+        }
+        if (tid == 0) s_err = 0;
+        __syncthreads();
+        const int64_t c0 = first(seg);
+        for (int e = tid; e < N; e += NTH) {
+            if (e < nb - 1) continue;                                /* (wrapped coefficients: never read) */
+            const bool live = (uint64_t)(c0 + e) < d.ncoef;
+            double r[NP];
+            uint64_t dg[NP];
+#pragma unroll
+            for (int j = 0; j < NP; j++) r[j] = live ? pl[j][e + (e >> 5)] : 0.0;
+            crt_digits<NP>(a.cc, r, dg);
+#pragma unroll
+            for (int j = 0; j < NP; j++) pl[j][e + (e >> 5)] = __longlong_as_double((long long)dg[j]);
+        }
+        __syncthreads();
+        /* limbs: coefficient k - j of limb k = s0 + u is element nb + 3 + u - j >= nb - 1 */
+        auto digit = [&](int j, int u) -> uint64_t {
+            const int e = nb + 3 + u;
+            return (uint64_t)__double_as_longlong(pl[j][e + (e >> 5)]);
+        };
+        auto vsum = [&](int u, uint64_t x) -> uint64_t {
+            uint64_t y = x;
+#pragma unroll
+            for (int j = 0; j < NP; j++) y += digit(j, u - j);
+            return y;
+        };
+        auto quot = [](uint64_t y) -> uint32_t {
+            uint32_t q = 0;
+#pragma unroll
+            for (int c = 1; c <= NP; c++) q += y >= (uint64_t)c * NTTM_B;
+            return q;
+        };
+        uint64_t wv[IT], GX[IT], GY[IT];
+        uint32_t ql[IT];
+#pragma unroll
+        for (int i = 0; i < IT; i++) {
+            const int w = wave + i * NW, u = w * 64 + lane;
+            wv[i] = GX[i] = GY[i] = 0; ql[i] = 0;
+            if (w < nw) {
+                const uint64_t k = s0 + u;
+                const uint64_t y = k < d.nc ? vsum(u, xk[i]) : 0;
+                const uint32_t q = quot(y);
+                uint32_t qp = __shfl_up(q, 1, 64);
+                if (lane == 0) qp = k >= 1 && k <= d.nc ? quot(vsum(u - 1, xp[i])) : 0u;
+                wv[i] = y - (uint64_t)q * NTTM_B + qp;
+                if (k >= d.nc) wv[i] = 0;
+                ql[i] = q;
+                const uint64_t g = __ballot(wv[i] >= NTTM_B), pr = __ballot(wv[i] == NTTM_B - 1);
+                GX[i] = g; GY[i] = g | pr;
+                if (lane == 0) { sgx[w] = g; sgy[w] = g | pr; }
+            }
+        }
+        __syncthreads();
+        /* the carry into every word for a carry of 0 (C0) and 1 (C1) into the segment; bit nw: out of it */
+        uint64_t C0, C1;
+        {
+            uint32_t f0 = 0, f1 = 0;
+            if (lane < nw) { f0 = add_cout(sgx[lane], sgy[lane], 0); f1 = add_cout(sgx[lane], sgy[lane], 1); }
+            const uint64_t G = __ballot(f0 != 0), GP = __ballot(f1 != 0);
+            C0 = (G + GP) ^ G ^ GP; C1 = (G + GP + 1) ^ G ^ GP;
+        }
+#pragma unroll
+        for (int i = 0; i < IT; i++) {
+            const int w = wave + i * NW, u = w * 64 + lane;
+            if (w < nw) {
+                const uint64_t k = s0 + u;
+                const uint32_t c = (uint32_t)(C0 >> w) & 1u;
+                const uint64_t CB = (GX[i] + GY[i] + c) ^ GX[i] ^ GY[i];      /* bit b: the carry into bit b */
+                const uint32_t oin = (uint32_t)(CB >> lane) & 1u;
+                const uint32_t oout = lane == 63 ? add_cout(GX[i], GY[i], c) : (uint32_t)(CB >> (lane + 1)) & 1u;
+                if (k < d.nc) ((GOut)d.c)[k] = wv[i] + oin - (oout ? NTTM_B : 0);
+                if (k + 1 == d.nc && !d.trunc) {                     /* the last limb: nothing may remain beyond it */
+                    const uint32_t c1 = (uint32_t)(C1 >> w) & 1u;
+                    const uint64_t CB1 = (GX[i] + GY[i] + c1) ^ GX[i] ^ GY[i];
+                    const uint32_t o1 = lane == 63 ? add_cout(GX[i], GY[i], c1) : (uint32_t)(CB1 >> (lane + 1)) & 1u;
+                    uint64_t extra = ql[i];
+#pragma unroll
+                    for (int e = 1; e < NP; e++)
+#pragma unroll
+                        for (int j = e; j < NP; j++) extra += digit(j, u + e - j);
+                    s_err = (extra + oout ? CRT_ST_E0 : 0u) | (extra + o1 ? CRT_ST_E1 : 0u);
+                }
+            }
+        }
+        asm volatile("" :: "v"(touch));
+        __syncthreads();                                             /* (the digits are read, s_err is stored) */
+        if (tid == 0)
+            a.status[d.first_block + seg] = ((uint32_t)(C0 >> nw) & 1u) | ((uint32_t)(C1 >> nw) & 1u) << 1 | s_err | (seg ? 0u : CRT_ST_FIRST);
+    }
+}
+
+/* limbs of a segment for a short operand of nb limbs (whole words; 0: too long a one) */
+uint64_t nttm_seg_len(uint64_t nb) { return nb < 1 || nb > ((uint64_t)1 << SMALL_LOG_MAX) - 3 - 512 ? 0 : (((uint64_t)1 << SMALL_LOG_MAX) - 3 - nb) & ~(uint64_t)63; }
+/* nprod products in segments, from device descriptors, or (ld null) the one product ld1, cd1: the longer operand as a, step =
+ * nttm_seg_len(nb), over the segments of a workgroup, tn the product's first workgroup, first_block its first segment among the status
+ * words.  The limbs are for a carry of 0 into every segment: nttm_crt_launch_carry(.., NTTM_CRT_SEGS) follows */
+int nttm_run_segments(int np, const LoadDesc *ld, const CrtDesc *cd, const LoadDesc *ld1, const CrtDesc *cd1, uint64_t nprod,
+                      uint64_t groups, const TwTables *fwd, const TwTables *inv, const double2 *ninv,
+                      const CrtConst &cc, uint32_t *scratch, uint32_t *ctl, hipStream_t s, double alg_bytes, uint64_t *stamps)
+{
+    if (np < 3 || np > NTTM_MAX_PRIMES || !nprod || !groups || (!ld != !cd) || (!ld && (!ld1 || !cd1 || nprod != 1)) || !ctl)
+        return nttm_fail(NTTM_EINVAL, "internal: products in segments");
+    if (!ld && (!cd1->step || !cd1->over || cd1->step != nttm_seg_len(ld1->nb))) return nttm_fail(NTTM_EINVAL, "internal: segments of %llu limbs", (unsigned long long)cd1->step);
+    if (groups > 0x7fffffffULL) return nttm_fail(NTTM_EINVAL, "internal: too many segments");
+    SegArgs a; memset(&a, 0, sizeof a);
+    a.ld = ld; a.cd = cd; a.nprod = nprod; a.status = scratch + CRT_CTL_WORDS; a.ctl = ctl; a.stamps = stamps; a.cc = cc;
+    if (ld1) a.ld1 = *ld1;
+    if (cd1) a.cd1 = *cd1;
+    for (int i = 0; i < np; i++) { a.stage[i] = fwd[i].stage; a.istage[i] = inv[i].stage; a.ninv[i] = ninv[i]; }
+    prof_begin("k_segments", alg_bytes, s);
+    if (np == 3) hipLaunchKernelGGL(k_segments<3>, dim3((unsigned)groups), dim3(3 * 256), 0, s, a);
+    else hipLaunchKernelGGL(k_segments<4>, dim3((unsigned)groups), dim3(4 * 256), 0, s, a);
+    prof_end(s);
+    return nttm_hip_check(hipGetLastError(), "k_segments launch");
+}

@@ -40,6 +40,12 @@ def pieces(nttm):
     (1 << 13, 20000, 4081),              # pieces of 4096 limbs: nearly all of a piece is overlap
     (1 << 13, 3 * 4096, 4096),
     (1 << 14, 70001, 129),
+    (1 << 12, 32768, 1),                 # segments of the result, one launch: 4032 limbs each
+    (1 << 12, 4032 * 3 - 61, 61),        # the result ends with a segment (4032 limbs) ...
+    (1 << 12, 4032 * 3 - 60, 61),        # ... and a limb after it
+    (1 << 12, 30011, 2100),
+    (1 << 12, 9001, 3581),               # the longest short operand: 512 limbs of 4096 points
+    (1 << 12, 70003, 700),
     (3 << 12, 60001, 2047),              # 3 2^k points
     (3 << 13, 50003, 6000),
 ])
@@ -83,3 +89,46 @@ def test_cut(pieces, w):
     lib = pieces(1 << 13)
     got = host(lib.mul_cut(dev(a), dev(b), 0, w))
     assert np.array_equal(got[:w], O.mul_school(a, b)[:w])
+
+
+@pytest.mark.parametrize("points", [None, 1 << 12])
+@pytest.mark.parametrize("cfg", [dict(), dict(nprimes=4)])
+@pytest.mark.parametrize("top", [False, True])
+def test_batch(pieces, points, cfg, top):
+    """a batch, by call and as a plan, whose uneven products go through segments (by the rule, or all that can): lengths, added
+    operands, several segments and products per workgroup, among products of other classes"""
+    import torch
+    rng = np.random.default_rng(11)
+    ops, s = [], 5
+    for i in range(70):
+        lo, hi = ((1, 300), (9000, 40000)) if i % 3 else ((1, 3500), (1, 5000))
+        na, nb = int(rng.integers(*hi)), int(rng.integers(*lo))
+        a, s = O.gen_limbs(na, s)
+        b, s = O.gen_limbs(nb, s)
+        x = O.gen_limbs(int(rng.integers(1, na + nb + 1)), s)[0] if i % 4 == 0 else None
+        if top:
+            a[:] = TOP; b[:] = TOP
+            if x is not None:
+                x[:] = TOP
+        ops.append((a, b, x) if i % 2 else (b, a, x))
+    say("batch", points, cfg, top)
+    lib = pieces(points, **cfg)
+    want = [O.mul_school(*o) for o in ops]
+    items = [(dev(a), dev(b), None if x is None else dev(x),
+              torch.full((len(w),), -1, dtype=torch.int64, device="cuda")) for (a, b, x), w in zip(ops, want)]
+    prods = lib.make_prods(items)
+    lib.mul_batch(prods)
+    lens = [int(np.nonzero(w)[0][-1]) + 1 for w in want]
+    assert [p.ncn for p in prods] == lens
+    for it, w in zip(items, want):
+        assert np.array_equal(host(it[3]), w)
+    for tune in (0, 1):
+        plan = lib.BatchPlan(prods, autotune=tune)
+        for _ in range(2):
+            for it in items:
+                it[3].fill_(-1)
+            plan.run()
+            assert list(plan.ncn()) == lens
+            for it, w in zip(items, want):
+                assert np.array_equal(host(it[3]), w)
+        plan.close()
