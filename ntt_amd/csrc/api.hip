@@ -853,6 +853,14 @@ static double seg_launch_us(uint64_t n, uint32_t per, uint64_t S)
 }
 static bool seg_forced(void) { return g_pieces_points == 1 << 12; }
 static bool seg_allowed(uint64_t S) { return S && !g_no_small && (g_pieces_points < 0 || seg_forced()); }
+/* the result shares memory with an operand: segments, which write limbs while others still read theirs, are not for it (the
+ * passes read every operand limb before the first result limb is written) */
+static bool result_over_operands(const uint64_t *c, size_t nc, const uint64_t *a, size_t na, const uint64_t *b, size_t nb,
+                                 const uint64_t *x, size_t nx)
+{
+    auto hit = [&](const uint64_t *p, size_t n) { return p && n && (uintptr_t)p < (uintptr_t)(c + nc) && (uintptr_t)c < (uintptr_t)(p + n); };
+    return hit(a, na) || hit(b, nb) || hit(x, nx);
+}
 /* one product: the segments of a workgroup that give it the least time, if that is below `most`; else 0 */
 static uint32_t choose_segments(size_t nc, size_t blen, double most)
 {
@@ -869,11 +877,13 @@ static uint32_t choose_segments(size_t nc, size_t blen, double most)
 }
 /* a product of a batch, whose launches fill the device either way: segments against the passes and the CRT of its own length
  * at 17 ps a point and prime from 2^16 points, 1.5 more for each bit below (measured 17.3 there, 19 at 2^15, 21 at 2^14) */
-static bool batch_segments(size_t na, size_t nb, int logn, int r3)
+static bool batch_segments(const nttm_prod &q, int logn, int r3)
 {
+    const size_t na = q.na, nb = q.nb;
     const size_t alen = std::max(na, nb), blen = std::min(na, nb);
     const uint64_t S = nttm_seg_len(blen);
     if (!seg_allowed(S) || (uint64_t)na + nb > 0xffffffffULL) return false;
+    if (result_over_operands(q.c, na + nb + (q.x ? 1 : 0), q.a, na, q.b, nb, q.x, q.x ? q.nx : 0)) return false;
     if (seg_forced()) return true;
     if (small_len(logn, r3) || alen < 2 * blen) return false;
     const double segs = ceil((double)(na + nb) / (double)S);
@@ -898,8 +908,9 @@ __global__ __launch_bounds__(256) void k_pieces(LoadDesc *ld, uint32_t *bmap, co
 /* the workspace of a one-transform product: the planes, its CRT descriptor (the pieces' descriptors) and the CRT's scratch
  * (bytes from ws).  n: points of the transforms, plane: of one prime's plane of A */
 struct CoreLayout { int np, logn, r3, par; uint32_t seg_per; uint64_t n, plane, ncoef, cnt, step; size_t nc, nc_full, off_desc, off_bmap, off_crt, bytes; };
-/* allow_par: one launch per pass for all primes, each with its own B plane (in the library's workspace) */
-static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout *L, bool allow_par = false)
+/* allow_par: one launch per pass for all primes, each with its own B plane (in the library's workspace), or the product in
+ * pieces or (allow_segs: no result over its operands) in segments */
+static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout *L, bool allow_par = false, bool allow_segs = true)
 {
     L->nc_full = na + nb + (has_x ? 1 : 0); L->nc = L->nc_full < wcut ? L->nc_full : wcut;
     RCK(choose_np(na < nb ? na : nb, &L->np));
@@ -912,7 +923,7 @@ static int core_layout(size_t na, size_t nb, bool has_x, size_t wcut, CoreLayout
     if (allow_par) {                                             /* (the library's own workspace) */
         const size_t alen = std::max(na, nb), blen = std::min(na, nb);
         const Pieces q = choose_pieces(L->np, alen, blen, L->logn, L->r3);
-        if (!small_len(L->logn, L->r3) && (L->seg_per = choose_segments(L->nc, blen, q.us))) {
+        if (allow_segs && !small_len(L->logn, L->r3) && (L->seg_per = choose_segments(L->nc, blen, q.us))) {
             L->step = nttm_seg_len(blen); L->cnt = (L->nc + L->step - 1) / L->step; L->par = 1;
             L->off_desc = L->off_crt = 0;
             L->bytes = nttm_crt_scratch_words(L->cnt) * 4 + 256;
@@ -985,7 +996,7 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
         return 0;
     }
     if (!nc) return 0;
-    CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws));
+    CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws, !result_over_operands(c, nc, a, na, b, nb, x, x ? nx : 0)));
     uint32_t *ctl = (uint32_t *)((char *)g.hpin + 128 * slot + 96);
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.plane = L.plane; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
@@ -1548,7 +1559,7 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
         int logn, r3;
         choose_len(q.na + q.nb - 1, &logn, &r3);
         if (logn > NTTM_LOGN_MAX) return nttm_fail(NTTM_EBOUND, "product %zu: transform above 2^%d", i, NTTM_LOGN_MAX);
-        groups[batch_segments(q.na, q.nb, logn, r3) ? SEG_CLASS : r3 * (NTTM_LOGN_MAX + 1) + logn].push_back(i);
+        groups[batch_segments(q, logn, r3) ? SEG_CLASS : r3 * (NTTM_LOGN_MAX + 1) + logn].push_back(i);
     }
     int np; RCK(choose_np(mn_max ? mn_max : 1, &np));
     for (size_t i = 0; i < N; i++) {
@@ -2140,7 +2151,8 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
         RCK(prod_kinds(mm, q.a, q.na, q.b, q.nb, q.x, q.nx, q.c, nc, ki, i));
         if (any_host(ki)) return nttm_fail(NTTM_EINVAL, "nttm_mul_each_async: product %zu: host memory (device memory only)", i);
         if (q.na && q.nb && fits_one(q.na, q.nb, nc)) {                /* (with every prime's B plane) */
-            CoreLayout L; RCK(core_layout(q.na, q.nb, q.x != nullptr, SIZE_MAX, &L, true));
+            CoreLayout L; 
+            RCK(core_layout(q.na, q.nb, q.x != nullptr, SIZE_MAX, &L, true, !result_over_operands(q.c, nc, q.a, q.na, q.b, q.nb, q.x, q.x ? q.nx : 0)));
             ws_max = std::max(ws_max, L.bytes);
         }
     }
@@ -2892,7 +2904,7 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
         if (logn > NTTM_LOGN_MAX) return fail(nttm_fail(NTTM_EBOUND, "product %zu: transform above 2^%d", i, NTTM_LOGN_MAX));
         int ln, r3b;
         choose_len(q.na + q.nb - 1, &ln, &r3b);
-        if (batch_segments(q.na, q.nb, ln, r3b)) segs.push_back(i);
+        if (batch_segments(q, ln, r3b)) segs.push_back(i);
         else cls[logn].push_back(i);
     }
     int rc = choose_np(mn_max ? mn_max : 1, &pl->np);

@@ -132,3 +132,21 @@ def test_batch(pieces, points, cfg, top):
             for it, w in zip(items, want):
                 assert np.array_equal(host(it[3]), w)
         plan.close()
+
+
+def test_result_over_operand(pieces):
+    """a result that overwrites its own operand is formed by the passes, which read every limb first"""
+    import torch
+    a, s = O.gen_limbs(60000, 3)
+    b, _ = O.gen_limbs(300, s)
+    say("result over operand")
+    lib = pieces()
+    want = O.mul_school(a, b)
+    for off in (0, 17, 4000):
+        buf = torch.zeros(70000, dtype=torch.int64, device="cuda")
+        buf[off:off + 60000] = dev(a)
+        lib.mul(buf[off:off + 60000], dev(b), out=buf[:60300])
+        assert np.array_equal(host(buf)[:60300], want)
+        buf[off:off + 60000] = dev(a)
+        lib.mul_batch(lib.make_prods([(buf[off:off + 60000], dev(b), None, buf[:60300])]))
+        assert np.array_equal(host(buf)[:60300], want)
