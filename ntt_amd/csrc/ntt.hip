@@ -217,9 +217,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
         }
         if (LT && s_lo + logR <= STW_LOG) {
             if (i == 0 && !(gw + s_lo < 4)) __syncthreads();        /* (no barrier has passed since the table was stored) */
-            if (active) ROUND_SWITCH(logR, round_compute<LR, INV, PTS, LTab>(v, pp, s_lo, stw, p, pinv);)
+            if (active) ROUND_SWITCH(logR, round_compute<LR, INV, PTS, LTab>(v, pp, s_lo, stw, p, pinv, GM >= 0 && i > 0, GM >= 0 && i + 1 < nr);)
         } else {
-            if (active) ROUND_SWITCH(logR, round_compute<LR, INV, PTS>(v, pp, s_lo, gtw, p, pinv);)
+            if (active) ROUND_SWITCH(logR, round_compute<LR, INV, PTS>(v, pp, s_lo, gtw, p, pinv, GM >= 0 && i > 0, GM >= 0 && i + 1 < nr);)
         }
         if (i + 1 < nr && active)
             ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
                     }
                 }
             }
-            ROUND_SWITCH(logR, round_compute<LR, INV, PTS, LTab>(v, pp, s_lo, stw, p, pinv);)
+            ROUND_SWITCH(logR, round_compute<LR, INV, PTS, LTab>(v, pp, s_lo, stw, p, pinv, i > 0, i + 1 < NR);)
             if (i + 1 < NR)
                 ROUND_SWITCH(logR, for_slots<LR, PTS>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
                     cur[e] = v[sl]; });)
@@ -578,9 +578,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
                                                                            uint32_t) { v[sl] = xs.at(e); });)
         }
         if (LT && i < 2) {                                       /* inverse rounds 0 and 1: stages 0..7 */
-            if (active) ROUND_SWITCH(logR, round_compute_mirror<LR, PTS>(v, pp, s_lo, stw, p, pinv);)
+            if (active) ROUND_SWITCH(logR, round_compute_mirror<LR, PTS>(v, pp, s_lo, stw, p, pinv, GM >= 0 && i > 0, GM >= 0 && i + 1 < nr);)
         } else {
-            if (active) ROUND_SWITCH(logR, round_compute<LR, true, PTS>(v, pp, s_lo, GTab(a.twi.stage), p, pinv);)
+            if (active) ROUND_SWITCH(logR, round_compute<LR, true, PTS>(v, pp, s_lo, GTab(a.twi.stage), p, pinv, GM >= 0 && i > 0, GM >= 0 && i + 1 < nr);)
         }
         if (i + 1 < nr && active)
             ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t,

@@ -15,10 +15,14 @@
  * row field, point j sits at global offset ob + j 2^(s_lo + lo) and at bit-reversed row kb + brev(j) 2^(m - s_lo - logR):
  * addresses and boundary-twiddle exponents of a group are a base plus compile-time multiples.  Each thread reads and
  * writes exactly the elements of its groups within a round, so one barrier separates consecutive rounds.
- * Lazy reduction (bounds of arith.h): the DIF reduces its sum path at odd levels and at a round's last level (values
- * entering a butterfly stay within [-2p, 2p]); the DIT reduces both outputs at a round's last level only (after levels
- * 0..3 the outputs are within 1.75p, 2.5p, 3.5p, 4.5p + 2, and every mul_shoup input within 4p; with the trivial
- * first level of a lowest-bits round, 2p, 2.75p + 1, 3.75p + 2, 4.75p + 3, mul_shoup inputs within 3.75p + 2).
+ * Lazy reduction.  For |x| <= k p, k <= 4, mul_shoup gives at most (1/2 + k/16) p, reduce p/2 + 1; sums are exact below 8p.
+ * The DIF follows every slot's bound from inputs within p (DifRed): a sum is reduced where it would take the next
+ * level's difference past 4p (above 2p), or at the last level above p.  13 reductions for 16 points in 4 levels, where one of
+ * every sum at odd levels took 16.  The DIT's outputs grow by less than 0.71 p a level: from inputs within p (and a trivial first
+ * level) 2, 2.625, 3.29, 3.995 p.  Rounds with another one after them leave their outputs so; that one reduces the half of
+ * its inputs that its first level does not multiply (then 1.25, 1.83, 2.45, 3.10 p), and a pass's last round reduces all
+ * outputs.  (Reducing all outputs of every round: 16 a round in place of 0, 8 and 24.)  Both together, ms:
+ * 2^27 x 2^27 limbs 22.16 to 21.98, 2^25 x 2^25 5.38 to 5.28, 4096 leaves as a plan 4.89 to 4.80.
  * Where the round's low row bits are known to be zero at compile time, twiddles w^0 = 1 are not multiplied: the DIF
  * difference then follows the sum path's rule, the DIT skips them at its first level (where all of them are 1). */
 #define PASS_PTS 16               /* points per thread of full tiles; tiles below 16 points use one thread */
@@ -68,47 +72,76 @@ __device__ __forceinline__ double2 tw_at(const CTab &tw, uint32_t, uint32_t fixe
     return make_double2(x[0], x[1]);
 }
 
+/* which outputs of each DIF level are reduced, from the slots' bounds in units of p (TRIV: the twiddles of slot 0 of every
+ * block are 1 and not multiplied) */
+template <int LOGR, bool TRIV> struct DifRed {
+    uint32_t mask[LOGR];
+    constexpr DifRed() : mask{}
+    {
+        constexpr int R = 1 << LOGR;
+        double b[R] = {};
+        for (int j = 0; j < R; j++) b[j] = 1.0;
+        for (int lev = 0; lev < LOGR; lev++) {
+            const int h = R >> (lev + 1);
+            const double most = lev == LOGR - 1 ? 1.0 : 2.0;
+            for (int jj = 0; jj < h; jj++)
+                for (int j = jj; j < R; j += 2 * h) {
+                    const double sm = b[j] + b[j + h];
+                    const bool one = TRIV && jj == 0;
+                    b[j] = sm; b[j + h] = one ? sm : 0.5 + sm / 16;
+                    for (int e = j; e <= j + h; e += h)
+                        if (b[e] > most) { mask[lev] |= 1u << e; b[e] = 0.5; }
+                }
+        }
+    }
+};
+
 template <int LOGR, typename TW>
 __device__ __forceinline__ void dif_group(double *v, int s_lo, uint32_t rlow, TW tw, double p, double pinv)
 {
     constexpr int R = 1 << LOGR;
+    constexpr DifRed<LOGR, false> rn{};
+    constexpr DifRed<LOGR, true> rt{};
 #pragma unroll
     for (int lev = 0; lev < LOGR; lev++) {
         const int k = LOGR - 1 - lev, h = 1 << k;
-        const bool red = (lev & 1) || lev == LOGR - 1;
+        const uint32_t red = NTTM_TRIVIAL_W(rlow, 0) ? rt.mask[lev] : rn.mask[lev];
 #pragma unroll
         for (int jj = 0; jj < h; jj++) {
-            /* a trivial twiddle: the difference follows the sum path's bound and reduction rule */
             const bool one = NTTM_TRIVIAL_W(rlow, jj);
             const double2 w = one ? make_double2(1.0, 0.0) : tw_at(tw, rlow, (1u << (s_lo + k)) + ((uint32_t)jj << s_lo));
 #pragma unroll
             for (int j = jj; j < R; j += 2 * h) {
                 const double u = v[j], x = v[j + h];
                 const double sm = u + x, df = u - x;
-                v[j] = red ? reduce(sm, p, pinv) : sm;
-                v[j + h] = one ? (red ? reduce(df, p, pinv) : df) : mul_shoup(df, w.x, w.y, p);
+                v[j] = (red >> j) & 1 ? reduce(sm, p, pinv) : sm;
+                v[j + h] = !one ? mul_shoup(df, w.x, w.y, p) : (red >> (j + h)) & 1 ? reduce(df, p, pinv) : df;
             }
         }
     }
 }
 
+/* one DIT butterfly level's inputs: wide: within 4p (at the round's first level), so u, and an x that is not multiplied, are
+ * reduced */
+__device__ __forceinline__ double dit_u(double u, bool wide, double p, double pinv) { return wide ? reduce(u, p, pinv) : u; }
+/* wide_in: the inputs are within 4p, else p; wide_out: the outputs may be left within 4p, else they are reduced */
 template <int LOGR, typename TW>
-__device__ __forceinline__ void dit_group(double *v, int s_lo, uint32_t rlow, TW tw, double p, double pinv)
+__device__ __forceinline__ void dit_group(double *v, int s_lo, uint32_t rlow, TW tw, double p, double pinv, bool wide_in = false,
+                                          bool wide_out = false)
 {
     constexpr int R = 1 << LOGR;
 #pragma unroll
     for (int lev = 0; lev < LOGR; lev++) {
         const int k = lev, h = 1 << k;
-        const bool red = lev == LOGR - 1;
+        const bool red = lev == LOGR - 1 && !wide_out, wide = lev == 0 && wide_in;
 #pragma unroll
         for (int jj = 0; jj < h; jj++) {
-            /* a trivial twiddle at the first level only (inputs within p: outputs within 2p, and the later bounds
-             * below hold with 0.25p to spare) */
             const bool one = lev == 0 && NTTM_TRIVIAL_W(rlow, jj);
             const double2 w = one ? make_double2(1.0, 0.0) : tw_at(tw, rlow, (1u << (s_lo + k)) + ((uint32_t)jj << s_lo));
 #pragma unroll
             for (int j = jj; j < R; j += 2 * h) {
-                const double u = v[j], x = one ? v[j + h] : mul_shoup(v[j + h], w.x, w.y, p);
+                const double u = dit_u(v[j], wide, p, pinv);
+                const double x = one ? dit_u(v[j + h], wide, p, pinv) : mul_shoup(v[j + h], w.x, w.y, p);
                 const double s1 = u + x, s2 = u - x;
                 v[j] = red ? reduce(s1, p, pinv) : s1;
                 v[j + h] = red ? reduce(s2, p, pinv) : s2;
@@ -154,7 +187,8 @@ __device__ __forceinline__ void for_slots(const PassPos &pp, int s_lo, F f)
 /* the radix step of one round on all PTS slots: PTS / R groups of R points */
 /* TW: GTab (a global stage table) or LTab (a table in LDS, named explicitly so that it stays restrict) */
 template <int LOGR, bool INV, int PTS, typename TW>
-__device__ __forceinline__ void round_compute(double *v, const PassPos &pp, int s_lo, TW tw, double p, double pinv)
+__device__ __forceinline__ void round_compute(double *v, const PassPos &pp, int s_lo, TW tw, double p, double pinv, bool wide_in = false,
+                                              bool wide_out = false)
 {
     constexpr int R = 1 << LOGR, G = PTS / R;
     const int L = pp.logw + s_lo;
@@ -162,7 +196,7 @@ __device__ __forceinline__ void round_compute(double *v, const PassPos &pp, int 
     for (int g = 0; g < G; g++) {
         const uint32_t tau = (uint32_t)(g * pp.nthr + pp.t);
         const uint32_t rlow = (tau & ((1u << L) - 1)) >> pp.logw;      /* row bits below s_lo */
-        if (INV) dit_group<LOGR, TW>(v + g * R, s_lo, rlow, tw, p, pinv);
+        if (INV) dit_group<LOGR, TW>(v + g * R, s_lo, rlow, tw, p, pinv, wide_in, wide_out);
         else dif_group<LOGR, TW>(v + g * R, s_lo, rlow, tw, p, pinv);
     }
 }
@@ -172,13 +206,13 @@ __device__ __forceinline__ void round_compute(double *v, const PassPos &pp, int 
  * w^0 = 1 taken from entry 1 (stage 0).  Lets a kernel keep one small table in LDS for both directions. */
 template <int LOGR>
 __device__ __forceinline__ void dit_group_mirror(double *v, int s_lo, uint32_t rlow, const double2 *tw, double p,
-                                                 double pinv)
+                                                 double pinv, bool wide_in, bool wide_out)
 {
     constexpr int R = 1 << LOGR;
 #pragma unroll
     for (int lev = 0; lev < LOGR; lev++) {
         const int k = lev, h = 1 << k, s = s_lo + k;
-        const bool red = lev == LOGR - 1;
+        const bool red = lev == LOGR - 1 && !wide_out, wide = lev == 0 && wide_in;
 #pragma unroll
         for (int jj = 0; jj < h; jj++) {
             const bool one = lev == 0 && NTTM_TRIVIAL_W(rlow, jj);
@@ -194,7 +228,8 @@ __device__ __forceinline__ void dit_group_mirror(double *v, int s_lo, uint32_t r
             }
 #pragma unroll
             for (int i = jj; i < R; i += 2 * h) {
-                const double u = v[i], x = one ? v[i + h] : mul_shoup(v[i + h], w.x, w.y, p);
+                const double u = dit_u(v[i], wide, p, pinv);
+                const double x = one ? dit_u(v[i + h], wide, p, pinv) : mul_shoup(v[i + h], w.x, w.y, p);
                 const double s1 = u + x, s2 = u - x;
                 v[i] = red ? reduce(s1, p, pinv) : s1;
                 v[i + h] = red ? reduce(s2, p, pinv) : s2;
@@ -204,7 +239,7 @@ __device__ __forceinline__ void dit_group_mirror(double *v, int s_lo, uint32_t r
 }
 template <int LOGR, int PTS>
 __device__ __forceinline__ void round_compute_mirror(double *v, const PassPos &pp, int s_lo, const double2 *tw, double p,
-                                                     double pinv)
+                                                     double pinv, bool wide_in = false, bool wide_out = false)
 {
     constexpr int R = 1 << LOGR, G = PTS / R;
     const int L = pp.logw + s_lo;
@@ -212,7 +247,7 @@ __device__ __forceinline__ void round_compute_mirror(double *v, const PassPos &p
     for (int g = 0; g < G; g++) {
         const uint32_t tau = (uint32_t)(g * pp.nthr + pp.t);
         const uint32_t rlow = (tau & ((1u << L) - 1)) >> pp.logw;
-        dit_group_mirror<LOGR>(v + g * R, s_lo, rlow, tw, p, pinv);
+        dit_group_mirror<LOGR>(v + g * R, s_lo, rlow, tw, p, pinv, wide_in, wide_out);
     }
 }
 

@@ -156,8 +156,8 @@ __global__ __launch_bounds__((NP << TL) / PTS) void k_small(SmallArgs a)
                 ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
                     v[sl] = xs.at(e); });)
             }
-            if (i == NR - 1 && LOGN > SW) { ROUND_SWITCH(logR, round_compute<LR, true, PTS>(v, pp, s_lo, gi, p, pinv);) }
-            else { ROUND_SWITCH(logR, round_compute_mirror<LR, PTS>(v, pp, s_lo, lt, p, pinv);) }
+            if (i == NR - 1 && LOGN > SW) { ROUND_SWITCH(logR, round_compute<LR, true, PTS>(v, pp, s_lo, gi, p, pinv, i > 0, i + 1 < NR);) }
+            else { ROUND_SWITCH(logR, round_compute_mirror<LR, PTS>(v, pp, s_lo, lt, p, pinv, i > 0, i + 1 < NR);) }
             ROUND_SWITCH(logR, for_slots<LR, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) {
                 xs.at(e) = v[sl]; });)
         }
@@ -433,8 +433,8 @@ __global__ __launch_bounds__(NP * 256) void k_segments(SegArgs a)
                 __syncthreads();
                 for_slots<4, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) { v[sl] = xs.at(e); });
             }
-            if (i == NR - 1) round_compute<4, true, PTS>(v, pp, s_lo, gi, p, pinv);
-            else round_compute_mirror<4, PTS>(v, pp, s_lo, lt, p, pinv);
+            if (i == NR - 1) round_compute<4, true, PTS>(v, pp, s_lo, gi, p, pinv, true, false);
+            else round_compute_mirror<4, PTS>(v, pp, s_lo, lt, p, pinv, i > 0, true);
             for_slots<4, PTS, true>(pp, s_lo, [&](int sl, uint32_t e, uint32_t, uint32_t, uint32_t) { xs.at(e) = v[sl]; });
         }
         /* the segment's x limbs are requested, the next one's operand limbs drawn into the L2 (a word of every line; in registers
