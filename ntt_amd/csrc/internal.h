@@ -92,12 +92,14 @@ struct PassJob {
     const LoadDesc *ldesc; int which;
     int do_in_scale, dfr_do_scale;
     uint64_t batch;                 /* transforms in this job's plane */
-    uint32_t block0, blocks;        /* a streamed pass: the job's blocks in the launch */
+    uint32_t blocks;                /* a streamed pass: the job's blocks in the launch, from JobSet::block0 on */
     double p, pinv;
     TwTables tw;
     double2 in_scale;               /* of the limbs (do_in_scale) or of the deferred twiddles (dfr_do_scale) */
 };
-struct JobSet { int n; PassJob j[NTTM_MAX_JOBS]; };
+/* block0: a streamed pass's first block of each job (beyond the jobs: no block's number), in one piece so that a block reads
+ * them with one load */
+struct JobSet { int n; uint32_t block0[NTTM_MAX_JOBS]; PassJob j[NTTM_MAX_JOBS]; };
 /* the double-fused pass's jobs: one per prime */
 struct FusedJob {
     double *x, *xb;                 /* A's and B's planes */

@@ -276,11 +276,17 @@ __device__ __forceinline__ void lds_barrier()
 template <int MODE, int GM, int GW, bool U = false>
 __global__ __launch_bounds__(STREAM_T) void k_pass_stream(PassArgs a, JobSet js)
 {
-    uint32_t job = 0;
-    while ((int)job + 1 < js.n && blockIdx.x >= js.j[job + 1].block0) job++;
+    /* (a loop over the jobs, a load in each step, took 1.4 us of a short pass: 8.6 against 7.4 us for 2^15 points) */
+    uint32_t job = 0, first = 0;
+#pragma unroll
+    for (int k = 1; k < NTTM_MAX_JOBS; k++) {
+        const uint32_t f = js.block0[k];
+        const bool past = blockIdx.x >= f;
+        job += past; first = past ? f : first;
+    }
     apply_job(a, js, job);
     stamp_clock(a.stamp);
-    const uint32_t blk = blockIdx.x - js.j[job].block0, nblk = js.j[job].blocks;
+    const uint32_t blk = blockIdx.x - first, nblk = js.j[job].blocks;
     hold(a.x); hold(a.pk.p); hold(a.pk.pinv);
     const uint32_t ntiles = (uint32_t)((a.batch << a.logn) >> (GM + GW));
     constexpr bool INV = MODE == PM_INV, LIMB = MODE == PM_FWD_LIMB;
@@ -877,9 +883,10 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
         uint32_t nb = 0;
         for (int k = 0; k < js.n; k++) {
             const uint64_t t = plan_tiles(g, a.logn, js.j[k].batch), share = std::max<uint64_t>(1, (uint64_t)g_ncu * t / all);
-            js.j[k].block0 = nb; js.j[k].blocks = (uint32_t)std::min(t, share);
+            js.block0[k] = nb; js.j[k].blocks = (uint32_t)std::min(t, share);
             nb += js.j[k].blocks;
         }
+        for (int k = js.n; k < NTTM_MAX_JOBS; k++) js.block0[k] = 0xffffffffu;
         const dim3 sgrid(nb);
 #define NTTM_STREAM_LAUNCH(M, W) \
         if (u && mode == PM_FWD) hipLaunchKernelGGL((k_pass_stream<PM_FWD, M, W, true>), sgrid, dim3(STREAM_T), 0, s, b, js); \
