@@ -132,6 +132,7 @@ struct Ctx {
     char *stage; size_t stage_bytes;         /* device copies of host-resident operands and results */
     size_t stage_chunk;                      /* staged bytes per sub-batch of a batch */
     char *chk; size_t chk_bytes;             /* device scratch of the residue post-condition */
+    uint64_t *xc; size_t xc_limbs;           /* copies of the x operands that lie under their results */
     char *bounce; size_t bounce_half;        /* pinned bounce buffer of the host copies: two halves */
     char *dl; size_t dl_half; hipEvent_t dlev[2];   /* pinned halves of the large downloads (nttm_copy_to_host) */
     hipEvent_t bev[2]; int bev_live[2];      /* the last copy through each half */
@@ -495,6 +496,7 @@ extern "C" void nttm_shutdown(void)
     if (g.stamps) (void)hipHostFree(g.stamps);
     if (g.stage) (void)hipFree(g.stage);
     if (g.chk) (void)hipFree(g.chk);
+    if (g.xc) (void)hipFree(g.xc);
     if (g.bounce) (void)hipHostFree(g.bounce);
     if (g.dl) (void)hipHostFree(g.dl);
     for (int k = 0; k < 2; k++) if (g.dlev[k]) (void)hipEventDestroy(g.dlev[k]);
@@ -853,13 +855,16 @@ static double seg_launch_us(uint64_t n, uint32_t per, uint64_t S)
 }
 static bool seg_forced(void) { return g_pieces_points == 1 << 12; }
 static bool seg_allowed(uint64_t S) { return S && !g_no_small && (g_pieces_points < 0 || seg_forced()); }
-/* the result shares memory with an operand: segments, which write limbs while others still read theirs, are not for it (the
- * passes read every operand limb before the first result limb is written) */
-static bool result_over_operands(const uint64_t *c, size_t nc, const uint64_t *a, size_t na, const uint64_t *b, size_t nb,
-                                 const uint64_t *x, size_t nx)
+/* the result shares memory with a or b: segments, which write limbs while others still read theirs, are not for it (the
+ * passes read every limb of both before the first result limb is written; an x under the result is read from a copy,
+ * x_apart) */
+static bool shares(const uint64_t *c, size_t nc, const uint64_t *p, size_t n)
 {
-    auto hit = [&](const uint64_t *p, size_t n) { return p && n && (uintptr_t)p < (uintptr_t)(c + nc) && (uintptr_t)c < (uintptr_t)(p + n); };
-    return hit(a, na) || hit(b, nb) || hit(x, nx);
+    return p && n && (uintptr_t)p < (uintptr_t)(c + nc) && (uintptr_t)c < (uintptr_t)(p + n);
+}
+static bool result_over_operands(const uint64_t *c, size_t nc, const uint64_t *a, size_t na, const uint64_t *b, size_t nb)
+{
+    return shares(c, nc, a, na) || shares(c, nc, b, nb);
 }
 /* one product: the segments of a workgroup that give it the least time, if that is below `most`; else 0 */
 static uint32_t choose_segments(size_t nc, size_t blen, double most)
@@ -883,7 +888,7 @@ static bool batch_segments(const nttm_prod &q, int logn, int r3)
     const size_t alen = std::max(na, nb), blen = std::min(na, nb);
     const uint64_t S = nttm_seg_len(blen);
     if (!seg_allowed(S) || (uint64_t)na + nb > 0xffffffffULL) return false;
-    if (result_over_operands(q.c, na + nb + (q.x ? 1 : 0), q.a, na, q.b, nb, q.x, q.x ? q.nx : 0)) return false;
+    if (result_over_operands(q.c, na + nb + (q.x ? 1 : 0), q.a, na, q.b, nb)) return false;
     if (seg_forced()) return true;
     if (small_len(logn, r3) || alen < 2 * blen) return false;
     const double segs = ceil((double)(na + nb) / (double)S);
@@ -996,7 +1001,7 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
         return 0;
     }
     if (!nc) return 0;
-    CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws, !result_over_operands(c, nc, a, na, b, nb, x, x ? nx : 0)));
+    CoreLayout L; RCK(core_layout(na, nb, x != nullptr, wcut, &L, !ws, !result_over_operands(c, nc, a, na, b, nb)));
     uint32_t *ctl = (uint32_t *)((char *)g.hpin + 128 * slot + 96);
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.plane = L.plane; hd.ncoef = L.ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
@@ -1265,6 +1270,76 @@ static int mul_grid(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     HIPCK(hipStreamSynchronize(s));
     return 0;
 }
+/* ---- a result over its own x -------------------------------------------------------------------------------------------
+ * The CRT's kernels read x while they write c, and a run's or block's first lanes need the limbs of x just before their
+ * own, which another run may have overwritten where the two share memory (the quotient of such a limb differs at every
+ * second edge).  Such an x is copied ahead into memory of the library's and read from there; an empty operand's c = x and the
+ * residue post-condition, which reads x again, take the copy too. */
+#define XCOPY_MAX 32
+struct XCopy { const uint64_t *src[XCOPY_MAX]; uint64_t *dst[XCOPY_MAX]; uint64_t n[XCOPY_MAX]; };
+__global__ __launch_bounds__(256) void k_copy_x(XCopy a)
+{
+    const uint64_t *src = a.src[blockIdx.y], n = a.n[blockIdx.y];
+    uint64_t *dst = a.dst[blockIdx.y];
+    for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (uint64_t)gridDim.x * 256) dst[k] = src[k];
+}
+static int xc_need(size_t limbs)
+{
+    if (limbs <= g.xc_limbs) return 0;
+    if (g.xc) { HIPCK(hipDeviceSynchronize()); HIPCK(hipFree(g.xc)); g.xc = nullptr; g.xc_limbs = 0; }
+    if (hipMalloc(&g.xc, limbs * 8) != hipSuccess) { (void)hipGetLastError(); return nttm_fail(NTTM_ENOMEM, "copy of x: %zu limbs", limbs); }
+    g.xc_limbs = limbs;
+    return 0;
+}
+/* whether a product's x is to be copied.  The one-kernel products read all of x before they write (every: copied too, for a
+ * caller that may give them another length) */
+static bool x_to_copy(const nttm_prod &q, bool every)
+{
+    const size_t nc = q.na + q.nb + (q.x ? 1 : 0);
+    if (!shares(q.c, nc, q.x, q.nx)) return false;
+    if (every || g.cfg.check || !q.na || !q.nb) return true;
+    int logn, r3;
+    choose_len(q.na + q.nb - 1, &logn, &r3);
+    return !small_len(logn, r3) || !fits_one(q.na, q.nb, nc);
+}
+/* limbs of the copies of N products; their launches, the copies back to back from dst, and the products with their x there */
+static size_t x_limbs(const nttm_prod *P, size_t N, bool every)
+{
+    size_t n = 0;
+    for (size_t i = 0; i < N; i++) if (x_to_copy(P[i], every)) n += P[i].nx;
+    return n;
+}
+static int copy_x(nttm_prod *Q, size_t N, bool every, uint64_t *dst, hipStream_t s)
+{
+    XCopy a;
+    int k = 0;
+    uint64_t most = 0;
+    auto flush = [&]() -> int {
+        if (!k) return 0;
+        const uint64_t blocks = std::min<uint64_t>((most + 2047) / 2048, 1024);   /* (8 limbs a thread) */
+        hipLaunchKernelGGL(k_copy_x, dim3((unsigned)blocks, (unsigned)k), dim3(256), 0, s, a);
+        k = 0; most = 0;
+        return nttm_hip_check(hipGetLastError(), "k_copy_x launch");
+    };
+    for (size_t i = 0; i < N; i++) {
+        if (!x_to_copy(Q[i], every)) continue;
+        a.src[k] = Q[i].x; a.dst[k] = dst; a.n[k] = Q[i].nx; k++;
+        most = std::max<uint64_t>(most, Q[i].nx);
+        Q[i].x = dst; dst += Q[i].nx;
+        if (k == XCOPY_MAX) RCK(flush());
+    }
+    return flush();
+}
+/* Q: left empty, or (an x under its result) P with those x operands copied */
+static int x_apart(const nttm_prod *P, size_t N, std::vector<nttm_prod> &Q, hipStream_t s)
+{
+    const size_t n = x_limbs(P, N, false);
+    if (!n) return 0;
+    RCK(xc_need(n));
+    Q.assign(P, P + N);
+    return copy_x(Q.data(), N, false, g.xc, s);
+}
+
 /* one transform when it holds the product, else the grid */
 static int mul_any(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b, size_t nb, const uint64_t *x, size_t nx,
                    hipStream_t s, size_t lowcut = 0, size_t w = SIZE_MAX)
@@ -1280,10 +1355,13 @@ static int mul_any(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b,
 static int mul_full(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b, size_t nb, const uint64_t *x, size_t nx,
                     hipStream_t s, size_t lowcut = 0, size_t w = SIZE_MAX)
 {
-    RCK(mul_any(c, a, na, b, nb, x, nx, s, lowcut, w));
-    if (!g.cfg.check || w != SIZE_MAX) return 0;
     nttm_prod q; memset(&q, 0, sizeof q);
     q.a = a; q.na = na; q.b = b; q.nb = nb; q.c = c; q.x = x; q.nx = x ? nx : 0;
+    std::vector<nttm_prod> Q;
+    RCK(x_apart(&q, 1, Q, s));
+    if (!Q.empty()) { q = Q[0]; x = q.x; }
+    RCK(mul_any(c, a, na, b, nb, x, nx, s, lowcut, w));
+    if (!g.cfg.check || w != SIZE_MAX) return 0;
     return check_products(&q, 1, s);
 }
 
@@ -1554,10 +1632,9 @@ template <typename F> static bool group_lengths(const GroupBuild &gb, const uint
     return bad;
 }
 
-/* the batch on device memory (every pointer of P classed MEM_DEV) */
-static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
+/* the batch on device memory (every pointer of P classed MEM_DEV), no x to be copied */
+static int mul_batch_apart(nttm_prod *P, size_t N, hipStream_t s)
 {
-    if (!N) return 0;
     /* validate; zero-operand products are written directly */
     size_t mn_max = 0;
     /* groups by transform length: 2^logn at [logn], 3 2^logn at [NTTM_LOGN_MAX + 1 + logn] */
@@ -1662,6 +1739,17 @@ static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
         q.ncn = n;
     }
     return g.cfg.check ? check_products(P, N, s) : 0;
+}
+
+static int mul_batch_dev(nttm_prod *P, size_t N, hipStream_t s)
+{
+    if (!N) return 0;
+    std::vector<nttm_prod> Q;
+    RCK(x_apart(P, N, Q, s));
+    if (Q.empty()) return mul_batch_apart(P, N, s);
+    const int rc = mul_batch_apart(Q.data(), N, s);
+    for (size_t i = 0; i < N; i++) P[i].ncn = Q[i].ncn;
+    return rc;
 }
 
 /* ---- host-resident operands: staging through HBM -----------------------------------------------------------------------
@@ -2164,8 +2252,8 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
         RCK(prod_kinds(mm, q.a, q.na, q.b, q.nb, q.x, q.nx, q.c, nc, ki, i));
         if (any_host(ki)) return nttm_fail(NTTM_EINVAL, "nttm_mul_each_async: product %zu: host memory (device memory only)", i);
         if (q.na && q.nb && fits_one(q.na, q.nb, nc)) {                /* (with every prime's B plane) */
-            CoreLayout L; 
-            RCK(core_layout(q.na, q.nb, q.x != nullptr, SIZE_MAX, &L, true, !result_over_operands(q.c, nc, q.a, q.na, q.b, q.nb, q.x, q.x ? q.nx : 0)));
+            CoreLayout L;
+            RCK(core_layout(q.na, q.nb, q.x != nullptr, SIZE_MAX, &L, true, !result_over_operands(q.c, nc, q.a, q.na, q.b, q.nb)));
             ws_max = std::max(ws_max, L.bytes);
         }
     }
@@ -2174,8 +2262,11 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
     RCK(hpin_need(128 * N + 8 * N + 256));
     RCK(stage_need(off_ncn + N * 8));
     std::vector<char> fl(N, 0);                                  /* 1: flags in pinned slot i */
+    std::vector<nttm_prod> Q;
+    RCK(x_apart(P, N, Q, s));
+    const nttm_prod *S = Q.empty() ? P : Q.data();
     for (size_t i = 0; i < N; i++) {
-        const nttm_prod &q = P[i];
+        const nttm_prod &q = S[i];
         const size_t nc = q.na + q.nb + (q.x ? 1 : 0);
         if (q.na && q.nb && !fits_one(q.na, q.nb, nc)) RCK(mul_any(q.c, q.a, q.na, q.b, q.nb, q.x, q.nx, s));
         else { RCK(mul_core(q.c, q.a, q.na, q.b, q.nb, q.x, q.nx, s, SIZE_MAX, nullptr, 0, 0, i)); fl[i] = 1; }
@@ -2192,7 +2283,7 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
             return nttm_fail(NTTM_ECHECK, "product %zu: crt: non-zero carry beyond the top limb (wrong residues)", i);
         P[i].ncn = hn[i];
     }
-    return g.cfg.check ? check_products(P, N, s) : 0;
+    return g.cfg.check ? check_products(S, N, s) : 0;
 }
 
 /* ---- the binary-splitting product tree ----------------------------------------------------------------------------------- */
@@ -2669,6 +2760,13 @@ extern "C" int nttm_crt(uint64_t *c, size_t nc, const uint64_t *const *planes, i
     const size_t pbytes = copy ? align_up((size_t)np * ncoef * 8, 256) : 0;
     const size_t crt_words = nttm_crt_scratch_words(nttm_crt_blocks(nc));
     RCK(ws_need(pbytes + 256 + crt_words * 4 + 256));
+    if (shares(c, nc, x, nx)) {                                  /* (x_apart) */
+        RCK(xc_need(nx));
+        nttm_prod q; memset(&q, 0, sizeof q);
+        q.na = nc; q.c = c; q.x = x; q.nx = nx;
+        RCK(copy_x(&q, 1, true, g.xc, s));
+        x = q.x;
+    }
     CrtDesc hd; memset(&hd, 0, sizeof hd);
     hd.ncoef = ncoef; hd.x = x; hd.nx = x ? nx : 0; hd.c = c; hd.nc = nc; hd.first_block = 0;
     if (copy) {
@@ -2770,6 +2868,7 @@ struct nttm_batch_plan {
     size_t off_z = 0;
     char *blob = nullptr;
     size_t blob_bytes = 0;
+    uint64_t *xc = nullptr;                                      /* the copies of x operands under their results */
     uint64_t *hstage = nullptr;                                  /* pinned: the lengths and flags, written by the runs */
     size_t hstage_words = 0;
     hipStream_t cs = nullptr;
@@ -2787,6 +2886,7 @@ static void plan_free(nttm_batch_plan *pl)
     if (pl->graph) (void)hipGraphDestroy(pl->graph);
     if (pl->cs) (void)hipStreamDestroy(pl->cs);
     if (pl->blob) (void)hipFree(pl->blob);
+    if (pl->xc) (void)hipFree(pl->xc);
     if (pl->hstage) (void)hipHostFree(pl->hstage);
     delete pl;
 }
@@ -2923,6 +3023,18 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
     int rc = choose_np(mn_max ? mn_max : 1, &pl->np);
     if (rc) return fail(rc);
     const int np = pl->np;
+    /* an x under its result: every run copies it first (x_apart) */
+    const nttm_prod *const P0 = P;
+    std::vector<nttm_prod> Q;
+    if (const size_t n = x_limbs(P, N, true)) {
+        if (hipMalloc(&pl->xc, n * 8) != hipSuccess) {
+            (void)hipGetLastError(); pl->xc = nullptr;
+            return fail(nttm_fail(NTTM_ENOMEM, "plan: copies of x: %zu limbs", n));
+        }
+        Q.assign(P, P + N);
+        if ((rc = copy_x(Q.data(), N, true, pl->xc, s))) return fail(rc);
+        P = Q.data();
+    }
     /* the schedule: per class k the radix-3 subset (products of at most 3 2^(k-2) coefficients) either takes 3 2^(k-2)
      * points or stays at 2^k; per group the tile and points per thread */
     TuneBuf tb;
@@ -3001,6 +3113,10 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
     g_prof_on = 0;                                               /* no event records inside the graph */
     if ((rc = nttm_hip_check(hipStreamBeginCapture(pl->cs, hipStreamCaptureModeRelaxed), "begin capture"))) { g_prof_on = prof0; return fail(rc); }
     uint64_t *hw = pl->hstage;
+    if (pl->xc) {
+        Q.assign(P0, P0 + N);
+        rc = copy_x(Q.data(), N, true, pl->xc, pl->cs);
+    }
     for (size_t i = 0; i < pl->gb.size() && !rc; i++) {
         const uint64_t cnt = pl->gb[i].cnt;
         rc = group_launch(pl->gb[i], np, A, pl->blob + pl->goff[i], pl->cs, hw, (uint32_t *)(hw + cnt));
