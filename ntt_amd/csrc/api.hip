@@ -1414,13 +1414,24 @@ struct GroupBuild {
     size_t planes_bytes = 0;                                     /* (np cnt + cnt_b) n doubles */
     size_t off_cd = 0, off_ld = 0, off_ldb = 0, off_bmap = 0, off_ctl = 0, off_ncn = 0, off_crt = 0, desc_bytes = 0;
 };
-/* products of a group that run together (a chunk), and whether all primes of a chunk share a launch per pass */
-static uint64_t chunk_products(uint64_t n) { return std::max<uint64_t>(1, g_chunk_points / n); }
-static bool chunk_merged(uint64_t n, uint64_t cn) { return n * cn <= std::max(g_chunk_points, g_par_points); }
-static size_t chunk_planes_bytes(int np, uint64_t n, uint64_t cnt)
+/* how a group of cnt products of n points runs: the products that run together (a chunk; the next one reuses their planes), and
+ * whether all primes of a chunk share a launch per pass, each with a B plane of its own.  Under a cap on the planes' bytes
+ * (0: none) fewer products a chunk, and where not even one has room for 2 np planes, prime after prime through np + 1 */
+struct GroupShape {
+    uint64_t cn;
+    bool merged;
+    size_t bytes(int np, uint64_t n) const { return (size_t)(merged ? 2 * np : np + 1) * cn * n * 8; }
+};
+static GroupShape group_shape(int np, uint64_t n, uint64_t cnt, size_t cap)
 {
-    const uint64_t cn = std::min(cnt, chunk_products(n));
-    return (size_t)(chunk_merged(n, cn) ? 2 * np : np + 1) * cn * n * 8;
+    GroupShape h;
+    h.cn = std::min(cnt, std::max<uint64_t>(1, g_chunk_points / n));
+    h.merged = n * h.cn <= std::max(g_chunk_points, g_par_points);
+    if (!cap || h.bytes(np, n) <= cap) return h;
+    const uint64_t room = cap / (n * 8);                         /* planes of one product */
+    h.merged = h.merged && room >= 2 * (uint64_t)np;
+    h.cn = std::max<uint64_t>(1, std::min(h.cn, room / (h.merged ? 2 * np : np + 1)));
+    return h;
 }
 #define SEG_CLASS (2 * (NTTM_LOGN_MAX + 1) + 12)   /* the group class of products in segments of 2^12 points (r3 = 2) */
 static uint64_t seg_blocks(const nttm_prod &q)
@@ -1483,7 +1494,7 @@ static void group_build_segments(GroupBuild &gb, const nttm_prod *P, const std::
     group_offsets(gb);
 }
 static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<size_t> &G, int np, int r3, int logn,
-                        int tile, int pts)
+                        int tile, int pts, size_t cap = 0)
 {
     gb.r3 = r3; gb.logn = logn; gb.tile = tile; gb.pts = pts;
     if (r3 == 2) { group_build_segments(gb, P, G); return; }
@@ -1493,8 +1504,9 @@ static void group_build(GroupBuild &gb, const nttm_prod *P, const std::vector<si
     gb.crt_per = gb.inv_m ? NTTM_CRT_RUNS : n <= 1024 ? 1 : 8;    /* (products of at most n + 1 limbs: 256-limb blocks) */
     gb.cd.assign(cnt, CrtDesc()); gb.ld.assign(cnt, LoadDesc()); gb.ldb.clear(); gb.bmap.clear(); gb.chunk.clear();
     gb.small = small_len(logn, r3);                              /* one kernel, no planes and no CRT blocks */
-    const uint64_t cmax = gb.small ? cnt : chunk_products(n);
-    gb.merged = chunk_merged(n, std::min(cnt, cmax));
+    const GroupShape shape = group_shape(np, n, cnt, cap);
+    const uint64_t cmax = gb.small ? cnt : shape.cn;
+    gb.merged = shape.merged;
     for (uint64_t c0 = 0; c0 < cnt; c0 += cmax) gb.chunk.push_back({c0, std::min(cmax, cnt - c0), 0, 0, 0, 0, 0.0});
     for (GroupBuild::Chunk &ch : gb.chunk) {
         ch.blk0 = gb.nblk;
@@ -1664,6 +1676,7 @@ static int mul_batch_apart(nttm_prod *P, size_t N, hipStream_t s)
      * precedes, on the caller's), and the lengths and flags are written straight to pinned memory.  One
      * synchronization at the end.  (Waiting per group left the device idle for 0.9 of the 4096 leaves' 6.6 ms.) */
     std::vector<size_t> order;
+    const size_t cap = g.cfg.workspace_bytes;
     size_t planes = 256, desc = 0, img = 0, words = 0;
     auto radix = [](size_t gi) { return (int)(gi / (NTTM_LOGN_MAX + 1)); };
     auto pts = [&](size_t gi) { return (uint64_t)(radix(gi) == 1 ? 3 : radix(gi) ? 8 : 1) << (gi % (NTTM_LOGN_MAX + 1)); };   /* (about 8 segments) */
@@ -1675,7 +1688,7 @@ static int mul_batch_apart(nttm_prod *P, size_t N, hipStream_t s)
         const uint64_t n = pts(gi), cnt = G.size();
         uint64_t blk = 0;
         for (size_t i : G) blk += r3 == 2 ? seg_blocks(P[i]) : prod_crt_blocks(logn, r3, n, P[i].na + P[i].nb + (P[i].x ? 1 : 0));
-        if (r3 != 2 && !small_len(logn, r3)) planes = std::max(planes, chunk_planes_bytes(np, n, cnt));
+        if (r3 != 2 && !small_len(logn, r3)) planes = std::max(planes, group_shape(np, n, cnt, cap).bytes(np, n));
         const size_t im = align_up(cnt * sizeof(CrtDesc), 256) + 2 * align_up(cnt * sizeof(LoadDesc), 256) +
                           align_up((r3 ? 3 : 1) * cnt * 4, 256) + 512;
         img += im;
@@ -1701,7 +1714,7 @@ static int mul_batch_apart(nttm_prod *P, size_t N, hipStream_t s)
             const std::vector<size_t> &G = groups[order[k]];
             GroupBuild &gb = gbs[k];
             const int logn = (int)(order[k] % (NTTM_LOGN_MAX + 1));
-            group_build(gb, P, G, np, radix(order[k]), logn, g.cfg.tile_log, batch_pts(logn));
+            group_build(gb, P, G, np, radix(order[k]), logn, g.cfg.tile_log, batch_pts(logn), cap);
             if (dpos + gb.desc_bytes > g.tdesc_bytes || ipos + gb.off_ncn > img || gb.planes_bytes > g.ws_bytes)
                 return nttm_fail(NTTM_EINVAL, "internal: a batch group exceeds its sizing");
             char *dbase = g.tdesc + dpos;
@@ -2359,6 +2372,7 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
     const int nlev = (int)len.size() - 1;                        /* levels of products */
     /* resources for every level, sized before the first launch: pools by level parity, planes, descriptors; each
      * product's length class kept for its level's grouping (-1: an empty operand) */
+    const size_t cap = g.cfg.workspace_bytes;
     size_t pool_max[2] = {1, 1}, planes_max = 0, desc_total = 0, img_total = 0, ngroups = 0;
     std::vector<int> lev_np(nlev + 1, 3);
     std::vector<std::vector<int8_t>> keys(nlev + 1);
@@ -2398,7 +2412,7 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
             if (logn > NTTM_LOGN_MAX) return 1;
             for (uint64_t c0 = 0; c0 < cnt_all; c0 += TREE_CHUNK) {   /* the group's chunks (below) */
                 const uint64_t cn = std::min<uint64_t>(TREE_CHUNK, cnt_all - c0), tb = r3 ? 3 * cn : cn;
-                if (!small_len(logn, r3)) planes_max = std::max(planes_max, chunk_planes_bytes(lev_np[k], npts, cn));
+                if (!small_len(logn, r3)) planes_max = std::max(planes_max, group_shape(lev_np[k], npts, cn, cap).bytes(lev_np[k], npts));
                 const size_t img = align_up(cn * sizeof(CrtDesc), 256) + 2 * align_up(cn * sizeof(LoadDesc), 256) +
                                    align_up(tb * 4, 256) + 256 + 256;
                 img_total += img;
@@ -2479,7 +2493,7 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
                 const std::vector<size_t> G(Gall.begin() + c0, Gall.begin() + std::min(Gall.size(), c0 + TREE_CHUNK));
                 const int r3 = gi > NTTM_LOGN_MAX, logn = gi % (NTTM_LOGN_MAX + 1);
                 GroupBuild gb;
-                group_build(gb, prods.data(), G, lev_np[k], r3, logn, g.cfg.tile_log, batch_pts(logn));
+                group_build(gb, prods.data(), G, lev_np[k], r3, logn, g.cfg.tile_log, batch_pts(logn), cap);
                 if (dpos + gb.desc_bytes > g.tdesc_bytes || ipos + gb.off_ncn > img_total || gb.planes_bytes > g.ws_bytes)
                     return nttm_fail(NTTM_EINVAL, "internal: tree plan exceeds its sizing (level %d)", k);
                 char *img = g.tpin + ipos, *dbase = g.tdesc + dpos;
