@@ -241,7 +241,10 @@ int nttm_crt(uint64_t *c, size_t nc, const uint64_t *const *planes, int np, size
              const uint64_t *x, size_t nx, void *stream);
 
 /* device-side time of the phases of the last nttm_mul / nttm_mul_add (ms): the forward transforms of b (limb load
- * fused), those of a with the fused pointwise product and the inverse transforms, the CRT */
+ * fused), those of a with the fused pointwise product and the inverse transforms, the CRT.  Where a launch holds more than
+ * one of them its time is shared out: the forward passes of both operands by the points each transforms, a product in
+ * segments as its first workgroup's time was.  An uneven product in pieces or segments, which transforms its shorter operand
+ * once, counts that one as b.  The CRT of 2^13 to 2^16 points includes the last inverse pass */
 int nttm_last_phase_ms(double *b_fwd_ms, double *a_fwd_pw_inv_ms, double *crt_ms);
 
 /* ---- live kernel timing (no reference counterpart; the reference times phases with events, E/rns_mul.c:548-587) ---- */

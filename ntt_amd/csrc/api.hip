@@ -141,6 +141,7 @@ struct Ctx {
     hipEvent_t pev[2 * NTTM_MAX_PRIMES];      /* around B's transform of each prime (phase times of nttm_mul) */
     double last_ms[3];
     uint64_t *stamps; int last_stamped;      /* pinned: the device clock at the last short product's phase boundaries */
+    double last_b;                           /* B's share of its joint forward launches (0: a product in segments) */
 };
 static Ctx g;
 static uint64_t g_init_count;
@@ -1012,7 +1013,7 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
                       sync ? g.stamps : nullptr));
         if (!sync) return 0;
         HIPCK(hipStreamSynchronize(s));
-        g.last_stamped = 1;
+        g.last_stamped = 1; g.last_b = 0.5;
         return ctl[1] & 1 ? nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond the top limb (wrong residues)") : 0;
     }
     if (ws) {
@@ -1026,14 +1027,12 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
         const LoadDesc ld{sw ? b : a, sw ? nb : na, sw ? a : b, sw ? na : nb};
         hd.step = L.step; hd.over = L.seg_per;
         uint64_t *st = sync ? g.stamps : nullptr;
-        if (st) st[0] = ~(uint64_t)0;
         RCK(run_segments(L.np, nullptr, nullptr, &ld, &hd, 1, (L.cnt + L.seg_per - 1) / L.seg_per, (uint32_t *)ws, ctl, s,
-                         8.0 * (double)(na + nb + nc + hd.nx), st ? st + 1 : nullptr));
-        RCK(nttm_crt_launch_carry(nullptr, &hd, 1, L.cnt, (uint32_t *)ws, ctl, s, NTTM_CRT_SEGS, st ? st + 2 : nullptr));
-        if (st) st[3] = 0;
+                         8.0 * (double)(na + nb + nc + hd.nx), st));
+        RCK(nttm_crt_launch_carry(nullptr, &hd, 1, L.cnt, (uint32_t *)ws, ctl, s, NTTM_CRT_SEGS, st ? st + 4 : nullptr));
         if (!sync) return 0;
         HIPCK(hipStreamSynchronize(s));
-        g.last_stamped = 1;
+        g.last_stamped = 1; g.last_b = 0.0;
         return ctl[1] & 1 ? nttm_fail(NTTM_ECHECK, "crt: non-zero carry beyond the top limb (wrong residues)") : 0;
     }
     double *A = (double *)ws, *Bp = A + (size_t)L.np * L.plane;
@@ -1070,6 +1069,7 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     if (!sync) return 0;
     HIPCK(hipStreamSynchronize(s));
     g.last_stamped = stamps != nullptr;
+    g.last_b = L.cnt ? 1.0 / (double)(1 + L.cnt) : 0.5;          /* (the pieces share one transform of B) */
     if (events) {
         float ms, tb = 0, t;
         for (int i = 0; i < L.np; i++) { HIPCK(hipEventElapsedTime(&t, g.pev[2 * i], g.pev[2 * i + 1])); tb += t; }
@@ -1386,8 +1386,13 @@ extern "C" int nttm_last_phase_ms(double *f, double *i, double *c)
         if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g.dev) != hipSuccess || khz <= 0) { (void)hipGetLastError(); khz = 100000; }
         const uint64_t *t = g.stamps;
         auto ms = [&](uint64_t a, uint64_t b) { return b > a ? (double)(b - a) / khz : 0.0; };
-        const double fwd = ms(t[0], t[1]);                       /* both operands' forward passes, one launch each */
-        g.last_ms[0] = 0.5 * fwd; g.last_ms[1] = 0.5 * fwd + ms(t[1], t[2]); g.last_ms[2] = ms(t[2], t[3]);
+        if (g.last_b > 0) {
+            const double fwd = ms(t[0], t[1]);                   /* both operands' forward passes, one launch each */
+            g.last_ms[0] = g.last_b * fwd; g.last_ms[1] = (1.0 - g.last_b) * fwd + ms(t[1], t[2]); g.last_ms[2] = ms(t[2], t[3]);
+        } else {                                                 /* segments: the launch shared out as its first workgroup's time was */
+            const double all = ms(t[0], t[4]), own = ms(t[0], t[2]), unit = own > 0 ? all / own : 0.0;
+            g.last_ms[0] = unit * ms(t[0], t[1]); g.last_ms[2] = unit * ms(0, t[3]); g.last_ms[1] = all - g.last_ms[0] - g.last_ms[2];
+        }
     }
     if (f) *f = g.last_ms[0];
     if (i) *i = g.last_ms[1];

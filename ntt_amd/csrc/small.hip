@@ -342,7 +342,8 @@ struct SegArgs {
     LoadDesc ld1; CrtDesc cd1;
     uint64_t nprod;
     uint32_t *status, *ctl;
-    uint64_t *stamps;
+    uint64_t *stamps;                           /* or null: block 0's clock at its start, after B's transforms and at its end, and
+                                                 * the time it spent on digits, limbs and carries */
     const double2 *stage[NTTM_MAX_PRIMES], *istage[NTTM_MAX_PRIMES];
     double2 ninv[NTTM_MAX_PRIMES];
     CrtConst cc;
@@ -414,6 +415,9 @@ __global__ __launch_bounds__(NP * 256) void k_segments(SegArgs a)
     const double2 ninv = a.ninv[pi];
 #pragma unroll
     for (int sl = 0; sl < PTS; sl++) bv[sl] = mul_shoup(v[sl], ninv.x, ninv.y, p);
+    const bool clk = a.stamps && blockIdx.x == 0;
+    uint64_t crt_ticks = 0;
+    if (clk) stamp_clock(a.stamps + 1);
 
     __syncthreads();                                                 /* B's last LDS reads before A's first writes */
     for (uint32_t seg = seg0; seg < seg1; seg++) {
@@ -459,6 +463,7 @@ __global__ __launch_bounds__(NP * 256) void k_segments(SegArgs a)
         }
         if (tid == 0) s_err = 0;
         __syncthreads();
+        if (clk) crt_ticks -= wall_clock64();
         const int64_t c0 = first(seg);
         for (int e = tid; e < N; e += NTH) {
             if (e < nb - 1) continue;                                /* (wrapped coefficients: never read) */
@@ -545,7 +550,9 @@ __global__ __launch_bounds__(NP * 256) void k_segments(SegArgs a)
         __syncthreads();                                             /* (the digits are read, s_err is stored) */
         if (tid == 0)
             a.status[d.first_block + seg] = ((uint32_t)(C0 >> nw) & 1u) | ((uint32_t)(C1 >> nw) & 1u) << 1 | s_err | (seg ? 0u : CRT_ST_FIRST);
+        if (clk) crt_ticks += wall_clock64();
     }
+    if (clk) { stamp_clock(a.stamps + 2); if (threadIdx.x == 0) a.stamps[3] = crt_ticks; }
 }
 
 /* limbs of a segment for a short operand of nb limbs (whole words; 0: too long a one) */

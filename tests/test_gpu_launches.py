@@ -108,6 +108,36 @@ def test_phase_times(schedule, n, par):
         assert all(p >= 0 for p in ph) and 0 < sum(ph) <= wall + 0.03
 
 
+# pieces (NTTM_PIECES points), segments, by the rule
+@pytest.mark.parametrize("points,na,nb", [(1 << 13, 1 << 18, 1), (None, 1000000, 1000), (1 << 12, 30011, 2100)])
+def test_phase_times_uneven(schedule, points, na, nb):
+    """an uneven product's short operand is transformed once (here for at most a 64th of the points, or in every workgroup of
+    segments): its phase is above 0 and, in pieces, below a 20th of the whole; every phase has a share"""
+    import time
+    import torch
+    if points:
+        os.environ["NTTM_PIECES"] = str(points)
+    try:
+        lib = schedule()
+    finally:
+        os.environ.pop("NTTM_PIECES", None)
+    a, s = O.gen_limbs(na, 3)
+    da, db = dev(a), dev(O.gen_limbs(nb, s)[0])
+    lib.mul(da, db)
+    for _ in range(3):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        lib.mul(da, db)
+        wall = 1e3 * (time.perf_counter() - t0)
+        ph = lib.last_phase_ms()
+        say("phases uneven", points, na, nb, ph, wall)
+        assert all(p > 0 for p in ph) and sum(ph) <= wall + 0.03
+        if nb == 1:
+            assert ph[0] < sum(ph) / 20
+        lib.mul(db, da)
+        assert all(p > 0 for p in lib.last_phase_ms())
+
+
 def _limbs(kind, n, s):
     if kind == "max":
         return np.full(n, O.B - 1, dtype=np.uint64), s
