@@ -2973,9 +2973,13 @@ static int tune_group(const nttm_prod *P, const std::vector<size_t> &G, int np, 
     }
     double best_ms = 1e30;
     hipEvent_t e0 = g.ev[0], e1 = g.ev[1];
-    for (int c = 0; c < 4; c++) {
+    /* the one-kernel products know neither tile nor points per thread: all four candidates are one launch, timed once for the
+     * choice of length, and the group keeps the configured values */
+    const bool one = small_len(logn, r3);
+    for (int c = 0; c < (one ? 1 : 4); c++) {
         GroupBuild gb;
-        group_build(gb, P, G, np, r3, logn, cand[c][0], cand[c][1]);
+        if (one) group_build(gb, P, G, np, r3, logn, g.cfg.tile_log, batch_pts(logn));
+        else group_build(gb, P, G, np, r3, logn, cand[c][0], cand[c][1]);
         const size_t off_d = align_up(gb.planes_bytes, 256);
         RCK(tb.need(off_d + gb.desc_bytes + 256));
         img.resize(gb.desc_bytes);
@@ -2993,7 +2997,7 @@ static int tune_group(const nttm_prod *P, const std::vector<size_t> &G, int np, 
             float f = 0; HIPCK(hipEventElapsedTime(&f, e0, e1));
             t = std::min(t, (double)f);
         }
-        (*ntried)++;
+        *ntried += one ? 4 : 1;
         if (t < best_ms) { best_ms = t; best = std::move(gb); }
     }
     *ms = best_ms;

@@ -146,6 +146,28 @@ def test_plan_reuses_remembered_choices(nttm):
         p3.close()
 
 
+def test_plan_times_one_kernel_group_once(nttm):
+    """products of one kernel each run alike under every candidate: one warm and two timed launches, and the plan reports
+    the configured tile and points per thread"""
+    import torch
+    a, s = O.gen_limbs(100, 3)
+    b, _ = O.gen_limbs(100, s)
+    c = [torch.empty(200, dtype=torch.int64, device="cuda") for _ in range(64)]
+    prods = nttm.make_prods([(dev(a), dev(b), None, x) for x in c])
+    say("plan one kernel")
+    default = nttm.BatchPlan(prods, autotune=False)
+    nttm.profile(True)
+    tuned = nttm.BatchPlan(prods, autotune=True)
+    launches = nttm.profile_read()
+    nttm.profile(False)
+    shape = lambda p: re.sub(r" ms=\S+", "", p.info().splitlines()[0])
+    assert launches["k_small"][0] == 3 and shape(tuned) == shape(default)
+    tuned.run()
+    assert all(np.array_equal(host(x), O.mul_school(a, b)) for x in c)
+    tuned.close()
+    default.close()
+
+
 def test_plan_leaf_workload_equals_eager(nttm):
     """the 4096-leaf workload (log-uniform lengths in [64, 65536], seeds 0x5EED0005/6) through an autotuned plan"""
     import torch
