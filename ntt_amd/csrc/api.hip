@@ -14,6 +14,7 @@
 #include <atomic>
 #include "internal.h"
 #include "plan.h"
+#include "segrule.h"
 
 int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s, const JobSet *jobs = nullptr);
 int nttm_run_fused2(const PassArgs &a, const FusedB &fb, const PassGeom &g, hipStream_t s, const FusedSet &js);
@@ -22,6 +23,7 @@ void nttm_set_pts(int pts);
 int nttm_get_pts(void);
 void nttm_set_fixed_shapes(int on);
 void nttm_set_stream(int on, int ncu);
+int nttm_ncu(void);
 #define NTTM_CRT_RUNS 0            /* the carry launch's blocks are k_inv_crt's runs, */
 #define NTTM_CRT_SEGS (-1)         /* or k_segments' segments */
 #define NTTM_FUSED_LOG 12          /* tile of the fused forward + pointwise + inverse pass (k_fused2) */
@@ -165,7 +167,7 @@ static uint64_t g_par_points = (uint64_t)1 << 24;
  * per chunk).  NTTM_CHUNK_POINTS overrides it. */
 static uint64_t g_chunk_points = (uint64_t)1 << 24;
 static int64_t g_pieces_points = -1;         /* NTTM_PIECES: 0 never in pieces, else pieces of that many points */
-static uint64_t g_inv_crt_points = (uint64_t)1 << 22;   /* the last inverse pass with the CRT (inv_crt_bits) */
+static uint64_t g_inv_crt_points = (uint64_t)1 << 22;   /* the last inverse pass with the CRT (inv_crt_bits): 2^14 points a CU */
 
 /* the workspace of nttm_mul_noalloc: a file-scope device array, one copy per GPU, held until the process ends.  Host
  * code never uses its name as an address (on the host it is a stand-in, not the device address): nttm_init looks up
@@ -462,7 +464,7 @@ extern "C" int nttm_init(int device, const nttm_config *cfg)
         g_chunk_points = c && strtoull(c, nullptr, 0) ? strtoull(c, nullptr, 0) : (uint64_t)1 << 24;
         const char *pp = getenv("NTTM_PIECES");
         g_pieces_points = pp ? (int64_t)strtoull(pp, nullptr, 0) : -1;
-        g_inv_crt_points = v && strtoull(v, nullptr, 0) ? strtoull(v, nullptr, 0) : (uint64_t)1 << 22;
+        g_inv_crt_points = v && strtoull(v, nullptr, 0) ? strtoull(v, nullptr, 0) : (uint64_t)nttm_ncu() << 14;
     }
     {
         const char *e = getenv("NTTM_TREE_LEVELWISE");
@@ -811,7 +813,8 @@ static bool fits_one(size_t na, size_t nb, size_t nc)
 struct Pieces { int logn, r3; uint64_t n, cnt, step; double us; };   /* cnt = 0: the product whole; us: the time to beat */
 /* a product's time by its passes, us: 12 for the call, 7 per launch (its own and its first and last tiles') and, per point and prime, 2.4 ps for the limb pass and 1.6 more where it
  * reads limbs, 3.6 a forward and 3.3 an inverse strided pass (9-bit rows 1.0 and 0.8 more), 3.8 (and the limbs) and 3.0 the radix-3 layers, 7.6
- * the double-fused pass; the CRT 2.5 per coefficient, 3.3 from pieces (kernel times of products of 2^20 to 2^28 points) */
+ * the double-fused pass; the CRT 2.5 per coefficient, 3.3 from pieces (kernel times of products of 2^20 to 2^28 points).  A
+ * partition of the device has its share of the CUs and of the memory */
 static double passes_us(int np, int logn, int r3, uint64_t cnt, uint64_t alen, uint64_t blen)
 {
     Plan pl; product_plan(&pl, logn, 1, product_tile_log(logn));
@@ -820,7 +823,7 @@ static double passes_us(int np, int logn, int r3, uint64_t cnt, uint64_t alen, u
     double fwd = r3 ? 3.8 + 3.6 * st : st ? 2.4 + 3.6 * (st - 1) : 0.0, inv = 3.3 * st + (r3 ? 3.0 : 0.0);
     for (int j = 0; j < st; j++) if (pl.p[j].m == 9) { fwd += 1.0; inv += 0.8; }
     return 12.0 + 7.0 * (2 * st + (r3 ? 2 : 0) + 3) + (cnt > 1 ? 4.0 : 0.0) +
-           1e-6 * np * (ca * (fwd + 7.6 + inv) + n * fwd + 1.6 * (double)(alen + blen) + (cnt > 1 ? 3.3 : 2.5) * (double)(alen + blen));
+           1e-6 * NTTM_CUS / nttm_ncu() * np * (ca * (fwd + 7.6 + inv) + n * fwd + 1.6 * (double)(alen + blen) + (cnt > 1 ? 3.3 : 2.5) * (double)(alen + blen));
 }
 static Pieces choose_pieces(int np, size_t alen, size_t blen, int logn, int r3)
 {
@@ -846,14 +849,6 @@ static Pieces choose_pieces(int np, size_t alen, size_t blen, int logn, int r3)
 /* whether products of this transform length run as one kernel each (small.hip): 2^k points up to 2^12 */
 static bool small_len(int logn, int r3) { return !r3 && !g_no_small && nttm_small_log(logn) != 0; }
 /* ---- products in segments of the result (k_segments): short operands of up to some 2000 limbs -------------------------------- */
-#define SEG_B_US 13.0              /* a workgroup (a CU has room for one): the short operand's transforms, ... */
-static double seg_us(uint64_t S) { return 21.0 + 10.0 * (double)S / 4096; }   /* ... and each segment of S limbs */
-/* the launch's time in workgroups of `per` segments, n workgroups in all */
-static double seg_launch_us(uint64_t n, uint32_t per, uint64_t S)
-{
-    const double r = (double)n / 256;
-    return (r <= 4 ? ceil(r) : r + 0.5) * (SEG_B_US + seg_us(S) * per);
-}
 static bool seg_forced(void) { return g_pieces_points == 1 << 12; }
 static bool seg_allowed(uint64_t S) { return S && !g_no_small && (g_pieces_points < 0 || seg_forced()); }
 /* the result shares memory with a or b: segments, which write limbs while others still read theirs, are not for it (the
@@ -874,15 +869,11 @@ static uint32_t choose_segments(size_t nc, size_t blen, double most)
     if (!seg_allowed(S)) return 0;
     const uint64_t segs = (nc + S - 1) / S;
     if (segs > 0x7fffffffULL) return 0;
-    uint32_t best = 0;
-    for (uint32_t per = 1; per <= 8; per++) {
-        const double us = 17.0 + seg_launch_us((segs + per - 1) / per, per, S);
-        if (us < most || (seg_forced() && !best)) { most = us; best = per; }
-    }
-    return best;
+    return seg_choose(segs, S, most, nttm_ncu(), seg_forced());
 }
 /* a product of a batch, whose launches fill the device either way: segments against the passes and the CRT of its own length
- * at 17 ps a point and prime from 2^16 points, 1.5 more for each bit below (measured 17.3 there, 19 at 2^15, 21 at 2^14) */
+ * at 17 ps a point and prime from 2^16 points, 1.5 more for each bit below (measured 17.3 there, 19 at 2^15, 21 at 2^14).  Both
+ * sides in time of the whole device: a partition takes longer for either alike */
 static bool batch_segments(const nttm_prod &q, int logn, int r3)
 {
     const size_t na = q.na, nb = q.nb;
@@ -894,7 +885,7 @@ static bool batch_segments(const nttm_prod &q, int logn, int r3)
     if (small_len(logn, r3) || alen < 2 * blen) return false;
     const double segs = ceil((double)(na + nb) / (double)S);
     const double ps = 17.0 + 1.5 * std::max(0, 16 - logn - (r3 ? 1 : 0));
-    return (segs * seg_us(S) + SEG_B_US * ceil(segs / 6)) / 256 < 0.95 * ps * 3e-6 * (double)((uint64_t)(r3 ? 3 : 1) << logn);
+    return (segs * seg_us(S) + SEG_B_US * ceil(segs / 6)) / NTTM_CUS < 0.95 * ps * 3e-6 * (double)((uint64_t)(r3 ? 3 : 1) << logn);
 }
 /* the descriptors of the pieces and the map to their one B operand: written by a kernel, since nothing on the host would
  * live until a copy of them has run in a call that does not wait */
@@ -1466,21 +1457,9 @@ static void group_build_segments(GroupBuild &gb, const nttm_prod *P, const std::
     gb.crt_per = NTTM_CRT_SEGS; gb.small = gb.share = false; gb.merged = true;
     gb.cd.assign(cnt, CrtDesc()); gb.ld.assign(cnt, LoadDesc()); gb.ldb.clear(); gb.bmap.clear();
     gb.chunk.assign(1, GroupBuild::Chunk{0, cnt, 0, cnt, 0, 0, 0.0});
-    /* segments of a workgroup, at most: a product's are shared out evenly, the products come longest first, and the launch ends
-     * within about a quarter of its longest workgroup.  (Every workgroup taken for a full one, in the callers' order: the 4096
-     * leaves' plan 4.70 ms, now 4.50.) */
-    double least = 0;
-    for (uint32_t per = 1; per <= 8; per++) {
-        double sum = 0, longest = 0;
-        uint64_t n = 0;
-        for (size_t i : G) {
-            const uint64_t sb = seg_blocks(P[i]), k = (sb + per - 1) / per;
-            const double us = SEG_B_US + seg_us(nttm_seg_len(std::min(P[i].na, P[i].nb))) * (double)((sb + k - 1) / k);
-            sum += us * (double)k; n += k; longest = std::max(longest, us);
-        }
-        const double us = n <= 256 ? longest : n <= 1024 ? ceil((double)n / 256) * longest : sum / 256 + longest / 4;
-        if (per == 1 || us < least) { least = us; gb.seg_per = per; }
-    }
+    std::vector<uint64_t> blocks(cnt), lens(cnt);
+    for (uint64_t j = 0; j < cnt; j++) { blocks[j] = seg_blocks(P[G[j]]); lens[j] = nttm_seg_len(std::min(P[G[j]].na, P[G[j]].nb)); }
+    gb.seg_per = seg_batch_per(blocks.data(), lens.data(), cnt, nttm_ncu());
     gb.seg_groups = 0;
     for (uint64_t j = 0; j < cnt; j++) {
         const nttm_prod &q = P[G[j]];

@@ -791,6 +791,7 @@ static int g_fixed_shapes = 1;                                  /* use the fixed
 void nttm_set_fixed_shapes(int on) { g_fixed_shapes = on != 0; }
 static int g_stream = 1, g_ncu = 256;                           /* streaming strided passes; CUs of the device */
 void nttm_set_stream(int on, int ncu) { g_stream = on != 0; g_ncu = ncu > 0 ? ncu : 256; }
+int nttm_ncu(void) { return g_ncu; }
 
 /* whether nttm_run_pass runs this forward pass as the streamed kernel (the condition in nttm_run_pass below) */
 bool nttm_fwd_pass_streams(const PassArgs &a, const PassGeom &g)

@@ -21,6 +21,9 @@
 #include "internal.h"
 #include "rounds.h"
 #include "crt_dev.h"
+#include "segrule.h"
+
+int nttm_ncu(void);
 
 #define SMALL_LOG_MIN 7
 #define SMALL_LOG_MAX 12
@@ -300,11 +303,11 @@ int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, cons
     for (int i = 0; i < np; i++) { a.stage[i] = fwd[i].stage; a.istage[i] = inv[i].stage; a.ninv[i] = ninv[i]; }
     /* Few products: a block each and 4 or 8 points a thread, so that more waves share a product's chain of rounds; many:
      * 16 points, and at least a wave per prime (12 waves a block at 2^11 points, whose 6 of one product leave room for no
-     * second block: waves of 144 registers start on the same SIMDs).  The line is 2^19 points, one block a CU at 2^11.
+     * second block: waves of 144 registers start on the same SIMDs).  The line is 2^11 points a CU, one block at 2^11.
      * A plan's replay, us, many / few: 2^7 points 1 product 22 / 18, 4096 32 / 27, 8192 42 / 43; 2^9 256 26 / 22, 2048 44 / 44;
      * 2^10 1 24 / 21, 512 33 / 31, 1024 45 / 62; 2^11 1 38 / 26, 256 43 / 29, 512 46 / 52, 8192 572 / 668 (6 waves of
      * 16 points: 789).  One 64 x 64 limb call 35 -> 27 us, 1000 x 1000 46 -> 40. */
-    const bool few = cnt <= ((uint64_t)1 << 19) >> logn;
+    const bool few = small_few(cnt, logn, nttm_ncu());
     const int tl = few ? (logn < 8 ? 8 : logn) : logn == 11 ? 12 : logn > 10 ? logn : 10, h = 1 << (tl - logn);
     const int pts = !few ? 16 : tl <= 8 ? 4 : tl <= 11 ? 8 : 16;
     const uint64_t blocks = (cnt + h - 1) / h;
