@@ -3108,6 +3108,7 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
     if (hipHostMalloc((void **)&pl->hstage, pl->hstage_words * 8, 0) != hipSuccess) {
         (void)hipGetLastError(); pl->hstage = nullptr; return fail(nttm_fail(NTTM_ENOMEM, "plan: pinned staging"));
     }
+    memset(pl->hstage, 0, pl->hstage_words * 8);                  /* (lengths asked for before any run: 0, and no flag) */
     /* capture every group's launches on a stream of the plan's own (default priority) */
     if ((rc = nttm_hip_check(hipStreamCreate(&pl->cs), "plan stream"))) return fail(rc);
     if ((rc = nttm_hip_check(hipStreamSynchronize(s), "plan tuning"))) return fail(rc);

@@ -146,6 +146,19 @@ def test_plan_reuses_remembered_choices(nttm):
         p3.close()
 
 
+def test_plan_lengths_before_a_run(nttm):
+    """0 and no error, for every kind of group and an empty operand; plans made and dropped before leave nothing behind"""
+    import torch
+    for _ in range(3):
+        ops = mixed_ops(41)
+        plan = nttm.BatchPlan(nttm.make_prods(device_items(ops)), autotune=False)
+        say("plan lengths before a run")
+        assert list(plan.ncn()) == [0] * len(ops)
+        plan.run()
+        assert any(plan.ncn())
+        plan.close()
+
+
 def test_plan_times_one_kernel_group_once(nttm):
     """products of one kernel each run alike under every candidate: one warm and two timed launches, and the plan reports
     the configured tile and points per thread"""
