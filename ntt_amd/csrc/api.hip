@@ -1010,8 +1010,14 @@ static int mul_core(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
     if (ws) {
         if (L.bytes > ws_cap) return nttm_fail(NTTM_EINVAL, "the product needs %zu bytes of workspace, above the %zu given", L.bytes, ws_cap);
     } else {
-        RCK(ws_need(L.bytes));
+        int rc = ws_need(L.bytes);
+        if (rc == NTTM_ENOMEM && L.par + L.cnt) {                 /* the device is nearly full: whole, prime after prime */
+            RCK(core_layout(na, nb, x != nullptr, wcut, &L));
+            rc = ws_need(L.bytes);
+        }
+        RCK(rc);
         ws = g.ws;
+        hd.plane = L.plane;
     }
     if (L.seg_per) {
         const bool sw = na < nb;
@@ -1107,11 +1113,13 @@ int nttm_mul_cyclic(uint64_t *v, const uint64_t *a, size_t na, const uint64_t *b
     bool par = L <= g_par_points;
     size_t planes_bytes = (size_t)(par ? 2 * np : np + 1) * L * 8;
     const size_t crt_bytes = nttm_crt_scratch_words(nttm_crt_blocks(nc)) * 4 + 256;
-    if (par && g.cfg.workspace_bytes && align_up(planes_bytes, 256) + 256 + crt_bytes > g.cfg.workspace_bytes) {
+    int rc = ws_need(align_up(planes_bytes, 256) + 256 + crt_bytes);
+    if (rc == NTTM_ENOMEM && par) {                               /* above the cap, or the device is nearly full */
         par = false; planes_bytes = (size_t)(np + 1) * L * 8;
+        rc = ws_need(align_up(planes_bytes, 256) + 256 + crt_bytes);
     }
+    RCK(rc);
     const size_t off_desc = align_up(planes_bytes, 256), off_crt = off_desc + 256;
-    RCK(ws_need(off_crt + crt_bytes));
     double *A = (double *)g.ws, *Bp = A + (size_t)np * L;
     RCK(product_transforms(np, logn, r3, 1, A, Bp, par ? L : 0, a, na, b, nb, nullptr, s, nullptr));
     CrtDesc hd; memset(&hd, 0, sizeof hd);
@@ -1429,6 +1437,15 @@ static GroupShape group_shape(int np, uint64_t n, uint64_t cnt, size_t cap)
     h.cn = std::max<uint64_t>(1, std::min(h.cn, room / (h.merged ? 2 * np : np + 1)));
     return h;
 }
+/* the workspace of the groups' planes under a cap (planes(cap) bytes); on a device nearly full, where that cannot be had, of the
+ * least planes the groups run with, *cap set so that they are built for it */
+template <typename F> static int ws_need_least(size_t *cap, F planes, bool defer = false)
+{
+    const int rc = ws_need(planes(*cap), defer);
+    if (rc != NTTM_ENOMEM) return rc;
+    *cap = 1;
+    return ws_need(planes(*cap), defer);
+}
 #define SEG_CLASS (2 * (NTTM_LOGN_MAX + 1) + 12)   /* the group class of products in segments of 2^12 points (r3 = 2) */
 static uint64_t seg_blocks(const nttm_prod &q)
 {
@@ -1660,8 +1677,7 @@ static int mul_batch_apart(nttm_prod *P, size_t N, hipStream_t s)
      * precedes, on the caller's), and the lengths and flags are written straight to pinned memory.  One
      * synchronization at the end.  (Waiting per group left the device idle for 0.9 of the 4096 leaves' 6.6 ms.) */
     std::vector<size_t> order;
-    const size_t cap = g.cfg.workspace_bytes;
-    size_t planes = 256, desc = 0, img = 0, words = 0;
+    size_t cap = g.cfg.workspace_bytes, desc = 0, img = 0, words = 0;
     auto radix = [](size_t gi) { return (int)(gi / (NTTM_LOGN_MAX + 1)); };
     auto pts = [&](size_t gi) { return (uint64_t)(radix(gi) == 1 ? 3 : radix(gi) ? 8 : 1) << (gi % (NTTM_LOGN_MAX + 1)); };   /* (about 8 segments) */
     for (size_t gi = 0; gi < groups.size(); gi++) {
@@ -1672,7 +1688,6 @@ static int mul_batch_apart(nttm_prod *P, size_t N, hipStream_t s)
         const uint64_t n = pts(gi), cnt = G.size();
         uint64_t blk = 0;
         for (size_t i : G) blk += r3 == 2 ? seg_blocks(P[i]) : prod_crt_blocks(logn, r3, n, P[i].na + P[i].nb + (P[i].x ? 1 : 0));
-        if (r3 != 2 && !small_len(logn, r3)) planes = std::max(planes, group_shape(np, n, cnt, cap).bytes(np, n));
         const size_t im = align_up(cnt * sizeof(CrtDesc), 256) + 2 * align_up(cnt * sizeof(LoadDesc), 256) +
                           align_up((r3 ? 3 : 1) * cnt * 4, 256) + 512;
         img += im;
@@ -1680,7 +1695,15 @@ static int mul_batch_apart(nttm_prod *P, size_t N, hipStream_t s)
         words += cnt + 2;
     }
     std::sort(order.begin(), order.end(), [&](size_t u, size_t v) { return pts(u) * groups[u].size() > pts(v) * groups[v].size(); });
-    RCK(ws_need(planes));
+    auto planes = [&](size_t c) {
+        size_t most = 256;
+        for (size_t gi : order) {
+            const int logn = (int)(gi % (NTTM_LOGN_MAX + 1));
+            if (radix(gi) != 2 && !small_len(logn, radix(gi))) most = std::max(most, group_shape(np, pts(gi), groups[gi].size(), c).bytes(np, pts(gi)));
+        }
+        return most;
+    };
+    RCK(ws_need_least(&cap, planes));
     RCK(tdesc_need(desc + 256));
     const size_t img0 = align_up(words * 8 + 256, 256);          /* the lengths and flags, then the descriptor images */
     RCK(hpin_need(img0 + img));
@@ -2255,7 +2278,8 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
         }
     }
     const size_t off_ncn = align_up(N * sizeof(CrtDesc), 256);
-    RCK(ws_need(ws_max));                                        /* sized once: no reallocation between launches */
+    const int rcw = ws_need(ws_max);                             /* sized once: no reallocation between launches, but */
+    if (rcw && rcw != NTTM_ENOMEM) return rcw;                   /* on a device nearly full, where each takes what it needs */
     RCK(hpin_need(128 * N + 8 * N + 256));
     RCK(stage_need(off_ncn + N * 8));
     std::vector<char> fl(N, 0);                                  /* 1: flags in pinned slot i */
@@ -2356,8 +2380,9 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
     const int nlev = (int)len.size() - 1;                        /* levels of products */
     /* resources for every level, sized before the first launch: pools by level parity, planes, descriptors; each
      * product's length class kept for its level's grouping (-1: an empty operand) */
-    const size_t cap = g.cfg.workspace_bytes;
-    size_t pool_max[2] = {1, 1}, planes_max = 0, desc_total = 0, img_total = 0, ngroups = 0;
+    size_t cap = g.cfg.workspace_bytes, pool_max[2] = {1, 1}, desc_total = 0, img_total = 0, ngroups = 0;
+    struct Need { int np; uint64_t n, cnt; };
+    std::vector<Need> need;                                      /* the groups with planes */
     std::vector<int> lev_np(nlev + 1, 3);
     std::vector<std::vector<int8_t>> keys(nlev + 1);
     std::vector<std::array<uint64_t, TREE_NKEY>> lev_cnt(nlev + 1);
@@ -2396,7 +2421,7 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
             if (logn > NTTM_LOGN_MAX) return 1;
             for (uint64_t c0 = 0; c0 < cnt_all; c0 += TREE_CHUNK) {   /* the group's chunks (below) */
                 const uint64_t cn = std::min<uint64_t>(TREE_CHUNK, cnt_all - c0), tb = r3 ? 3 * cn : cn;
-                if (!small_len(logn, r3)) planes_max = std::max(planes_max, group_shape(lev_np[k], npts, cn, cap).bytes(lev_np[k], npts));
+                if (!small_len(logn, r3)) need.push_back({lev_np[k], npts, cn});
                 const size_t img = align_up(cn * sizeof(CrtDesc), 256) + 2 * align_up(cn * sizeof(LoadDesc), 256) +
                                    align_up(tb * 4, 256) + 256 + 256;
                 img_total += img;
@@ -2426,7 +2451,11 @@ static int bs_tree_planned(const nttm_bs_node *leaves, size_t n, uint64_t *p, si
      * after the tree's final synchronization (a failed call's, at the next call's start) */
     if (g.ndfree || g.nhfree) { HIPCK(hipDeviceSynchronize()); free_deferred(); }
     RCK(bsp_need(0, pool_max[0], true)); RCK(bsp_need(1, pool_max[1], true));
-    RCK(ws_need(planes_max ? planes_max : 256, true));
+    RCK(ws_need_least(&cap, [&](size_t c) {
+        size_t most = 256;
+        for (const Need &x : need) most = std::max(most, group_shape(x.np, x.n, x.cnt, c).bytes(x.np, x.n));
+        return most;
+    }, true));
     RCK(tdesc_need(desc_total + 512, true));
     RCK(tpin_need(img_total + 8 * ngroups + 2048, true));
     RCK(side_stream());
@@ -2935,16 +2964,16 @@ static void memo_put(const TuneMemo &e)
 }
 /* the fastest (tile, points per thread) for one group of products, timed on the stream; *ms its time.  reuse: a
  * remembered choice for the same class is taken untimed (*ms scaled from its time per product; *nreused counts it) */
-static int tune_group(const nttm_prod *P, const std::vector<size_t> &G, int np, int r3, int logn, bool tune, TuneBuf &tb,
+static int tune_group(const nttm_prod *P, const std::vector<size_t> &G, int np, int r3, int logn, size_t cap, bool tune, TuneBuf &tb,
                       std::vector<char> &img, hipStream_t s, GroupBuild &best, double *ms, int *ntried, bool reuse = false,
                       int *nreused = nullptr)
 {
     static const int cand[4][2] = {{12, 16}, {13, 16}, {12, 8}, {13, 8}};
     *ms = 0;
-    if (!tune) { group_build(best, P, G, np, r3, logn, g.cfg.tile_log, batch_pts(logn)); return 0; }
+    if (!tune) { group_build(best, P, G, np, r3, logn, g.cfg.tile_log, batch_pts(logn), cap); return 0; }
     if (reuse) {
         if (const TuneMemo *m = memo_find(np, r3, logn, G.size())) {
-            group_build(best, P, G, np, r3, logn, m->tile, m->pts);
+            group_build(best, P, G, np, r3, logn, m->tile, m->pts, cap);
             *ms = m->ms_per * (double)G.size();
             if (nreused) (*nreused)++;
             return 0;
@@ -2957,8 +2986,8 @@ static int tune_group(const nttm_prod *P, const std::vector<size_t> &G, int np, 
     const bool one = small_len(logn, r3);
     for (int c = 0; c < (one ? 1 : 4); c++) {
         GroupBuild gb;
-        if (one) group_build(gb, P, G, np, r3, logn, g.cfg.tile_log, batch_pts(logn));
-        else group_build(gb, P, G, np, r3, logn, cand[c][0], cand[c][1]);
+        if (one) group_build(gb, P, G, np, r3, logn, g.cfg.tile_log, batch_pts(logn), cap);
+        else group_build(gb, P, G, np, r3, logn, cand[c][0], cand[c][1], cap);
         const size_t off_d = align_up(gb.planes_bytes, 256);
         RCK(tb.need(off_d + gb.desc_bytes + 256));
         img.resize(gb.desc_bytes);
@@ -2984,12 +3013,9 @@ static int tune_group(const nttm_prod *P, const std::vector<size_t> &G, int np, 
     return 0;
 }
 
-extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune, nttm_batch_plan **out, void *stream)
+/* a plan whose groups' planes take at most cap bytes where they can (0: any) */
+static int plan_create(const nttm_prod *P, size_t N, int autotune, size_t cap, nttm_batch_plan **out, hipStream_t s)
 {
-    if (!g.init) return nttm_fail(NTTM_ESTATE, "not initialised");
-    if (!out || (N && !P)) return nttm_fail(NTTM_EINVAL, "nttm_batch_plan_create arguments");
-    *out = nullptr;
-    hipStream_t s = (hipStream_t)stream;
     /* the graph has the operands' addresses built in: device memory only */
     {
         MemMap mm;
@@ -3055,19 +3081,19 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
         GroupBuild a, b3, b2;
         double ta = 0, t3 = 0, t2 = 0;
         if (tune && !S3.empty()) {                               /* both variants timed */
-            if ((rc = tune_group(P, C, np, 0, k, true, tb, img, s, a, &ta, &pl->candidates, reuse, &pl->reused))) return fail(rc);
-            if ((rc = tune_group(P, S3, np, 1, k - 2, true, tb, img, s, b3, &t3, &pl->candidates, reuse, &pl->reused)))
+            if ((rc = tune_group(P, C, np, 0, k, cap, true, tb, img, s, a, &ta, &pl->candidates, reuse, &pl->reused))) return fail(rc);
+            if ((rc = tune_group(P, S3, np, 1, k - 2, cap, true, tb, img, s, b3, &t3, &pl->candidates, reuse, &pl->reused)))
                 return fail(rc);
-            if (!S2.empty() && (rc = tune_group(P, S2, np, 0, k, true, tb, img, s, b2, &t2, &pl->candidates, reuse, &pl->reused)))
+            if (!S2.empty() && (rc = tune_group(P, S2, np, 0, k, cap, true, tb, img, s, b2, &t2, &pl->candidates, reuse, &pl->reused)))
                 return fail(rc);
             if (ta <= t3 + t2) { pl->gb.push_back(std::move(a)); pl->gidx.push_back(C); pl->gms.push_back(ta); continue; }
         } else if (S3.empty()) {
-            if ((rc = tune_group(P, C, np, 0, k, tune, tb, img, s, a, &ta, &pl->candidates, reuse, &pl->reused))) return fail(rc);
+            if ((rc = tune_group(P, C, np, 0, k, cap, tune, tb, img, s, a, &ta, &pl->candidates, reuse, &pl->reused))) return fail(rc);
             pl->gb.push_back(std::move(a)); pl->gidx.push_back(C); pl->gms.push_back(ta);
             continue;
         } else {                                                 /* untuned: the library's rule */
-            if ((rc = tune_group(P, S3, np, 1, k - 2, false, tb, img, s, b3, &t3, &pl->candidates))) return fail(rc);
-            if (!S2.empty() && (rc = tune_group(P, S2, np, 0, k, false, tb, img, s, b2, &t2, &pl->candidates))) return fail(rc);
+            if ((rc = tune_group(P, S3, np, 1, k - 2, cap, false, tb, img, s, b3, &t3, &pl->candidates))) return fail(rc);
+            if (!S2.empty() && (rc = tune_group(P, S2, np, 0, k, cap, false, tb, img, s, b2, &t2, &pl->candidates))) return fail(rc);
         }
         pl->gb.push_back(std::move(b3)); pl->gidx.push_back(S3); pl->gms.push_back(t3);
         if (!S2.empty()) { pl->gb.push_back(std::move(b2)); pl->gidx.push_back(S2); pl->gms.push_back(t2); }
@@ -3135,6 +3161,15 @@ extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune
     if ((rc = nttm_hip_check(hipGraphInstantiate(&pl->exec, pl->graph, nullptr, nullptr, 0), "graph instantiate"))) return fail(rc);
     *out = pl;
     return 0;
+}
+
+extern "C" int nttm_batch_plan_create(const nttm_prod *P, size_t N, int autotune, nttm_batch_plan **out, void *stream)
+{
+    if (!g.init) return nttm_fail(NTTM_ESTATE, "not initialised");
+    if (!out || (N && !P)) return nttm_fail(NTTM_EINVAL, "nttm_batch_plan_create arguments");
+    *out = nullptr;
+    const int rc = plan_create(P, N, autotune, 0, out, (hipStream_t)stream);
+    return rc == NTTM_ENOMEM ? plan_create(P, N, autotune, 1, out, (hipStream_t)stream) : rc;   /* (the least planes) */
 }
 
 extern "C" int nttm_batch_plan_run(nttm_batch_plan *pl, void *stream)

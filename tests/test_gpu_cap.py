@@ -95,3 +95,69 @@ def test_large(capped, cap):
     lib.mul_batch(lib.make_prods([(da, db, None, c)]))
     assert O.tref_res(a, b, host(c))
     assert np.array_equal(host(c), host(lib.mul(da, db)))
+
+
+def test_device_nearly_full(capped):
+    """no cap, but room on the device for np + 1 planes of 2^24 points (512 MiB) and not for 2 np (768): single, each, batch,
+    plan, cyclic and tree"""
+    import torch
+    n = 1 << 23
+    a, s = O.gen_limbs(n, 3)
+    b, _ = O.gen_limbs(n, s)
+    da, db, c = dev(a), dev(b), torch.empty(2 * n, dtype=torch.int64, device="cuda")
+    lib = capped()
+    want = lib.mul(da, db).clone()
+    lib.mul_batch(lib.make_prods([(da, db, None, c)]))
+    leaves = [(da[:n - 1], db), (db[:n - 1], da)]
+    tree = [t.clone() for t in lib.bs_tree(leaves)]
+    cyc = lib.mul_cyclic(da, db, 2 * n)
+    assert torch.equal(c, want) and O.tref_res(a, b, host(want))
+
+    def calls():
+        prods = lib.make_prods([(da, db, None, c)])
+        yield "mul", lambda: lib.mul(da, db, out=c), lambda: torch.equal(c, want)
+        yield "each", lambda: lib.mul_each_async(prods), lambda: torch.equal(c, want)
+        yield "batch", lambda: lib.mul_batch(prods), lambda: torch.equal(c, want)
+        for tune in (0, 1):
+            yield "plan", lambda: planned(prods, tune), lambda: torch.equal(c, want)
+
+    def planned(prods, tune):
+        plan = lib.BatchPlan(prods, autotune=tune)
+        plan.run()
+        plan.ncn()
+        plan.close()
+    most = fill(3 << 30)                                          # (once: it takes seconds)
+    for name, call, ok in calls():
+        lib = capped()
+        c.fill_(-1)
+        held = fill(640 << 20)
+        say("nearly full", name, torch.cuda.mem_get_info()[0] >> 20)
+        call()
+        assert ok(), name
+        del held
+    lib = capped()
+    held = fill((640 + 4 * 128 + 80) << 20)                       # (and the root's and the level's two numbers, the descriptors)
+    say("nearly full tree", torch.cuda.mem_get_info()[0] >> 20)
+    got = lib.bs_tree(leaves)
+    assert all(torch.equal(g, w) for g, w in zip(got, tree))
+    del held, got
+    lib = capped()
+    held = fill((640 + 130) << 20)
+    say("nearly full cyclic", torch.cuda.mem_get_info()[0] >> 20)
+    got = lib.mul_cyclic(da, db, 2 * n)
+    assert torch.equal(got, cyc)
+    del held, most
+    torch.cuda.empty_cache()
+
+
+def fill(leave):
+    """device memory held so that about `leave` bytes are free"""
+    import torch
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    held = []
+    while True:
+        left = torch.cuda.mem_get_info()[0] - leave
+        if left < 8 << 20:
+            return held
+        held.append(torch.empty(min(left, 32 << 30), dtype=torch.uint8, device="cuda"))
