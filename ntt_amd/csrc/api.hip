@@ -36,8 +36,6 @@ int nttm_run_f64_to_canon(double *x, uint64_t count, const PrimeK &pk, hipStream
 int nttm_run_pw_u64(uint64_t *x, const uint64_t *y, uint64_t count, const PrimeK &pk, hipStream_t s);
 int nttm_run_load_planes(double *dst, uint64_t plane, const uint64_t *src, uint64_t nlimbs, uint64_t npoints, int np,
                          const PrimeK *pk, const double2 *scale, int out_u64, hipStream_t s);
-int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which, uint64_t count, int logn, int np,
-                        const PrimeK *pk, const double2 *scale, hipStream_t s);
 /* the CRT of products whose blocks are [blk0, blk0 + nblk) of the launch's block numbering (limbs for a carry in of 0),
  * then every block's carry; nttm_crt_launch_one: both for one product */
 int nttm_crt_launch_limbs(const CrtDesc *desc_dev, const CrtDesc *one, uint64_t nprod, uint64_t blk0, uint64_t nblk, int np,
@@ -251,7 +249,7 @@ static int build_tables(void)
 {
     const size_t nst = (size_t)1 << NTTM_STAGE_LOG;
     const size_t nbq = (size_t)4 << NTTM_BQ_LOG, nb3 = nbq + 1, ncol = (size_t)2 << 12;
-    const size_t per_dir = nst + nbq + nb3 + ncol, total = (size_t)NTTM_MAX_PRIMES * 2 * per_dir;
+    const size_t per_dir = nst + nbq + nb3, per_prime = 2 * per_dir + ncol, total = (size_t)NTTM_MAX_PRIMES * per_prime;
     std::vector<double2> h(total);
     for (int i = 0; i < NTTM_MAX_PRIMES; i++) {
         const uint64_t p = NTTM_PRIMES[i];
@@ -260,7 +258,7 @@ static int build_tables(void)
         g.root3x32[i] = h_powmod(gen, ((p - 1) >> 32) / 3, p);
         for (int dir = 0; dir < 2; dir++) {
             const uint64_t w32 = dir ? h_inv(g.root32[i], p) : g.root32[i];
-            double2 *st = &h[((size_t)i * 2 + dir) * per_dir], *bq = st + nst;
+            double2 *st = &h[i * per_prime + dir * per_dir], *bq = st + nst;
             double2 *b3 = bq + nbq;
             const uint64_t W3 = dir ? h_inv(g.root3x32[i], p) : g.root3x32[i];
             for (int k = 0; k < 4; k++) {                                /* b3[k 2^8 + x] = W3^(x 2^(8k)) */
@@ -272,7 +270,7 @@ static int build_tables(void)
             }
             b3[nbq] = h_shoup(h_powmod(g.root3x32[i], (uint64_t)1 << 32, p), p);   /* the forward cube root */
             double2 *co = b3 + nb3;
-            for (int m = 3; m <= 4; m++) {                               /* (unused in the forward direction) */
+            for (int m = 3; dir && m <= 4; m++) {                        /* (the inverse direction's only) */
                 const uint64_t wm = h_powmod(w32, (uint64_t)1 << (32 - 12 - m), p);
                 uint64_t v = 1;
                 for (size_t c = 0; c < ((size_t)1 << 12); c++) { co[((size_t)(m - 3) << 12) + c] = h_shoup(v, p); v = h_mulmod(v, wm, p); }
@@ -296,9 +294,9 @@ static int build_tables(void)
     HIPCK(hipMemcpy(g.tables, h.data(), total * sizeof(double2), hipMemcpyHostToDevice));
     for (int i = 0; i < NTTM_MAX_PRIMES; i++)
         for (int dir = 0; dir < 2; dir++) {
-            const double2 *st = g.tables + ((size_t)i * 2 + dir) * per_dir;
+            const double2 *st = g.tables + i * per_prime + dir * per_dir;
             TwTables t; t.stage = st; t.bq = st + nst;
-            t.b3 = t.bq + nbq; t.col = t.b3 + nb3;
+            t.b3 = t.bq + nbq; t.col = dir ? t.b3 + nb3 : nullptr;
             if (dir) g.twi[i] = t; else g.twf[i] = t;
         }
     return 0;

@@ -439,40 +439,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         const uint32_t b = (uint32_t)row * RUN_BLOCKS + ch0 + g;
         if (lane == 0) a.status[d.first_block + b] = st | (b == 0 ? CRT_ST_FIRST : 0u);
     };
-    /* CNT rows from row0 on: their x limbs requested, their digits side by side (one coefficient's are a serial chain) */
-#define RUN_ROWS(CNT, ROW0) { \
-        uint64_t xv[CNT], dg[CNT][NP]; \
+    /* the run's limbs in one row: the x limb requested, the residues (the previous row's in a row's first four lanes) to digits */
+#define RUN_ROW(ROW) { \
+        const int rw = (ROW), k = (rw << RUN_LO) + col[g]; \
+        uint64_t xv = 0, dg[NP]; \
+        if (nx && col[g] < COLS && k >= 0 && k < nx) xv = *(GIn)((GByte)d.x + 8u * (uint32_t)k); \
+        const bool coef = col[g] < COLS && k >= 0 && k < ncoef; \
+        double rz[NP]; \
         _Pragma("unroll") \
-        for (int u = 0; u < CNT; u++) { \
-            const int k = (((ROW0) + u) << RUN_LO) + col[g]; \
-            xv[u] = 0; \
-            if (nx && col[g] < COLS && k >= 0 && k < nx) xv[u] = *(GIn)((GByte)d.x + 8u * (uint32_t)k); \
+        for (int p = 0; p < NP; p++) { \
+            const double here = rw < R ? r[p][g][rw < R ? rw : 0] : 0.0, prev = rw ? r[p][g][rw ? rw - 1 : 0] : 0.0; \
+            rz[p] = coef ? (wrap ? prev : here) : 0.0; \
         } \
-        _Pragma("unroll") \
-        for (int u = 0; u < CNT; u++) { \
-            const int rw = (ROW0) + u, k = (rw << RUN_LO) + col[g]; \
-            const bool coef = col[g] < COLS && k >= 0 && k < ncoef; \
-            double rz[NP]; \
-            _Pragma("unroll") \
-            for (int p = 0; p < NP; p++) { \
-                const double here = rw < R ? r[p][g][rw < R ? rw : 0] : 0.0, prev = rw ? r[p][g][rw ? rw - 1 : 0] : 0.0; \
-                rz[p] = coef ? (wrap ? prev : here) : 0.0; \
-            } \
-            crt_digits<NP>(a.cc, rz, dg[u]); \
-        } \
-        _Pragma("unroll") \
-        for (int u = 0; u < CNT; u++) finish(g, (ROW0) + u, dg[u], xv[u]); \
+        crt_digits<NP>(a.cc, rz, dg); \
+        finish(g, rw, dg, xv); \
     }
-    constexpr int U = R < 1 ? R : 1;
 #pragma unroll
     for (int g = 0; g < G; g++) {
         if (ch0 + g >= RUN_BLOCKS) break;
         const bool wrap = col[g] < 0;
 #pragma unroll
-        for (int row = 0; row < R; row += U) RUN_ROWS(U, row)
-        if (ch0 + g == 0) RUN_ROWS(1, R)                         /* the limbs from 2^logn on: the last coefficients' upper digits */
+        for (int row = 0; row < R; row++) RUN_ROW(row)
+        if (ch0 + g == 0) RUN_ROW(R)                             /* the limbs from 2^logn on: the last coefficients' upper digits */
     }
-#undef RUN_ROWS
+#undef RUN_ROW
 }
 
 /* c[0 .. n) += *carry (0 or 1), the carry rippling through the leading limbs equal to B - 1 (one workgroup, 2048

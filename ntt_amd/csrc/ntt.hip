@@ -25,13 +25,7 @@ __device__ __forceinline__ double input_limb_raw(const PassArgs &a, uint64_t gi,
     else { src = a.limbs; nl = a.nlimbs; }
     return k < nl ? limb_to_res(((GLimb)src)[k], p, pinv) : 0.0;
 }
-__device__ __forceinline__ double input_limb(const PassArgs &a, uint64_t gi, double p, double pinv)
-{
-    double x = input_limb_raw(a, gi, p, pinv);
-    if (a.do_in_scale) x = mul_shoup(x, a.in_scale.x, a.in_scale.y, p);
-    return x;
-}
-/* input_limb with the operand of the last transform looked up kept: consecutive elements of one transform (the slots
+/* the scaled element with the operand of the last transform looked up kept: consecutive elements of one transform (the slots
  * of a group) read its descriptor once */
 struct LimbCache {
     uint64_t b = ~(uint64_t)0, nl = 0;
@@ -607,14 +601,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
 }
 
-/* limbs -> residues of np primes, zero-extended to npoints; optional per-prime scale (n^-1 folded into one operand).
- * Batched form: product j of a length group takes points [j n, (j+1) n) of every plane, operand a or b of desc[j]. */
+/* limbs -> residues of np primes, zero-extended to npoints; optional per-prime scale */
 struct LoadArgs {
     double *dst;                 /* plane i at dst + i * plane */
     uint64_t plane;
-    const uint64_t *src;         /* single operand, or null with desc */
+    const uint64_t *src;
     uint64_t nlimbs, npoints;
-    const LoadDesc *desc; int which, logn;
     int np, do_scale, out_u64;
     PrimeK pk[NTTM_MAX_PRIMES];
     double2 scale[NTTM_MAX_PRIMES];
@@ -622,17 +614,8 @@ struct LoadArgs {
 __global__ __launch_bounds__(NTTM_THREADS) void k_load(LoadArgs a)
 {
     const uint64_t stride = (uint64_t)gridDim.x * NTTM_THREADS;
-    const uint64_t nmask = ((uint64_t)1 << a.logn) - 1;
     for (uint64_t i = (uint64_t)blockIdx.x * NTTM_THREADS + threadIdx.x; i < a.npoints; i += stride) {
-        uint64_t x;
-        if (a.desc) {
-            const LoadDesc &d = a.desc[i >> a.logn];
-            const uint64_t k = i & nmask;
-            const uint64_t nl = a.which ? d.nb : d.na;
-            x = k < nl ? (a.which ? d.b : d.a)[k] : 0;
-        } else {
-            x = i < a.nlimbs ? a.src[i] : 0;
-        }
+        const uint64_t x = i < a.nlimbs ? a.src[i] : 0;
         for (int k = 0; k < a.np; k++) {
             double v = limb_to_res(x, a.pk[k].p, a.pk[k].pinv);
             if (a.do_scale) v = mul_shoup(v, a.scale[k].x, a.scale[k].y, a.pk[k].p);
@@ -987,23 +970,11 @@ int nttm_run_load_planes(double *dst, uint64_t plane, const uint64_t *src, uint6
                          const PrimeK *pk, const double2 *scale, int out_u64, hipStream_t s)
 {
     LoadArgs a; memset(&a, 0, sizeof a);
-    a.dst = dst; a.plane = plane; a.src = src; a.nlimbs = nlimbs; a.npoints = npoints; a.desc = nullptr; a.logn = 0;
+    a.dst = dst; a.plane = plane; a.src = src; a.nlimbs = nlimbs; a.npoints = npoints;
     a.out_u64 = out_u64;
     load_common(a, np, pk, scale);
     prof_begin("k_load", 8.0 * (double)nlimbs + 8.0 * np * (double)npoints, s);
     hipLaunchKernelGGL(k_load, dim3(grid_for(npoints)), dim3(NTTM_THREADS), 0, s, a);
-    prof_end(s);
-    return nttm_hip_check(hipGetLastError(), "k_load launch");
-}
-int nttm_run_load_batch(double *dst, uint64_t plane, const void *desc, int which, uint64_t count, int logn, int np,
-                        const PrimeK *pk, const double2 *scale, hipStream_t s)
-{
-    LoadArgs a; memset(&a, 0, sizeof a);
-    a.dst = dst; a.plane = plane; a.src = nullptr; a.npoints = count << logn; a.desc = (const LoadDesc *)desc;
-    a.which = which; a.logn = logn; a.out_u64 = 0;
-    load_common(a, np, pk, scale);
-    prof_begin("k_load", 16.0 * np * (double)a.npoints, s);
-    hipLaunchKernelGGL(k_load, dim3(grid_for(a.npoints)), dim3(NTTM_THREADS), 0, s, a);
     prof_end(s);
     return nttm_hip_check(hipGetLastError(), "k_load launch");
 }
