@@ -76,7 +76,8 @@ enum { NTTM_R3_AUTO = 0,       /* 3 2^k where it fits and moves fewer bytes than
 
 typedef struct nttm_config {
     int nprimes;                /* 0: choose per product (3 while the bound allows, else 4); 3 or 4: fixed */
-    size_t workspace_bytes;     /* 0: grow on demand; else the cap of the library's device workspace */
+    size_t workspace_bytes;     /* 0: grow on demand; else the cap of the library's device workspace (the residue planes and the
+                                 * CRT's scratch; descriptors, copies and plans' memory are beside it) */
     int tile_log;               /* points per tile of the strided transform passes, log2: 12 or 13 (0: default) */
     int pts;                    /* transform points per thread: 8 or 16 (0: default) */
     int radix3;                 /* NTTM_R3_*: when products use 3 2^k lengths (0: NTTM_R3_AUTO) */
@@ -135,7 +136,8 @@ int nttm_check_product(const uint64_t *c, size_t nc, const uint64_t *a, size_t n
                        const uint64_t *x, size_t nx, void *stream);
 /* N independent products; P is HOST memory; its a, b, x, c may each be device or host memory (host arrays staged, see
  * the top; a batch with more than 1 GiB of host arrays runs as consecutive sub-batches).  Products are grouped by
- * transform length and run batched; ncn is filled on return (the call synchronizes the stream). */
+ * transform length (those by a short operand in segments of the result) and run batched; ncn is filled on return (the call
+ * synchronizes the stream). */
 int nttm_mul_batch(nttm_prod *P, size_t N, void *stream);
 /* a node of a binary-splitting tree: P and Q as device limb arrays */
 typedef struct nttm_bs_node {
@@ -178,9 +180,10 @@ int nttm_limbs_mod(uint64_t *res, const uint64_t *x, size_t n, const uint64_t *q
  * (E/verify.c:18).  Synchronous. */
 int nttm_e_write_packed(const char *path, const uint64_t *frac, size_t m, uint64_t d_out, void *stream);
 /* a batch fixed once and run many times (the binary-splitting leaves' repeated rns_mul_batch calls, E/rns_mul.c:792):
- * the products are grouped by transform length; with autotune != 0 each group's schedule is chosen by timing the
- * candidates on these operands -- per length class, 3 2^k points for the products that fit them or 2^(k+2); per group,
- * a strided-pass tile of 2^12 or 2^13 points and 8 or 16 points per thread -- else the library's defaults are taken.
+ * the products are grouped by transform length, those by a short operand that go in segments of the result in a group of
+ * their own; with autotune != 0 each length group's schedule is chosen by timing the candidates on these operands -- per
+ * length class, 3 2^k points for the products that fit them or 2^(k+2); per group, a strided-pass tile of 2^12 or 2^13
+ * points and 8 or 16 points per thread (one-kernel products know neither) -- else the library's defaults are taken.
  * The choices are remembered until nttm_shutdown, per prime count, transform length and group size; autotune == 2
  * takes the remembered choice of a group of the same size, else of the nearest size in the same power-of-two class,
  * without timing it (autotune == 1 times every group and refreshes what is remembered).

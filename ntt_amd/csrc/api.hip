@@ -1089,8 +1089,8 @@ struct ResChunkH { const uint64_t *x; uint64_t n; };          /* must match digi
  * cyclic convolution c_k = sum_(i + j = k mod L) a_i b_j, i.e. a b mod (x^L - 1) at x = B before its carries wrap (the
  * caller folds v modulo B^L - 1).  The transforms are DFTs of length L, so the pointwise product gives the cyclic
  * convolution directly; each c_k has at most min(na, nb) terms, the bound of an ordinary product.  na, nb <= L, device
- * pointers.  flag null: synchronous; else the launches only, the CRT's flag word copied to the pinned word *flag (bit
- * 0 set: a carry beyond the top limb), read by the caller after it synchronizes the stream.  The Newton reciprocal's
+ * pointers.  flag null: synchronous; else the launches only, *flag the pinned word that the carry launch writes (bit 0
+ * set: a carry beyond the top limb), read by the caller after it synchronizes the stream.  The Newton reciprocal's
  * wrapped product (GMP's mpn_mulmod_bnm1 plays this part there). */
 int nttm_mul_cyclic(uint64_t *v, const uint64_t *a, size_t na, const uint64_t *b, size_t nb, size_t L, hipStream_t s,
                     const uint32_t **flag)
@@ -1363,7 +1363,7 @@ static int mul_full(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b
 }
 
 /* c = a b on device memory without a synchronization where it fits one transform (no residue check configured): the
- * launches only, the CRT's flag word copied to the pinned word *flag (bit 0 set: a carry beyond the top limb), which
+ * launches only, *flag the pinned word that the product's last launch writes (bit 0 set: a carry beyond the top limb), which
  * the caller reads after synchronizing the stream; *flag = null when the product ran synchronously (a grid) */
 int nttm_mul_launch(uint64_t *c, const uint64_t *a, size_t na, const uint64_t *b, size_t nb, hipStream_t s,
                     const uint32_t **flag)

@@ -1,8 +1,9 @@
 /* arith.h - exact modular arithmetic of the product library, host + device.
  *
- * Residues are FP64 values that hold integers exactly.  Primes are p = c 2^k + 1 < 2^50 (k >= 32), so every live value
- * lies in [-p, p] (|v| < 2^50) and sums of two stay below 2^52: FP64 add/sub/FMA on them are exact, and the full-rate
- * FP64 pipe of CDNA4 does the modular products.  Bounds below use u = 2^-53 and p < 2^50.
+ * Residues are FP64 values that hold integers exactly.  Primes are p = c 2^k + 1 < 2^50 (k >= 32).  Values between passes lie
+ * in [-p, p], those between the levels and rounds of a pass within 4p < 2^52 (radix.h), and sums of two stay within
+ * 8p < 2^53: FP64 add/sub/FMA on them are exact, and the full-rate FP64 pipe of CDNA4 does the modular products.  Bounds
+ * below use u = 2^-53 and p < 2^50.
  *
  *  rint_prod(a, b)       a b rounded once to the nearest integer, for |a b| < 2^51: fma(a, b, C) - C with C = 1.5 2^52
  *                        (the FMA result lies in [2^52, 2^53), where the FP64 spacing is 1; the subtraction is exact).

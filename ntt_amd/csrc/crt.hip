@@ -333,8 +333,8 @@ __global__ __launch_bounds__(256) void k_carry(const CrtDesc *desc, CrtDesc one,
  * every limb's lower digits and the quotient before the first limb come by shuffles.  A wave's run of 60 limbs is
  * one ballot word and one block of the carry launch.  For m < 4 a wave takes two runs, every load requested at once.
  * It replaces a pass over the planes (16 B read and written per point and prime) and the CRT's reads (8 B): bound by
- * vector issue, about 290 instructions per coefficient, of which 1 in 16 is spent on the four repeated columns, at 2 to 5
- * waves per SIMD.  4096 products of 64 to 65536 limbs: 1.15 ms against 0.64 (inverse pass) + 0.65 (k_crt). */
+ * vector issue, 269 instructions per coefficient at m = 1, 283, 323 and 368 at m = 4, of which 1 in 16 is spent on the four
+ * repeated columns, at 86, 86, 62 and 68% of the issue rate (2 to 5 waves per SIMD).  4096 products of 64 to 65536 limbs: 1.15 ms against 0.64 (inverse pass) + 0.65 (k_crt). */
 struct InvCrtArgs {
     const CrtDesc *desc; uint64_t nprod;        /* null: the one product `one` */
     CrtDesc one;

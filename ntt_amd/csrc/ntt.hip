@@ -916,9 +916,9 @@ int nttm_run_pass(bool inv, const PassArgs &a, const PassGeom &g, hipStream_t s,
     return nttm_hip_check(hipGetLastError(), "k_pass launch");
 }
 
-/* Bound by vector issue (166 of 178 vector instructions a point are FP64).  A block's first loads wait for nothing but its
+/* Bound by vector issue (82% of the rate; 160.5 of 171.5 vector instructions a point are FP64).  A block's first loads wait for nothing but its
  * arguments: the LDS table's entry is requested before B's tile and stored behind it, and limbs are read through
- * global-space pointers (2.06 -> 1.97 ms per launch at 2^28 points). */
+ * global-space pointers (2.06 -> 1.97 ms per launch at 2^28 points; with the lazy reductions 1.91). */
 /* the double-fused last pass of every prime of js: a = A's common arguments (its operand where a transform is a single
  * pass: limbs or descriptors; a.ymode and a.scale unused), fb = B's */
 int nttm_run_fused2(const PassArgs &a, const FusedB &fb, const PassGeom &g, hipStream_t s, const FusedSet &js)

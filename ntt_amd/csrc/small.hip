@@ -12,11 +12,12 @@
  *     natural order;
  *   - digits: each coefficient's residues are replaced in place by its base-10^18 digits (crt_digits);
  *   - limbs: words of 64 limbs, one per wave and step.  Product limbs run to n + 2 (n coefficients, two digits more), so
- *     a product has W = n / 64 + 1 words and a block at most 65.  A word's carry chain is one addition of its ballot
- *     masks (crt.hip), and the chain over the words the same once more: lane l holds word l's carry out for either
- *     carry in, a product's last word passes nothing on.
- * Bound by vector issue as k_fused2 is: 2846 vector instructions per wave and prime at n = 4096 and about 160 per
- * coefficient for the digits. */
+ *     a product has W = n / 64 + 1 words: 65 at most, and a block's 66 at most (two products of 2^11 points).  A word's
+ *     carry chain is one addition of its ballot masks (crt.hip), and the chain over up to 65 words the same once more:
+ *     lane l holds word l's carry out for either carry in, a product's last word passes nothing on.  Blocks of more words
+ *     have a chain per product.
+ * Bound by vector issue and, with one block a CU at n = 4096, by latency: 4606 vector instructions a wave at 69% of the issue
+ * rate there (three primes, 8192 products 1.23 ms), 4323 at 87% at n = 1024 (32768 products 0.94 ms). */
 #include <string.h>
 #include "internal.h"
 #include "rounds.h"
@@ -336,7 +337,7 @@ int nttm_run_small(int np, int logn, const LoadDesc *ld, const CrtDesc *cd, cons
  * forward, pointwise product and inverse of every prime, digits and limbs as in k_small, so that nothing but operand and
  * result limbs crosses memory.  A segment is one block of the carry launch.  The overlapping limbs are transformed twice:
  * the rules that choose it (choose_segments, batch_segments) weigh that.
- * Bound by vector issue and latency at one workgroup a CU (12 waves, 115 KiB of LDS): 13 us for the short operand and 26 to 31
+ * Bound by vector issue (64% of the issue rate) and latency at one workgroup a CU (12 waves, 115 KB of LDS): 13 us for the short operand and 26 to 31
  * for a segment of 2048 to 4032 limbs.  Through passes of 2^13 points and more, us, before / now: 500 products of
  * 8000 x 500 limbs 458 / 210, of 60000 x 1000 1743 / 1178, 8 of 60000 x 300 72 / 50; one of 1000000 x 1000 116 / 88,
  * of 20000000 x 300 2660 / 625 (in pieces 1080). */
