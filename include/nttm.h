@@ -11,7 +11,7 @@
  * unless stated, and returns NTTM_EINVAL, before any launch, for host memory, memory of another device or a range
  * that runs past the end of its device allocation.
  * A product's c may share memory with its own x, in any way, and, where one transform holds the product, with its a
- * and b; it may not share memory with anything another product of the same call reads or writes.
+ * and b; in a batch or a plan it may not share memory with anything that another product of it reads or writes.
  *
  * Streams and synchronization: work runs on the given HIP stream (a hipStream_t passed as void *, NULL = the null
  * stream) on the device selected by nttm_init.  These entries return with the stream drained (they read flags or

@@ -2281,11 +2281,13 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
     RCK(hpin_need(128 * N + 8 * N + 256));
     RCK(stage_need(off_ncn + N * 8));
     std::vector<char> fl(N, 0);                                  /* 1: flags in pinned slot i */
-    std::vector<nttm_prod> Q;
-    RCK(x_apart(P, N, Q, s));
-    const nttm_prod *S = Q.empty() ? P : Q.data();
+    /* an x under its result is copied at its product's turn (x_apart): the products before it may have written it */
+    std::vector<nttm_prod> Q(P, P + N);
+    RCK(xc_need(x_limbs(P, N, false)));
+    uint64_t *xd = g.xc;
     for (size_t i = 0; i < N; i++) {
-        const nttm_prod &q = S[i];
+        if (x_to_copy(P[i], false)) { RCK(copy_x(&Q[i], 1, false, xd, s)); xd += Q[i].nx; }
+        const nttm_prod &q = Q[i];
         const size_t nc = q.na + q.nb + (q.x ? 1 : 0);
         if (q.na && q.nb && !fits_one(q.na, q.nb, nc)) RCK(mul_any(q.c, q.a, q.na, q.b, q.nb, q.x, q.nx, s));
         else { RCK(mul_core(q.c, q.a, q.na, q.b, q.nb, q.x, q.nx, s, SIZE_MAX, nullptr, 0, 0, i)); fl[i] = 1; }
@@ -2302,7 +2304,7 @@ extern "C" int nttm_mul_each_async(nttm_prod *P, size_t N, void *stream)
             return nttm_fail(NTTM_ECHECK, "product %zu: crt: non-zero carry beyond the top limb (wrong residues)", i);
         P[i].ncn = hn[i];
     }
-    return g.cfg.check ? check_products(S, N, s) : 0;
+    return g.cfg.check ? check_products(Q.data(), N, s) : 0;
 }
 
 /* ---- the binary-splitting product tree ----------------------------------------------------------------------------------- */

@@ -125,6 +125,26 @@ def test_many_and_empty(lib):
         plan.close()
 
 
+@pytest.mark.parametrize("na,nb", [(40, 25), (3500, 3501), (30011, 2100)])
+def test_chain(lib, na, nb):
+    """the one-call-each forms over one accumulator: every product adds to what the one before it left"""
+    import torch
+    n, s = lib(), 5
+    x, s = O.gen_limbs(na + nb, s)
+    ops, want = [], x
+    for i in range(4):
+        a, s = O.gen_limbs(na, s)
+        b, s = O.gen_limbs(nb, s)
+        ops.append((dev(a), dev(b)))
+        want = O.mul_school(a, b, want[:na + nb])
+    say("chain over x", na, nb)
+    for call in (n.mul_each, n.mul_each_async):
+        buf = torch.zeros(na + nb + 1, dtype=torch.int64, device="cuda")
+        buf[:na + nb] = dev(x)
+        call(n.make_prods([(a, b, buf[:na + nb], buf) for a, b in ops]))
+        assert np.array_equal(host(buf), want)
+
+
 @pytest.mark.parametrize("shift", [0, 7, -7])
 def test_grid_and_crt(lib, shift):
     """a grid under a workspace cap, and the CRT primitive"""
